@@ -48,12 +48,22 @@
 
 #include <algorithm>
 #include <map>
+#include <type_traits>
 #include <vector>
 
 #include "cgm_internal.h"
 #include "cgm_special.h"
 
 using namespace cgm;
+
+// One work-group's share of a tile's W (k_tile_ws): block columns j0, j0 + 1
+// and the block rows from i0 on.
+struct Strip {
+  long woff;   // the tile's first block in W16
+  int bloc;    // the tile's first block row among its map's
+  int nB;      // block rows of the tile
+  int i0, j0;
+};
 
 struct cgm_tiles {
   cgm_context* ctx = nullptr;
@@ -63,6 +73,7 @@ struct cgm_tiles {
   int M2 = 0;               // unknowns per tile (T * T)
   bool reduced = false;     // T >= 64: reduced form
   int maps = 0;             // maps factored by the last cgm_tiles_factor (1: shared)
+  bool maps1 = true;        // the layout below is that of one map
   rocblas_handle h = nullptr;
   size_t bytes = 0;         // device memory held
   // dense form (T <= 32)
@@ -75,15 +86,24 @@ struct cgm_tiles {
   long* woff = nullptr;            // [B][nt * nt] offset of W_t in W16 (half2 elements)
   float* kscale = nullptr;         // [B][nt * nt] largest |W_t| entry
   int* ids = nullptr;              // [B][nt * nt] factor members (tiles with n_t > 0), by size
-  int* eloc = nullptr;             // [B][nt * nt] index of each tile's first block in its map's block list
-  int* btab = nullptr;             // block lists of the maps: tile << 16 | block row << 8 | block column
-  size_t btab_cap = 0;
-  int* bstart = nullptr;           // [B] first entry of each map's block list in btab
-  int* bcount = nullptr;           // [B] blocks of each map
-  int bcount_max = 0;              // largest block count over the factored maps
+  int* bloc = nullptr;             // [B][nt * nt] each tile's first block row among its map's
+  int* sloc = nullptr;             // [B][nt * nt] each tile's first entry in spos
+  Strip* stab = nullptr;           // strip lists of the maps, largest first
+  int* spos = nullptr;             // by tile, [si][64]: place of strip (si, sj) in the map's list
+  size_t stab_cap = 0, spos_cap = 0;
+  int* sstart = nullptr;           // [B] first entry of each map's list in stab
+  int* scount = nullptr;           // [B] strips of each map
+  int* ssize = nullptr;            // [B] block rows of a map's strips
+  int scount_max = 0;              // largest strip count over the factored maps
+  long plen_max = 0;               // largest scount * (2 + ssize)
+  int xblk_max = 0;                // largest number of block rows of a map
   int nbmax = 0;                   // largest number of block rows of a tile
-  float2* Pw = nullptr;            // [sys][bcount_max][2][kBlkW] partial products (apply)
+  float4* Pw = nullptr;            // [group][strip][2 + ssize][64 systems of the group] partial products (apply)
   size_t pw_cap = 0;
+  unsigned* Xs = nullptr;          // [group][xblk_max][kXsBlk] inputs in FP16 parts (apply)
+  size_t xs_cap = 0;
+  float* xinv = nullptr;           // [sys][nt * nt] inverse scales of the inputs (apply)
+  size_t xinv_cap = 0;
   long* koff = nullptr;            // [B][nt * nt] offset of each member's matrix in Kw
   int* nl = nullptr;               // [B][nt * nt] each member's matrix side (n_t padded to kBlk)
   __half2* W16 = nullptr;          // W_t / kscale_t in FP16: the kBlkW x kBlkW blocks (i, j <= i) of the
@@ -116,6 +136,8 @@ constexpr int kPadTo = 16;                   // n_t is padded to a multiple of t
 constexpr unsigned short kPadCol = 0xFFFF;   // cell index of a padding slot
 constexpr int kBlk = 128;                    // block of the Gauss-Jordan inversion (reduced form)
 constexpr int kBlkW = 128;                   // block of the symmetric storage of W (apply)
+constexpr int kSplits = 3;                   // FP16 parts of one FP32 input value (apply)
+constexpr int kXsBlk = kSplits * 16 * kBlkW; // dwords of one block row's inputs in Xs (apply)
 
 template <typename P>
 int grow(cgm_tiles* t, P** p, size_t* cap, size_t need) {
@@ -569,170 +591,410 @@ k_tile_red_pack(const float2* __restrict__ Kw, const int* __restrict__ ncol, con
 // reduced form: application
 // ---------------------------------------------------------------------------
 
-// Two-component shuffle across the wave.
-__device__ inline float2 shfl_xor2(float2 v, int o) {
-  return make_float2(__shfl_xor(v.x, o, 64), __shfl_xor(v.y, o, 64));
-}
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef unsigned int uint4_t __attribute__((ext_vector_type(4)));
+typedef unsigned int uint2_t __attribute__((ext_vector_type(2)));
 
-// One stage of the transposing butterfly: the 2H values of every lane become
-// H, each the sum of the lane's and its partner's (lane ^ o) value of the
-// same column, the upper half kept by the lanes with bit o set.
-template <int H>
-__device__ inline void bfly_stage(float2* c, int lane, int o) {
-  const bool up = lane & o;
-#pragma unroll
-  for (int k = 0; k < H; ++k) {
-    const float2 send = up ? c[k] : c[k + H];
-    const float2 keep = up ? c[k + H] : c[k];
-    c[k] = cadd(keep, shfl_xor2(send, o));
-  }
-}
+constexpr int kXsRow = kBlkW + 4;        // LDS stride of one column of inputs (bank-conflict free 16-byte reads)
 
-// W_t is complex symmetric (W_t = (D_S^{-1} - G_SS)^{-1}, G symmetric), so
-// only its lower triangle is stored, in kBlkW x kBlkW blocks.  A work-group
-// takes block e = (i, j) of its system s's map block list and writes two
-// partial products of kBlkW values (scaled W16): B x_j (for block
-// row i) and, for j < i, B^T x_i (for block row j), x_i, x_j the tile's
-// input at the cells of S in block rows i and j (io.v scaled by
-// 1 / *(io.nrm + s sNrm bytes) when io.nrm is given).  Lane l of every wave
-// holds rows 2l, 2l + 1 of the block (one 8-byte load per column), the four
-// waves take 32 columns each; the row sums meet in LDS, and the 32 column
-// sums of each wave are reduced across its lanes by a transposing butterfly
-// (lane l ends with column l / 2).  Systems with *(done + s sd bytes) set
-// are skipped.  The grid is (8 ceil(blocks / 8), systems): work-group L in
-// dispatch order (on XCD L % 8) takes system (L / 8) % systems and block
-// 8 (L / (8 systems)) + L % 8, so the systems of one block run back to back
-// on one XCD and, on a shared map, its L2 serves the block's later reads
-// (16 systems at N = 512 fetch 1.5 times W from HBM, not 16 times).  One
-// system keeps block e = L.
-template <int T>
-__global__ void __launch_bounds__(256)
-k_tile_ws(const __half2* __restrict__ W16, const long* __restrict__ woff, const int* __restrict__ ncol,
-          const unsigned short* __restrict__ cols, const int* __restrict__ btab, const int* __restrict__ bstart,
-          const int* __restrict__ bcount, int maps1, FnoIO io, float2* __restrict__ Pw, long spw,
+// Position of row p of a block row among its inputs and products, and the row
+// at a position: in every 32 rows the even ones first, as the MFMA operands of
+// k_tile_ws hold them.
+__device__ inline int xpos(int p) { return (p & ~31) | (p & 1) << 4 | (p & 31) >> 1; }
+__device__ inline int xrow(int q) { return (q & ~31) | (q & 15) << 1 | (q >> 4 & 1); }
+
+// The tile inputs x_t[S] of system blockIdx.y and tile blockIdx.x (io.v scaled
+// by 1 / *(io.nrm + s sNrm bytes) when io.nrm is given), as the right-hand
+// operand of k_tile_ws: every value is scaled by the power of two that brings
+// the tile's largest component to [2^14, 2^15) and cut into kSplits FP16
+// parts, x = hi + mid + lo, which hold all 24 bits of the FP32 value (down to
+// 2^-39 of the tile's largest).  Group v = s / VP of the systems, column
+// n(s) = s % VP: with VP = 16 one dword (re, im) per value and column n; with
+// VP = 8 the two columns 2n and 2n + 1 hold (re, -im) and (im, re).  Layout
+// [group][block row][part][16 columns][kBlkW], rows at xpos().  xinv[s][tile] is the inverse
+// of the scale.  Each map's tiles own xblk[map] block rows (bloc: the tile's
+// first).  A few tiles and systems leave CUs idle: then `parts` work-groups
+// share a tile (blockIdx.x = tile * parts + part), each finding the maximum of
+// all of it and writing its share.
+template <int T, int VP>
+__global__ void __launch_bounds__(1024)
+k_tile_xs(const int* __restrict__ ncol, const unsigned short* __restrict__ cols, const int* __restrict__ bloc,
+          int maps1, int parts, FnoIO io, unsigned* __restrict__ Xs, long sXs, float* __restrict__ xinv,
           const int* __restrict__ done, long sd, int N) {
-  constexpr int M2 = T * T, B = kBlkW;
-  __shared__ float2 xj[B], xi[B];
-  __shared__ float4 red[3][64];
+  constexpr int M2 = T * T;
+  constexpr int PT = M2 / 1024;  // values per thread
+  __shared__ float red[16];
   const int nt = N / T;
-  const int nsys = gridDim.y;
-  const long L = (long)blockIdx.y * gridDim.x + blockIdx.x;
-  const long q = L >> 3;
-  const int s = (int)(q % nsys), map = maps1 ? 0 : s, e = (int)((q / nsys) * 8 + (L & 7));
-  if (e >= bcount[map]) return;
+  const int s = blockIdx.y, t = blockIdx.x / parts, part = blockIdx.x % parts;
   if (done && *boff(done, (long)s * sd)) return;
-  const int pk = btab[bstart[map] + e];
-  const int t = pk >> 16, i = (pk >> 8) & 255, j = pk & 255;
-  const long tb = (long)map * nt * nt + t;
+  const long tb = (long)(maps1 ? 0 : s) * nt * nt + t;
   const int n = ncol[tb];
+  if (n == 0) return;
+  const int np = (n + kBlkW - 1) / kBlkW * kBlkW;
   const unsigned short* ct = cols + tb * M2;
   float sc = 1.f;
   if (io.nrm) {
     const double d = *boff(io.nrm, (long)s * io.sNrm);
     sc = d > 0.0 ? (float)(1.0 / d) : 0.f;
   }
-  {
-    const int h = threadIdx.x >> 7, r = threadIdx.x & (B - 1);
-    const int p = (h ? i : j) * B + r;
-    float2 xv = make_float2(0.f, 0.f);
-    if (p < n) {
-      const int c = ct[p];
-      if (c != kPadCol) {
-        xv = io.v[(long)s * io.sV + tile_cell(t, c, nt, T, N)];
-        xv.x *= sc;
-        xv.y *= sc;
+  const float2* v = io.v + (long)s * io.sV;
+  float2 xv[PT];
+  int cell[PT];
+  float mx = 0.f;
+#pragma unroll
+  for (int k = 0; k < PT; ++k) {
+    const int p = threadIdx.x + 1024 * k;
+    cell[k] = ct[p < M2 ? p : 0];
+    if (p >= n) cell[k] = kPadCol;
+  }
+#pragma unroll
+  for (int k = 0; k < PT; ++k) {  // padding slots load a cell too, so that no load waits behind a branch
+    xv[k] = v[tile_cell(t, cell[k] == kPadCol ? 0 : cell[k], nt, T, N)];
+    xv[k].x = cell[k] == kPadCol ? 0.f : xv[k].x * sc;
+    xv[k].y = cell[k] == kPadCol ? 0.f : xv[k].y * sc;
+    mx = fmaxf(mx, fmaxf(fabsf(xv[k].x), fabsf(xv[k].y)));
+  }
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 16; ++k) mx = fmaxf(mx, red[k]);
+  // scale 2^e: the exponent is clamped so that the scale and its inverse are normal numbers
+  int e = 0;
+  if (mx > 0.f && mx < __builtin_huge_valf()) e = 141 - (int)(__float_as_uint(mx) >> 23);
+  e = e > 126 ? 126 : (e < -126 ? -126 : e);
+  const float up = __uint_as_float((unsigned)(e + 127) << 23);
+  if (threadIdx.x == 0) xinv[(long)s * nt * nt + t] = __uint_as_float((unsigned)(127 - e) << 23);
+  const int col = s % VP;
+  unsigned* X = Xs + (long)(maps1 ? s / VP : s) * sXs + (long)bloc[tb] * kXsBlk;
+#pragma unroll
+  for (int k = 0; k < PT; ++k) {
+    const int p = threadIdx.x + 1024 * k;
+    if (p >= np) break;
+    if (k % parts != part) continue;
+    float re = xv[k].x * up, im = xv[k].y * up;
+    unsigned* Xp = X + (long)(p / kBlkW) * kXsBlk + xpos(p % kBlkW);
+#pragma unroll
+    for (int q = 0; q < kSplits; ++q) {
+      const _Float16 a = (_Float16)re, b = (_Float16)im;
+      re -= (float)a;
+      im -= (float)b;
+      const unsigned ua = __builtin_bit_cast(unsigned short, a), ub = __builtin_bit_cast(unsigned short, b);
+      if constexpr (VP == 16) {
+        Xp[(q * 16 + col) * kBlkW] = ua | ub << 16;
+      } else {
+        const int cn = maps1 ? 2 * col : 0;
+        Xp[(q * 16 + cn) * kBlkW] = ua | (ub ^ 0x8000u) << 16;
+        Xp[(q * 16 + cn + 1) * kBlkW] = ub | ua << 16;
       }
     }
-    (h ? xi : xj)[r] = xv;
   }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r0 = 2 * lane, q0 = 32 * wave;
-  typedef unsigned int u2v_t __attribute__((ext_vector_type(2)));
-  const u2v_t* Bp =
-      reinterpret_cast<const u2v_t*>(W16 + woff[tb] + (long)(i * (i + 1) / 2 + j) * B * B + r0);
-  const float2 x0 = xi[r0], x1 = xi[r0 + 1];
-  const bool off = i != j;  // uniform over the work-group
-  float2* P = Pw + (long)s * spw + (long)e * 2 * B;
-  float ax = 0.f, ay = 0.f, bx = 0.f, by = 0.f;
-#pragma unroll 1
-  for (int g = 0; g < 2; ++g) {
-    uint2 w[16];  // each vector load is copied out at once (rows r0 and r0 + 1)
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const u2v_t l = __builtin_nontemporal_load(Bp + (long)(q0 + 16 * g + u) * (B / 2));
-      w[u] = make_uint2(l.x, l.y);
-    }
-    float2 c[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const float2 xv = xj[q0 + 16 * g + u];
-      const float2 k0 = __half22float2(__builtin_bit_cast(__half2, w[u].x));
-      const float2 k1 = __half22float2(__builtin_bit_cast(__half2, w[u].y));
-      ax += k0.x * xv.x - k0.y * xv.y;
-      ay += k0.x * xv.y + k0.y * xv.x;
-      bx += k1.x * xv.x - k1.y * xv.y;
-      by += k1.x * xv.y + k1.y * xv.x;
-      c[u] = cadd(cmul(k0, x0), cmul(k1, x1));
-    }
-    if (off) {  // the 16 column sums of B^T x_i over the wave: lane l ends with column l / 4
-      bfly_stage<8>(c, lane, 32);
-      bfly_stage<4>(c, lane, 16);
-      bfly_stage<2>(c, lane, 8);
-      bfly_stage<1>(c, lane, 4);
-      c[0] = cadd(c[0], shfl_xor2(c[0], 2));
-      c[0] = cadd(c[0], shfl_xor2(c[0], 1));
-      if ((lane & 3) == 0) P[B + q0 + 16 * g + (lane >> 2)] = c[0];
-    }
-  }
-  if (wave > 0) red[wave - 1][lane] = make_float4(ax, ay, bx, by);
-  __syncthreads();
-  if (wave > 0) return;
-#pragma unroll
-  for (int w = 0; w < 3; ++w) {
-    const float4 o = red[w][lane];
-    ax += o.x;
-    ay += o.y;
-    bx += o.z;
-    by += o.w;
-  }
-  P[r0] = make_float2(ax, ay);
-  P[r0 + 1] = make_float2(bx, by);
 }
 
-// u_t of block row blockIdx.x % nbmax of tile blockIdx.x / nbmax, system
-// blockIdx.y: the partial products of the blocks (i, j <= i) of the row and
-// (k > i, i) of the column, summed in that fixed order, times the tile's
-// scale, written to U at the cells of S.
-template <int T>
-__global__ void __launch_bounds__(kBlkW)
-k_tile_wsum(const float* __restrict__ ksc, const int* __restrict__ ncol, const unsigned short* __restrict__ cols,
-            const int* __restrict__ eloc, int maps1, int nbmax, const float2* __restrict__ Pw, long spw,
+// The products with W_t of up to VP = 8 NT systems of one map.  W_t is complex
+// symmetric (W_t = (D_S^{-1} - G_SS)^{-1}, G symmetric), so only its lower
+// triangle is stored, in kBlkW x kBlkW blocks.  A work-group takes a strip of
+// them: block columns j0 = 2 sj and j0 + 1 of its tile, block rows i of
+// [si R, si R + R) with i >= j0 (R = 2, 4 or 8, by map), and forms for every
+// block (i, j) B x_j (added up over the two columns, per row) and, for j < i,
+// B^T x_i (added up over the rows, per column): 2 + R partial products of kBlkW
+// values per system, which k_tile_wsum adds up.
+//
+// What bounds it is the stream of W (64 KB a block), which is read once.  The
+// contraction runs on the matrix cores (FP16 inputs, FP32 sums): W is FP16 as
+// stored, and the FP32 inputs enter as three FP16 parts (k_tile_xs), so the
+// products are those of the FP32 values.  Complex arithmetic is real arithmetic
+// on interleaved parts: a dword (re, im) of W meets the dword (re, -im) of x
+// for the real part and (im, re) for the imaginary part, 16 complex values of
+// K per MFMA.
+//   B x_j:    lane (a, g) of wave w loads rows 32 w + 2 a, 2 a + 1 of four
+//             columns (8 bytes each, 128-byte segments); the four columns'
+//             values of one row are that lane's 8 K-values of an MFMA.
+//   B^T x_i:  the same registers, transposed by the matrix core: an MFMA with
+//             a 0/1 right operand that picks the real (imaginary) parts leaves
+//             column a's values of rows 4 g .. 4 g + 3 in lane (a, g), which
+//             are then packed back to FP16 (exactly) as the left operand.  (A
+//             second read of the block in the other layout cost as much as the
+//             first: the blocks in flight exceed an XCD's L2.)
+// Rows and columns are taken in the order of xpos().  x_j of the two columns
+// stays in LDS; a wave needs x_i at its own 32 rows only, which go straight to
+// registers, so the loop over the rows has no barrier.  A wave's sums of B^T x_i
+// run over its own rows and are added up over the four waves at the end.  Each
+// of the 16 KB that a wave needs of a block is loaded again for the next block
+// as soon as it is used, D steps of 2 KB ahead; every such load is issued
+// unconditionally (the last block again where there is no next), so that the
+// compiler's waits know how many loads are younger than the ones waited for.
+//
+// At N = 512, T = 128 on a map of the benchmark (1.33 GB of W; a plain
+// non-temporal read of as much takes 190 us): one system 242 us (5.5 TB/s),
+// 16 systems 337 us.  The vector-ALU kernel before it, which took one block
+// and one system at a time, took 272 and 3,000 us (202 us of arithmetic per
+// system).  One FP16 part instead of three would save 19 us at one system.
+// Two groups of 4 waves with 8 K-steps in flight took 249 us; R = 4 and 16
+// (rows per strip) instead of 8 took 252 and 241 us.
+template <int NT>
+__global__ void __launch_bounds__(256, 2)
+k_tile_ws(const unsigned* __restrict__ W16, const Strip* __restrict__ stab, const int* __restrict__ sstart,
+          const int* __restrict__ scount, const int* __restrict__ ssize, int maps1, int nsys,
+          const unsigned* __restrict__ Xs, long sXs, float4_t* __restrict__ Pw, long spw,
+          const int* __restrict__ done, long sd) {
+  constexpr int B = kBlkW, VP = 8 * NT, KS = B / 16;
+  constexpr int D = NT == 1 ? 4 : 2;                // K-steps of W in flight (2 KB per wave each)
+  constexpr int kSlot = kSplits * 16 * kXsRow;      // dwords of one block row's inputs in LDS
+  __shared__ unsigned lds[2 * kSlot];
+  const int grp = blockIdx.y, map = maps1 ? 0 : grp;
+  if ((int)blockIdx.x >= scount[map]) return;
+  const int nv = maps1 ? (nsys - grp * VP < VP ? nsys - grp * VP : VP) : 1;
+  if (done) {  // uniform over the work-group
+    bool all = true;
+    for (int k = 0; k < nv; ++k) all &= *boff(done, (long)((maps1 ? grp * VP : grp) + k) * sd) != 0;
+    if (all) return;
+  }
+  const int R = ssize[map];
+  const Strip sp = stab[sstart[map] + blockIdx.x];
+  const int nB = sp.nB, j0 = sp.j0, i0 = sp.i0, iend = i0 + R < nB ? i0 + R : nB;
+  const int ibeg = i0 > j0 ? i0 : j0;
+  const int tid = threadIdx.x, lane = tid & 63, a = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // in a scalar register, with all that follows from it
+  const unsigned* Wt = W16 + sp.woff + 32 * w;
+  const unsigned voff = (8 * g * B + 2 * a) * sizeof(unsigned);
+  const unsigned* X = Xs + (long)grp * sXs + (long)sp.bloc * kXsBlk;
+  const int ncols = NT == 2 ? nv : 2 * nv;  // columns in use: the others are not copied, and their sums not kept
+
+  uint2_t A[D][4];
+  const auto load_a = [&](int i, int j, int k) {  // K-step k: columns 32 (k / 2) + 8 g + 2 c + k % 2, positions 16 k + 4 g + c
+    const char* Bp = reinterpret_cast<const char*>(Wt + (long)(i * (i + 1) / 2 + j) * B * B + (32 * (k >> 1) + (k & 1)) * B);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      A[k % D][c] = __builtin_nontemporal_load(reinterpret_cast<const uint2_t*>(Bp + voff + 2 * c * B * sizeof(unsigned)));
+  };
+  // x_i at the wave's rows, loaded a block ahead of its first use and before the loads of W that follow it
+  uint4_t xr[2][kSplits], xn[2][kSplits];
+  const auto load_x = [&](int i, uint4_t (*to)[kSplits]) {
+    const unsigned* xi = X + (long)i * kXsBlk + 32 * w + a * B + 4 * g;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < kSplits; ++q) to[h][q] = *reinterpret_cast<const uint4_t*>(xi + q * 16 * B + 16 * h);
+  };
+  load_x(ibeg == j0 && ibeg + 1 < iend ? ibeg + 1 : ibeg, xr);
+#pragma unroll
+  for (int k = 0; k < D; ++k) load_a(ibeg, j0, k);
+
+  {  // x_j of the two columns, the columns in use, into LDS
+    const unsigned* src = X + (long)j0 * kXsBlk;
+    const int per = ncols * (B / 4), all = (j0 + 1 < nB ? 2 : 1) * kSplits * per;
+    for (int e0 = tid; e0 < all; e0 += 4 * 256) {
+      uint4_t v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int e = e0 + u * 256 < all ? e0 + u * 256 : tid, q = e / per, r = (e - q * per) >> 5, c = e & 31;
+        v[u] = *reinterpret_cast<const uint4_t*>(src + (q * 16 + r) * B + 4 * c);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int e = e0 + u * 256, q = e / per, r = (e - q * per) >> 5, c = e & 31;
+        if (e < all) *reinterpret_cast<uint4_t*>(lds + (q * 16 + r) * kXsRow + 4 * c) = v[u];
+      }
+    }
+  }
+  // the 0/1 operands: value 4 g + c of the K-step to column a, real or imaginary part
+  half8_t Ire, Iim;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const _Float16 one = (_Float16)(4 * g + c == a ? 1.f : 0.f);
+    Ire[2 * c] = one;
+    Ire[2 * c + 1] = (_Float16)0.f;
+    Iim[2 * c] = (_Float16)0.f;
+    Iim[2 * c + 1] = one;
+  }
+  const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+  float4_t Z[2][KS][NT];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) Z[h][k][n] = zero;
+
+  // partial products: [strip][2 columns, R rows][positions / 4][system][re, im] float4
+  const long qlen = 64 * nv;
+  float4_t* P = Pw + (long)grp * spw + (long)blockIdx.x * (2 + R) * qlen;
+  const auto put_p = [&](float4_t* Pq, int k, const float4_t* acc) {  // positions 16 k + 4 g .. + 3
+    float4_t* q = Pq + (k * 4 + g) * 2 * nv;
+    if constexpr (NT == 2) {
+      if (a < nv) {
+        q[2 * a] = acc[0];
+        q[2 * a + 1] = acc[1];
+      }
+    } else {
+      if (a < 2 * nv) q[a] = acc[0];
+    }
+  };
+  const auto mac = [&](half8_t h, uint4_t v, float4_t* acc) {
+    if constexpr (NT == 2) {
+      const half8_t re = __builtin_bit_cast(half8_t, v ^ 0x80000000u);
+      const half8_t im = __builtin_bit_cast(half8_t, (v >> 16) | (v << 16));
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h, re, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h, im, acc[1], 0, 0, 0);
+    } else {
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h, __builtin_bit_cast(half8_t, v), acc[0], 0, 0, 0);
+    }
+  };
+  float4_t Y[2 * NT];
+  // block (i, j): its row sums to Y, with `columns` its column sums to Zj (not on the diagonal, where the block is whole and its row
+  // sums are all), and the loads of block (ni, nj)
+  const auto product = [&](auto columns, int i, int j, int ni, int nj, const unsigned* xj, float4_t (&Zj)[KS][NT]) {
+    int xoff = a * kXsRow + 4 * g;
+    asm volatile("" : "+v"(xoff));  // x_j is read from LDS for every block: 96 registers otherwise
+    unsigned keep = i != j ? 0xFFFFFFFFu : 0u;
+    asm volatile("" : "+v"(keep));  // masked, not branched around: see load_a
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      half8_t f[2];
+      {
+        const uint2_t* Ak = A[k % D];
+        f[0] = __builtin_bit_cast(half8_t, (uint4_t{Ak[0].x, Ak[1].x, Ak[2].x, Ak[3].x}));
+        f[1] = __builtin_bit_cast(half8_t, (uint4_t{Ak[0].y, Ak[1].y, Ak[2].y, Ak[3].y}));
+      }
+      if (k + D < KS) load_a(i, j, k + D);
+      else load_a(ni, nj, k + D - KS);
+#pragma unroll
+      for (int q = 0; q < kSplits; ++q) {
+        const uint4_t v = *reinterpret_cast<const uint4_t*>(xj + xoff + q * 16 * kXsRow + 16 * k);
+        mac(f[0], v, Y);
+        mac(f[1], v, Y + NT);
+      }
+      if constexpr (decltype(columns)::value) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const float4_t re = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[h], Ire, zero, 0, 0, 0);
+          const float4_t im = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[h], Iim, zero, 0, 0, 0);
+          uint4_t tr;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) tr[c] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(re[c], im[c])) & keep;
+          const half8_t ft = __builtin_bit_cast(half8_t, tr);
+#pragma unroll
+          for (int q = 0; q < kSplits; ++q) mac(ft, xr[h][q], Zj[k]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of their use
+    }
+  };
+  const auto store_y = [&](int i) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) put_p(P + (2 + i - i0) * qlen, 2 * w + h, Y + h * NT);
+  };
+  __syncthreads();
+  int i = ibeg;
+  if (i == j0) {
+#pragma unroll
+    for (int k = 0; k < 2 * NT; ++k) Y[k] = zero;
+    const bool more = i + 1 < iend;
+    product(std::false_type(), i, j0, more ? i + 1 : i, j0, lds, Z[0]);
+    store_y(i);
+    ++i;
+  }
+  for (; i < iend; ++i) {
+    const bool more = i + 1 < iend;
+#pragma unroll
+    for (int k = 0; k < 2 * NT; ++k) Y[k] = zero;
+    product(std::true_type(), i, j0, i, j0 + 1, lds, Z[0]);
+    if constexpr (NT == 1) load_x(more ? i + 1 : i, xn);
+    product(std::true_type(), i, j0 + 1, more ? i + 1 : i, more ? j0 : j0 + 1, lds + kSlot, Z[1]);
+    store_y(i);
+    if constexpr (NT == 1) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < kSplits; ++q) xr[h][q] = xn[h][q];
+    } else {
+      load_x(more ? i + 1 : i, xr);
+    }
+  }
+  // Z over the four waves: wave w keeps positions 32 w .. 32 w + 31
+  float4_t* red = reinterpret_cast<float4_t*>(lds);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if ((k >> 1) != w) red[((w - (w > (k >> 1))) * KS + k) * 64 + lane] = Z[h][k][n];
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if ((k >> 1) == w) Z[h][k][n] += (red[k * 64 + lane] + red[(KS + k) * 64 + lane]) + red[(2 * KS + k) * 64 + lane];
+    }
+    if (j0 + h < nB)
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if ((k >> 1) == w) put_p(P + h * qlen, k, Z[h][k]);
+  }
+}
+
+// u_t of block row blockIdx.x % nbmax of tile blockIdx.x / nbmax, systems of
+// group blockIdx.z, 64 of the 64 nv values (float4: four rows) a system group
+// has per block row: the partial products of the strips of the row and
+// of the column, in four interleaved sums (one per slice of 64 threads, each in
+// a fixed order) added up in LDS, times the tile's scales, written to U at the
+// cells of S.
+template <int T, int VP>
+__global__ void __launch_bounds__(256)
+k_tile_wsum(const float* __restrict__ ksc, const float* __restrict__ xinv, const int* __restrict__ ncol,
+            const unsigned short* __restrict__ cols, const int* __restrict__ sloc, const int* __restrict__ spos,
+            const int* __restrict__ ssize, int maps1, int nsys, int nbmax, const float4_t* __restrict__ Pw, long spw,
             float2* __restrict__ U, const int* __restrict__ done, long sd, int N) {
   constexpr int M2 = T * T, B = kBlkW;
+  __shared__ float4_t red[4][64];
   const int nt = N / T;
-  const int s = blockIdx.y, map = maps1 ? 0 : s;
+  const int grp = blockIdx.z, map = maps1 ? 0 : grp;
+  const int nv = maps1 ? (nsys - grp * VP < VP ? nsys - grp * VP : VP) : 1;
+  if ((int)blockIdx.y >= nv) return;
   const int t = blockIdx.x / nbmax, i = blockIdx.x % nbmax;
   const long tb = (long)map * nt * nt + t;
   const int n = ncol[tb], nB = (n + B - 1) / B;
   if (i >= nB) return;
+  const int R = ssize[map], si = i / R, sj = i >> 1;
+  const int nS = (nB + R - 1) / R;
+  const int e = threadIdx.x & 63, sl = threadIdx.x >> 6;
+  const long qlen = 64 * nv;
+  const float4_t* P = Pw + (long)grp * spw + 64 * blockIdx.y + e;
+  const int* pos = spos + sloc[tb];  // place of each of the tile's strips in the map's list, [si][64]
+  float4_t acc = {0.f, 0.f, 0.f, 0.f};
+  // terms 0 .. sj: row sums of strips (si, 0 .. sj); then column sums of (si .. nS - 1, sj)
+  const int terms = sj + 1 + nS - si;
+#pragma unroll 4
+  for (int k = sl; k < terms; k += 4) {
+    const int r = k <= sj ? si : si + k - sj - 1, c = k <= sj ? k : sj;
+    acc += P[((long)pos[r * 64 + c] * (2 + R) + (k <= sj ? 2 + i - si * R : (i & 1))) * qlen];
+  }
+  red[sl][e] = acc;
+  __syncthreads();
+  if (threadIdx.x >= 32) return;
+  const int e2 = 32 * blockIdx.y + threadIdx.x;
+  const int v = e2 % nv, h = e2 / nv;
+  const int pos0 = 4 * h;  // its first position in the block row
+  const int s = (maps1 ? grp * VP : grp) + v;
   if (done && *boff(done, (long)s * sd)) return;
-  const int r = threadIdx.x, p = i * B + r;
-  const float2* P = Pw + (long)s * spw + (long)eloc[tb] * 2 * B;
-  float2 acc = make_float2(0.f, 0.f);
-  for (int j = 0; j <= i; ++j) acc = cadd(acc, P[(long)(i * (i + 1) / 2 + j) * 2 * B + r]);
-  for (int k = i + 1; k < nB; ++k) acc = cadd(acc, P[(long)(k * (k + 1) / 2 + i) * 2 * B + B + r]);
-  if (p < n) {
-    const int c = cols[tb * M2 + p];
-    if (c != kPadCol) {
-      const float m = ksc[tb];
-      U[((long)s * nt * nt + t) * M2 + c] = make_float2(acc.x * m, acc.y * m);
+  const int f = 2 * threadIdx.x;
+  const float4_t re = (red[0][f] + red[1][f]) + (red[2][f] + red[3][f]);
+  const float4_t im = (red[0][f + 1] + red[1][f + 1]) + (red[2][f + 1] + red[3][f + 1]);
+  const float k1 = ksc[tb], k2 = xinv[(long)s * nt * nt + t];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int p = i * B + xrow(pos0 + r);
+    if (p < n) {
+      const int c = cols[tb * M2 + p];
+      if (c != kPadCol) U[((long)s * nt * nt + t) * M2 + c] = make_float2(re[r] * k1 * k2, im[r] * k1 * k2);
     }
   }
 }
 
 // z = x + Y (Y in tile-major order) for system blockIdx.y; x is io.v scaled
-// as in k_tile_ws and is written to io.vw when io.nrm and io.vw are given.
+// as in k_tile_xs and is written to io.vw when io.nrm and io.vw are given.
 template <int T>
 __global__ void __launch_bounds__(256)
 k_tile_combine(FnoIO io, const float2* __restrict__ Y, const int* __restrict__ done, long sd, int N) {
@@ -753,6 +1015,18 @@ k_tile_combine(FnoIO io, const float2* __restrict__ Y, const int* __restrict__ d
   if (io.nrm && io.vw) io.vw[(long)s * io.sV + e] = xv;
   const float2 g = Y[((long)s * nt * nt + (i / T) * nt + j / T) * (T * T) + (i % T) * T + j % T];
   io.z[(long)s * io.sZ + e] = cadd(xv, g);
+}
+
+// Inputs and partial products of the applications to scratch_sys systems.
+// One map serves groups of 8 or 16 systems; systems with maps of their own
+// are groups of one.
+int grow_products(cgm_tiles* t) {
+  const size_t sys = (size_t)std::max(t->scratch_sys, 1);
+  const size_t groups = t->maps1 ? (sys + 15) / 16 : sys, per = t->maps1 ? std::min<size_t>(sys, 16) : 1;
+  int rc = grow(t, &t->Pw, &t->pw_cap, groups * t->plen_max * 64 * per);
+  if (!rc) rc = grow(t, &t->Xs, &t->xs_cap, groups * t->xblk_max * kXsBlk);
+  if (!rc) rc = grow(t, &t->xinv, &t->xinv_cap, sys * t->nt * t->nt);
+  return rc;
 }
 
 int ensure_scratch(cgm_tiles* t, int nsys) {
@@ -778,7 +1052,35 @@ int ensure_scratch(cgm_tiles* t, int nsys) {
   }
   t->scratch_sys = nsys;
   t->bytes += (2 * n + tm) * sizeof(float2) * nsys;
-  return grow(t, &t->Pw, &t->pw_cap, (size_t)nsys * t->bcount_max * 2 * kBlkW);
+  return grow_products(t);
+}
+
+// u_t = W_t x_t[S] of every tile for nsys systems; NT = 1: groups of up to 8
+// systems of one map (or one system with its own map), NT = 2: up to 16.  Each
+// column of the MFMAs is one system's, so a system's result does not depend on
+// the others or on NT.
+template <int T, int NT>
+int launch_ws(const cgm_tiles* tl, hipStream_t st, const FnoIO& io, const int* done, long sd, int nsys,
+              hipEvent_t* ev) {
+  constexpr int VP = 8 * NT;
+  const int ntiles = tl->nt * tl->nt;
+  const int m1 = tl->maps1 ? 1 : 0;
+  const int groups = m1 ? (nsys + VP - 1) / VP : nsys;
+  const int per = m1 ? std::min(nsys, VP) : 1;
+  const int parts = ntiles * nsys < 128 ? 4 : 1;
+  const long spw = tl->plen_max * 64 * per, sxs = (long)tl->xblk_max * kXsBlk;
+  float4_t* Pw = reinterpret_cast<float4_t*>(tl->Pw);
+  hipLaunchKernelGGL((k_tile_xs<T, VP>), dim3(ntiles * parts, nsys), dim3(1024), 0, st, tl->ncol, tl->cols, tl->bloc, m1, parts, io,
+                     tl->Xs, sxs, tl->xinv, done, sd, tl->N);
+  if (ev) CGM_HIP(hipEventRecord(ev[0], st));
+  hipLaunchKernelGGL((k_tile_ws<NT>), dim3(tl->scount_max, groups), dim3(256), 0, st,
+                     reinterpret_cast<const unsigned*>(tl->W16), tl->stab, tl->sstart, tl->scount, tl->ssize, m1, nsys, tl->Xs, sxs, Pw, spw, done, sd);
+  if (ev) CGM_HIP(hipEventRecord(ev[1], st));
+  hipLaunchKernelGGL((k_tile_wsum<T, VP>), dim3(ntiles * tl->nbmax, per, groups), dim3(256), 0, st, tl->kscale,
+                     tl->xinv, tl->ncol, tl->cols, tl->sloc, tl->spos, tl->ssize, m1, nsys, tl->nbmax, Pw, spw, tl->U,
+                     done, sd, tl->N);
+  CGM_HIP(hipGetLastError());
+  return CGM_SUCCESS;
 }
 
 // ev, when given: events recorded around k_tile_ws (live timing).
@@ -793,25 +1095,15 @@ int launch_apply_red(const cgm_tiles* tl, hipStream_t st, const FnoIO& io, const
     cgm_set_last_error("%d systems exceed the tile convolution's batch limit", nsys);
     return CGM_ERROR_UNSUPPORTED;
   }
-  const int maps1 = tl->maps == 1 ? 1 : 0;
-  const long spw = (long)tl->bcount_max * 2 * kBlkW;
-  if (tl->bcount_max > 0) {
-    if (ev) CGM_HIP(hipEventRecord(ev[0], st));
-    if (tl->T == 64)
-      hipLaunchKernelGGL((k_tile_ws<64>), dim3((tl->bcount_max + 7) / 8 * 8, nsys), dim3(256), 0, st, tl->W16, tl->woff, tl->ncol,
-                         tl->cols, tl->btab, tl->bstart, tl->bcount, maps1, io, tl->Pw, spw, done, sd, tl->N);
-    else
-      hipLaunchKernelGGL((k_tile_ws<128>), dim3((tl->bcount_max + 7) / 8 * 8, nsys), dim3(256), 0, st, tl->W16, tl->woff, tl->ncol,
-                         tl->cols, tl->btab, tl->bstart, tl->bcount, maps1, io, tl->Pw, spw, done, sd, tl->N);
-    CGM_HIP(hipGetLastError());
-    if (ev) CGM_HIP(hipEventRecord(ev[1], st));
-    if (tl->T == 64)
-      hipLaunchKernelGGL((k_tile_wsum<64>), dim3(ntiles * tl->nbmax, nsys), dim3(kBlkW), 0, st, tl->kscale, tl->ncol,
-                         tl->cols, tl->eloc, maps1, tl->nbmax, tl->Pw, spw, tl->U, done, sd, tl->N);
-    else
-      hipLaunchKernelGGL((k_tile_wsum<128>), dim3(ntiles * tl->nbmax, nsys), dim3(kBlkW), 0, st, tl->kscale, tl->ncol,
-                         tl->cols, tl->eloc, maps1, tl->nbmax, tl->Pw, spw, tl->U, done, sd, tl->N);
-    CGM_HIP(hipGetLastError());
+  if (tl->scount_max > 0) {
+    if (tl->T == 64) {
+      rc = tl->maps1 && nsys > 8 ? launch_ws<64, 2>(tl, st, io, done, sd, nsys, ev)
+                                 : launch_ws<64, 1>(tl, st, io, done, sd, nsys, ev);
+    } else {
+      rc = tl->maps1 && nsys > 8 ? launch_ws<128, 2>(tl, st, io, done, sd, nsys, ev)
+                                 : launch_ws<128, 1>(tl, st, io, done, sd, nsys, ev);
+    }
+    if (rc) return rc;
   } else if (ev) {  // no cell of chi != 0: nothing streamed
     CGM_HIP(hipEventRecord(ev[0], st));
     CGM_HIP(hipEventRecord(ev[1], st));
@@ -848,14 +1140,15 @@ int layout_reduced(cgm_tiles* t, const std::vector<int>& nc, int maps) {
   const int nb = ntiles * maps;
   constexpr long BB = (long)kBlkW * kBlkW;
   std::vector<long> off(nb);
-  std::vector<int> eloc(nb), btab, bstart(maps), bcount(maps);
+  std::vector<int> bloc(nb), sloc(nb), spos, sstart(maps), scount(maps), ssize(maps);
+  std::vector<Strip> stab;
   long total = 0;
   t->kept.assign(maps, 0.0);
-  t->nbmax = 0;
-  t->bcount_max = 0;
+  t->nbmax = t->scount_max = t->xblk_max = 0;
+  t->plen_max = 0;
+  t->maps1 = maps == 1;
   for (int m = 0; m < maps; ++m) {
-    bstart[m] = (int)btab.size();
-    int le = 0;
+    int rows = 0;
     for (int tl = 0; tl < ntiles; ++tl) {
       const int k = m * ntiles + tl;
       const int nB = (nc[k] + kBlkW - 1) / kBlkW;
@@ -863,25 +1156,63 @@ int layout_reduced(cgm_tiles* t, const std::vector<int>& nc, int maps) {
       off[k] = total;
       total += nblk * BB;
       t->kept[m] += (double)nblk * BB;
-      eloc[k] = le;
-      le += nblk;
+      bloc[k] = rows;
+      rows += nB;
       t->nbmax = std::max(t->nbmax, nB);
-      for (int i = 0; i < nB; ++i)
-        for (int j = 0; j <= i; ++j) btab.push_back(tl << 16 | i << 8 | j);
     }
-    bcount[m] = le;
-    t->bcount_max = std::max(t->bcount_max, le);
+    struct Item { int work, tile, i, j; };
+    std::vector<Item> items;
+    // long strips move fewer partial products and short ones keep more
+    // work-groups busy: the longest of which each CU gets two or more
+    int R = 8;
+    for (;; R /= 2) {
+      items.clear();
+      for (int tl = 0; tl < ntiles; ++tl) {
+        const int nB = (nc[m * ntiles + tl] + kBlkW - 1) / kBlkW;
+        for (int i = 0; i * R < nB; ++i)
+          for (int j = 0; 2 * j < std::min(nB, i * R + R); ++j) {
+            int work = 0;
+            for (int r = i * R; r < std::min(nB, i * R + R); ++r) work += std::max(0, std::min(2, r - 2 * j + 1));
+            items.push_back({work, tl, i, j});
+          }
+      }
+      if (R == 2 || items.size() >= 1024) break;
+    }
+    const int spos0 = (int)spos.size();
+    int slots = 0;
+    for (int tl = 0; tl < ntiles; ++tl) {
+      sloc[m * ntiles + tl] = spos0 + slots;
+      slots += ((nc[m * ntiles + tl] + kBlkW - 1) / kBlkW + R - 1) / R * 64;
+    }
+    spos.resize(spos0 + slots);
+    std::stable_sort(items.begin(), items.end(), [](const Item& x, const Item& y) { return x.work > y.work; });
+    sstart[m] = (int)stab.size();
+    for (size_t k = 0; k < items.size(); ++k) {
+      spos[sloc[m * ntiles + items[k].tile] + items[k].i * 64 + items[k].j] = (int)k;
+      const int q = m * ntiles + items[k].tile;
+      stab.push_back({off[q], bloc[q], (nc[q] + kBlkW - 1) / kBlkW, items[k].i * R, items[k].j * 2});
+    }
+    scount[m] = (int)items.size();
+    ssize[m] = R;
+    t->scount_max = std::max(t->scount_max, scount[m]);
+    t->plen_max = std::max(t->plen_max, (long)scount[m] * (2 + R));
+    t->xblk_max = std::max(t->xblk_max, rows);
   }
   int rc;
   if ((rc = grow(t, &t->W16, &t->w16_cap, (size_t)std::max(total, 1L)))) return rc;
-  if ((rc = grow(t, &t->btab, &t->btab_cap, std::max<size_t>(btab.size(), 1)))) return rc;
-  if ((rc = grow(t, &t->Pw, &t->pw_cap, (size_t)t->scratch_sys * t->bcount_max * 2 * kBlkW))) return rc;
+  if ((rc = grow(t, &t->stab, &t->stab_cap, std::max<size_t>(stab.size(), 1)))) return rc;
+  if ((rc = grow(t, &t->spos, &t->spos_cap, std::max<size_t>(spos.size(), 1)))) return rc;
+  if ((rc = grow_products(t))) return rc;
   CGM_HIP(hipMemcpyAsync(t->woff, off.data(), sizeof(long) * nb, hipMemcpyHostToDevice, st));
-  CGM_HIP(hipMemcpyAsync(t->eloc, eloc.data(), sizeof(int) * nb, hipMemcpyHostToDevice, st));
-  if (!btab.empty())
-    CGM_HIP(hipMemcpyAsync(t->btab, btab.data(), sizeof(int) * btab.size(), hipMemcpyHostToDevice, st));
-  CGM_HIP(hipMemcpyAsync(t->bstart, bstart.data(), sizeof(int) * maps, hipMemcpyHostToDevice, st));
-  CGM_HIP(hipMemcpyAsync(t->bcount, bcount.data(), sizeof(int) * maps, hipMemcpyHostToDevice, st));
+  CGM_HIP(hipMemcpyAsync(t->bloc, bloc.data(), sizeof(int) * nb, hipMemcpyHostToDevice, st));
+  CGM_HIP(hipMemcpyAsync(t->sloc, sloc.data(), sizeof(int) * nb, hipMemcpyHostToDevice, st));
+  if (!stab.empty()) {
+    CGM_HIP(hipMemcpyAsync(t->stab, stab.data(), sizeof(Strip) * stab.size(), hipMemcpyHostToDevice, st));
+    CGM_HIP(hipMemcpyAsync(t->spos, spos.data(), sizeof(int) * spos.size(), hipMemcpyHostToDevice, st));
+  }
+  CGM_HIP(hipMemcpyAsync(t->sstart, sstart.data(), sizeof(int) * maps, hipMemcpyHostToDevice, st));
+  CGM_HIP(hipMemcpyAsync(t->scount, scount.data(), sizeof(int) * maps, hipMemcpyHostToDevice, st));
+  CGM_HIP(hipMemcpyAsync(t->ssize, ssize.data(), sizeof(int) * maps, hipMemcpyHostToDevice, st));
   CGM_HIP(hipStreamSynchronize(st));  // the host vectors are read by the copies above
   return CGM_SUCCESS;
 }
@@ -1054,11 +1385,15 @@ int tiles_maps(const cgm_tiles* t) { return t->maps; }
 // Algorithmic bytes of one application to nsys systems: the inverse entries
 // streamed (dense form: every entry of every tile in FP32, once per system or
 // once per group of four right-hand sides of one map; reduced form: the FP16
-// entries of W of the map each system uses) plus v in and z out.
+// entries of W, once per system or once per group of sixteen right-hand sides
+// of one map) plus v in and z out.
 double apply_bytes(const cgm_tiles* tl, int nsys) {
   double e = 0.0;
   if (tl->reduced) {
-    for (int s = 0; s < nsys; ++s) e += tl->kept[tl->maps == 1 ? 0 : s] * 4.0;
+    if (tl->maps == 1)
+      e = tl->kept[0] * 4.0 * ((nsys + 15) / 16);
+    else
+      for (int s = 0; s < nsys; ++s) e += tl->kept[s] * 4.0;
   } else {
     const int streams = (tl->maps == 1 && nsys > 1) ? (nsys + 3) / 4 : nsys;
     if (tl->maps == 1)
@@ -1144,9 +1479,11 @@ extern "C" int cgm_tiles_create(cgm_ctx_t c, int T, int batch, cgm_tiles_t* out)
     alloc((void**)&t->kscale, sizeof(float) * nb);
     alloc((void**)&t->ids, sizeof(int) * nb);
     alloc((void**)&t->koff, sizeof(long) * nb);
-    alloc((void**)&t->eloc, sizeof(int) * nb);
-    alloc((void**)&t->bstart, sizeof(int) * batch);
-    alloc((void**)&t->bcount, sizeof(int) * batch);
+    alloc((void**)&t->bloc, sizeof(int) * nb);
+    alloc((void**)&t->sloc, sizeof(int) * nb);
+    alloc((void**)&t->sstart, sizeof(int) * batch);
+    alloc((void**)&t->scount, sizeof(int) * batch);
+    alloc((void**)&t->ssize, sizeof(int) * batch);
     alloc((void**)&t->nl, sizeof(int) * nb);
     alloc((void**)&t->info, sizeof(int) * nb);
     if (ok && plan_init(t->P, T) != CGM_SUCCESS) ok = false;
@@ -1172,7 +1509,8 @@ extern "C" int cgm_tiles_destroy(cgm_tiles_t t) {
   if (!t) return CGM_SUCCESS;
   (void)hipSetDevice(t->device);
   void* ptrs[] = {t->K,    t->ipiv, t->info, t->ncol, t->cols, t->woff, t->kscale,
-                  t->ids,  t->eloc, t->btab, t->bstart, t->bcount, t->Pw, t->koff, t->nl,
+                  t->ids,  t->bloc, t->sloc, t->stab, t->spos, t->sstart, t->scount, t->ssize,
+                  t->Pw,   t->Xs,   t->xinv, t->koff, t->nl,
                   t->W16,  t->Kw,   t->Pb,    t->Rw,   t->Cw,
                   t->U,    t->Y,    t->Tm,   t->tw32, t->tw64, t->blkT,  t->gq};
   for (void* p : ptrs)

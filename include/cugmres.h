@@ -366,15 +366,16 @@ int cgm_tiles_factor(cgm_tiles_t tiles, const cgm_complex128* dev_block, const f
                      int maps);
 /* y[b] = P x[b] for b < batch ([batch][N*N]; map b, or the one map).
  * Asynchronous on the context stream.  With one map and several systems the
- * reduced form (T >= 64) runs the systems of each W block back to back on one
- * XCD, whose L2 serves the repeated reads (16 systems fetch W from HBM about
- * 1.5 times per call); the dense form (T <= 32) applies each inverse to four
- * systems per pass. */
+ * reduced form (T >= 64) applies W to up to 16 systems per pass over it on the
+ * matrix cores (FP32 inputs as three FP16 parts each, FP32 sums); the dense
+ * form (T <= 32) applies each inverse to four systems per pass.  A system's
+ * result does not depend on the others. */
 int cgm_tiles_apply(cgm_tiles_t tiles, const cgm_complex64* dev_x, cgm_complex64* dev_y, int batch);
 /* Algorithmic bytes of one cgm_tiles_apply over `batch` systems: the inverse
  * entries it streams (every entry of every tile in FP32 for T <= 32, once per
  * group of four right-hand sides of one map; the stored FP16 blocks of W for
- * T >= 64, once per system) plus 16 * N*N per system. */
+ * T >= 64, once per group of sixteen right-hand sides of one map) plus
+ * 16 * N*N per system. */
 int cgm_tiles_apply_bytes(cgm_tiles_t tiles, int batch, double* bytes);
 /* Diagnostics: fills the inverses of one map with synthetic values (no
  * factorisation) and returns in *ms the average device time of `reps`

@@ -364,6 +364,41 @@ def test_reduced_tiles_shared_map_many_rhs_and_batched_solves(orc):
     ctx.close()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,systems", [(64, 1), (64, 8), (64, 9), (64, 17), (128, 3), (128, 16)])
+def test_reduced_tiles_system_groups_and_scales(orc, T, systems):
+    """Groups of 8 and 16 systems of one map and their remainders, on tiles of
+    0, 1, 12 and 32 block rows of W (T = 64) and an odd number of them: every
+    system against the oracle's reduced form (1e-2 and 2.5e-2, the FP16 storage
+    of W), equal bit for bit to its own application, and scaled by 2^60 and
+    2^-60 with its input (the inputs are scaled by powers of two before they
+    are cut into FP16 parts, so nothing rounds differently)."""
+    import torch
+    from cugmres_amd import problems, solver, tiles as gt
+    from oracle import tiles
+    N = 128
+    print(f"tiles groups T={T} systems={systems}", flush=True)
+    ctx = solver.Context(N, 0)
+    ref_blk = orc.baseline_green_block(N, problems.KH)
+    chi = _sparse_pattern_map(N, 4)
+    tl = gt.Tiles(ctx, T, 1).factor(ctx.block_helmholtz(problems.KH), ctx.to_device(chi, "f32"))
+    rng = np.random.default_rng(systems)
+    V = (rng.standard_normal((systems, N * N)) + 1j * rng.standard_normal((systems, N * N))).astype(np.complex64)
+    dV = torch.as_tensor(V).to(ctx.device)
+    y = tl.apply(dV)
+    R = tiles.tile_reduced(ref_blk, chi, N, T)
+    for k in range(systems):
+        yk = y[k].cpu().numpy()
+        if k in (0, systems - 1):
+            assert rel(yk, tiles.tile_apply_reduced(R, ref_blk, V[k].astype(np.complex128), N, T)) < (
+                1e-2 if T == 64 else 2.5e-2)
+        assert torch.equal(tl.apply(dV[k].contiguous()), y[k]), k
+    for e in (60, -60):
+        assert torch.equal(tl.apply(dV * 2.0 ** e), y * 2.0 ** e), e
+    tl.close()
+    ctx.close()
+
+
 def _oracle_right_pc_gmres(A, P, b, tol, m=400):
     """Unrestarted right-preconditioned GMRES in FP64 numpy (CGS2), for the
     reference solutions of the tests above: x = P y, min ||b - A P y||."""
