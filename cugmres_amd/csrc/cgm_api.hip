@@ -139,6 +139,7 @@ extern "C" int cgm_create(cgm_ctx_t* out, int N, int device) {
     return CGM_ERROR_ALLOC;
   }
   CGM_HIP(hipMemset(c->st, 0, sizeof(DevState)));
+  if ((rc = pass_lds_limits(c->M))) { cgm_destroy(c); return rc; }
   if ((rc = cgm_autotune(c))) { cgm_destroy(c); return rc; }
   *out = c;
   return CGM_SUCCESS;
@@ -153,7 +154,7 @@ extern "C" int cgm_autotune(cgm_ctx_t c) {
   CGM_CHECK(c, CGM_ERROR_INVALID_VALUE, "null context");
   CGM_HIP(hipSetDevice(c->device));
   const int N = c->N, M = c->M;
-  const int nt = fft_threads(M);
+  const int nt = pass_threads(M, false);
   const long n = (long)N * N;
   const size_t H = (size_t)M / 2 + 1;
   float2 *x = nullptr, *gq = nullptr;
@@ -185,7 +186,7 @@ extern "C" int cgm_autotune(cgm_ctx_t c) {
   float best1 = 1e30f, best2 = 1e30f, best3 = 1e30f;
   int r1 = P.rows1, c2 = P.cols2, r3 = P.rows3;
   for (int k : cand) {
-    if (k * nt > pass_max_threads(M, false) || (size_t)k * lds_len(M, false) * sizeof(float2) > 65536) continue;
+    if (k * nt > pass_max_threads(M, false) || (size_t)k * lds_len(M) * sizeof(float2) > 65536) continue;
     Plan Q = P;
     Q.rows1 = Q.rows3 = k;
     const float t1 = time_it([&] { rc |= launch_pass1<float>(Q, c->stream, x, nullptr, chi, nullptr, kModeForward, c->T32, c->tw32, nullptr); });
@@ -198,10 +199,10 @@ extern "C" int cgm_autotune(cgm_ctx_t c) {
       if (t2 < best2) { best2 = t2; c2 = k; }
     }
   }
-  // M = 1024: the register-resident one-wave kernel of each pass against
-  // the tuned LDS-staged radix-8 one, at batches of 1, 4 and 16
-  // vectors; a pass takes the register-resident kernel from the smallest batch
-  // at which it is faster at that batch and at every larger one
+  // M = 1024: the one-wave form of each pass (16 elements per thread) against
+  // the tuned two-wave one (8), at batches of 1, 4 and 16 vectors; a pass takes
+  // the one-wave form from the smallest batch at which it is faster at that
+  // batch and at every larger one
   int wide_from[3] = {0, 0, 0};
   float wide_us[3][3] = {}, lds_us[3][3] = {};
   if (!rc && M == 1024) {
@@ -442,6 +443,8 @@ extern "C" int cgm_block_reference(cgm_ctx_t c, double k, double sr, double sc, 
 static int matvec32(cgm_context* c, const float2* gq, const float* chi, const float2* x,
                     const float2* b, float2* y, int mode, const double* norm_ptr, float2* xw,
                     const int* done) {
+  if (!b && !norm_ptr && !done && mode <= kModeGreen && small_matvec<float>(c->plan))
+    return launch_small<float, float2>(c->plan, c->stream, x, chi, gq, y, mode, c->tw32);
   int rc = launch_pass1<float>(c->plan, c->stream, x, xw, chi, norm_ptr, mode, c->T32, c->tw32, done);
   if (!rc) rc = launch_pass2<float, float2>(c->plan, c->stream, c->T32, gq, c->tw32, done);
   // pass 3 reads the (possibly rescaled) input written back by pass 1
@@ -457,6 +460,8 @@ static int ensure_T64(cgm_context* c) {
 
 static int matvec64(cgm_context* c, const double2* gq, const double* chi, const double2* x,
                     const double2* b, double2* y, int mode) {
+  if (!b && mode <= kModeGreen && small_matvec<double>(c->plan64))
+    return launch_small<double, double2>(c->plan64, c->stream, x, chi, gq, y, mode, c->tw64);
   int rc = ensure_T64(c);
   if (!rc) rc = launch_pass1<double>(c->plan64, c->stream, x, nullptr, chi, nullptr, mode, c->T64, c->tw64, nullptr);
   if (!rc) rc = launch_pass2<double, double2>(c->plan64, c->stream, c->T64, gq, c->tw64, nullptr);
@@ -493,14 +498,17 @@ extern "C" int cgm_matvec_batched(cgm_ctx_t c, const cgm_complex64* gamma, const
   CGM_CHECK(chi_stride == 0 || chi_stride >= (long)c->N * c->N, CGM_ERROR_INVALID_VALUE,
             "chi_stride must be 0 (shared map) or >= N*N");
   CGM_HIP(hipSetDevice(c->device));
-  int rc = ensure_T32B(c, batch);
-  if (rc) return rc;
   const long n = (long)c->N * c->N;
   BatchStrides bs;
   bs.x = n;
   bs.chi = chi_stride;
   bs.y = n;
   bs.T = (long)c->N * c->M;
+  if (small_matvec<float>(c->plan))
+    return launch_small<float, float2>(c->plan, c->stream, (const float2*)x, chi, (const float2*)gamma, (float2*)y,
+                                       mode, c->tw32, batch, bs);
+  int rc = ensure_T32B(c, batch);
+  if (rc) return rc;
   rc = launch_pass1<float>(c->plan, c->stream, (const float2*)x, nullptr, chi, nullptr, mode, c->T32B, c->tw32,
                            nullptr, batch, bs);
   if (!rc) rc = launch_pass2<float, float2>(c->plan, c->stream, c->T32B, (const float2*)gamma, c->tw32, nullptr,

@@ -133,7 +133,7 @@ template <int M, int EPD, int BS>
 __global__ void __launch_bounds__(BS) k_arn_a(FusedArgs a) {
   batch_offset(a);
   const int dn = a.st->done;  // tested once this block's loads are in flight
-  constexpr int NT = FftShape<M>::NT;
+  constexpr int NT = FftShape<M, kFftE<M>>::NT;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   float2* smem = reinterpret_cast<float2*>(smem_raw);
   const int N = a.N, R = a.R, j = a.j;
@@ -145,12 +145,12 @@ __global__ void __launch_bounds__(BS) k_arn_a(FusedArgs a) {
   const int t = tid % NT, rl = fa ? tid / NT : 0;
   FftTwiddles<float, M> tws;
   if (fa) tws.load(a.tw, t);
-  constexpr int ML = LdsLen<float, M>::value;
+  constexpr int ML = LdsLen<M>::value;
   float2* buf = smem + rl * ML;
   const bool tail = a.tail != 0;
   // the row values of pass 3 and this thread's u values, loaded before the
   // done test so that their latency overlaps it
-  constexpr int EPT = FftShape<M>::EPT;
+  constexpr int EPT = FftShape<M, kFftE<M>>::EPT;
   float2 trow[EPT];
   if (!tail && fa) {
     const int row = r0 + rl;
@@ -173,12 +173,13 @@ __global__ void __launch_bounds__(BS) k_arn_a(FusedArgs a) {
   }
   if (dn) return;
   if (!tail) {
+    reg_fft<float, M, +1, false, true>(trow, buf, tws, t, fa);  // columns < N are used
+    FftSync<M>::stage();
     if (fa) {
 #pragma unroll
-      for (int k = 0; k < EPT; ++k) buf[lpad<float>(t + k * NT)] = trow[k];
+      for (int k = 0; k < EPT / 2; ++k) buf[lpad(t + k * NT)] = trow[k];
     }
     __syncthreads();
-    lds_fft<float, M, +1, false, true>(buf, tws, t, fa);  // columns < N are used
   }
   // ---- z = u - G(.), u and z of the block's R*N elements staged in LDS -------
   // (the FFT rows are no longer needed once every thread has read its values)
@@ -196,7 +197,7 @@ __global__ void __launch_bounds__(BS) k_arn_a(FusedArgs a) {
       uu[k] = u;
       if (!tail) {
         const float2 xin = xpre[k];
-        float2 tv = smem[r * ML + lpad<float>(c)];
+        float2 tv = smem[r * ML + lpad(c)];
         tv.x *= a.inv_mm;
         tv.y *= a.inv_mm;
         if (a.mode == kModeAdjoint) {
@@ -479,7 +480,7 @@ template <int M, int EPD, int BS>
 __global__ void __launch_bounds__(BS) k_arn_b(FusedArgs a) {
   batch_offset(a);
   const int dn = a.st->done;  // tested once this block's u, z and basis loads are issued
-  constexpr int NT = FftShape<M>::NT;
+  constexpr int NT = FftShape<M, kFftE<M>>::NT;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   float2* smem = reinterpret_cast<float2*>(smem_raw);
   const int N = a.N, R = a.R, j = a.j;
@@ -577,7 +578,7 @@ __global__ void __launch_bounds__(BS) k_arn_b(FusedArgs a) {
         w.y *= ch;
       }
     }
-    if (r < R && !a.flex) smem[r * LdsLen<float, M>::value + lpad<float>(c)] = w;
+    if (r < R && !a.flex) smem[r * LdsLen<M>::value + lpad(c)] = w;
   }
   if (a.flex) {
     // ||u_{j+1}||: block partial, the last block sums them in a fixed order
@@ -600,18 +601,24 @@ __global__ void __launch_bounds__(BS) k_arn_b(FusedArgs a) {
     return;
   }
   if (a.tail) return;  // u_m needs no matvec (block-uniform)
-  constexpr int ZE = fft_lo_read_end<M>();  // zeros the transform reads
-  for (int e = tid; e < R * (ZE - N); e += BS) {
-    const int r = e / (ZE - N), c = N + e % (ZE - N);
-    smem[r * LdsLen<float, M>::value + lpad<float>(c)] = make_float2(0.f, 0.f);
-  }
   __syncthreads();
-  float2* buf = smem + rl * LdsLen<float, M>::value;
-  lds_fft<float, M, -1, true>(buf, tws, t, fa);  // the rows are zero from N <= M/2 on
+  float2* buf = smem + rl * LdsLen<M>::value;
+  constexpr int EPT = FftShape<M, kFftE<M>>::EPT;
+  float2 v[EPT];
+  if (fa) {
+#pragma unroll
+    for (int k = 0; k < EPT / 2; ++k) {  // the rows are zero from N <= M/2 on
+      const int e = t + k * NT;
+      v[k] = e < N ? buf[lpad(e)] : make_float2(0.f, 0.f);
+    }
+  }
+  FftSync<M>::stage();
+  reg_fft<float, M, -1, true>(v, buf, tws, t, fa);
   if (fa) {
     const int row = r0 + rl;
     if (row < N) {
-      for (int e = t; e < M; e += NT) a.T[tpos(row, e, N)] = buf[lpad<float>(e)];
+#pragma unroll
+      for (int k = 0; k < EPT; ++k) a.T[tpos(row, t + k * NT, N)] = v[k];
     }
   }
 }
@@ -695,7 +702,7 @@ int launch_fused(hipStream_t st, int which, const FusedLaunch& L) {
   a.sSt = L.sSt;
   a.sHist = L.sHist;
   // the row FFTs, then u and z of the block staged in the same space
-  size_t lds = (size_t)a.R * lds_len(M, false) * sizeof(float2);
+  size_t lds = (size_t)a.R * lds_len(M) * sizeof(float2);
   const size_t stage = (size_t)2 * fs.bs * epd * sizeof(float2);
   if (lds < stage) lds = stage;
 #define CGM_FUSED_LAUNCH(NN, EPD, BSZ)                                                          \

@@ -1,5 +1,8 @@
-// LDS-resident self-sorting Stockham FFT for one transform of compile-time
-// length M, executed by NT = M / EPT threads that each hold EPT elements.
+// Self-sorting Stockham FFT for one transform of compile-time length M, executed
+// by NT = M / EPT threads that each hold EPT elements in registers: element
+// t + NT k in register k of thread t, for the input and for the output.  Every
+// stage is a DFT over registers; between two stages the data cross threads
+// through LDS once.
 //
 // Stage s with radix R over span Ns (product of earlier radices): butterfly
 // j in [0, M/R) reads x[j + r*M/R], multiplies by exp(sign*2*pi*i*r*(j%Ns)/(Ns*R)),
@@ -13,53 +16,80 @@
 namespace cgm {
 
 // ---- LDS layout ---------------------------------------------------------------
-// Single-precision transforms keep one pad element after every 8 in LDS:
-// element e sits at e + e/8.  The first radix-8 stage writes x[8j + r] (64-byte
-// lane stride for complex64), which without the pad lands every lane of a
-// wave in the same few banks; with it the stride is 72 bytes and the writes
-// spread over all banks, while stride-1 reads stay contiguous.  Double
-// transforms (the one-off spectrum and the FP64 refinement) are unpadded so
-// that a 4096-point row still fits 64 KiB.
-template <typename T> __host__ __device__ constexpr int lpad(int e) { return sizeof(T) == 4 ? e + (e >> 3) : e; }
-template <typename T, int M> struct LdsLen {
-  static constexpr int value = sizeof(T) == 4 ? M + M / 8 : M;
+// Transforms keep one pad element after every 8 in LDS: element e sits at
+// e + e/8.  The first radix-8 stage writes x[8j + r] (64-byte lane stride for
+// complex64), which without the pad lands every lane of a wave in the same few
+// banks; with it the stride is 72 bytes and the writes spread over all banks,
+// while stride-1 reads stay contiguous.
+__host__ __device__ constexpr int lpad(int e) { return e + (e >> 3); }
+template <int M> struct LdsLen {
+  static constexpr int value = M + M / 8;
 };
 
 // ---- radix plans ------------------------------------------------------------
-// Elements per thread: 8 for powers of two (radices 8/4/2), 12 for 3*2^k
-// (radices 3/4/2).  Radices must divide EPT so that every thread owns exactly
-// EPT/R butterflies per stage.
-template <int M> struct FftShape {
+// E elements per thread.  Radices must divide E, so that every thread owns
+// exactly E/R butterflies per stage.
+//   powers of two: E = 8 (radices 8, then 4 or 2, or 4 4 in place of 8 2) or 16 (the fewest stages of
+//                  at most 16, as even as possible: 128 = 16 8, 1024 = 16 8 8);
+//   3 * 2^k:       E = 12 (a radix-12 first stage, then 4s and a 2) or 24 (12,
+//                  then 8s and a 4 or 2).
+// Fewer stages exchange less through LDS; more elements per thread take more
+// registers and leave fewer threads.
+template <int M, int E> struct FftShape {
   static constexpr bool pow2 = (M & (M - 1)) == 0;
-  static constexpr int EPT = pow2 ? 8 : 12;
-  static constexpr int NT = M / EPT;
+  static constexpr int EPT = E;
+  static constexpr int NT = M / E;
   // work-group size bound used for launch_bounds: groups of transforms fill 256 threads
   static constexpr int WG = NT > 256 ? NT : 256;
+  static_assert(pow2 ? (E == 8 || E == 16) : (E == 12 || E == 24), "elements per thread");
 };
+// Elements per thread without a reason for more.
+template <int M> constexpr int kFftE = (M & (M - 1)) == 0 ? 8 : 12;
 
-template <int M> __host__ __device__ constexpr int fft_num_stages() {
-  int n = M, k = 0;
-  if ((M & (M - 1)) == 0) {
-    while (n % 8 == 0 && n > 1) { n /= 8; ++k; }
-    if (n > 1) ++k;
-  } else {
-    while (n % 3 == 0) { n /= 3; ++k; }
-    while (n % 4 == 0) { n /= 4; ++k; }
-    if (n > 1) ++k;
-  }
+constexpr int fft_log2(int n) {
+  int k = 0;
+  while (n > 1) { n >>= 1; ++k; }
   return k;
 }
-
-template <int M> __host__ __device__ constexpr int fft_radix(int s) {
-  int n = M, k = 0;
-  if ((M & (M - 1)) == 0) {
-    while (n % 8 == 0 && n > 1) { if (k == s) return 8; n /= 8; ++k; }
-    return n;  // remainder 2 or 4
-  } else {
-    while (n % 3 == 0) { if (k == s) return 3; n /= 3; ++k; }
-    while (n % 4 == 0) { if (k == s) return 4; n /= 4; ++k; }
-    return n;  // remainder 2
+// Radix of stage s (0: there is no such stage).
+template <int M, int E> __host__ __device__ constexpr int fft_radix(int s) {
+  int n = M;
+  if constexpr (E == 16) {
+    int left = (fft_log2(M) + 3) / 4;
+    for (int k = 0; left > 0; ++k, --left) {
+      const int e = (fft_log2(n) + left - 1) / left;
+      if (k == s) return 1 << e;
+      n >>= e;
+    }
+    return 0;
   }
+  int k = 0;
+  if (E == 12 || E == 24) {
+    if (s == 0) return 12;
+    n /= 12;
+    ++k;
+  }
+  const int top = E == 12 ? 4 : 8;
+  if (E == 8) {  // 8s, and two 4s rather than an 8 and a 2
+    while (n > 1) {
+      const int r = n == 16 ? 4 : n % 8 == 0 ? 8 : n;
+      if (k == s) return r;
+      n /= r;
+      ++k;
+    }
+    return 0;
+  }
+  while (n % top == 0 && n > 1) {
+    if (k == s) return top;
+    n /= top;
+    ++k;
+  }
+  return k == s && n > 1 ? n : 0;  // remainder
+}
+template <int M, int E> __host__ __device__ constexpr int fft_num_stages() {
+  int k = 0;
+  while (fft_radix<M, E>(k) > 0) ++k;
+  return k;
 }
 
 // ---- small DFTs in registers -------------------------------------------------
@@ -109,9 +139,9 @@ __device__ inline void dft8(cplx<T>* v) {
   dft4<T, SIGN>(o);
   const T h = T(0.70710678118654752440);
   // w8^1 = (1 + SIGN i)/sqrt2, w8^2 = SIGN i, w8^3 = (-1 + SIGN i)/sqrt2
-  cplx<T> o1 = cmul(o[1], mk(h, T(SIGN) * h));
+  cplx<T> o1 = mk(h * (o[1].x - T(SIGN) * o[1].y), h * (o[1].y + T(SIGN) * o[1].x));
   cplx<T> o2 = mul_si<T, SIGN>(o[2]);
-  cplx<T> o3 = cmul(o[3], mk(-h, T(SIGN) * h));
+  cplx<T> o3 = mk(-h * (o[3].x + T(SIGN) * o[3].y), h * (T(SIGN) * o[3].x - o[3].y));
   v[0] = cadd(e[0], o[0]);
   v[4] = csub(e[0], o[0]);
   v[1] = cadd(e[1], o1);
@@ -122,12 +152,22 @@ __device__ inline void dft8(cplx<T>* v) {
   v[7] = csub(e[3], o3);
 }
 
+// 12-point DFT: n = 3 m + p, k = k1 + 4 k2; 4-point DFTs over m, the twiddles
+// exp(SIGN 2 pi i p k1 / 12), 3-point DFTs over p.  LO: v[6 ..] are zero and
+// not read.
+template <typename T, int SIGN, bool LO> __device__ inline void dft12(cplx<T>* v);
+// 16-point DFT: n = 4 m + p, k = k1 + 4 k2, the same way with twiddles exp(SIGN 2
+// pi i p k1 / 16).  LO: v[8 ..] are zero and not read.
+template <typename T, int SIGN, bool LO> __device__ inline void dft16(cplx<T>* v);
+
 template <typename T, int SIGN, int R>
 __device__ inline void dft(cplx<T>* v) {
   if constexpr (R == 2) dft2<T, SIGN>(v[0], v[1]);
   else if constexpr (R == 3) dft3<T, SIGN>(v);
   else if constexpr (R == 4) dft4<T, SIGN>(v);
   else if constexpr (R == 8) dft8<T, SIGN>(v);
+  else if constexpr (R == 12) dft12<T, SIGN, false>(v);
+  else if constexpr (R == 16) dft16<T, SIGN, false>(v);
 }
 
 // The same DFTs when the upper half of the inputs, v[R/2 .. R-1], is zero
@@ -141,12 +181,93 @@ __device__ inline void dft4_lo(cplx<T>* v) {  // v[2] = v[3] = 0
   v[1] = cadd(a, d);
   v[3] = csub(a, d);
 }
+template <typename T, int SIGN, bool LO>
+__device__ inline void dft12(cplx<T>* v) {
+  cplx<T> a[3][4];
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+#pragma unroll
+    for (int m = 0; m < (LO ? 2 : 4); ++m) a[p][m] = v[3 * m + p];
+    if constexpr (LO) dft4_lo<T, SIGN>(a[p]);
+    else dft4<T, SIGN>(a[p]);
+  }
+  const T c = T(0.86602540378443864676), h = T(0.5);  // cos, sin of pi/6
+  a[1][1] = cmul(a[1][1], mk(c, T(SIGN) * h));
+  a[1][2] = cmul(a[1][2], mk(h, T(SIGN) * c));
+  a[1][3] = mul_si<T, SIGN>(a[1][3]);
+  a[2][1] = cmul(a[2][1], mk(h, T(SIGN) * c));
+  a[2][2] = cmul(a[2][2], mk(-h, T(SIGN) * c));
+  a[2][3] = mk(-a[2][3].x, -a[2][3].y);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    cplx<T> b[3] = {a[0][k], a[1][k], a[2][k]};
+    dft3<T, SIGN>(b);
+    v[k] = b[0];
+    v[k + 4] = b[1];
+    v[k + 8] = b[2];
+  }
+}
+// a * exp(SIGN 2 pi i Q / 16)
+template <typename T, int SIGN, int Q>
+__device__ inline cplx<T> rot16(cplx<T> a) {
+  constexpr T h = T(0.70710678118654752440);
+  constexpr T c1 = T(0.92387953251128675613), s1 = T(0.38268343236508977173);  // cos, sin of pi/8
+  if constexpr (Q == 4) {
+    return mul_si<T, SIGN>(a);
+  } else if constexpr (Q == 2) {
+    return mk(h * (a.x - SIGN * a.y), h * (a.y + SIGN * a.x));
+  } else if constexpr (Q == 6) {
+    return mk(-h * (a.x + SIGN * a.y), h * (SIGN * a.x - a.y));
+  } else if constexpr (Q == 1) {
+    return cmul(a, mk(c1, SIGN * s1));
+  } else if constexpr (Q == 3) {
+    return cmul(a, mk(s1, SIGN * c1));
+  } else {
+    static_assert(Q == 9, "twiddles of the 16-point DFT");
+    return cmul(a, mk(-c1, -SIGN * s1));
+  }
+}
+
+template <typename T, int SIGN, bool LO>
+__device__ inline void dft16(cplx<T>* v) {
+  cplx<T> a[4][4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+#pragma unroll
+    for (int m = 0; m < (LO ? 2 : 4); ++m) a[p][m] = v[4 * m + p];
+    if constexpr (LO)
+      dft4_lo<T, SIGN>(a[p]);
+    else
+      dft4<T, SIGN>(a[p]);
+  }
+  a[1][1] = rot16<T, SIGN, 1>(a[1][1]);
+  a[1][2] = rot16<T, SIGN, 2>(a[1][2]);
+  a[1][3] = rot16<T, SIGN, 3>(a[1][3]);
+  a[2][1] = rot16<T, SIGN, 2>(a[2][1]);
+  a[2][2] = rot16<T, SIGN, 4>(a[2][2]);
+  a[2][3] = rot16<T, SIGN, 6>(a[2][3]);
+  a[3][1] = rot16<T, SIGN, 3>(a[3][1]);
+  a[3][2] = rot16<T, SIGN, 6>(a[3][2]);
+  a[3][3] = rot16<T, SIGN, 9>(a[3][3]);
+#pragma unroll
+  for (int k1 = 0; k1 < 4; ++k1) {
+    cplx<T> b[4] = {a[0][k1], a[1][k1], a[2][k1], a[3][k1]};
+    dft4<T, SIGN>(b);
+#pragma unroll
+    for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = b[k2];
+  }
+}
+
 template <typename T, int SIGN, int R>
 __device__ inline void dft_lo(cplx<T>* v) {
   if constexpr (R == 2) {
     v[1] = v[0];
   } else if constexpr (R == 4) {
     dft4_lo<T, SIGN>(v);
+  } else if constexpr (R == 12) {
+    dft12<T, SIGN, true>(v);
+  } else if constexpr (R == 16) {
+    dft16<T, SIGN, true>(v);
   } else {
     static_assert(R == 8, "half-zero inputs need an even radix");
     cplx<T> e[4] = {v[0], v[2], v[0], v[0]};  // v[4], v[6] are zero
@@ -154,9 +275,9 @@ __device__ inline void dft_lo(cplx<T>* v) {
     dft4_lo<T, SIGN>(e);
     dft4_lo<T, SIGN>(o);
     const T h = T(0.70710678118654752440);
-    cplx<T> o1 = cmul(o[1], mk(h, T(SIGN) * h));
+    cplx<T> o1 = mk(h * (o[1].x - T(SIGN) * o[1].y), h * (o[1].y + T(SIGN) * o[1].x));
     cplx<T> o2 = mul_si<T, SIGN>(o[2]);
-    cplx<T> o3 = cmul(o[3], mk(-h, T(SIGN) * h));
+    cplx<T> o3 = mk(-h * (o[3].x + T(SIGN) * o[3].y), h * (T(SIGN) * o[3].x - o[3].y));
     v[0] = cadd(e[0], o[0]);
     v[4] = csub(e[0], o[0]);
     v[1] = cadd(e[1], o1);
@@ -169,31 +290,31 @@ __device__ inline void dft_lo(cplx<T>* v) {
 }
 
 // Twiddles of one thread for every stage with span NS > 1, flattened:
-// stage S, butterfly b, r = 1..R-1 at tw_offset<M>(S) + b*(R-1) + r-1.
-template <int M> __host__ __device__ constexpr int fft_stage_span(int S) {
+// stage S, butterfly b, r = 1..R-1 at fft_tw_offset<M, E>(S) + b*(R-1) + r-1.
+template <int M, int E> __host__ __device__ constexpr int fft_stage_span(int S) {
   int ns = 1;
-  for (int s = 0; s < S; ++s) ns *= fft_radix<M>(s);
+  for (int s = 0; s < S; ++s) ns *= fft_radix<M, E>(s);
   return ns;
 }
-template <int M> __host__ __device__ constexpr int fft_tw_offset(int S) {
+template <int M, int E> __host__ __device__ constexpr int fft_tw_offset(int S) {
   int off = 0;
   for (int s = 0; s < S; ++s)
-    if (fft_stage_span<M>(s) > 1) off += (FftShape<M>::EPT / fft_radix<M>(s)) * (fft_radix<M>(s) - 1);
+    if (fft_stage_span<M, E>(s) > 1) off += (FftShape<M, E>::EPT / fft_radix<M, E>(s)) * (fft_radix<M, E>(s) - 1);
   return off;
 }
-template <int M> __host__ __device__ constexpr int fft_tw_count() {
-  return fft_tw_offset<M>(fft_num_stages<M>());
+template <int M, int E> __host__ __device__ constexpr int fft_tw_count() {
+  return fft_tw_offset<M, E>(fft_num_stages<M, E>());
 }
 
-template <typename T, int M, int S>
+template <typename T, int M, int E, int S>
 __device__ inline void fft_load_tw(cplx<T>* reg, const cplx<T>* __restrict__ tw, int t) {
-  if constexpr (S < fft_num_stages<M>()) {
-    constexpr int R = fft_radix<M>(S);
-    constexpr int NS = fft_stage_span<M>(S);
+  if constexpr (S < fft_num_stages<M, E>()) {
+    constexpr int R = fft_radix<M, E>(S);
+    constexpr int NS = fft_stage_span<M, E>(S);
     if constexpr (NS > 1) {
-      constexpr int NB = FftShape<M>::EPT / R;
-      constexpr int NT = FftShape<M>::NT;
-      constexpr int OFF = fft_tw_offset<M>(S);
+      constexpr int NB = FftShape<M, E>::EPT / R;
+      constexpr int NT = FftShape<M, E>::NT;
+      constexpr int OFF = fft_tw_offset<M, E>(S);
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         const int k = (t + b * NT) % NS;
@@ -201,97 +322,136 @@ __device__ inline void fft_load_tw(cplx<T>* reg, const cplx<T>* __restrict__ tw,
         for (int r = 1; r < R; ++r) reg[OFF + b * (R - 1) + r - 1] = tw[(r * k) * (M / (NS * R))];
       }
     }
-    fft_load_tw<T, M, S + 1>(reg, tw, t);
+    fft_load_tw<T, M, E, S + 1>(reg, tw, t);
   }
 }
 
-// One Stockham stage for the butterflies owned by thread t.  LO: the inputs
-// j + r M/R with r >= R/2 (the upper half of the data, first stage only)
-// are zero and not read.  HI: only the outputs below M/2 (r < R/2 of the
-// last stage) are wanted and written.
-template <typename T, int M, int SIGN, int R, int NS, int OFF, bool LO = false, bool HI = false>
-__device__ inline void fft_stage(cplx<T>* buf, const cplx<T>* reg, int t, bool active = true) {
-  constexpr int EPT = FftShape<M>::EPT;
-  constexpr int NT = FftShape<M>::NT;
-  constexpr int NB = EPT / R;        // butterflies per thread
-  constexpr int MR = M / R;
-  // Threads outside the transform (active = false) skip the data work but
-  // reach the same two barriers: the barriers stay outside any branch, so a
-  // wave whose lanes are partly inside the transform (rows * NT not a multiple
-  // of 64) still executes exactly two of them.
-  static_assert(!LO || (NS == 1 && R % 2 == 0), "half-zero inputs: first stage, even radix");
-  static_assert(!HI || (NS * R == M && R % 2 == 0), "half outputs: last stage, even radix");
-  cplx<T> v[NB][R];
-  if (active) {
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int j = t + b * NT;
-#pragma unroll
-      for (int r = 0; r < (LO ? R / 2 : R); ++r) v[b][r] = buf[lpad<T>(j + r * MR)];
-    }
+// A thread's twiddles: registers loaded once per kernel (before the data, so the
+// table reads overlap the first global loads) and reused by every forward and
+// inverse transform the thread takes part in.  With 12 double elements they
+// would take over 100 registers; there they are read from the table (in the L1)
+// where they are used (FP64 product at N = 700: 65.6 instead of 72.5 us; with 8
+// elements it is the slower form, N = 1024: 86 instead of 83 us).
+template <typename T, int M, int E = kFftE<M>> struct FftTwiddles {
+  static constexpr bool late = sizeof(T) == 8 && E == 12;
+  static constexpr int K = late || fft_tw_count<M, E>() == 0 ? 1 : fft_tw_count<M, E>();
+  cplx<T> reg[K];
+  const cplx<T>* tab;
+  __device__ inline void load(const cplx<T>* __restrict__ tw, int t) {
+    if constexpr (late) tab = tw;
+    else fft_load_tw<T, M, E, 0>(reg, tw, t);
   }
-  __syncthreads();
+  // Keeps the compiler from holding table values from one transform to the next.
+  __device__ inline void refresh() {
+    if constexpr (late) asm volatile("" : "+s"(tab));
+  }
+  // r-th twiddle of butterfly b of stage S with span NS and radix R
+  template <int S, int NS, int R>
+  __device__ inline cplx<T> get(int t, int b, int r) const {
+    if constexpr (late) return tab[(r * ((t + b * (M / E)) % NS)) * (M / (NS * R))];
+    constexpr int OFF = fft_tw_offset<M, E>(S);  // a constant, so that the registers are indexed by constants
+    return reg[late ? 0 : OFF + b * (R - 1) + r - 1];
+  }
+};
+
+// Orders one wave's LDS writes before its later reads (no instruction: the
+// wave's LDS accesses complete in issue order; this keeps the compiler from
+// moving them across).
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Transforms of at most 64 threads lie within one wave: thread t of the
+// transform is lane (t + NT * k) of its wave, since NT is a power of two and
+// the groups of NT threads start at multiples of it.  Their stages are ordered
+// by the wave's own LDS order and take no work-group barrier: the waves of a
+// work-group run through their transforms independently.
+template <int M, int E = kFftE<M>> struct FftSync {
+  static constexpr bool one_wave = FftShape<M, E>::NT <= 64 && 64 % FftShape<M, E>::NT == 0;
+  static __device__ inline void stage() {
+    if constexpr (one_wave) wave_lds_sync();
+    else __syncthreads();
+  }
+};
+
+// Where element e of a transform sits in its LDS buffer.
+struct LdsRow {
+  __device__ inline int operator()(int e) const { return lpad(e); }
+};
+
+// Stage S of a transform and the ones after it.  Threads outside the
+// transform (active = false) skip the data work but reach the same
+// synchronisations: these stay outside any branch, so a wave whose lanes are
+// partly inside the transform still executes all of them.
+template <typename T, int M, int E, int SIGN, int S, int NS, bool LO, bool HI, typename IX>
+__device__ inline void fft_stages(cplx<T>* v, cplx<T>* buf, const FftTwiddles<T, M, E>& tws, int t, bool active, IX at) {
+  constexpr int R = fft_radix<M, E>(S);
+  constexpr int EPT = E;
+  constexpr int NT = FftShape<M, E>::NT;
+  constexpr int NB = EPT / R;  // butterflies per thread: j = t + b NT reads registers b + r NB
+  constexpr bool lo = LO && S == 0 && R % 2 == 0;
+  constexpr bool last = S + 1 == fft_num_stages<M, E>();
+  static_assert(!LO || fft_radix<M, E>(0) % 2 == 0, "half-zero inputs need an even first radix");
+  static_assert(!HI || fft_radix<M, E>(fft_num_stages<M, E>() - 1) % 2 == 0, "half outputs need an even last radix");
+  cplx<T> u[NB][R];
   if (active) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int j = t + b * NT;
-      const int k = j % NS;
+#pragma unroll
+      for (int r = 0; r < (lo ? R / 2 : R); ++r) u[b][r] = v[b + r * NB];
       if constexpr (NS > 1) {
 #pragma unroll
         for (int r = 1; r < R; ++r) {
-          cplx<T> w = reg[OFF + b * (R - 1) + r - 1];
+          cplx<T> w = tws.template get<S, NS, R>(t, b, r);
           if (SIGN > 0) w.y = -w.y;
-          v[b][r] = cmul(v[b][r], w);
+          u[b][r] = cmul(u[b][r], w);
         }
       }
-      if constexpr (LO)
-        dft_lo<T, SIGN, R>(v[b]);
+      if constexpr (lo)
+        dft_lo<T, SIGN, R>(u[b]);
       else
-        dft<T, SIGN, R>(v[b]);
-      const int base = (j / NS) * NS * R + k;
-#pragma unroll
-      for (int r = 0; r < (HI ? R / 2 : R); ++r) buf[lpad<T>(base + r * NS)] = v[b][r];
+        dft<T, SIGN, R>(u[b]);
     }
   }
-  __syncthreads();
-}
-
-template <typename T, int M, int SIGN, int S, int NS, bool LO, bool HI>
-__device__ inline void fft_stages(cplx<T>* buf, const cplx<T>* reg, int t, bool active) {
-  if constexpr (S < fft_num_stages<M>()) {
-    constexpr int R = fft_radix<M>(S);
-    constexpr bool lo = LO && S == 0 && R % 2 == 0;
-    constexpr bool hi = HI && S == fft_num_stages<M>() - 1 && R % 2 == 0;
-    fft_stage<T, M, SIGN, R, NS, fft_tw_offset<M>(S), lo, hi>(buf, reg, t, active);
-    fft_stages<T, M, SIGN, S + 1, NS * R, LO, HI>(buf, reg, t, active);
+  if constexpr (last) {
+    if (active) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < (HI ? R / 2 : R); ++r) v[b + r * NB] = u[b][r];
+    }
+  } else {
+    if constexpr (S > 0) FftSync<M, E>::stage();  // the previous exchange is read
+    if (active) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const int j = t + b * NT;
+        const int base = (j / NS) * NS * R + j % NS;
+#pragma unroll
+        for (int r = 0; r < R; ++r) buf[at(base + r * NS)] = u[b][r];
+      }
+    }
+    FftSync<M, E>::stage();
+    if (active) {
+#pragma unroll
+      for (int k = 0; k < EPT; ++k) v[k] = buf[at(t + k * NT)];
+    }
+    fft_stages<T, M, E, SIGN, S + 1, NS * R, LO, HI>(v, buf, tws, t, active, at);
   }
 }
 
-// Per-thread twiddle registers, loaded once per kernel (before the data, so
-// the table reads overlap the first global loads) and reused by every
-// forward and inverse transform the thread takes part in.
-template <typename T, int M> struct FftTwiddles {
-  static constexpr int K = fft_tw_count<M>() > 0 ? fft_tw_count<M>() : 1;
-  cplx<T> reg[K];
-  __device__ inline void load(const cplx<T>* __restrict__ tw, int t) { fft_load_tw<T, M, 0>(reg, tw, t); }
-};
-
-// Length of the zero padding a transform with LO still reads: the first
-// stage of an even first radix never reads buf[M/2 ..], so zero-padded data
-// need zeros only up to M/2 there (up to M otherwise).
-template <int M> __host__ __device__ constexpr int fft_lo_read_end() { return fft_radix<M>(0) % 2 == 0 ? M / 2 : M; }
-
-// Full transform of the M elements of buf (LDS, padded layout lpad<T>) by
-// threads t in [0, NT).  The caller
-// must have synchronised the work-group after filling buf; on return buf
-// holds the result and the group is synchronised.  LO: buf[M/2 ..] is zero
-// (zero-padded data; used when the first radix is even, the upper half is
-// then never read).  HI: only the outputs below M/2 are used (when the last
-// radix is even the others are not written and buf[M/2 ..] is left as it
-// was).
-template <typename T, int M, int SIGN, bool LO = false, bool HI = false>
-__device__ inline void lds_fft(cplx<T>* buf, const FftTwiddles<T, M>& tws, int t, bool active = true) {
-  fft_stages<T, M, SIGN, 0, 1, LO, HI>(buf, tws.reg, t, active);
+// Length-M transform of v (element t + NT k in v[k]) by threads t in [0, NT),
+// in place; buf is M elements of LDS (element e at buf[at(e)]) that no other
+// thread uses and that the transform's own threads are done with (FftSync<M, E>::stage()
+// before the call if they were not, and before buf is used again after it).
+// LO: the upper half of the input is zero (v[EPT/2 ..] is not read).  HI: only
+// the outputs below M/2 are formed (v[k], k < EPT/2).
+template <typename T, int M, int SIGN, bool LO = false, bool HI = false, int E = kFftE<M>, typename IX = LdsRow>
+__device__ inline void reg_fft(cplx<T>* v, cplx<T>* buf, const FftTwiddles<T, M, E>& tws, int t, bool active = true,
+                               IX at = IX()) {
+  fft_stages<T, M, E, SIGN, 0, 1, LO, HI>(v, buf, tws, t, active, at);
 }
 
 }  // namespace cgm

@@ -42,12 +42,15 @@ struct Plan {
   int rows1, rows3;  // rows per work-group in passes 1 and 3
   int cols2;         // columns per work-group in pass 2
   int wide1_batch, wide2_batch, wide3_batch;  // M = 1024, complex64: launches of at
-                     // least this many vectors take the register-resident
-                     // pass 1 / 2 / 3 (0: never)
+                     // least this many vectors take the 16-element (one-wave)
+                     // transforms in pass 1 / 2 / 3 (0: never)
 };
 
 int plan_init(Plan& P, int N);
 int fft_threads(int M);
+int pass_threads(int M, bool fp64);
+// Lets the kernels of size M that ask for more than 64 KB of LDS have it (current device).
+int pass_lds_limits(int M);
 int choose_embedding(int N);
 int pass_max_threads(int M, bool fp64);
 
@@ -62,6 +65,12 @@ template <typename T>
 int launch_pass3(const Plan& P, hipStream_t st, const cplx<T>* Tm, const cplx<T>* x, const T* chi,
                  const cplx<T>* b, cplx<T>* y, int mode, const cplx<T>* tw, const int* done,
                  int B = 1, const BatchStrides& bs = BatchStrides());
+
+// The whole product in one launch, on grids where small_matvec() says so.
+template <typename T> bool small_matvec(const Plan& P);
+template <typename T, typename G>
+int launch_small(const Plan& P, hipStream_t st, const cplx<T>* x, const T* chi, const G* gq, cplx<T>* y, int mode,
+                 const cplx<T>* tw, int B = 1, const BatchStrides& bs = BatchStrides());
 
 int spectrum_from_block(const Plan& P, hipStream_t st, const double2* blk, const double2* tw64,
                         float2* gq32, double2* gq64);

@@ -80,6 +80,9 @@ extern "C" int cgm_matvec_batched_noalloc(cgm_ctx_t c, const cgm_complex64* gamm
   bs.chi = chi_stride;
   bs.y = n;
   bs.T = (long)c->N * c->M;
+  if (small_matvec<float>(c->plan))
+    return launch_small<float, float2>(c->plan, c->stream, (const float2*)x, chi, (const float2*)gamma, (float2*)y,
+                                       mode, c->tw32, batch, bs);
   int rc = launch_pass1<float>(c->plan, c->stream, (const float2*)x, nullptr, chi, nullptr, mode, Tm, c->tw32,
                                nullptr, batch, bs);
   if (!rc) rc = launch_pass2<float, float2>(c->plan, c->stream, Tm, (const float2*)gamma, c->tw32, nullptr, batch, bs);

@@ -14,7 +14,13 @@
 //                       by Ghat[:, c], inverse FFT, keep rows < N -> T[:, c]
 //   pass 3  row i < N:  inverse FFT of T[i, :], crop to N, scale 1/M^2 and
 //                       combine with x (and b for a residual) -> y[i, :]
-// T is N x M row-major (complex), so only N of the M rows are ever stored.
+// T is N x M in column panels (tpos), so only N of the M rows are ever stored.
+//
+// The passes hold their transforms in registers and cross threads through LDS
+// between stages only (cgm_fft.h): S stages take S - 1 exchanges, where transforms
+// kept in LDS took S + 1.  N = 301, two vectors: 33.4 -> 24.1 us; N = 512, 16
+// vectors: 124 -> 107 us (20 + 58 + 25; pass 2 is bound by its vector
+// arithmetic, about 40 us at full issue, passes 1 and 3 by memory).
 #include <math.h>
 #include <string.h>
 
@@ -30,13 +36,24 @@ namespace cgm {
 // Work-group bound: float kernels accept tiles up to 1024 threads (autotuned
 // rows/columns per work-group); double kernels keep the tighter bound that
 // avoids register spills of the FP64 transforms.
-template <typename T, int M> struct PassWG {
-  static constexpr int value =
-      (sizeof(T) == 4 && FftShape<M>::pow2) ? (FftShape<M>::WG > 1024 ? FftShape<M>::WG : 1024) : FftShape<M>::WG;
+// Elements per thread of the pass kernels: 16 saves one of four stages at 2048
+// and 4096 points in single precision (N = 1024, four vectors: 128 against 157
+// us); at 128-512 points the fewer waves cost more (N = 128, one vector: 15.1
+// against 11.0 us), and so do the registers of 16 double elements (N = 1024:
+// 90.6 against 82.7 us) and of 24 elements at 3 * 2^k (N = 384: 50.8 against 38.3 us).
+template <typename T, int M> constexpr int kPassE = sizeof(T) == 4 && (M == 2048 || M == 4096) ? 16 : kFftE<M>;
+// At M = 1024 in single precision both 8 and 16 pay, by pass and batch (the
+// autotuner's radix plan): with 16 a transform is one wave (radices 16, 8, 8),
+// with 8 two waves and a stage more.
+constexpr int kWideE = 16;
+template <typename T, int M, int E> struct PassWG {
+  using Shape = FftShape<M, E>;
+  static constexpr int want = sizeof(T) == 8 ? 0 : E == 8 ? 1024 : 0;
+  static constexpr int value = Shape::WG > want ? Shape::WG : want;
 };
 
-template <typename T, int M>
-__global__ void __launch_bounds__((PassWG<T, M>::value))
+template <typename T, int M, int E>
+__global__ void __launch_bounds__((PassWG<T, M, E>::value))
 k_pass1(const cplx<T>* __restrict__ x, cplx<T>* xw, const T* __restrict__ chi,
         const double* __restrict__ norm_ptr, int mode, cplx<T>* __restrict__ Tm, int N,
         int rows_per_wg, const cplx<T>* __restrict__ tw, const int* __restrict__ done, BatchStrides bs) {
@@ -52,24 +69,24 @@ k_pass1(const cplx<T>* __restrict__ x, cplx<T>* xw, const T* __restrict__ chi,
   const int dn = done ? *done : 0;  // tested once the row loads are in flight
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* smem = reinterpret_cast<cplx<T>*>(smem_raw);
-  constexpr int NT = FftShape<M>::NT;
-  constexpr int EPT = FftShape<M>::EPT;
+  constexpr int NT = FftShape<M, E>::NT;
+  constexpr int EPT = E;
   const int t = threadIdx.x % NT;
   const int rl = threadIdx.x / NT;
   const int row = blockIdx.x * rows_per_wg + rl;
-  constexpr int ML = LdsLen<T, M>::value;
-  cplx<T>* buf = smem + rl * ML;
+  cplx<T>* buf = smem + rl * LdsLen<M>::value;
   const bool live = row < N;
   const long rb = (long)row * N;
   const bool mul = mode == kModeForward || mode == kModeResidual;
-  FftTwiddles<T, M> tws;
+  FftTwiddles<T, M, E> tws;
   tws.load(tw, t);
-  cplx<T> xv[EPT];
-  T cv[EPT];
+  // the row is zero from N <= M/2 on: registers EPT/2 .. stay unused
+  cplx<T> v[EPT];
+  T cv[EPT / 2];
 #pragma unroll
-  for (int k = 0; k < EPT; ++k) {
+  for (int k = 0; k < EPT / 2; ++k) {
     const int e = t + k * NT;
-    xv[k] = (live && e < N) ? x[rb + e] : mk(T(0), T(0));
+    v[k] = (live && e < N) ? x[rb + e] : mk(T(0), T(0));
     cv[k] = (live && e < N && mul) ? chi[rb + e] : T(1);
   }
   if (dn) return;
@@ -79,24 +96,23 @@ k_pass1(const cplx<T>* __restrict__ x, cplx<T>* xw, const T* __restrict__ chi,
     s = nv > 0.0 ? T(1.0 / nv) : T(0);
   }
 #pragma unroll
-  for (int k = 0; k < EPT; ++k) {
+  for (int k = 0; k < EPT / 2; ++k) {
     const int e = t + k * NT;
-    cplx<T> v = xv[k];
     if (norm_ptr) {
-      v = cscale(v, s);
-      if (xw && live && e < N) xw[rb + e] = v;
+      v[k] = cscale(v[k], s);
+      if (xw && live && e < N) xw[rb + e] = v[k];
     }
-    if (e < fft_lo_read_end<M>()) buf[lpad<T>(e)] = mul ? cscale(v, cv[k]) : v;
+    if (mul) v[k] = cscale(v[k], cv[k]);
   }
-  __syncthreads();
-  lds_fft<T, M, -1, true>(buf, tws, t);  // the row is zero from N <= M/2 on
+  reg_fft<T, M, -1, true, false, E>(v, buf, tws, t);
   if (live) {
-    for (int e = t; e < M; e += NT) Tm[tpos(row, e, N)] = buf[lpad<T>(e)];
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) Tm[tpos(row, t + k * NT, N)] = v[k];
   }
 }
 
-template <typename T, typename G, int M>
-__global__ void __launch_bounds__((PassWG<T, M>::value))
+template <typename T, typename G, int M, int E>
+__global__ void __launch_bounds__((PassWG<T, M, E>::value))
 k_pass2(cplx<T>* __restrict__ Tm, const G* __restrict__ gq, int N, int cols_per_wg,
         const cplx<T>* __restrict__ tw, const int* __restrict__ done, BatchStrides bs) {
   Tm += (long)blockIdx.y * bs.T;
@@ -104,20 +120,21 @@ k_pass2(cplx<T>* __restrict__ Tm, const G* __restrict__ gq, int N, int cols_per_
   const int dn = done ? *done : 0;  // tested once the column loads are in flight
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* smem = reinterpret_cast<cplx<T>*>(smem_raw);
-  constexpr int NT = FftShape<M>::NT;
+  constexpr int NT = FftShape<M, E>::NT;
+  constexpr int EPT = E;
   constexpr int H = M / 2 + 1;
-  constexpr int ML = LdsLen<T, M>::value;
+  constexpr int ML = LdsLen<M>::value;
   const int grp = xcd_tile(blockIdx.x, gridDim.x);
   const int c0 = grp * cols_per_wg;
   const int nthr = blockDim.x;  // cols_per_wg * NT
-  FftTwiddles<T, M> tws;
-  tws.load(tw, threadIdx.x % NT);
-  // gather the column tile: consecutive threads read consecutive columns.
-  // Single precision: N <= M/2 + 1, so each thread gathers at most EPT/2 + 1
-  // values into registers before the done test; double precision (whose
-  // registers are spoken for) tests first and gathers straight to LDS.
-  if constexpr (sizeof(T) == 4) {
-    constexpr int GR = FftShape<M>::EPT / 2 + 1;
+  const int t = threadIdx.x % NT;
+  const int cl = threadIdx.x / NT;
+  FftTwiddles<T, M, E> tws;
+  tws.load(tw, t);
+  // gather the column tile: consecutive threads read consecutive columns; N <=
+  // M/2, so each thread gathers at most EPT/2 values
+  constexpr int GR = EPT / 2;
+  {
     cplx<T> gv[GR];
 #pragma unroll
     for (int k = 0; k < GR; ++k) {
@@ -133,342 +150,58 @@ k_pass2(cplx<T>* __restrict__ Tm, const G* __restrict__ gq, int N, int cols_per_
       const int idx = threadIdx.x + k * nthr;
       if (idx < N * cols_per_wg) {
         const int r = idx / cols_per_wg, c = idx - r * cols_per_wg;
-        smem[c * ML + lpad<T>(r)] = gv[k];
+        smem[c * ML + lpad(r)] = gv[k];
       }
     }
-  } else {
-    if (dn) return;
-    for (int idx = threadIdx.x; idx < N * cols_per_wg; idx += nthr) {
-      const int r = idx / cols_per_wg, c = idx - r * cols_per_wg;
-      smem[c * ML + lpad<T>(r)] = Tm[tpos(r, c0 + c, N)];
-    }
   }
-  for (int idx = threadIdx.x; idx < (fft_lo_read_end<M>() - N) * cols_per_wg; idx += nthr) {
-    const int r = N + idx / cols_per_wg, c = idx % cols_per_wg;
-    smem[c * ML + lpad<T>(r)] = mk(T(0), T(0));
-  }
-  __syncthreads();
-  const int t = threadIdx.x % NT;
-  const int cl = threadIdx.x / NT;
-  cplx<T>* buf = smem + cl * ML;
-  lds_fft<T, M, -1, true>(buf, tws, t);  // rows N.. are zero
+  // the column's multipliers, loaded ahead of the transform
   const int col = c0 + cl;
   const int cq = col <= M - col ? col : M - col;
   const G* grow = gq + (long)cq * H;
-  for (int e = t; e < M; e += NT) {
-    const int fr = e <= M - e ? e : M - e;
-    const G g = grow[fr];
-    buf[lpad<T>(e)] = cmul(buf[lpad<T>(e)], mk(T(g.x), T(g.y)));
-  }
-  __syncthreads();
-  lds_fft<T, M, +1, false, true>(buf, tws, t);  // rows < N are kept
-  for (int idx = threadIdx.x; idx < N * cols_per_wg; idx += nthr) {
-    const int r = idx / cols_per_wg, c = idx - r * cols_per_wg;
-    Tm[tpos(r, c0 + c, N)] = smem[c * ML + lpad<T>(r)];
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Register-resident 1024-point transforms, one wave per transform (complex64,
-// M = 1024; the autotuner chooses them per pass and batch size).  Lane l
-// holds element l + 64 q in register q (q < 16), and the transform is the
-// Stockham sequence of radices 16, 16, 4:
-//   stage 0: a 16-point DFT over the registers, written to LDS as x[16 l + r];
-//   stage 1: reads x[l + 64 r], twiddles exp(s 2 pi i r (l % 16) / 256),
-//            16-point DFT, writes x[256 (l / 16) + l % 16 + 16 r];
-//   stage 2: butterflies j = l + 64 b (b < 4) read x[j + 256 r], twiddles
-//            exp(s 2 pi i r j / 1024), 4-point DFT; X[j + 256 r] stays in
-//            register b + 4 r, i.e. X[l + 64 q] in register q again.
-// The forward output is therefore the inverse's input layout, and the column
-// pass multiplies by the spectrum in registers between the two.  Two LDS
-// exchanges per transform, in the wave's own region of kWL elements with one
-// pad element after every 16: every access pattern above then falls in
-// distinct banks within each group of 16 lanes.  A wave orders its own LDS
-// accesses, so a transform needs no work-group barrier.
-// ---------------------------------------------------------------------------
-constexpr int kWL = 1024 + 1024 / 16;  // LDS elements per wave
-__device__ inline int wpad(int e) { return e + (e >> 4); }
-
-// Orders one wave's LDS writes before its later reads (no instruction: the
-// wave's LDS accesses complete in issue order; this keeps the compiler from
-// moving them across).
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// a * exp(SIGN 2 pi i Q / 16)
-template <int SIGN, int Q>
-__device__ inline float2 rot16(float2 a) {
-  constexpr float h = 0.70710678118654752440f;
-  constexpr float c1 = 0.92387953251128675613f, s1 = 0.38268343236508977173f;  // cos, sin of pi/8
-  if constexpr (Q == 4) {
-    return mul_si<float, SIGN>(a);
-  } else if constexpr (Q == 2) {
-    return make_float2(h * (a.x - SIGN * a.y), h * (a.y + SIGN * a.x));
-  } else if constexpr (Q == 6) {
-    return make_float2(-h * (a.x + SIGN * a.y), h * (SIGN * a.x - a.y));
-  } else if constexpr (Q == 1) {
-    return cmul(a, make_float2(c1, SIGN * s1));
-  } else if constexpr (Q == 3) {
-    return cmul(a, make_float2(s1, SIGN * c1));
-  } else {
-    static_assert(Q == 9, "twiddles of the 16-point DFT");
-    return cmul(a, make_float2(-c1, -SIGN * s1));
-  }
-}
-
-// v[k] <- sum_n v[n] exp(SIGN 2 pi i n k / 16) with n = 4 m + p: four 4-point
-// DFTs over m, the twiddles exp(SIGN 2 pi i p k1 / 16), then four 4-point DFTs
-// over p give X[k1 + 4 k2].  LO: v[8 ..] are zero and not read.
-template <int SIGN, bool LO>
-__device__ inline void dft16(float2* v) {
-  float2 a[4][4];
+  G g[EPT];
+  const auto load_g = [&] {
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-#pragma unroll
-    for (int m = 0; m < (LO ? 2 : 4); ++m) a[p][m] = v[4 * m + p];
-    if constexpr (LO)
-      dft4_lo<float, SIGN>(a[p]);
-    else
-      dft4<float, SIGN>(a[p]);
-  }
-  a[1][1] = rot16<SIGN, 1>(a[1][1]);
-  a[1][2] = rot16<SIGN, 2>(a[1][2]);
-  a[1][3] = rot16<SIGN, 3>(a[1][3]);
-  a[2][1] = rot16<SIGN, 2>(a[2][1]);
-  a[2][2] = rot16<SIGN, 4>(a[2][2]);
-  a[2][3] = rot16<SIGN, 6>(a[2][3]);
-  a[3][1] = rot16<SIGN, 3>(a[3][1]);
-  a[3][2] = rot16<SIGN, 6>(a[3][2]);
-  a[3][3] = rot16<SIGN, 9>(a[3][3]);
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1) {
-    float2 b[4] = {a[0][k1], a[1][k1], a[2][k1], a[3][k1]};
-    dft4<float, SIGN>(b);
-#pragma unroll
-    for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = b[k2];
-  }
-}
-
-// The twiddles of lane l for stages 1 and 2 (forward sign; the inverse uses
-// their conjugates), from the table tw[q] = exp(-2 pi i q / 1024).
-struct WaveTw {
-  float2 s1[15];  // r = 1..15: exp(-2 pi i r (l % 16) / 256)
-  float2 s2[12];  // b = 0..3, r = 1..3 at 3 b + r - 1: exp(-2 pi i r (l + 64 b) / 1024)
-  __device__ inline void load(const float2* __restrict__ tw, int l) {
-    const int k = l & 15;
-#pragma unroll
-    for (int r = 1; r < 16; ++r) s1[r - 1] = tw[4 * r * k];
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int r = 1; r < 4; ++r) s2[3 * b + r - 1] = tw[r * (l + 64 * b)];
-  }
-};
-
-template <int SIGN>
-__device__ inline float2 twid(float2 a, float2 w) {
-  if (SIGN > 0) w.y = -w.y;
-  return cmul(a, w);
-}
-
-// Stages 0 and 1 of a transform of v (in the register layout above); on
-// return stage 1's output is in X.  LO: v[8 ..] are zero and not read.
-template <int SIGN, bool LO>
-__device__ inline void wfft_head(float2* v, float2* __restrict__ X, const WaveTw& w, int l) {
-  dft16<SIGN, LO>(v);
-#pragma unroll
-  for (int r = 0; r < 16; ++r) X[wpad(16 * l + r)] = v[r];
-  wave_lds_sync();
-#pragma unroll
-  for (int r = 0; r < 16; ++r) v[r] = X[wpad(l + 64 * r)];
-#pragma unroll
-  for (int r = 1; r < 16; ++r) v[r] = twid<SIGN>(v[r], w.s1[r - 1]);
-  dft16<SIGN, false>(v);
-  const int base = 256 * (l >> 4) + (l & 15);
-#pragma unroll
-  for (int r = 0; r < 16; ++r) X[wpad(base + 16 * r)] = v[r];
-  wave_lds_sync();
-}
-
-// Forward transform; v[q] = x[l + 64 q] with x[n] = 0 for n >= 512 (v[8 ..]
-// not read) becomes v[q] = X[l + 64 q] for all 16 q.
-__device__ inline void wfft_fwd_lo(float2* v, float2* __restrict__ X, const WaveTw& w, int l) {
-  wfft_head<-1, true>(v, X, w, l);
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    float2 u[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) u[r] = X[wpad(l + 64 * b + 256 * r)];
-#pragma unroll
-    for (int r = 1; r < 4; ++r) u[r] = twid<-1>(u[r], w.s2[3 * b + r - 1]);
-    dft4<float, -1>(u);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[b + 4 * r] = u[r];
-  }
-  wave_lds_sync();
-}
-
-// Inverse (unnormalised) transform of v[q] = Y[l + 64 q]; only the outputs
-// below 512 are formed: v[q] = y[l + 64 q] for q < 8.
-__device__ inline void wfft_inv_hi(float2* v, float2* __restrict__ X, const WaveTw& w, int l) {
-  wfft_head<1, false>(v, X, w, l);
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    float2 u[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) u[r] = X[wpad(l + 64 * b + 256 * r)];
-#pragma unroll
-    for (int r = 1; r < 4; ++r) u[r] = twid<1>(u[r], w.s2[3 * b + r - 1]);
-    dft4<float, 1>(u);
-    v[b] = u[0];
-    v[b + 4] = u[1];
-  }
-  wave_lds_sync();
-}
-
-// Pass 2, M = 1024: a work-group of four waves takes half a column panel
-// (N rows x 4 columns, kPW / 2 contiguous values per row), staged through LDS
-// with a row stride of 5 values for coalesced global accesses; wave g then
-// transforms column g of it forward, multiplies by the spectrum column and
-// transforms back, keeping rows < N.
-template <typename G>
-__global__ void __launch_bounds__(256)
-k_pass2w(float2* __restrict__ Tm, const G* __restrict__ gq, int N, const float2* __restrict__ tw,
-         const int* __restrict__ done, BatchStrides bs) {
-  constexpr int M = 1024;
-  constexpr int H = M / 2 + 1;
-  constexpr int kC = kPW / 2;  // columns per work-group
-  constexpr int kRS = kC + 1;  // staging row stride
-  static_assert(512 * kRS <= 4 * kWL, "the staged half panel fits the work-group's LDS");
-  __shared__ float2 lds[4 * kWL];
-  Tm += (long)blockIdx.y * bs.T;
-  done = boff(done, (long)blockIdx.y * bs.st);
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int panel = tile >> 1;
-  const int grp = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int col = tile * kC + grp;
-  WaveTw w;
-  w.load(tw, lane);
-  float2* S = lds;
-  float2* g0 = Tm + (long)panel * N * kPW + (tile & 1) * kC;
-  for (int e = threadIdx.x; e < N * kC; e += 256) S[(e >> 2) * kRS + (e & 3)] = g0[(long)(e >> 2) * kPW + (e & 3)];
-  __syncthreads();
-  if (done && *done) return;  // uniform over the work-group
-  float2 v[16];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int n = lane + 64 * q;
-    v[q] = n < N ? S[n * kRS + grp] : make_float2(0.f, 0.f);
-  }
-  __syncthreads();  // the staging area is reused by the transforms
-  float2* X = lds + grp * kWL;
-  wfft_fwd_lo(v, X, w, lane);
-  const int cq = col <= M - col ? col : M - col;
-  const G* grow = gq + (long)cq * H;
-#pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int k = lane + 64 * q;
-    const G g = grow[k <= M - k ? k : M - k];
-    v[q] = cmul(v[q], make_float2((float)g.x, (float)g.y));
-  }
-  wfft_inv_hi(v, X, w, lane);
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int n = lane + 64 * q;
-    if (n < N) S[n * kRS + grp] = v[q];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < N * kC; e += 256) g0[(long)(e >> 2) * kPW + (e & 3)] = S[(e >> 2) * kRS + (e & 3)];
-}
-
-// Passes 1 and 3 for M = 1024 with the same transforms: one wave per row,
-// four rows per work-group.  Pass 1 loads row i of chi .* x (lane l, register
-// q: element l + 64 q), transforms it forward and writes T[i][l + 64 q].
-// Pass 3 reads that layout, transforms it back, and lane l combines element
-// l + 64 q of the row with x.  Only the plain operator modes (y = x - G(chi x),
-// x - chi G(x), G x) without input scaling take these kernels.
-__global__ void __launch_bounds__(256)
-k_pass1w(const float2* __restrict__ x, const float* __restrict__ chi, int mul, float2* __restrict__ Tm, int N,
-         const float2* __restrict__ tw, const int* __restrict__ done, BatchStrides bs) {
-  __shared__ float2 lds[4 * kWL];
-  {
-    const long kb = blockIdx.y;
-    x += kb * bs.x;
-    if (chi) chi += kb * bs.chi;
-    Tm += kb * bs.T;
-    done = boff(done, kb * bs.st);
-  }
-  const int grp = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + grp;
-  if (row >= N) return;  // no work-group barriers below
-  const long rb = (long)row * N;
-  WaveTw w;
-  w.load(tw, lane);
-  float2 v[16];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int n = lane + 64 * q;
-    float2 e = make_float2(0.f, 0.f);
-    if (n < N) {
-      e = x[rb + n];
-      if (mul) {
-        const float c = chi[rb + n];
-        e.x *= c;
-        e.y *= c;
-      }
+    for (int k = 0; k < EPT; ++k) {
+      const int e = t + k * NT;
+      g[k] = grow[e <= M - e ? e : M - e];
     }
-    v[q] = e;
+  };
+  if constexpr (!FftTwiddles<T, M, E>::late) load_g();  // else the registers are worth more than the latency
+  __syncthreads();
+  cplx<T>* buf = smem + cl * ML;
+  cplx<T> v[EPT];
+#pragma unroll
+  for (int k = 0; k < EPT / 2; ++k) {
+    const int e = t + k * NT;
+    v[k] = e < N ? buf[lpad(e)] : mk(T(0), T(0));
   }
-  if (done && *done) return;
-  wfft_fwd_lo(v, lds + grp * kWL, w, lane);
+  FftSync<M, E>::stage();
+  reg_fft<T, M, -1, true, false, E>(v, buf, tws, t);  // rows N.. are zero
+  if constexpr (FftTwiddles<T, M, E>::late) load_g();
+  tws.refresh();
 #pragma unroll
-  for (int q = 0; q < 16; ++q) Tm[tpos(row, lane + 64 * q, N)] = v[q];
-}
-
-__global__ void __launch_bounds__(256)
-k_pass3w(const float2* __restrict__ Tm, const float2* __restrict__ x, const float* __restrict__ chi,
-         float2* __restrict__ y, int mode, int N, float inv, const float2* __restrict__ tw,
-         const int* __restrict__ done, BatchStrides bs) {
-  __shared__ float2 lds[4 * kWL];
-  {
-    const long kb = blockIdx.y;
-    Tm += kb * bs.T;
-    x += kb * bs.x;
-    if (chi) chi += kb * bs.chi;
-    y += kb * bs.y;
-    done = boff(done, kb * bs.st);
+  for (int k = 0; k < EPT; ++k) v[k] = cmul(v[k], mk(T(g[k].x), T(g[k].y)));
+  FftSync<M, E>::stage();
+  reg_fft<T, M, +1, false, true, E>(v, buf, tws, t);  // rows < N are kept
+  FftSync<M, E>::stage();
+#pragma unroll
+  for (int k = 0; k < EPT / 2; ++k) {
+    const int e = t + k * NT;
+    if (e < N) buf[lpad(e)] = v[k];
   }
-  const int grp = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + grp;
-  if (row >= N) return;  // no work-group barriers below
-  WaveTw w;
-  w.load(tw, lane);
-  float2 v[16];
+  __syncthreads();
 #pragma unroll
-  for (int q = 0; q < 16; ++q) v[q] = Tm[tpos(row, lane + 64 * q, N)];
-  if (done && *done) return;
-  wfft_inv_hi(v, lds + grp * kWL, w, lane);
-  const long rb = (long)row * N;
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int n = lane + 64 * q;
-    if (n < N) {
-      const float2 g = cscale(v[q], inv);
-      float2 o;
-      if (mode == kModeForward) o = csub(x[rb + n], g);
-      else if (mode == kModeAdjoint) o = csub(x[rb + n], cscale(g, chi[rb + n]));
-      else o = g;
-      y[rb + n] = o;
+  for (int k = 0; k < GR; ++k) {
+    const int idx = threadIdx.x + k * nthr;
+    if (idx < N * cols_per_wg) {
+      const int r = idx / cols_per_wg, c = idx - r * cols_per_wg;
+      Tm[tpos(r, c0 + c, N)] = smem[c * ML + lpad(r)];
     }
   }
 }
 
-template <typename T, int M>
-__global__ void __launch_bounds__((PassWG<T, M>::value))
+template <typename T, int M, int E>
+__global__ void __launch_bounds__((PassWG<T, M, E>::value))
 k_pass3(const cplx<T>* __restrict__ Tm, const cplx<T>* __restrict__ x, const T* __restrict__ chi,
         const cplx<T>* __restrict__ b, cplx<T>* __restrict__ y, int mode, int N, int rows_per_wg,
         T inv, const cplx<T>* __restrict__ tw, const int* __restrict__ done, BatchStrides bs) {
@@ -481,25 +214,30 @@ k_pass3(const cplx<T>* __restrict__ Tm, const cplx<T>* __restrict__ x, const T* 
     y += k * bs.y;
     done = boff(done, k * bs.st);
   }
-  if (done && *done) return;
+  const int dn = done ? *done : 0;  // tested once the row loads are in flight
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* smem = reinterpret_cast<cplx<T>*>(smem_raw);
-  constexpr int NT = FftShape<M>::NT;
+  constexpr int NT = FftShape<M, E>::NT;
+  constexpr int EPT = E;
   const int t = threadIdx.x % NT;
   const int rl = threadIdx.x / NT;
   const int row = blockIdx.x * rows_per_wg + rl;
-  constexpr int ML = LdsLen<T, M>::value;
-  cplx<T>* buf = smem + rl * ML;
+  cplx<T>* buf = smem + rl * LdsLen<M>::value;
   const bool live = row < N;
-  FftTwiddles<T, M> tws;
+  FftTwiddles<T, M, E> tws;
   tws.load(tw, t);
-  for (int e = t; e < M; e += NT) buf[lpad<T>(e)] = live ? Tm[tpos(row, e, N)] : mk(T(0), T(0));
-  __syncthreads();
-  lds_fft<T, M, +1, false, true>(buf, tws, t);  // columns < N are used
+  cplx<T> v[EPT];
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) v[k] = live ? Tm[tpos(row, t + k * NT, N)] : mk(T(0), T(0));
+  if (dn) return;
+  reg_fft<T, M, +1, false, true, E>(v, buf, tws, t);  // columns < N are used
   if (!live) return;
   const long rb = (long)row * N;
-  for (int e = t; e < N; e += NT) {
-    const cplx<T> g = cscale(buf[lpad<T>(e)], inv);
+#pragma unroll
+  for (int k = 0; k < EPT / 2; ++k) {
+    const int e = t + k * NT;
+    if (e >= N) continue;
+    const cplx<T> g = cscale(v[k], inv);
     cplx<T> o;
     switch (mode) {
       case kModeForward: o = csub(x[rb + e], g); break;
@@ -512,45 +250,197 @@ k_pass3(const cplx<T>* __restrict__ Tm, const cplx<T>* __restrict__ x, const T* 
   }
 }
 
+// ---------------------------------------------------------------------------
+// The whole product in one launch, for grids whose M x M embedding fits the
+// LDS of one work-group with room to spare (complex64: M <= 96, i.e. N <= 48;
+// complex128: M <= 64).
+// Work-group blockIdx.x takes vector blockIdx.x through the three passes with T
+// in LDS: element (r, c) at r * RS + r / 8 + c + c / 8, whose pads keep the
+// stage-0 writes (stride 8) of rows and columns off each other's banks.  Every
+// transform lies in one wave (FftSync), so the work-group meets only between the
+// passes.  The transforms are those of k_pass1..3: results are equal bit for bit.
+//
+// Such a product is a chain of latencies: three launches that each wait for the
+// one before, with a few work-groups each.  N = 24, one vector: 6.5 us instead of
+// 12.1 (FP64: 7.0 instead of 13.6); N = 48, four vectors: 12.4 instead of 13.3.
+// At M = 128 one CU's LDS traffic costs more than the launches (N = 64, one
+// vector: 14.5 against 10.6 us).
+// ---------------------------------------------------------------------------
+template <int M> struct SmallShape {
+  static constexpr int E = kFftE<M>;
+  static constexpr int NT = FftShape<M, E>::NT;
+  static constexpr int want = M * NT < 64 ? 64 : (M * NT + 63) / 64 * 64;
+  static constexpr int BS = want > 1024 ? 1024 : want;
+  static constexpr int RS = M + M / 8 + 1;
+  static constexpr int len = M * RS + M / 8;  // elements of T
+};
+struct LdsGridRow {
+  __device__ inline int operator()(int e) const { return e + (e >> 3); }
+};
+template <int RS> struct LdsGridCol {
+  __device__ inline int operator()(int e) const { return e * RS + (e >> 3); }
+};
+
+template <typename T, typename G, int M>
+__global__ void __launch_bounds__(SmallShape<M>::BS)
+k_matvec_small(const cplx<T>* __restrict__ x, const T* __restrict__ chi, const G* __restrict__ gq,
+               cplx<T>* __restrict__ y, int mode, int N, T inv, const cplx<T>* __restrict__ tw, BatchStrides bs) {
+  using S = SmallShape<M>;
+  constexpr int E = S::E, NT = S::NT, EPT = E, PER = S::BS / NT, RS = S::RS, H = M / 2 + 1;
+  __shared__ __align__(16) cplx<T> buf[S::len];
+  static_assert(FftSync<M, E>::one_wave, "one wave per transform");
+  x += (long)blockIdx.x * bs.x;
+  if (chi) chi += (long)blockIdx.x * bs.chi;
+  y += (long)blockIdx.x * bs.y;
+  const int t = threadIdx.x % NT, l = threadIdx.x / NT;
+  const bool mul = mode == kModeForward;
+  FftTwiddles<T, M, E> tws;
+  tws.load(tw, t);
+  // rows i < N: chi .* x, forward
+  for (int r0 = 0; r0 < N; r0 += PER) {
+    const int r = r0 + l;
+    const bool live = r < N;
+    cplx<T>* row = buf + r * RS + (r >> 3);
+    cplx<T> v[EPT];
+#pragma unroll
+    for (int k = 0; k < EPT / 2; ++k) {
+      const int e = t + k * NT;
+      const bool in = live && e < N;
+      v[k] = in ? x[(long)r * N + e] : mk(T(0), T(0));
+      if (mul && in) v[k] = cscale(v[k], chi[(long)r * N + e]);
+    }
+    reg_fft<T, M, -1, true, false, E>(v, row, tws, t, live, LdsGridRow());
+    FftSync<M, E>::stage();
+    if (live) {
+#pragma unroll
+      for (int k = 0; k < EPT; ++k) row[LdsGridRow()(t + k * NT)] = v[k];
+    }
+  }
+  __syncthreads();
+  // columns: forward, times the spectrum, inverse
+  for (int c0 = 0; c0 < M; c0 += PER) {
+    const int c = c0 + l;
+    const bool live = c < M;
+    cplx<T>* col = buf + c + (c >> 3);
+    const int cq = c <= M - c ? c : M - c;
+    G g[EPT];
+    cplx<T> v[EPT];
+    if (live) {
+#pragma unroll
+      for (int k = 0; k < EPT; ++k) {
+        const int e = t + k * NT;
+        g[k] = gq[(long)cq * H + (e <= M - e ? e : M - e)];
+      }
+#pragma unroll
+      for (int k = 0; k < EPT / 2; ++k) {
+        const int e = t + k * NT;
+        v[k] = e < N ? col[LdsGridCol<RS>()(e)] : mk(T(0), T(0));
+      }
+    }
+    FftSync<M, E>::stage();
+    reg_fft<T, M, -1, true, false, E>(v, col, tws, t, live, LdsGridCol<RS>());
+    if (live) {
+#pragma unroll
+      for (int k = 0; k < EPT; ++k) v[k] = cmul(v[k], mk(T(g[k].x), T(g[k].y)));
+    }
+    FftSync<M, E>::stage();
+    reg_fft<T, M, +1, false, true, E>(v, col, tws, t, live, LdsGridCol<RS>());
+    FftSync<M, E>::stage();
+    if (live) {
+#pragma unroll
+      for (int k = 0; k < EPT / 2; ++k) {
+        const int e = t + k * NT;
+        if (e < N) col[LdsGridCol<RS>()(e)] = v[k];
+      }
+    }
+  }
+  __syncthreads();
+  // rows: inverse, crop, scale, combine with x
+  for (int r0 = 0; r0 < N; r0 += PER) {
+    const int r = r0 + l;
+    const bool live = r < N;
+    cplx<T>* row = buf + r * RS + (r >> 3);
+    const long rb = (long)r * N;
+    cplx<T> v[EPT], xv[EPT / 2];
+    T cv[EPT / 2];
+#pragma unroll
+    for (int k = 0; k < EPT / 2; ++k) {
+      const int e = t + k * NT;
+      const bool in = live && e < N;
+      xv[k] = in && mode != kModeGreen ? x[rb + e] : mk(T(0), T(0));
+      cv[k] = in && mode == kModeAdjoint ? chi[rb + e] : T(1);
+    }
+    if (live) {
+#pragma unroll
+      for (int k = 0; k < EPT; ++k) v[k] = row[LdsGridRow()(t + k * NT)];
+    }
+    FftSync<M, E>::stage();
+    reg_fft<T, M, +1, false, true, E>(v, row, tws, t, live, LdsGridRow());
+#pragma unroll
+    for (int k = 0; k < EPT / 2; ++k) {
+      const int e = t + k * NT;
+      if (!live || e >= N) continue;
+      const cplx<T> g = cscale(v[k], inv);
+      cplx<T> o = g;
+      if (mode == kModeForward) o = csub(xv[k], g);
+      else if (mode == kModeAdjoint) o = csub(xv[k], cscale(g, cv[k]));
+      y[rb + e] = o;
+    }
+  }
+}
+
 // Full-size 2-D FFT helpers for the one-off spectrum precompute (FP64).
 template <typename T, int M, int SIGN>
-__global__ void __launch_bounds__(FftShape<M>::WG)
+__global__ void __launch_bounds__((FftShape<M, kFftE<M>>::WG))
 k_fft_rows(cplx<T>* __restrict__ data, int rows, int rows_per_wg, const cplx<T>* __restrict__ tw) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* smem = reinterpret_cast<cplx<T>*>(smem_raw);
-  constexpr int NT = FftShape<M>::NT;
+  constexpr int NT = FftShape<M, kFftE<M>>::NT;
+  constexpr int EPT = FftShape<M, kFftE<M>>::EPT;
   const int t = threadIdx.x % NT, rl = threadIdx.x / NT;
   const int row = blockIdx.x * rows_per_wg + rl;
-  cplx<T>* buf = smem + rl * M;
   const bool live = row < rows;
   FftTwiddles<T, M> tws;
   tws.load(tw, t);
-  for (int e = t; e < M; e += NT) buf[e] = live ? data[(long)row * M + e] : mk(T(0), T(0));
-  __syncthreads();
-  lds_fft<T, M, SIGN>(buf, tws, t);
+  cplx<T> v[EPT];
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) v[k] = live ? data[(long)row * M + t + k * NT] : mk(T(0), T(0));
+  reg_fft<T, M, SIGN>(v, smem + rl * LdsLen<M>::value, tws, t);
   if (live)
-    for (int e = t; e < M; e += NT) data[(long)row * M + e] = buf[e];
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) data[(long)row * M + t + k * NT] = v[k];
 }
 
 template <typename T, int M, int SIGN>
-__global__ void __launch_bounds__(FftShape<M>::WG)
+__global__ void __launch_bounds__((FftShape<M, kFftE<M>>::WG))
 k_fft_cols(cplx<T>* __restrict__ data, int cols_per_wg, const cplx<T>* __restrict__ tw) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* smem = reinterpret_cast<cplx<T>*>(smem_raw);
-  constexpr int NT = FftShape<M>::NT;
+  constexpr int NT = FftShape<M, kFftE<M>>::NT;
+  constexpr int EPT = FftShape<M, kFftE<M>>::EPT;
+  constexpr int ML = LdsLen<M>::value;
   const int c0 = blockIdx.x * cols_per_wg;
   for (int idx = threadIdx.x; idx < M * cols_per_wg; idx += blockDim.x) {
     const int r = idx / cols_per_wg, c = idx % cols_per_wg;
-    smem[c * M + r] = data[(long)r * M + c0 + c];
+    smem[c * ML + lpad(r)] = data[(long)r * M + c0 + c];
   }
   __syncthreads();
   const int t = threadIdx.x % NT, cl = threadIdx.x / NT;
   FftTwiddles<T, M> tws;
   tws.load(tw, t);
-  lds_fft<T, M, SIGN>(smem + cl * M, tws, t);
+  cplx<T>* buf = smem + cl * ML;
+  cplx<T> v[EPT];
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) v[k] = buf[lpad(t + k * NT)];
+  FftSync<M>::stage();
+  reg_fft<T, M, SIGN>(v, buf, tws, t);
+  FftSync<M>::stage();
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) buf[lpad(t + k * NT)] = v[k];
+  __syncthreads();
   for (int idx = threadIdx.x; idx < M * cols_per_wg; idx += blockDim.x) {
     const int r = idx / cols_per_wg, c = idx % cols_per_wg;
-    data[(long)r * M + c0 + c] = smem[c * M + r];
+    data[(long)r * M + c0 + c] = smem[c * ML + lpad(r)];
   }
 }
 
@@ -635,7 +525,17 @@ __global__ void k_quarter(const double2* __restrict__ E, G* __restrict__ gq, int
 
 int fft_threads(int M) {
   switch (M) {
-#define X(m) case m: return FftShape<m>::NT;
+#define X(m) case m: return FftShape<m, kFftE<m>>::NT;
+    CGM_FOR_EACH_M(X)
+#undef X
+  }
+  return 0;
+}
+
+// Threads of one transform in the pass kernels.
+int pass_threads(int M, bool fp64) {
+  switch (M) {
+#define X(m) case m: return fp64 ? FftShape<m, kPassE<double, m>>::NT : FftShape<m, kPassE<float, m>>::NT;
     CGM_FOR_EACH_M(X)
 #undef X
   }
@@ -645,7 +545,8 @@ int fft_threads(int M) {
 // Largest work-group (threads) the pass kernels of size M accept.
 int pass_max_threads(int M, bool fp64) {
   switch (M) {
-#define X(m) case m: return fp64 ? PassWG<double, m>::value : PassWG<float, m>::value;
+#define X(m) \
+  case m: return fp64 ? PassWG<double, m, kPassE<double, m>>::value : PassWG<float, m, kPassE<float, m>>::value;
     CGM_FOR_EACH_M(X)
 #undef X
   }
@@ -672,22 +573,22 @@ int launch_pass1(const Plan& P, hipStream_t st, const cplx<T>* x, cplx<T>* xw, c
                  int B, const BatchStrides& bs) {
   const int M = P.M, N = P.N;
   if constexpr (sizeof(T) == 4) {
-    if (M == 1024 && P.wide1_batch > 0 && B >= P.wide1_batch && !xw && !norm_ptr &&
-        (mode == kModeForward || mode == kModeAdjoint || mode == kModeGreen)) {
-      hipLaunchKernelGGL(k_pass1w, dim3((N + 3) / 4, B), dim3(256), 0, st, (const float2*)x, (const float*)chi,
-                         (int)(mode == kModeForward), (float2*)Tm, N, (const float2*)tw, done, bs);
+    if (M == 1024 && P.wide1_batch > 0 && B >= P.wide1_batch) {
+      constexpr int E = kWideE, R = 256 / FftShape<1024, E>::NT;
+      hipLaunchKernelGGL((k_pass1<T, 1024, E>), dim3((N + R - 1) / R, B), dim3(256),
+                         R * lds_len(M) * sizeof(cplx<T>), st, x, xw, chi, norm_ptr, mode, Tm, N, R, tw, done, bs);
       return hipGetLastError() == hipSuccess ? CGM_SUCCESS : CGM_ERROR_DEVICE;
     }
   }
   const int rows = P.rows1;
   const int grid = (N + rows - 1) / rows;
-  const int threads = rows * fft_threads(M);
-  const size_t lds = (size_t)rows * lds_len(M, sizeof(T) == 8) * sizeof(cplx<T>);
-  if (threads > pass_max_threads(M, sizeof(T) == 8) || lds > 65536) return CGM_ERROR_UNSUPPORTED;
+  const int threads = rows * pass_threads(M, sizeof(T) == 8);
+  const size_t lds = (size_t)rows * lds_len(M) * sizeof(cplx<T>);
+  if (threads > pass_max_threads(M, sizeof(T) == 8) || lds > kMaxLds) return CGM_ERROR_UNSUPPORTED;
   switch (M) {
 #define X(m)                                                                                 \
   case m:                                                                                    \
-    hipLaunchKernelGGL((k_pass1<T, m>), dim3(grid, B), dim3(threads), lds, st, x, xw, chi,   \
+    hipLaunchKernelGGL((k_pass1<T, m, kPassE<T, m>>), dim3(grid, B), dim3(threads), lds, st, x, xw, chi,   \
                        norm_ptr, mode, Tm, N, rows, tw, done, bs);                            \
     break;
     CGM_FOR_EACH_M(X)
@@ -703,20 +604,21 @@ int launch_pass2(const Plan& P, hipStream_t st, cplx<T>* Tm, const G* gq, const 
   const int M = P.M, N = P.N;
   if constexpr (sizeof(T) == 4) {
     if (M == 1024 && P.wide2_batch > 0 && B >= P.wide2_batch) {
-      hipLaunchKernelGGL((k_pass2w<G>), dim3(M / (kPW / 2), B), dim3(256), 0, st, (float2*)Tm, gq, N, (const float2*)tw,
-                         done, bs);
+      constexpr int E = kWideE, C = 256 / FftShape<1024, E>::NT;
+      hipLaunchKernelGGL((k_pass2<T, G, 1024, E>), dim3(M / C, B), dim3(C * FftShape<1024, E>::NT),
+                         C * lds_len(M) * sizeof(cplx<T>), st, Tm, gq, N, C, tw, done, bs);
       return hipGetLastError() == hipSuccess ? CGM_SUCCESS : CGM_ERROR_DEVICE;
     }
   }
   const int cols = P.cols2;
   const int grid = M / cols;
-  const int threads = cols * fft_threads(M);
-  const size_t lds = (size_t)cols * lds_len(M, sizeof(T) == 8) * sizeof(cplx<T>);
-  if (threads > pass_max_threads(M, sizeof(T) == 8) || lds > 65536 || M % cols) return CGM_ERROR_UNSUPPORTED;
+  const int threads = cols * pass_threads(M, sizeof(T) == 8);
+  const size_t lds = (size_t)cols * lds_len(M) * sizeof(cplx<T>);
+  if (threads > pass_max_threads(M, sizeof(T) == 8) || lds > kMaxLds || M % cols) return CGM_ERROR_UNSUPPORTED;
   switch (M) {
 #define X(m)                                                                                  \
   case m:                                                                                     \
-    hipLaunchKernelGGL((k_pass2<T, G, m>), dim3(grid, B), dim3(threads), lds, st, Tm, gq, N,    \
+    hipLaunchKernelGGL((k_pass2<T, G, m, kPassE<T, m>>), dim3(grid, B), dim3(threads), lds, st, Tm, gq, N,    \
                        cols, tw, done, bs);                                                   \
     break;
     CGM_FOR_EACH_M(X)
@@ -732,24 +634,24 @@ int launch_pass3(const Plan& P, hipStream_t st, const cplx<T>* Tm, const cplx<T>
                  int B, const BatchStrides& bs) {
   const int M = P.M, N = P.N;
   if constexpr (sizeof(T) == 4) {
-    if (M == 1024 && P.wide3_batch > 0 && B >= P.wide3_batch && !b &&
-        (mode == kModeForward || mode == kModeAdjoint || mode == kModeGreen)) {
-      hipLaunchKernelGGL(k_pass3w, dim3((N + 3) / 4, B), dim3(256), 0, st, (const float2*)Tm, (const float2*)x,
-                         (const float*)chi, (float2*)y, mode, N, (float)(1.0 / ((double)M * (double)M)),
-                         (const float2*)tw, done, bs);
+    if (M == 1024 && P.wide3_batch > 0 && B >= P.wide3_batch) {
+      constexpr int E = kWideE, R = 256 / FftShape<1024, E>::NT;
+      hipLaunchKernelGGL((k_pass3<T, 1024, E>), dim3((N + R - 1) / R, B), dim3(256),
+                         R * lds_len(M) * sizeof(cplx<T>), st, Tm, x, chi, b, y, mode, N, R,
+                         T(1.0 / ((double)M * (double)M)), tw, done, bs);
       return hipGetLastError() == hipSuccess ? CGM_SUCCESS : CGM_ERROR_DEVICE;
     }
   }
   const int rows = P.rows3;
   const int grid = (N + rows - 1) / rows;
-  const int threads = rows * fft_threads(M);
-  const size_t lds = (size_t)rows * lds_len(M, sizeof(T) == 8) * sizeof(cplx<T>);
-  if (threads > pass_max_threads(M, sizeof(T) == 8) || lds > 65536) return CGM_ERROR_UNSUPPORTED;
+  const int threads = rows * pass_threads(M, sizeof(T) == 8);
+  const size_t lds = (size_t)rows * lds_len(M) * sizeof(cplx<T>);
+  if (threads > pass_max_threads(M, sizeof(T) == 8) || lds > kMaxLds) return CGM_ERROR_UNSUPPORTED;
   const T inv = T(1.0 / ((double)M * (double)M));
   switch (M) {
 #define X(m)                                                                                   \
   case m:                                                                                      \
-    hipLaunchKernelGGL((k_pass3<T, m>), dim3(grid, B), dim3(threads), lds, st, Tm, x, chi, b,   \
+    hipLaunchKernelGGL((k_pass3<T, m, kPassE<T, m>>), dim3(grid, B), dim3(threads), lds, st, Tm, x, chi, b,   \
                        y, mode, N, rows, inv, tw, done, bs);                                   \
     break;
     CGM_FOR_EACH_M(X)
@@ -758,6 +660,38 @@ int launch_pass3(const Plan& P, hipStream_t st, const cplx<T>* Tm, const cplx<T>
   }
   return hipGetLastError() == hipSuccess ? CGM_SUCCESS : CGM_ERROR_DEVICE;
 }
+
+// y = A x, A^T x or G x of B vectors in one launch, where the grid is small
+// enough (small_matvec); modes FORWARD, ADJOINT, GREEN.  The embedding has to
+// fit the 160 KB of LDS of one work-group.  Within that, one launch is the
+// better form at every batch: it moves x, chi and y and nothing else.
+template <typename T>
+bool small_matvec(const Plan& P) {
+  return P.M <= (sizeof(T) == 4 ? 96 : 64);
+}
+template <typename T, typename G>
+int launch_small(const Plan& P, hipStream_t st, const cplx<T>* x, const T* chi, const G* gq, cplx<T>* y, int mode,
+                 const cplx<T>* tw, int B, const BatchStrides& bs) {
+  const T inv = T(1.0 / ((double)P.M * (double)P.M));
+  switch (P.M) {
+#define X(m)                                                                                                      \
+  case m:                                                                                                         \
+    if constexpr (m <= (sizeof(T) == 4 ? 96 : 64))                                                                \
+      hipLaunchKernelGGL((k_matvec_small<T, G, m>), dim3(B), dim3(SmallShape<m>::BS), 0, st, x, chi, gq, y, mode, \
+                         P.N, inv, tw, bs);                                                                       \
+    break;
+    X(16) X(24) X(32) X(48) X(64) X(96)
+#undef X
+    default: return CGM_ERROR_UNSUPPORTED;
+  }
+  return hipGetLastError() == hipSuccess ? CGM_SUCCESS : CGM_ERROR_DEVICE;
+}
+template bool small_matvec<float>(const Plan&);
+template bool small_matvec<double>(const Plan&);
+template int launch_small<float, float2>(const Plan&, hipStream_t, const float2*, const float*, const float2*, float2*,
+                                         int, const float2*, int, const BatchStrides&);
+template int launch_small<double, double2>(const Plan&, hipStream_t, const double2*, const double*, const double2*,
+                                           double2*, int, const double2*, int, const BatchStrides&);
 
 template int launch_pass1<float>(const Plan&, hipStream_t, const float2*, float2*, const float*,
                                  const double*, int, float2*, const float2*, const int*, int,
@@ -775,6 +709,19 @@ template int launch_pass3<float>(const Plan&, hipStream_t, const float2*, const 
 template int launch_pass3<double>(const Plan&, hipStream_t, const double2*, const double2*,
                                   const double*, const double2*, double2*, int, const double2*,
                                   const int*, int, const BatchStrides&);
+
+int pass_lds_limits(int M) {
+  const auto allow = [](const void* f) { return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds); };
+  if (M == 4096) {  // a 4096-point FP64 transform
+    constexpr int E = kPassE<double, 4096>;
+    CGM_HIP(allow((const void*)k_pass1<double, 4096, E>));
+    CGM_HIP(allow((const void*)k_pass2<double, double2, 4096, E>));
+    CGM_HIP(allow((const void*)k_pass3<double, 4096, E>));
+    CGM_HIP(allow((const void*)k_fft_rows<double, 4096, -1>));
+    CGM_HIP(allow((const void*)k_fft_cols<double, 4096, -1>));
+  }
+  return CGM_SUCCESS;
+}
 
 int plan_init(Plan& P, int N) {
   P.N = N;
@@ -803,14 +750,16 @@ int spectrum_from_block(const Plan& P, hipStream_t st, const double2* blk, const
   hipLaunchKernelGGL(k_embed, dim3((MM + 255) / 256), dim3(256), 0, st, blk, E, N, M);
   const int nt = fft_threads(M);
   const int rows = groups_for(M, 256);
-  const size_t lds = (size_t)rows * M * sizeof(double2);
+  int cols = rows;
+  while (M % cols) cols /= 2;
+  const size_t lds = (size_t)rows * lds_len(M) * sizeof(double2);
   switch (M) {
 #define X(m)                                                                                   \
   case m:                                                                                      \
     hipLaunchKernelGGL((k_fft_rows<double, m, -1>), dim3((M + rows - 1) / rows),                \
                        dim3(rows * nt), lds, st, E, M, rows, tw64);                             \
-    hipLaunchKernelGGL((k_fft_cols<double, m, -1>), dim3(M / P.cols2), dim3(P.cols2 * nt),      \
-                       (size_t)P.cols2 * M * sizeof(double2), st, E, P.cols2, tw64);            \
+    hipLaunchKernelGGL((k_fft_cols<double, m, -1>), dim3(M / cols), dim3(cols * nt),            \
+                       (size_t)cols * lds_len(M) * sizeof(double2), st, E, cols, tw64);            \
     break;
     CGM_FOR_EACH_M(X)
 #undef X

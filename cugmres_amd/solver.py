@@ -66,8 +66,8 @@ class Context:
 
     def radix_plan(self):
         """The autotuner's radix plan at M = 1024: {'wide_from_batch': [pass 1, 2, 3],
-        'wave_us' / 'lds_us': [pass][batch 1, 4, 16] for the one-wave register kernel
-        and the LDS-staged radix-8 kernel}."""
+        'wave_us' / 'lds_us': [pass][batch 1, 4, 16] for the one-wave form (16 elements
+        per lane) and the two-wave form (8)}."""
         wb = (_c.c_int * 3)()
         w = (_c.c_float * 9)()
         l_ = (_c.c_float * 9)()
