@@ -146,6 +146,10 @@ SIGNATURES = {
     "cgm_G_x_fft_matvec_T": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_uint]),
     "cgm_cuSolve_LES": (ctypes.c_int, [c_void_p, c_void_p, ctypes.c_int, c_void_p, c_void_p, c_void_p,
                                        c_void_p]),
+    "cgm_block_orthonormalise": (ctypes.c_int, [c_void_p, c_void_p, ctypes.c_int, c_void_p, c_void_p, ctypes.c_int,
+                                                ctypes.c_long, ctypes.c_double, c_void_p]),
+    "cgm_block_combine": (ctypes.c_int, [c_void_p, c_void_p, ctypes.c_int, c_void_p, c_void_p, ctypes.c_int,
+                                         ctypes.c_long]),
     "cgm_malloc": (ctypes.c_int, [ctypes.POINTER(c_void_p), ctypes.c_size_t]),
     "cgm_free": (ctypes.c_int, [c_void_p]),
     "cgm_memcpy_h2d": (ctypes.c_int, [c_void_p, c_void_p, ctypes.c_size_t]),

@@ -25,7 +25,11 @@ Vectors are rows: B and X are (s, n), the basis is ((m + 1) s, n).  The core
 `block_gmres` takes the operator and the preconditioner as callables on such
 row blocks, so it runs on CPU tensors as well as on the device;
 `solve_map` wires it to a Context and a Tiles object."""
+import ctypes
+
 import numpy as np
+
+from ._lib import check, lib
 
 
 class BlockBreakdown(Exception):
@@ -100,6 +104,43 @@ def cholqr2(torch, W):
     return V, S2 @ S1
 
 
+class _DeviceSteps:
+    """The orthonormalisation of a block step by the library's kernels
+    (cgm_block_orthonormalise: up to 16 right-hand sides, complex64 rows of a
+    multiple of 64 values) in the place of project, update and cholqr2, whose
+    some hundred launches per step took longer than their arithmetic."""
+
+    MAX_S = 16
+
+    def __init__(self, ctx):
+        self.ctx = ctx
+        self.torch = ctx.torch
+
+    def takes(self, B):
+        return B.shape[0] <= self.MAX_S and B.shape[1] % 64 == 0
+
+    def orthonormalise(self, Vb, k, W):
+        """W (s, n) against the rows Vb[:k], the result to Vb[k:k + s]; returns
+        the device array [H (k, s); S (s, s)] and the flag behind it."""
+        s, n = W.shape
+        h = self.torch.empty((k + s) * s + 1, dtype=self.torch.complex128, device=W.device)
+        check(lib().cgm_block_orthonormalise(self.ctx.handle, _ptr(Vb), k, _ptr(W), _ptr(Vb[k:]), s, n, 1e-12, _ptr(h)),
+              "cgm_block_orthonormalise")
+        return h
+
+    def combine(self, Vb, Y):
+        """(V Y)^T for Y (k, s) complex128 on the device."""
+        k, s = Y.shape
+        U = self.torch.empty((s, Vb.shape[1]), dtype=Vb.dtype, device=Vb.device)
+        check(lib().cgm_block_combine(self.ctx.handle, _ptr(Vb), k, _ptr(Y), _ptr(U), s, Vb.shape[1]),
+              "cgm_block_combine")
+        return U
+
+
+def _ptr(t):
+    return ctypes.c_void_p(t.data_ptr())
+
+
 class _HessQR:
     """Householder QR of a block upper-Hessenberg matrix built one block column
     (height (j + 2) s, width s) at a time, and the rotated right-hand side
@@ -141,7 +182,7 @@ class _HessQR:
 
 
 def block_gmres(torch, apply_A, apply_P, B, X=None, restart=64, tol=1e-6, max_cycles=20, residual=None,
-                on_step=None, stall_window=10, stall_ratio=0.9):
+                on_step=None, stall_window=10, stall_ratio=0.9, steps_on=None):
     """Right-preconditioned block GMRES(restart) for A X_c = B_c, every row c
     of B (s, n) a right-hand side; restart counts block steps.
 
@@ -155,7 +196,9 @@ def block_gmres(torch, apply_A, apply_P, B, X=None, restart=64, tol=1e-6, max_cy
     cycle the estimates are driven to tol / 2.  A cycle also ends at the
     working precision's floor: when, with every estimate within 20 x tol and
     1e-4 times the cycle's starting residual, the largest one has not fallen
-    below stall_ratio times its value stall_window steps before.  Returns (X, info)
+    below stall_ratio times its value stall_window steps before.  steps_on
+    (optional, a _DeviceSteps object) orthonormalises each block step; without
+    it torch's products do.  Returns (X, info)
     with info["rel_residual"] (per row, from residual()), info["converged"]
     (per row), info["block_steps"], info["cycles"] and info["breakdowns"]."""
     s, n = B.shape
@@ -167,6 +210,24 @@ def block_gmres(torch, apply_A, apply_P, B, X=None, restart=64, tol=1e-6, max_cy
     bnorm = np.where(bnorm > 0, bnorm, 1.0)
     Vb = torch.empty(((restart + 1) * s, n), dtype=dt, device=dev)
     on_device = dev.type == "cuda"
+    if steps_on is not None:  # one pinned buffer for every step's Hessenberg column and flag
+        pinned = torch.empty((restart + 2) * s * s + 1, dtype=torch.complex128, pin_memory=True)
+
+    def stalled(hist, start):
+        return (len(hist) > stall_window and hist[-1] <= 20 * tol and hist[-1] <= 1e-4 * start
+                and hist[-1] > stall_ratio * hist[-1 - stall_window])
+
+    def orthonormalise(k, W):
+        """W against Vb[:k], the result in Vb[k:k + rows of W]: the pinned [H; S]
+        and flag, valid once the event has passed."""
+        h = steps_on.orthonormalise(Vb, k, W)
+        r = W.shape[0]
+        hh = pinned[:h.numel()]
+        hh.copy_(h, non_blocking=True)
+        ev = torch.cuda.Event()
+        ev.record()
+        return hh[:-1].reshape(k + r, r), hh[-1:], ev
+
     steps = cycles = breaks = 0
     R = resid(X)
     rel = torch.linalg.vector_norm(R.to(torch.complex128), dim=1).cpu().numpy() / bnorm
@@ -178,18 +239,29 @@ def block_gmres(torch, apply_A, apply_P, B, X=None, restart=64, tol=1e-6, max_cy
         idx = torch.as_tensor(active, device=dev)
         Ra = R.index_select(0, idx).to(dt)
         sa = int(active.size)
+
+        def start_block(Rc):
+            if steps_on is None:
+                V0, S0 = cholqr2(torch, Rc)
+                Vb[:V0.shape[0]] = V0.to(dt)
+                return S0.cpu().numpy()
+            S0, flag, ev = orthonormalise(0, Rc.clone())
+            ev.synchronize()
+            if float(flag[0].real) != 0.0:
+                raise BlockBreakdown("dependent columns")
+            return S0.numpy().copy()
+
         try:
-            V0, S0 = cholqr2(torch, Ra)
+            S0 = start_block(Ra)
         except BlockBreakdown:
             # dependent residuals: this cycle takes the first column alone, the
             # others follow in later cycles from their updated residuals
             sa = 1
             idx = idx[:1]
             Ra = Ra[:1]
-            V0, S0 = cholqr2(torch, Ra)
+            S0 = start_block(Ra)
             active = active[:1]
-        Vb[:sa] = V0.to(dt)
-        qr = _HessQR(S0.cpu().numpy(), restart)
+        qr = _HessQR(S0, restart)
         bn = bnorm[active]
         start = float(rel[active].max())
         hist = []
@@ -199,6 +271,31 @@ def block_gmres(torch, apply_A, apply_P, B, X=None, restart=64, tol=1e-6, max_cy
             Vk = Vb[:k]
             W = W_next if W_next is not None else apply_A(apply_P(Vb[j * sa:k]))
             W_next = None
+            if steps_on is not None:
+                Hh, flag, ev = orthonormalise(k, W)
+                steps += 1
+                # the next step's operator and tile inverses are queued behind
+                # the copy of the Hessenberg column: the device computes them
+                # while the host updates the QR
+                if j + 1 < restart:
+                    W_next = apply_A(apply_P(Vb[k:k + sa]))
+                ev.synchronize()
+                Hcol = Hh.numpy()
+                if float(flag[0].real) != 0.0:
+                    breaks += 1
+                    Hcol = Hcol.copy()
+                    Hcol[k:] = 0.0
+                    qr.add(Hcol)
+                    break
+                est = qr.add(Hcol) / bn
+                if on_step is not None:
+                    on_step(steps, est)
+                if bool((est <= 0.5 * tol).all()):
+                    break
+                hist.append(float(est.max()))
+                if stalled(hist, start):
+                    break
+                continue
             H1 = project(torch, Vk, W)                              # (k, sa) = V^H W
             W = update(torch, W, Vk, H1)
             H2 = project(torch, Vk, W)
@@ -234,11 +331,13 @@ def block_gmres(torch, apply_A, apply_P, B, X=None, restart=64, tol=1e-6, max_cy
             if bool((est <= 0.5 * tol).all()):
                 break
             hist.append(float(est.max()))
-            if (len(hist) > stall_window and hist[-1] <= 20 * tol and hist[-1] <= 1e-4 * start
-                    and hist[-1] > stall_ratio * hist[-1 - stall_window]):
+            if stalled(hist, start):
                 break
         Y = torch.as_tensor(qr.solve(), device=dev)                  # (qr.k sa, sa)
-        U = (Y.T.to(dt) @ Vb[:qr.k * sa])                            # (sa, n): (V Y)^T
+        if steps_on is not None and Y.shape[0] > 0:
+            U = steps_on.combine(Vb, Y.contiguous())                 # (sa, n): (V Y)^T
+        else:
+            U = (Y.T.to(dt) @ Vb[:qr.k * sa])
         Xa = X.index_select(0, idx) + apply_P(U).to(X.dtype)
         X = X.index_copy(0, idx, Xa.to(X.dtype))
         R = resid(X)
@@ -276,6 +375,7 @@ def solve_map(ctx, gamma, chi, B, tiles=None, X=None, restart=64, tol=1e-6, max_
     def apply_P(Y):
         return tiles.apply(Y.contiguous()) if tiles is not None else Y
 
+    dev = _DeviceSteps(ctx)
     residual = None
     if gamma64 is not None and chi64 is not None:
         B64 = B.to(torch.complex128)
@@ -286,4 +386,4 @@ def solve_map(ctx, gamma, chi, B, tiles=None, X=None, restart=64, tol=1e-6, max_
             return torch.stack([B64[c] - ctx.matvec_c128(gamma64, chi64, X64[c].contiguous(), _lib.OP_FORWARD)
                                 for c in range(s)])
     return block_gmres(torch, apply_A, apply_P, B, X=X, restart=restart, tol=tol, max_cycles=max_cycles,
-                       residual=residual, on_step=on_step)
+                       residual=residual, on_step=on_step, steps_on=dev if dev.takes(B) else None)

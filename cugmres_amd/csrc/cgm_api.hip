@@ -95,6 +95,7 @@ extern "C" int cgm_destroy(cgm_ctx_t c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   krylov_free(c->ws);
   lr_free(c->lr);
+  block_free(c->blk);
   if (c->lrt.created)
     for (hipEvent_t e : c->lrt.ev) (void)hipEventDestroy(e);
   void* ptrs[] = {c->tw32, c->tw64, c->T32, c->T64, c->st, c->chi_tmp, c->vec_tmp, c->v64a, c->chi32, c->zb,

@@ -238,6 +238,15 @@ int lr_cycle(LrWs& w, hipStream_t st, DevState* dst, DevState* hst, long sst, in
              long shist, float2* x, long sx, const LrStep& precond, const LrStep& matvec, LrTiming* tm = nullptr);
 int lr_scale(hipStream_t st, const float2* u, long su, float2* z, long sz, long n, const DevState* dst, long sst,
              int B);
+// Workspace of the block orthonormalisation (cgm_block.hip): grown as needed,
+// freed with the context; capacities in bytes.
+struct BlockWs {
+  double2* part = nullptr;  // projection partials
+  float2* h32 = nullptr;    // coefficients of the update
+  double2* gram = nullptr;  // Gram partials, then the 16 x 16 M and S
+  size_t part_cap = 0, h32_cap = 0, gram_cap = 0;
+};
+void block_free(BlockWs& B);
 // Device address of the allocation-free matvec's scratch array on `device`
 // (cgm_noalloc.hip), taken once per device; the device must be current.
 int noalloc_init(int device);
@@ -298,6 +307,7 @@ struct cgm_context {
   float mask_chi = 0.f;
   float tuned_us[3] = {0.f, 0.f, 0.f};  // autotuned pass 1/2/3 times
   float tuned_wide_us[3][3] = {}, tuned_lds_us[3][3] = {};  // [pass][batch 1/4/16], microseconds
+  cgm::BlockWs blk;  // block GMRES workspace (lazy)
   int path = 0;  // Arnoldi kernels: 0 = fused lagged CGS2 where supported, 1 = two-pass CGS2
   cgm::KrylovWs ws;
   cgm::LrWs lr;                  // long-recurrence FGMRES workspace (lazy)

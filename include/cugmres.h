@@ -423,6 +423,26 @@ int cgm_gmres_refine_pc(cgm_ctx_t ctx, const cgm_complex64* dev_gamma,
                         const cgm_complex128* dev_b, cgm_complex128* dev_x, const cgm_precond* pc,
                         const cgm_refine_params* params, cgm_refine_result* result);
 
+/* ---- block GMRES ----------------------------------------------------------- */
+/* One block step's orthonormalisation for s <= 16 right-hand sides (vectors
+ * are rows of n complex values, n a multiple of 64, 16-byte aligned):
+ * H = V^H W and W -= (V H)^T twice (CGS2) against the k basis rows, then
+ * W^T = out^T S with out orthonormal by CholQR2 (Gram matrices, Cholesky factors
+ * and the s x s transforms in FP64; projections with FP32 products, FP64 sums
+ * over chunks).  w is overwritten; k = 0 orthonormalises w alone.
+ * dev_h receives k*s + s*s + 1 complex128: H of both passes (k x s), S (s x s),
+ * and a flag (re): 0, 1 = a Gram matrix was not positive definite, 2 = its
+ * smallest pivot is at most tol times its largest diagonal entry (out and S
+ * then hold no use).  Asynchronous on the context stream; the workspace
+ * belongs to the context and grows with k and n.  No counterpart in the
+ * reference, which projects one vector at a time
+ * (B/CUDA_GMRES/GMRES.cuh:289-303). */
+int cgm_block_orthonormalise(cgm_ctx_t ctx, const cgm_complex64* dev_basis, int k, cgm_complex64* dev_w,
+                             cgm_complex64* dev_out, int s, long n, double tol, cgm_complex128* dev_h);
+/* u[c] = sum_i y[i][c] basis[i] for y (k x s, complex128) and s <= 16 rows u. */
+int cgm_block_combine(cgm_ctx_t ctx, const cgm_complex64* dev_basis, int k, const cgm_complex128* dev_y,
+                      cgm_complex64* dev_u, int s, long n);
+
 /* ---- reference-compatible entry points ------------------------------------ */
 /* The reference's plane wave exp(-i k i) with k = 2*3.14f/(N/6.f)
  * (B/CUDA_GMRES/GMRES_kernels.cuh:12,557-572), on the device. */

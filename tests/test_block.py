@@ -214,3 +214,59 @@ def test_block_gmres_on_the_helmholtz_operator_with_oracle_tiles(orc):
     ref = np.linalg.solve(A, B.T).T
     assert rel(X.numpy(), ref) < 1e-8
     assert info["block_steps"] < n // s
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,s", [(64, 0, 1), (64, 3, 2), (192, 63, 16), (4096, 0, 16), (4096, 64, 16), (4096, 65, 5),
+                                   (9216, 208, 13), (65536, 400, 16), (36864, 1, 16)])
+def test_device_orthonormalisation(n, k, s):
+    """cgm_block_orthonormalise at the edges of its tiles (64 basis rows, 128
+    cells, 16 block rows): W = V H + out S, out orthonormal and orthogonal to
+    V.  Tolerances: the update's FP32 sums of k products and the rounding of the
+    rows to complex64 leave a few 6e-8 sqrt(k + 16) relative to W (2e-6 at
+    k = 400); the Gram matrix of rows rounded to complex64 is the identity to
+    2 x 6e-8 x sqrt(16) per entry."""
+    import ctypes
+    import torch
+    from cugmres_amd import solver
+    from cugmres_amd._lib import check, lib
+    print(f"block orthonormalisation n={n} k={k} s={s}", flush=True)
+    ctx = solver.Context(64, 0)
+    rng = np.random.default_rng(n + k + s)
+
+    def rnd(r):
+        return rng.standard_normal((r, n)) + 1j * rng.standard_normal((r, n))
+    V = np.ascontiguousarray(np.linalg.qr(rnd(k).T)[0].T.astype(np.complex64)) if k else np.zeros((1, n), np.complex64)
+    C = rng.standard_normal((s, max(k, 1))) + 1j * rng.standard_normal((s, max(k, 1)))
+    W = (rnd(s) / np.sqrt(n) + (C @ V if k else 0)).astype(np.complex64)
+    dV, dW = torch.as_tensor(V).to(ctx.device), torch.as_tensor(W).to(ctx.device)
+    out = torch.empty((s, n), dtype=torch.complex64, device=ctx.device)
+    h = torch.zeros((k + s) * s + 1, dtype=torch.complex128, device=ctx.device)
+
+    def call(w):
+        check(lib().cgm_block_orthonormalise(ctx.handle, ctypes.c_void_p(dV.data_ptr()), k, ctypes.c_void_p(w.data_ptr()),
+                                             ctypes.c_void_p(out.data_ptr()), s, n, 1e-12,
+                                             ctypes.c_void_p(h.data_ptr())), "cgm_block_orthonormalise")
+        torch.cuda.synchronize()
+        return h.cpu().numpy()
+    hh = call(dW.clone())
+    assert hh[-1] == 0
+    H, S = hh[:k * s].reshape(k, s), hh[k * s:-1].reshape(s, s)
+    Q = out.cpu().numpy().astype(np.complex128)
+    Vd = V.astype(np.complex128)
+    # vectors are rows and columns of H belong to them: W^T = V^T H + Q^T S
+    R = W.astype(np.complex128).T - Q.T @ S - (Vd.T @ H if k else 0)
+    assert np.linalg.norm(R) < 2e-6 * np.linalg.norm(W)
+    assert np.abs(Q.conj() @ Q.T - np.eye(s)).max() < 5e-7
+    if k:
+        assert np.abs(Vd.conj() @ Q.T).max() < 2e-6
+        assert np.linalg.norm(H - (Vd.conj() @ W.T)) < 2e-6 * np.linalg.norm(W)
+        u = torch.empty((s, n), dtype=torch.complex64, device=ctx.device)
+        Y = torch.as_tensor(np.ascontiguousarray(H)).to(ctx.device)
+        check(lib().cgm_block_combine(ctx.handle, ctypes.c_void_p(dV.data_ptr()), k, ctypes.c_void_p(Y.data_ptr()),
+                                      ctypes.c_void_p(u.data_ptr()), s, n), "cgm_block_combine")
+        assert np.linalg.norm(u.cpu().numpy() - (Vd.T @ H).T) < 2e-6 * np.linalg.norm(W)
+    if s > 1:   # a repeated vector is flagged
+        dW[s - 1] = dW[0]
+        assert call(dW)[-1].real in (1.0, 2.0)
+    ctx.close()
