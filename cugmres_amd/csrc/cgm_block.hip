@@ -20,6 +20,7 @@
 // The MFMA used is 16 x 16 x 4 in FP32: lane (a, g) holds A[a][g], B[g][a] and
 // D[4 g + r][a].
 #include "cgm_internal.h"
+#include "cgm_reduce.h"
 
 using namespace cgm;
 
@@ -43,9 +44,9 @@ __device__ inline double2 dfmac(double2 a, double2 b, double2 c) {  // conj(a) b
 // Partial sums of H[i][c] = sum_x conj(V_i[x]) W_c[x] over chunk blockIdx.x (ch
 // cells, a multiple of 128) for the 64 basis rows of blockIdx.y, to
 // part[(chunk * kp + i) * 16 + c] (kp: k padded to 64).  Lane (a, g) of a wave
-// loads 8 consecutive cells (64 bytes) of basis row a of each of four row tiles
-// and of block row a: the m-th of them is K-value g of MFMA m, so nothing is
-// shuffled.  Re = Vr Wr + Vi Wi, Im = Vr Wi - Vi Wr.  Rows from k on repeat row
+// loads cells 8 h + 2 g, + 1 (h < 4; 64 bytes of a row per load) of basis row a of
+// each of four row tiles and of block row a: each is K-value g of an MFMA, so
+// nothing is shuffled.  Re = Vr Wr + Vi Wi, Im = Vr Wi - Vi Wr.  Rows from k on repeat row
 // k - 1 and are dropped by k_bp_red, block rows from s on are zero.
 __global__ void __launch_bounds__(256)
 k_bp_proj(const float2* __restrict__ V, const float2* __restrict__ W, long n, int k, int s, int ch, int kp,
@@ -58,29 +59,39 @@ k_bp_proj(const float2* __restrict__ V, const float2* __restrict__ W, long n, in
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int i = r0 + 16 * t + a;
-    vp[t] = V + (long)(i < k ? i : k - 1) * n + 8 * g;
+    vp[t] = V + (long)(i < k ? i : k - 1) * n + 2 * g;
   }
-  const float2* wp = W + (long)(a < s ? a : 0) * n + 8 * g;
+  const float2* wp = W + (long)(a < s ? a : 0) * n + 2 * g;
   f4_t re[4], p[4], q[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) re[t] = p[t] = q[t] = f4_t{0.f, 0.f, 0.f, 0.f};
-  for (long x = x0 + 32 * w; x < x1; x += 128) {
-    f4_t wv[4], vv[4][4];
+  f4_t wv[4], vv[4][4];
+  const auto load = [&](long x) {
 #pragma unroll
-    for (int h = 0; h < 4; ++h) wv[h] = *reinterpret_cast<const f4_t*>(wp + x + 2 * h);
+    for (int h = 0; h < 4; ++h) wv[h] = *reinterpret_cast<const f4_t*>(wp + x + 8 * h);
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int h = 0; h < 4; ++h) vv[t][h] = __builtin_nontemporal_load(reinterpret_cast<const f4_t*>(vp[t] + x + 2 * h));
-    if (a >= s)
+      for (int h = 0; h < 4; ++h) vv[t][h] = __builtin_nontemporal_load(reinterpret_cast<const f4_t*>(vp[t] + x + 8 * h));
+  };
+  long x = x0 + 32 * w;
+  if (x < x1) load(x);
+  for (; x < x1; x += 128) {
+    f4_t wc[4], vc[4][4];
 #pragma unroll
-      for (int h = 0; h < 4; ++h) wv[h] = f4_t{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < 4; ++h) {
+      wc[h] = a < s ? wv[h] : f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) vc[t][h] = vv[t][h];
+    }
+    load(x + 128 < x1 ? x + 128 : x);  // the next cells, while these are multiplied
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
-      const float wr = wv[m >> 1][2 * (m & 1)], wi = wv[m >> 1][2 * (m & 1) + 1];
+      const float wr = wc[m >> 1][2 * (m & 1)], wi = wc[m >> 1][2 * (m & 1) + 1];
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const float vr = vv[t][m >> 1][2 * (m & 1)], vi = vv[t][m >> 1][2 * (m & 1) + 1];
+        const float vr = vc[t][m >> 1][2 * (m & 1)], vi = vc[t][m >> 1][2 * (m & 1) + 1];
         re[t] = mfma(vr, wr, re[t]);
         p[t] = mfma(vr, wi, p[t]);
         q[t] = mfma(vi, wr, q[t]);
@@ -109,24 +120,30 @@ k_bp_proj(const float2* __restrict__ V, const float2* __restrict__ W, long n, in
   }
 }
 
-// H over the chunks: H32 (kp x 16, zero from k and s on) for the update, and
-// H64 (k x s): set by the first pass, added to by the second.
+// H over the chunks, in four interleaved sums: H32 (kp x 16, zero from k and s
+// on) for the update, and H64 (k x s): set by the first pass, added to by the
+// second.
 __global__ void __launch_bounds__(256)
 k_bp_red(const double2* __restrict__ part, int chunks, int k, int s, int kp, float2* __restrict__ H32,
          double2* __restrict__ H64, int second) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= kp * kS) return;
-  const int i = e / kS, c = e % kS;
+  __shared__ double2 red[4][64];
+  const int l = threadIdx.x & 63, sl = threadIdx.x >> 6;
+  const int e = blockIdx.x * 64 + l;  // kp is a multiple of 64
   double2 h = make_double2(0.0, 0.0);
-  if (i < k && c < s) {
 #pragma unroll 8
-    for (int u = 0; u < chunks; ++u) {
-      const double2 v = part[(long)u * kp * kS + e];
-      h.x += v.x;
-      h.y += v.y;
-    }
+  for (int u = sl; u < chunks; u += 4) {
+    const double2 v = part[(long)u * kp * kS + e];
+    h.x += v.x;
+    h.y += v.y;
+  }
+  red[sl][l] = h;
+  __syncthreads();
+  if (sl) return;
+  const int i = e / kS, c = e % kS;
+  if (i < k && c < s) {
     // as the update takes it
-    const float2 f = make_float2((float)h.x, (float)h.y);
+    const float2 f = make_float2((float)((red[0][l].x + red[1][l].x) + (red[2][l].x + red[3][l].x)),
+                                 (float)((red[0][l].y + red[1][l].y) + (red[2][l].y + red[3][l].y)));
     double2* o = H64 + (long)i * s + c;
     *o = second ? make_double2(o->x + f.x, o->y + f.y) : make_double2(f.x, f.y);
     H32[e] = f;
@@ -150,17 +167,38 @@ k_bp_coef(const double2* __restrict__ Y, int k, int s, int kp, float2* __restric
 }
 
 // Gram partial of the block's kX cells in LDS (rows of kLd): entry (a, b) =
-// sum_x conj(b_a[x]) b_b[x] by thread 16 a + b.
+// sum_x conj(b_a[x]) b_b[x].  A thread takes 2 x 2 entries over a quarter of the
+// cells (two LDS values per product instead of four); the quarters meet in red.
 template <typename C>
-__device__ inline void gram_part(const C* blk, double2* __restrict__ out) {
-  const int a = threadIdx.x >> 4, b = threadIdx.x & 15;
-  double2 acc = make_double2(0.0, 0.0);
-#pragma unroll 8
-  for (int x = 0; x < kX; ++x) {
-    const C u = blk[a * kLd + x], v = blk[b * kLd + x];
-    acc = dfmac(make_double2(u.x, u.y), make_double2(v.x, v.y), acc);
+__device__ inline void gram_part(const C* blk, double2 (*red)[kS * kS], double2* __restrict__ out) {
+  const int q = threadIdx.x >> 6, a = 2 * ((threadIdx.x >> 3) & 7), b = 2 * (threadIdx.x & 7);
+  double2 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = make_double2(0.0, 0.0);
+#pragma unroll 4
+  for (int x = q; x < kX; x += 4) {
+    double2 u[2], v[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const C cu = blk[(a + i) * kLd + x], cv = blk[(b + i) * kLd + x];
+      u[i] = make_double2(cu.x, cu.y);
+      v[i] = make_double2(cv.x, cv.y);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = dfmac(u[i], v[j], acc[i][j]);
   }
-  out[(long)blockIdx.x * kS * kS + threadIdx.x] = acc;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) red[q][(a + i) * kS + b + j] = acc[i][j];
+  __syncthreads();
+  const int e = threadIdx.x;
+  out[(long)blockIdx.x * kS * kS + e] = make_double2((red[0][e].x + red[1][e].x) + (red[2][e].x + red[3][e].x),
+                                                     (red[0][e].y + red[1][e].y) + (red[2][e].y + red[3][e].y));
 }
 
 // Out = In - (V H)^T for the kX cells of work-group blockIdx.x (In null: zero).
@@ -237,7 +275,7 @@ k_bp_upd(const float2* V, const float2* __restrict__ H32, const float2* In, floa
       q[1] = make_float2(o[r][2], o[r][3]);
     }
     __syncthreads();
-    gram_part(blk, gpart);
+    gram_part(blk, reinterpret_cast<double2(*)[kS * kS]>(reinterpret_cast<char*>(red) + 32768), gpart);
   }
 }
 
@@ -246,90 +284,93 @@ k_bp_upd(const float2* V, const float2* __restrict__ H32, const float2* In, floa
 // S = L^H.  Second: M = X M, S = L^H S, written to Sout (s x s).  *flag: 1 when a
 // pivot is not positive, 2 when the smallest |L_ii|^2 is at most tol times the
 // largest diagonal entry of G (M, S then hold no use); kept from the first.
-__global__ void __launch_bounds__(1024)
-k_bp_chol(const double2* __restrict__ gpart, int nparts, int s, double tol, int second, double2* __restrict__ M,
-          double2* __restrict__ S, double2* __restrict__ Sout, double2* __restrict__ flag) {
-  __shared__ double2 A[kS][kS + 1], X[kS][kS + 1];
-  __shared__ double2 red[4][kS * kS];
-  const int tid = threadIdx.x, e = tid & 255, sl = tid >> 8;
+//
+// kCholWgs work-groups add up their share of the partials; the last one to
+// arrive (its ticket is reset) adds up the shares and factors.  Step q of the
+// elimination updates the trailing part of G and of the right-hand side
+// (identity, for the inverse) from column q and row q as they stand, so a step
+// is one barrier.
+constexpr int kCholWgs = 16;
+__global__ void __launch_bounds__(256)
+k_bp_chol(const double2* __restrict__ gpart, int nparts, int s, double tol, int second, double2* __restrict__ share,
+          unsigned* ticket, double2* __restrict__ M, double2* __restrict__ S, double2* __restrict__ Sout,
+          double2* __restrict__ flag) {
+  __shared__ double2 A[kS][kS + 1], X[kS][kS + 1], L[kS][kS + 1], g[kS * kS];
+  const int e = threadIdx.x, i = e >> 4, j = e & 15;
   double2 acc = make_double2(0.0, 0.0);
 #pragma unroll 8
-  for (int u = sl; u < nparts; u += 4) {
+  for (int u = blockIdx.x; u < nparts; u += kCholWgs) {
     const double2 v = gpart[(long)u * kS * kS + e];
     acc.x += v.x;
     acc.y += v.y;
   }
-  red[sl][e] = acc;
-  __syncthreads();
-  const int i = e >> 4, j = e & 15;
-  if (sl == 0) {
-    const int t = j * kS + i;
-    const auto sum = [&](int q) {
-      return make_double2((red[0][q].x + red[1][q].x) + (red[2][q].x + red[3][q].x),
-                          (red[0][q].y + red[1][q].y) + (red[2][q].y + red[3][q].y));
-    };
-    const double2 u = sum(e), v = sum(t);
-    A[i][j] = i < s && j < s ? make_double2(0.5 * (u.x + v.x), 0.5 * (u.y - v.y)) : make_double2(i == j ? 1.0 : 0.0, 0.0);
-    X[i][j] = make_double2(0.0, 0.0);
+  put2(&share[blockIdx.x * kS * kS + e], acc.x, acc.y);
+  if (!arrive_last(ticket)) return;
+  if (e == 0) reset_ticket(ticket);
+  acc = make_double2(0.0, 0.0);
+  double2 v[kCholWgs];
+#pragma unroll
+  for (int u = 0; u < kCholWgs; ++u) v[u] = get2(&share[u * kS * kS + e]);
+#pragma unroll
+  for (int u = 0; u < kCholWgs; ++u) {
+    acc.x += v[u].x;
+    acc.y += v[u].y;
   }
+  g[e] = acc;
+  __syncthreads();
+  const double2 t = g[j * kS + i];
+  const double2 m1 = second ? M[e] : make_double2(0.0, 0.0), s1 = second ? S[e] : make_double2(0.0, 0.0);
+  A[i][j] = i < s && j < s ? make_double2(0.5 * (acc.x + t.x), 0.5 * (acc.y - t.y)) : make_double2(i == j ? 1.0 : 0.0, 0.0);
+  X[i][j] = make_double2(i == j ? 1.0 : 0.0, 0.0);
   __syncthreads();
   double dmax = 0.0;
   for (int q = 0; q < s; ++q) dmax = A[q][q].x > dmax ? A[q][q].x : dmax;
-  __syncthreads();
   bool bad = false;
   double lmin = __builtin_huge_val();
-  for (int q = 0; q < kS; ++q) {  // right-looking, L in the lower triangle
+  for (int q = 0; q < kS; ++q) {
     const double d = A[q][q].x;
     bad |= !(d > 0.0);
     if (q < s && d < lmin) lmin = d;
-    const double r = d > 0.0 ? sqrt(d) : 1.0;
-    __syncthreads();
-    if (tid < kS && tid >= q) {
-      const double2 v = A[tid][q];
-      A[tid][q] = tid == q ? make_double2(r, 0.0) : make_double2(v.x / r, v.y / r);
-    }
-    __syncthreads();
-    if (sl == 0 && j > q && i >= j) {  // A[i][j] -= L[i][q] conj(L[j][q])
-      const double2 u = A[i][q], v = A[j][q];
-      A[i][j].x -= u.x * v.x + u.y * v.y;
-      A[i][j].y -= u.y * v.x - u.x * v.y;
-    }
-    __syncthreads();
-  }
-  // X = inv(conj(L)), column tid by forward substitution
-  if (tid < kS) {
-    for (int r = tid; r < kS; ++r) {
-      double2 b = make_double2(r == tid ? 1.0 : 0.0, 0.0);
-      for (int q = tid; q < r; ++q) {  // b -= conj(L[r][q]) X[q][tid]
-        const double2 l = A[r][q], x = X[q][tid];
-        b.x -= l.x * x.x + l.y * x.y;
-        b.y -= l.x * x.y - l.y * x.x;
+    const double r = d > 0.0 ? 1.0 / sqrt(d) : 1.0;
+    const double2 ai = A[i][q], aj = A[j][q], xq = X[q][j];
+    const double2 li = make_double2(ai.x * r, ai.y * r), lj = make_double2(aj.x * r, aj.y * r);
+    if (j == q) L[i][q] = i > q ? li : make_double2(i == q && d > 0.0 ? sqrt(d) : 0.0, 0.0);
+    if (i > q) {
+      if (j > q && i >= j) {  // A[i][j] -= L[i][q] conj(L[j][q])
+        A[i][j].x -= li.x * lj.x + li.y * lj.y;
+        A[i][j].y -= li.y * lj.x - li.x * lj.y;
       }
-      const double l = A[r][r].x;
-      X[r][tid] = make_double2(b.x / l, b.y / l);
+      // X[i][j] -= conj(L[i][q]) X[q][j] / L[q][q]
+      const double2 x = make_double2(xq.x * r, xq.y * r);
+      X[i][j].x -= li.x * x.x + li.y * x.y;
+      X[i][j].y -= li.x * x.y - li.y * x.x;
     }
+    __syncthreads();
   }
-  __syncthreads();
-  const bool dep = lmin <= tol * dmax;
-  if (tid == 0) {
-    const double f = bad ? 1.0 : dep ? 2.0 : 0.0;
+  {  // the rows of the inverse over their pivots
+    const double l = L[i][i].x;
+    X[i][j] = j <= i ? make_double2(X[i][j].x / l, X[i][j].y / l) : make_double2(0.0, 0.0);
+  }
+  if (e == 0) {
+    const double f = bad ? 1.0 : lmin <= tol * dmax ? 2.0 : 0.0;
     if (!second || flag->x == 0.0) *flag = make_double2(f, 0.0);
   }
-  // L^H (upper triangular)
-  const double2 lh = j >= i ? make_double2(A[j][i].x, -A[j][i].y) : make_double2(0.0, 0.0);
-  double2 m = X[i][j], t = lh;
-  if (second) {
-    m = t = make_double2(0.0, 0.0);
-    for (int q = 0; q < kS; ++q) {
-      m = dfma(X[i][q], M[q * kS + j], m);
-      if (q >= i) t = dfma(make_double2(A[q][i].x, -A[q][i].y), S[q * kS + j], t);
-    }
-    __syncthreads();  // every entry of M is read before it is replaced
+  if (!second) {
+    M[e] = X[i][j];
+    S[e] = j >= i ? make_double2(L[j][i].x, -L[j][i].y) : make_double2(0.0, 0.0);  // L^H
+    return;
   }
-  if (sl) return;
+  __syncthreads();
+  A[i][j] = m1;
+  __syncthreads();
+  double2 m = make_double2(0.0, 0.0), w = make_double2(0.0, 0.0);
+  for (int q = 0; q <= i; ++q) m = dfma(X[i][q], A[q][j], m);
+  __syncthreads();
+  A[i][j] = s1;
+  __syncthreads();
+  for (int q = i; q < kS; ++q) w = dfma(make_double2(L[q][i].x, -L[q][i].y), A[q][j], w);
   M[e] = m;
-  if (!second) S[e] = t;
-  else if (i < s && j < s) Sout[i * s + j] = t;
+  if (i < s && j < s) Sout[i * s + j] = w;
 }
 
 // The kX cells of the block at x0, rows from s on zero, into LDS.
@@ -353,7 +394,7 @@ __device__ inline double2 apply_row(const double2* Ml, const float2* blk, int c,
 __global__ void __launch_bounds__(256)
 k_bp_gram(const float2* __restrict__ W, long n, int s, const double2* __restrict__ M, double2* __restrict__ gpart) {
   __shared__ float2 blk[kS * kLd];
-  __shared__ double2 v1[kS * kLd];
+  __shared__ double2 v1[kS * kLd], red[4][kS * kS];
   __shared__ double2 Ml[kS * kS];
   const long x0 = (long)blockIdx.x * kX;
   Ml[threadIdx.x] = M[threadIdx.x];
@@ -363,7 +404,7 @@ k_bp_gram(const float2* __restrict__ W, long n, int s, const double2* __restrict
 #pragma unroll 2
   for (int x = threadIdx.x & 15; x < kX; x += 16) v1[c * kLd + x] = apply_row(Ml, blk, c, x);
   __syncthreads();
-  gram_part(v1, gpart);
+  gram_part(v1, red, gpart);
 }
 
 __global__ void __launch_bounds__(256)
@@ -425,23 +466,36 @@ extern "C" int cgm_block_orthonormalise(cgm_ctx_t c, const cgm_complex64* basis,
   int rc;
   if ((rc = ensure((void**)&B.part, &B.part_cap, sizeof(double2) * kS * (size_t)(k ? kp : 1) * chunks))) return rc;
   if ((rc = ensure((void**)&B.h32, &B.h32_cap, sizeof(float2) * kS * (size_t)(kp + kRows)))) return rc;
-  if ((rc = ensure((void**)&B.gram, &B.gram_cap, sizeof(double2) * kS * kS * (size_t)(wgs + 2)))) return rc;
+  if ((rc = ensure((void**)&B.gram, &B.gram_cap, sizeof(double2) * kS * kS * (size_t)(wgs + 2 + kCholWgs)))) return rc;
+  if (!B.ticket) {
+    unsigned* p = nullptr;
+    CGM_HIP(hipMalloc((void**)&p, sizeof(unsigned)));
+    if (hipMemset(p, 0, sizeof(unsigned)) != hipSuccess) {
+      (void)hipFree(p);
+      cgm_set_last_error("block orthonormalisation: ticket clear failed");
+      return CGM_ERROR_DEVICE;
+    }
+    B.ticket = p;
+  }
   const float2* V = (const float2*)basis;
   float2* W = (float2*)w;
-  double2 *H = (double2*)h, *M = B.gram + (size_t)wgs * kS * kS, *S = M + kS * kS;
+  double2 *H = (double2*)h, *M = B.gram + (size_t)wgs * kS * kS, *S = M + kS * kS,
+          *share = S + kS * kS;
   double2 *Sout = H + (long)k * s, *flag = Sout + s * s;
   for (int pass = 0; pass < 2 && k; ++pass) {
     hipLaunchKernelGGL(k_bp_proj, dim3(chunks, groups), dim3(256), 0, st, V, W, n, k, s, ch, kp, B.part);
-    hipLaunchKernelGGL(k_bp_red, dim3((kp * kS + 255) / 256), dim3(256), 0, st, B.part, chunks, k, s, kp, B.h32, H, pass);
+    hipLaunchKernelGGL(k_bp_red, dim3(kp * kS / 64), dim3(256), 0, st, B.part, chunks, k, s, kp, B.h32, H, pass);
     if (pass == 0)
       hipLaunchKernelGGL((k_bp_upd<false>), dim3(wgs), dim3(256), 0, st, V, B.h32, W, W, n, k, s, B.gram);
     else
       hipLaunchKernelGGL((k_bp_upd<true>), dim3(wgs), dim3(256), 0, st, V, B.h32, W, W, n, k, s, B.gram);
   }
   if (!k) hipLaunchKernelGGL((k_bp_upd<true>), dim3(wgs), dim3(256), 0, st, W, B.h32, W, W, n, 0, s, B.gram);
-  hipLaunchKernelGGL(k_bp_chol, dim3(1), dim3(1024), 0, st, B.gram, wgs, s, tol, 0, M, S, Sout, flag);
+  hipLaunchKernelGGL(k_bp_chol, dim3(kCholWgs), dim3(256), 0, st, B.gram, wgs, s, tol, 0, share, B.ticket, M, S, Sout,
+                     flag);
   hipLaunchKernelGGL(k_bp_gram, dim3(wgs), dim3(256), 0, st, W, n, s, M, B.gram);
-  hipLaunchKernelGGL(k_bp_chol, dim3(1), dim3(1024), 0, st, B.gram, wgs, s, tol, 1, M, S, Sout, flag);
+  hipLaunchKernelGGL(k_bp_chol, dim3(kCholWgs), dim3(256), 0, st, B.gram, wgs, s, tol, 1, share, B.ticket, M, S, Sout,
+                     flag);
   hipLaunchKernelGGL(k_bp_out, dim3(wgs), dim3(256), 0, st, W, n, s, M, (float2*)out);
   CGM_HIP(hipGetLastError());
   return CGM_SUCCESS;
@@ -471,6 +525,7 @@ void block_free(BlockWs& B) {
   if (B.part) (void)hipFree(B.part);
   if (B.h32) (void)hipFree(B.h32);
   if (B.gram) (void)hipFree(B.gram);
+  if (B.ticket) (void)hipFree(B.ticket);
   B = BlockWs();
 }
 }  // namespace cgm

@@ -243,7 +243,8 @@ int lr_scale(hipStream_t st, const float2* u, long su, float2* z, long sz, long 
 struct BlockWs {
   double2* part = nullptr;  // projection partials
   float2* h32 = nullptr;    // coefficients of the update
-  double2* gram = nullptr;  // Gram partials, then the 16 x 16 M and S
+  double2* gram = nullptr;  // Gram partials, then the 16 x 16 M, S and the shares of the sums
+  unsigned* ticket = nullptr;
   size_t part_cap = 0, h32_cap = 0, gram_cap = 0;
 };
 void block_free(BlockWs& B);

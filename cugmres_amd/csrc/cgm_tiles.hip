@@ -187,15 +187,20 @@ k_tile_build(const double2* __restrict__ g, const float* __restrict__ chi, long 
 }
 
 // y_t = K_t x_t for NV vectors that share the tile's inverse (one map) or
-// one vector per map (NV = 1).  blockIdx.x = tile, blockIdx.y = group of NV
-// systems; system s reads io.v + s sV, scaled by 1 / *(io.nrm + s sNrm bytes)
-// when io.nrm is given (the scaled input is written to io.vw + s sV when
-// io.vw is given), writes io.z + s sZ, and is skipped once
+// one vector per map (NV = 1).  System s reads io.v + s sV, scaled by 1 /
+// *(io.nrm + s sNrm bytes) when io.nrm is given (the scaled input is written to
+// io.vw + s sV when io.vw is given), writes io.z + s sZ, and is skipped once
 // *(done + s sd bytes) is set.
-template <int M2, int NV>
-__global__ void __launch_bounds__(M2)
-k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restrict__ done, long sd, int N, int T,
-             int nsys) {
+//
+// Tiles of side 8: one wave per tile (blockIdx.x) and group of NV systems
+// (blockIdx.y), one row per lane.  Splitting a tile's 64 columns over waves, as
+// k_tile_apply does below, costs more than it gives there (N = 512, four
+// systems: 25.6 against 28.0 us).
+template <int NV>
+__global__ void __launch_bounds__(64)
+k_tile_apply8(const float2* __restrict__ K, long sK, FnoIO io, const int* __restrict__ done, long sd, int N, int T,
+              int nsys) {
+  constexpr int M2 = 64;
   constexpr int kU = 8;  // columns of the inverse loaded ahead
   __shared__ float2 xs[NV][M2];
   const int nt = N / T;
@@ -250,18 +255,163 @@ k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restr
     if (live[v]) io.z[(long)(s0 + v) * io.sZ + cell] = acc[v];
 }
 
+// Tiles of side 16 and 32: blockIdx.x = tile and block of 128 rows, blockIdx.y =
+// group of NV systems.
+//
+// The stream of K bounds it (8 T^4 bytes per tile; column-major, so rows are
+// independent and a row block needs no sum with another).  A wave reads two
+// rows per lane (1 KB of a column per load) of every eighth group of four
+// columns, kU loads ahead; the waves' sums meet in LDS.  Eight waves on 128 rows,
+// instead of one thread per row through all columns, keep 16 waves per CU on 256
+// tiles of side 16 where there were four, and 64 tiles of side 32 on all CUs.
+// One / four / sixteen systems of one map, us: N = 256, T = 16 (134 MB): 20.7 /
+// 34.3 / 48.9 before, 21.0 / 23.3 / 48 now; N = 512, T = 16 (537 MB): 90.6 / 101 /
+// 387 before, 87 / 97 / 210 now; N = 256, T = 32 (537 MB): 201 / 210 / 202 before,
+// 88 / 96 / 215 now.  Non-temporal loads are slower (the inverses of smaller
+// grids stay in the Infinity Cache): 25.3 / 26.5 / 55 at N = 256, T = 16.
+constexpr int kTileWaves = 8;
+template <int M2, int NV>
+__global__ void __launch_bounds__(64 * kTileWaves)
+k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restrict__ done, long sd, int N, int T,
+             int nsys) {
+  constexpr int kWaves = kTileWaves;
+  constexpr int RB = 128, kBlocks = M2 / RB;
+  constexpr int kUnit = 4;             // loads of one turn of a wave
+  constexpr int kU = NV > 4 ? 4 : 8;   // loads ahead: one turn or two
+  static_assert(M2 % (2 * kUnit * kWaves) == 0, "whole rounds of loads");
+  __shared__ float2 xs[M2][NV];
+  __shared__ float4 red[kWaves / 2][NV][64];
+  const int nt = N / T;
+  const int t = blockIdx.x / kBlocks, rb = blockIdx.x % kBlocks;
+  const int a = t / nt, b = t % nt;
+  const int s0 = blockIdx.y * NV;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  bool live[NV];
+  bool any = false;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int s = s0 + v;
+    live[v] = s < nsys && !(done && *boff(done, (long)s * sd));
+    any |= live[v];
+  }
+  if (!any) return;  // uniform over the work-group
+  const float4* Kt = reinterpret_cast<const float4*>(K + (long)(NV == 1 ? s0 : 0) * sK + (long)t * M2 * M2 + rb * RB) + lane;
+  typedef float f4v __attribute__((ext_vector_type(4)));
+  const auto load = [&](int q) { return *reinterpret_cast<const f4v*>(Kt + (long)q * (M2 / 2)); };  // rows 2 lane, + 1
+  f4v k[kU];
+  // load u of a round: the wave's turns come in the same order for every NV, so
+  // a system's sums do not depend on the others
+  constexpr int kStep = kU * kWaves;
+  const auto col = [&](int u) { return (u / kUnit * kWaves + w) * kUnit + u % kUnit; };
+#pragma unroll
+  for (int u = 0; u < kU; ++u) k[u] = load(col(u));
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int s = s0 + v;
+    float sc = 1.f;
+    if (live[v] && io.nrm) {
+      const double d = *boff(io.nrm, (long)s * io.sNrm);
+      sc = d > 0.0 ? (float)(1.0 / d) : 0.f;
+    }
+    for (int r = threadIdx.x; r < M2; r += 64 * kWaves) {
+      const long cell = (long)(a * T + r / T) * N + b * T + r % T;
+      float2 xv = make_float2(0.f, 0.f);
+      if (live[v]) {
+        xv = io.v[(long)s * io.sV + cell];
+        if (io.nrm) {
+          xv.x *= sc;
+          xv.y *= sc;
+          if (io.vw && rb == 0) io.vw[(long)s * io.sV + cell] = xv;
+        }
+      }
+      xs[r][v] = xv;
+    }
+  }
+  __syncthreads();
+  float4 acc[NV];  // the two rows
+#pragma unroll
+  for (int v = 0; v < NV; ++v) acc[v] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int q = 0; q < M2; q += kStep) {
+    f4v c[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) c[u] = k[u];
+    const int qn = q + kStep < M2 ? q + kStep : q;
+#pragma unroll
+    for (int u = 0; u < kU; ++u) k[u] = load(qn + col(u));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const float2 xv = xs[q + col(u)][v];
+        acc[v].x += c[u][0] * xv.x - c[u][1] * xv.y;
+        acc[v].y += c[u][0] * xv.y + c[u][1] * xv.x;
+        acc[v].z += c[u][2] * xv.x - c[u][3] * xv.y;
+        acc[v].w += c[u][2] * xv.y + c[u][3] * xv.x;
+      }
+    }
+  }
+  // sums of the eight waves: the upper four to the lower four, then those four
+  const auto add = [](float4& o, const float4& p) {
+    o.x += p.x;
+    o.y += p.y;
+    o.z += p.z;
+    o.w += p.w;
+  };
+  if (w >= kWaves / 2)
+#pragma unroll
+    for (int v = 0; v < NV; ++v) red[w - kWaves / 2][v][lane] = acc[v];
+  __syncthreads();
+  if (w < kWaves / 2)
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      add(acc[v], red[w][v][lane]);
+      red[w][v][lane] = acc[v];
+    }
+  __syncthreads();
+  for (int e = threadIdx.x; e < NV * 64; e += 64 * kWaves) {
+    const int v = e / 64, l = e % 64;
+    const int s = s0 + v;
+    if (s >= nsys || (done && *boff(done, (long)s * sd))) continue;
+    float4 o = red[0][v][l];
+#pragma unroll
+    for (int u = 1; u < kWaves / 2; ++u) add(o, red[u][v][l]);
+    const int r = rb * RB + 2 * l;  // T is even: the two rows are neighbours on the grid
+    const long cell = (long)(a * T + r / T) * N + b * T + r % T;
+    float2* z = io.z + (long)s * io.sZ + cell;
+    z[0] = make_float2(o.x, o.y);
+    z[1] = make_float2(o.z, o.w);
+  }
+}
+
+// Systems per pass over the inverses of one map.
+int dense_group(int M2, int nsys) {
+  if (M2 == 64) return nsys > 1 ? 4 : 1;
+  return nsys > 4 ? 8 : nsys > 2 ? 4 : nsys;
+}
+
 template <int M2>
 int launch_apply_m(const cgm_tiles* tl, hipStream_t st, const FnoIO& io, const int* done, long sd, int nsys) {
   const long sK = (long)tl->nt * tl->nt * M2 * M2;
   const int ntiles = tl->nt * tl->nt;
-  if (tl->maps == 1 && nsys > 1) {
-    constexpr int NV = 4;
-    const int groups = (nsys + NV - 1) / NV;
-    hipLaunchKernelGGL((k_tile_apply<M2, NV>), dim3(ntiles, groups), dim3(M2), 0, st, tl->K, 0L, io, done, sd,
-                       tl->N, tl->T, nsys);
+  const int nv = tl->maps == 1 ? dense_group(M2, nsys) : 1;
+  const int groups = (nsys + nv - 1) / nv;
+  if constexpr (M2 == 64) {
+    if (nv == 4)
+      hipLaunchKernelGGL(k_tile_apply8<4>, dim3(ntiles, groups), dim3(64), 0, st, tl->K, 0L, io, done, sd, tl->N, tl->T, nsys);
+    else
+      hipLaunchKernelGGL(k_tile_apply8<1>, dim3(ntiles, groups), dim3(64), 0, st, tl->K, sK, io, done, sd, tl->N, tl->T, nsys);
   } else {
-    hipLaunchKernelGGL((k_tile_apply<M2, 1>), dim3(ntiles, nsys), dim3(M2), 0, st, tl->K, sK, io, done, sd, tl->N,
-                       tl->T, nsys);
+#define CGM_DENSE(NV, S)                                                                                              \
+  hipLaunchKernelGGL((k_tile_apply<M2, NV>), dim3(ntiles * (M2 / 128), groups), dim3(64 * kTileWaves), 0, st, tl->K, S, \
+                     io, done, sd, tl->N, tl->T, nsys)
+    switch (nv) {
+      case 8: CGM_DENSE(8, 0L); break;
+      case 4: CGM_DENSE(4, 0L); break;
+      case 2: CGM_DENSE(2, 0L); break;
+      default: CGM_DENSE(1, sK); break;
+    }
+#undef CGM_DENSE
   }
   CGM_HIP(hipGetLastError());
   return CGM_SUCCESS;
@@ -1384,7 +1534,7 @@ int tiles_maps(const cgm_tiles* t) { return t->maps; }
 
 // Algorithmic bytes of one application to nsys systems: the inverse entries
 // streamed (dense form: every entry of every tile in FP32, once per system or
-// once per group of four right-hand sides of one map; reduced form: the FP16
+// once per group of eight (T = 8: four) right-hand sides of one map; reduced form: the FP16
 // entries of W, once per system or once per group of sixteen right-hand sides
 // of one map) plus v in and z out.
 double apply_bytes(const cgm_tiles* tl, int nsys) {
@@ -1395,7 +1545,8 @@ double apply_bytes(const cgm_tiles* tl, int nsys) {
     else
       for (int s = 0; s < nsys; ++s) e += tl->kept[s] * 4.0;
   } else {
-    const int streams = (tl->maps == 1 && nsys > 1) ? (nsys + 3) / 4 : nsys;
+    const int group = tl->maps == 1 ? dense_group(tl->M2, nsys) : 1;
+    const int streams = (nsys + group - 1) / group;
     if (tl->maps == 1)
       e = tl->kept[0] * 8.0 * streams;
     else

@@ -367,12 +367,12 @@ int cgm_tiles_factor(cgm_tiles_t tiles, const cgm_complex128* dev_block, const f
  * Asynchronous on the context stream.  With one map and several systems the
  * reduced form (T >= 64) applies W to up to 16 systems per pass over it on the
  * matrix cores (FP32 inputs as three FP16 parts each, FP32 sums); the dense
- * form (T <= 32) applies each inverse to four systems per pass.  A system's
+ * form (T <= 32) applies each inverse to eight systems per pass (T = 8: four).  A system's
  * result does not depend on the others. */
 int cgm_tiles_apply(cgm_tiles_t tiles, const cgm_complex64* dev_x, cgm_complex64* dev_y, int batch);
 /* Algorithmic bytes of one cgm_tiles_apply over `batch` systems: the inverse
  * entries it streams (every entry of every tile in FP32 for T <= 32, once per
- * group of four right-hand sides of one map; the stored FP16 blocks of W for
+ * group of eight (T = 8: four) right-hand sides of one map; the stored FP16 blocks of W for
  * T >= 64, once per group of sixteen right-hand sides of one map) plus
  * 16 * N*N per system. */
 int cgm_tiles_apply_bytes(cgm_tiles_t tiles, int batch, double* bytes);
