@@ -265,9 +265,9 @@ k_tile_apply8(const float2* __restrict__ K, long sK, FnoIO io, const int* __rest
 // instead of one thread per row through all columns, keep 16 waves per CU on 256
 // tiles of side 16 where there were four, and 64 tiles of side 32 on all CUs.
 // One / four / sixteen systems of one map, us: N = 256, T = 16 (134 MB): 20.7 /
-// 34.3 / 48.9 before, 21.0 / 23.3 / 48 now; N = 512, T = 16 (537 MB): 90.6 / 101 /
-// 387 before, 87 / 97 / 210 now; N = 256, T = 32 (537 MB): 201 / 210 / 202 before,
-// 88 / 96 / 215 now.  Non-temporal loads are slower (the inverses of smaller
+// 34.3 / 48.9 before, 21.7 / 22.5 / 47 now; N = 512, T = 16 (537 MB): 90.6 / 101 /
+// 387 before, 88 / 95 / 207 now; N = 256, T = 32 (537 MB): 201 / 210 / 202 before,
+// 89 / 95 / 198 now.  Non-temporal loads are slower (the inverses of smaller
 // grids stay in the Infinity Cache): 25.3 / 26.5 / 55 at N = 256, T = 16.
 constexpr int kTileWaves = 8;
 template <int M2, int NV>
@@ -279,8 +279,10 @@ k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restr
   constexpr int kUnit = 4;             // loads of one turn of a wave
   constexpr int kU = NV > 4 ? 4 : 8;   // loads ahead: one turn or two
   static_assert(M2 % (2 * kUnit * kWaves) == 0, "whole rounds of loads");
-  __shared__ float2 xs[M2][NV];
-  __shared__ float4 red[kWaves / 2][NV][64];
+  constexpr size_t kXsLen = sizeof(float2) * M2 * NV, kRedLen = sizeof(float4) * (kWaves / 2) * NV * 64;
+  __shared__ __align__(16) unsigned char smem[kXsLen > kRedLen ? kXsLen : kRedLen];  // the inputs, then the waves' sums
+  float2(*xs)[NV] = reinterpret_cast<float2(*)[NV]>(smem);
+  float4(*red)[NV][64] = reinterpret_cast<float4(*)[NV][64]>(smem);
   const int nt = N / T;
   const int t = blockIdx.x / kBlocks, rb = blockIdx.x % kBlocks;
   const int a = t / nt, b = t % nt;
@@ -313,6 +315,7 @@ k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restr
       const double d = *boff(io.nrm, (long)s * io.sNrm);
       sc = d > 0.0 ? (float)(1.0 / d) : 0.f;
     }
+#pragma unroll 1
     for (int r = threadIdx.x; r < M2; r += 64 * kWaves) {
       const long cell = (long)(a * T + r / T) * N + b * T + r % T;
       float2 xv = make_float2(0.f, 0.f);
@@ -344,10 +347,11 @@ k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restr
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
         const float2 xv = xs[q + col(u)][v];
-        acc[v].x += c[u][0] * xv.x - c[u][1] * xv.y;
-        acc[v].y += c[u][0] * xv.y + c[u][1] * xv.x;
-        acc[v].z += c[u][2] * xv.x - c[u][3] * xv.y;
-        acc[v].w += c[u][2] * xv.y + c[u][3] * xv.x;
+        // two fused multiply-adds each (a product of its own and an addition otherwise)
+        acc[v].x = fmaf(-c[u][1], xv.y, fmaf(c[u][0], xv.x, acc[v].x));
+        acc[v].y = fmaf(c[u][1], xv.x, fmaf(c[u][0], xv.y, acc[v].y));
+        acc[v].z = fmaf(-c[u][3], xv.y, fmaf(c[u][2], xv.x, acc[v].z));
+        acc[v].w = fmaf(c[u][3], xv.x, fmaf(c[u][2], xv.y, acc[v].w));
       }
     }
   }
@@ -358,6 +362,7 @@ k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restr
     o.z += p.z;
     o.w += p.w;
   };
+  __syncthreads();  // the inputs are read
   if (w >= kWaves / 2)
 #pragma unroll
     for (int v = 0; v < NV; ++v) red[w - kWaves / 2][v][lane] = acc[v];
