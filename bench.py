@@ -854,8 +854,8 @@ def profile_fno(ctx, net, dchi, db, batch=1):
     # For one vector the row kernels of
     # layers 0-2 form B_x themselves (inverse x-DFT from the mixed modes) and
     # k_invx runs for layer 3 only; for more, k_invx forms every B_x.  The
-    # stand-alone row projection runs only in the backward pass.  Algorithmic
-    # bytes per launch: BF16 activations 64 B per cell, complex64 vectors 8 B,
+    # row projection with the weight-gradient partials (k_back_rows) runs only
+    # in the backward pass.  Algorithmic bytes per launch: BF16 activations 64 B per cell, complex64 vectors 8 B,
     # chi 4 B; FP32 row projections 4 KiB per grid row, x-DFT partials
     # 128 KiB per 64 rows, spectral weights 4 MiB per layer, mixed modes
     # 128 KiB per vector, row twiddles 256 B per row, BF16 per-row mixing
@@ -864,7 +864,7 @@ def profile_fno(ctx, net, dchi, db, batch=1):
     part = (N // 64) * 16384 * 8   # x-DFT partials: one per 64 rows
     Bv = batch
     bx = 128 * 1024 if batch == 1 else N * 2048   # B_x source per vector: modes (folded) or k_invx's rows
-    bytes_ = {"fno_lift": Bv * (n * (4 + 8) + N * 4096), "fno_rowproj": Bv * (n * 64 + N * 4096),
+    bytes_ = {"fno_lift": Bv * (n * (4 + 8) + N * 4096), "fno_rowproj": Bv * (n * 128 + N * 4096) + min(512, Bv * N) * 4224,
               "fno_dftx": Bv * (N * 4096 + part) + N * 256, "fno_mix": Bv * (part + 16384 * 8) + 4 * 1024 * 1024,
               "fno_invx": Bv * (16384 * 8 + N * 2048) + N * 256,
               "fno_cell_gemm": Bv * (n * 128 + N * 4096 + bx) + N * 256,

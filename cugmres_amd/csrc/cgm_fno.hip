@@ -37,7 +37,7 @@
 // 1 + 3 x 3 + 4 launches for one sample, 1 + 4 x 4 for more.  h0 is a
 // pointwise function of (chi, v): outside training it never reaches global
 // memory, and layer 0's cell GEMM lifts its row again.  The
-// backward pass has the separate kernels (k_rowproj, k_pixel) with the roles
+// backward pass has separate kernels (k_back_rows, k_back_cells) with the roles
 // transposed.
 //
 // Activations are BF16, channel-last ([sample][x][y][32], 64 bytes per cell);
@@ -62,7 +62,7 @@ constexpr int C = 32;   // channels
 constexpr int KY = 16;  // retained column frequencies
 constexpr int KX = 32;  // retained row frequencies
 constexpr int XC = 32;  // fewest rows per partial of k_dftx (sizes the partials)
-constexpr int S = 36;   // LDS row stride (bf16) of k_rowproj: 16-bank offset between lane groups
+constexpr int S = 36;   // LDS row stride (bf16) of a lifted row: 16-bank offset between lane groups
 constexpr int kLayerParams = C * C + C + KX * KY * C * C * 2;
 constexpr long kOffLayer0 = 4 * C;
 constexpr long layer_off(int l) { return kOffLayer0 + (long)l * kLayerParams; }
@@ -110,77 +110,192 @@ __device__ inline bool skip(const int* done) { return done && *done; }
 
 __device__ const double kOne = 1.0;  // the norm of a vector that needs no scaling
 
-// ---------------------------------------------------------------------------
-// Row projection (one grid row x of one sample per iteration):
+// Gradient of the last activation, dh4[p][c] = d0 W_out[c][0] + d1 W_out[c][1]
+// with (d0, d1) = dz[p] / s, at 8 channels c0..c0+7 (w: their 16 entries of
+// W_out, from dproj_weights).  The one rounding of dh4: every kernel that
+// needs it forms it from the 8 bytes of dz, so its 64 bytes per cell are
+// never stored.  One product is rounded before the sum: the first at
+// channels 1, 5, ... and from 30 on the second factor's, elsewhere the other
+// way round.  The choice decides a BF16 rounding now and then, which the
+// layers below amplify to 1e-3 of a weight's gradient: it is fixed, so that
+// a training run is reproducible across versions of these kernels.
+__device__ inline void dproj_weights(const float* __restrict__ Wout, int c0, float* w) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) w[k] = Wout[2 * c0 + k];
+  if (c0 + 8 == C) {  // channels 30 and 31 take their factors in the other order
+    const float t6 = w[12], t7 = w[14];
+    w[12] = w[13];
+    w[14] = w[15];
+    w[13] = t6;
+    w[15] = t7;
+  }
+}
+__device__ inline bf16x8 dproj8(float2 dz, float is, int c0, const float* w) {
+  const float d0 = dz.x * is, d1 = dz.y * is;
+  const float e0 = c0 + 8 == C ? d1 : d0, e1 = c0 + 8 == C ? d0 : d1;  // channels 6, 7 of the eight
+  bf16x8 h;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float a = k < 6 ? d0 : e0, b = k < 6 ? d1 : e1;
+    h[k] = (bf16)((k & 3) == 1 ? __builtin_fmaf(a, w[2 * k], b * w[2 * k + 1])
+                               : __builtin_fmaf(b, w[2 * k + 1], a * w[2 * k]));
+  }
+  return h;
+}
+
+// Four K values of a column of a row-major BF16 tile in LDS: the 16 lanes of
+// a group read four rows of 16 elements (lane j the elements 4 (j % 4).. of
+// row j / 4) and lane j receives column j.  Two of these are an MFMA operand
+// whose K runs over the tile's rows.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ inline bf16x8 ld_tr(const bf16* p0, const bf16* p1) {
+  typedef __attribute__((address_space(3))) s16x4 lds4;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)p0);
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)p1);
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// Sums of NV values over the 16 lanes whose index e is 0..15 (lane = e ST +
+// fixed): each step exchanges one half of the values and keeps the other, NV
+// exchanges in all where NV full reductions take 4 NV.  Afterwards v[j], j <
+// NV / 16, is the sum of value e NV / 16 + j (NV < 16: v[0] that of value
+// e / (16 / NV), in all of its lanes).
+template <int NV, int ST, int M = 8>
+__device__ inline void lane16_sums(float* v, int e) {
+  if constexpr (NV > 1) {
+    constexpr int H = NV / 2;
+    const bool up = e & M;
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+      const float give = up ? v[k] : v[k + H], keep = up ? v[k + H] : v[k];
+      v[k] = keep + __shfl_xor(give, M * ST, 64);
+    }
+    if constexpr (M > 1) lane16_sums<H, ST, M / 2>(v, e);
+  } else {
+    v[0] += __shfl_xor(v[0], M * ST, 64);
+    if constexpr (M > 1) lane16_sums<1, ST, M / 2>(v, e);
+  }
+}
+
+// First kernel of a layer's backward pass, one grid row per iteration:
 //   out[r][a][c] = sum_y Xt[a][y] Y[r][y][c]                  (Xt: 32 x N basis)
-// and with WZ also the weight-gradient partials of this block
-//   part[blk][a][c] += sum_y Z[r][y][a] Y[r][y][c],  part[blk][C*C + c] += sum_y Y[r][y][c].
-// Wave w owns output tile (a-tile w >> 1, c-tile w & 1); Y (and Z) of the row
-// are staged in LDS (row stride S) and read back as MFMA B (and A) operands.
-template <bool WZ>
-__global__ void __launch_bounds__(256) k_rowproj(const bf16* __restrict__ Xt, const bf16* __restrict__ Y,
-                                                 const bf16* __restrict__ Z, float* __restrict__ out,
-                                                 float* __restrict__ part, int N, int rows,
-                                                 const int* done) {
-  if (skip(done)) return;
+// and the block's weight-gradient partials (Y = the gradient of the layer's
+// pre-activations, Z = the layer's input)
+//   part[blk][a][c] = sum_r,y Z[r][y][a] Y[r][y][c],  part[blk][C*C + c] = sum_r,y Y[r][y][c].
+// DZ: Y is dh4, formed from dz (dproj8); otherwise Y is read.
+//
+// Bound by the reads of Y and Z (128 bytes per cell, with DZ 72).  The row
+// is staged in LDS row-major, 64 bytes per cell, and both operands whose K
+// runs over y come from transposing reads; 8 rows apart, the two 32-byte
+// halves of a cell are exchanged, so that the 8 rows a half wave touches lie
+// in different banks.  Waves 0-3 hold the four 16 x 16 tiles of out, waves
+// 4-7 those of the weight gradient; the next row's NC 16-byte items per
+// thread are in flight meanwhile.  NC = ceil(N / 128), in steps 1, 2, 4, 8;
+// the 16 rows of Xt a wave needs stay in its registers up to NC = 2
+// (beyond, they would leave room for one work-group per CU).  At N = 256, 8
+// samples: 16 us (15 with DZ), 4.2 TB/s; with 16-bit LDS reads for the
+// operands, one work-group of 4 waves per CU and no loads in flight during
+// the products the same work took 38 us.  512 work-groups (two per CU): 1,024
+// take 18 us and twice the partials.
+template <int NC, bool DZ>
+__global__ void __launch_bounds__(512, NC <= 4 ? 4 : 2) k_back_rows(const bf16* __restrict__ Xt, const bf16* __restrict__ Y,
+                                                   const float2* __restrict__ dz, const float* __restrict__ Wout,
+                                                   float is, const bf16* __restrict__ Z,
+                                                   float* __restrict__ out, float* __restrict__ part, int N,
+                                                   int rows) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   bf16* ly = reinterpret_cast<bf16*>(smem_raw);
-  bf16* lz = ly + (long)N * S;
+  bf16* lz = ly + (long)N * C;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int i = lane & 15, g = lane >> 4;
-  const int ta = w >> 1, tc = w & 1;
-  f32x4 accz = {0.f, 0.f, 0.f, 0.f};
-  float accb = 0.f;
-  for (int r = blockIdx.x; r < rows; r += gridDim.x) {
-    const bf16* Yr = Y + (long)r * N * C;
-    const bf16* Zr = WZ ? Z + (long)r * N * C : nullptr;
-    __syncthreads();
-    for (int q = tid; q < N * 4; q += 256) {
-      const int y = q >> 2, c8 = (q & 3) * 8;
-      const u32x4 val = *(const u32x4*)(Yr + (long)y * C + c8);
-      u32x2* d = reinterpret_cast<u32x2*>(ly + y * S + c8);
-      d[0] = u32x2{val[0], val[1]};
-      d[1] = u32x2{val[2], val[3]};
-      if (WZ) {
-        const u32x4 vz = *(const u32x4*)(Zr + (long)y * C + c8);
-        u32x2* dz = reinterpret_cast<u32x2*>(lz + y * S + c8);
-        dz[0] = u32x2{vz[0], vz[1]};
-        dz[1] = u32x2{vz[2], vz[3]};
-      }
-    }
-    __syncthreads();
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int y0 = 0; y0 < N; y0 += 32) {
-      const bf16x8 a = ld8(Xt + (long)(16 * ta + i) * N + y0 + 8 * g);
-      bf16x8 b;
+  const int ta = (w >> 1) & 1, tc = w & 1;
+  const bool wz = w >= 4;
+  const int items = N * 4;
+  const int c8 = (tid & 3) * 8;  // this thread's channels (512 % 4 == 0)
+  constexpr bool XR = NC <= 2;
+  constexpr int NX = XR ? 4 * NC : 1;  // K steps of 32 held
+  bf16x8 xa[NX];
+  const bf16* xrow = Xt + (long)(16 * ta + i) * N + 8 * g;
+  if (XR) {
 #pragma unroll
-      for (int v = 0; v < 8; ++v) b[v] = ly[(y0 + 8 * g + v) * S + 16 * tc + i];
-      acc = mma(a, b, acc);
-      if (WZ) {
-        bf16x8 az;
-#pragma unroll
-        for (int v = 0; v < 8; ++v) az[v] = lz[(y0 + 8 * g + v) * S + 16 * ta + i];
-        accz = mma(az, b, accz);
-      }
-    }
-    float* o = out + (long)r * C * C;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) o[(16 * ta + 4 * g + v) * C + 16 * tc + i] = acc[v];
-    if (WZ)
-      for (int y = tid >> 5; y < N; y += 8) accb += (float)ly[y * S + (tid & 31)];
+    for (int u = 0; u < NX; ++u) xa[u] = ld8(xrow + (32 * u < N ? 32 * u : 0));
   }
-  if (WZ) {
-    float* pp = part + (long)blockIdx.x * (C * C + C);
+  float wo[16];
+  if (DZ) dproj_weights(Wout, c8, wo);
+  u32x4 vy[NC], vz[NC];
+  float2 vd[NC];
+  auto load = [&](long r) {
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      int q = tid + 512 * k;
+      q = q < items ? q : items - 1;
+      if (DZ)
+        vd[k] = dz[r * N + (q >> 2)];
+      else
+        vy[k] = *reinterpret_cast<const u32x4*>(Y + r * N * C + (long)q * 8);
+      vz[k] = *reinterpret_cast<const u32x4*>(Z + r * N * C + (long)q * 8);
+    }
+  };
+  // operand addresses within a K step of 32 rows (rows y with (y >> 3) & 1 == g & 1)
+  const int row8 = (8 * g + (i >> 2)) * C + 4 * (i & 3);
+  const bf16* pb = ly + row8 + 16 * (tc ^ (g & 1));
+  const bf16* pz = lz + row8 + 16 * (ta ^ (g & 1));
+  f32x4 accz = {0.f, 0.f, 0.f, 0.f};
+  float accb[8] = {};
+  load(blockIdx.x);
+  for (int r = blockIdx.x; r < rows; r += gridDim.x) {
+    __syncthreads();  // the previous row has been read
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      const int q = tid + 512 * k;
+      if (DZ) vy[k] = __builtin_bit_cast(u32x4, dproj8(vd[k], is, c8, wo));
+      if (q < items) {
+        const int y = q >> 2, o = y * C + (c8 ^ ((y & 8) << 1));
+        *reinterpret_cast<u32x4*>(ly + o) = vy[k];
+        *reinterpret_cast<u32x4*>(lz + o) = vz[k];
+        const bf16x8 hv = __builtin_bit_cast(bf16x8, vy[k]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) accb[j] += (float)hv[j];
+      }
+    }
+    __syncthreads();
+    load(r + (int)gridDim.x < rows ? r + gridDim.x : r);
+    if (!wz) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      if (XR) {
+#pragma unroll
+        for (int u = 0; u < NX; ++u)
+          if (32 * u < N) acc = mma(xa[u], ld_tr(pb + 32 * u * C, pb + 32 * u * C + 4 * C), acc);
+      } else {
+        for (int y0 = 0; y0 < N; y0 += 64) {  // N % 64 == 0
+          const bf16x8 a0 = ld8(xrow + y0), a1 = ld8(xrow + y0 + 32);
+          acc = mma(a0, ld_tr(pb + y0 * C, pb + y0 * C + 4 * C), acc);
+          acc = mma(a1, ld_tr(pb + (y0 + 32) * C, pb + (y0 + 32) * C + 4 * C), acc);
+        }
+      }
+      float* o = out + (long)r * C * C;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) o[(16 * ta + 4 * g + v) * C + 16 * tc + i] = acc[v];
+    } else {
+#pragma unroll 4
+      for (int y0 = 0; y0 < N; y0 += 32)
+        accz = mma(ld_tr(pz + y0 * C, pz + y0 * C + 4 * C), ld_tr(pb + y0 * C, pb + y0 * C + 4 * C), accz);
+    }
+  }
+  float* pp = part + (long)blockIdx.x * (C * C + C);
+  if (wz) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) pp[(16 * ta + 4 * g + v) * C + 16 * tc + i] = accz[v];
-    __shared__ float sb[256];
-    sb[tid] = accb;
-    __syncthreads();
-    if (tid < C) {
-      float sacc = 0.f;
-      for (int k = 0; k < 8; ++k) sacc += sb[tid + 32 * k];
-      pp[C * C + tid] = sacc;
-    }
+  }
+  __shared__ float sb[8][C];
+  lane16_sums<8, 4>(accb, lane >> 2);
+  if (!(lane & 4)) sb[w][c8 + (lane >> 3)] = accb[0];
+  __syncthreads();
+  if (tid < C) {
+    float t = 0.f;
+    for (int k = 0; k < 8; ++k) t += sb[k][tid];
+    pp[C * C + tid] = t;
   }
 }
 
@@ -343,16 +458,18 @@ __global__ void __launch_bounds__(256) k_mix(const float2* __restrict__ upart, i
 //   B_x = (S1 - S2) + i (S3 + S4),  B_{N-x} = (S1 + S2) + i (S4 - S3).
 // Pair p >= 1 is rows (p, N - p); pair 0 is rows 0 and N/2, whose twiddles
 // are 1 and (-1)^kx = (-1)^kxi (N even, kx = kxi or N - 32 + kxi).  The
-// block's 2 XP x 32 x 32 outputs are assembled in LDS and leave as 16-byte
-// stores of whole 2 KiB rows.  Every block reads its sample's 128 KiB of
-// modes: XP = 8 from 8 vectors and XP = 4 from 4 (fewer reads), XP = 1 for
-// fewer (enough blocks).
+// block's 2 XP x 32 x 32 outputs are assembled in LDS, where the 16-byte
+// chunk j of channel ch is at j ^ (ch / 4 % 4) (a wave's writes, one word per
+// channel, then touch 32 banks and not 4), and leave as 16-byte stores of
+// whole 2 KiB rows.  Every block reads its sample's 128 KiB of modes, so XP
+// is the largest that still gives every CU a block (N = 256, 8 samples: XP 4
+// takes 6.8 us; XP 8, half the CUs, and unswizzled 2-byte LDS writes 10.2).
 template <int XP>
 __global__ void __launch_bounds__(512) k_invx(const float2* __restrict__ V, bf16* __restrict__ out,
                                               const float2* __restrict__ Ex, int N, const int* done) {
   if (skip(done)) return;
   __shared__ float2 se[XP][KX];
-  __shared__ __align__(16) bf16 lt[2 * XP][C][C];
+  __shared__ __align__(16) unsigned int lt[2 * XP][C * C / 2];  // pairs (2ky, 2ky + 1)
   const int p0 = blockIdx.x * XP, b = blockIdx.z;
   const int tid = threadIdx.x;
   if (tid < XP * KX) {
@@ -360,6 +477,11 @@ __global__ void __launch_bounds__(512) k_invx(const float2* __restrict__ V, bf16
     se[pl][q] = Ex[(long)q * N + p0 + pl];
   }
   const int ch = tid & 31, ky = tid >> 5;
+  const int slot = ch * (C / 2) + (ky ^ (((ch >> 2) & 3) << 2));
+  auto pack = [](float re, float im) {
+    struct P2 { bf16 v[2]; } p{{(bf16)re, (bf16)im}};
+    return __builtin_bit_cast(unsigned int, p);
+  };
   float2 vq[KX];
 #pragma unroll
   for (int q = 0; q < KX; ++q) vq[q] = V[(((long)b * KX + q) * KY + ky) * C + ch];
@@ -375,11 +497,9 @@ __global__ void __launch_bounds__(512) k_invx(const float2* __restrict__ V, bf16
       s3 += vq[q].x * e.y;
       s4 += vq[q].y * e.x;
     }
-    lt[pl][ch][2 * ky] = (bf16)(s1 - s2);
-    lt[pl][ch][2 * ky + 1] = (bf16)(s3 + s4);
+    lt[pl][slot] = pack(s1 - s2, s3 + s4);
     if (p0 + pl > 0) {
-      lt[XP + pl][ch][2 * ky] = (bf16)(s1 + s2);
-      lt[XP + pl][ch][2 * ky + 1] = (bf16)(s4 - s3);
+      lt[XP + pl][slot] = pack(s1 + s2, s4 - s3);
     } else {  // row N/2
       float t1 = 0.f, t2 = 0.f;
 #pragma unroll
@@ -387,56 +507,87 @@ __global__ void __launch_bounds__(512) k_invx(const float2* __restrict__ V, bf16
         t1 += vq[q].x - vq[q + 1].x;
         t2 += vq[q].y - vq[q + 1].y;
       }
-      lt[XP][ch][2 * ky] = (bf16)t1;
-      lt[XP][ch][2 * ky + 1] = (bf16)t2;
+      lt[XP][slot] = pack(t1, t2);
     }
   }
   __syncthreads();
   // staged row r: x = p0 + r (r < XP), else N - (p0 + r - XP), pair 0's N/2
-  const u32x4* src = reinterpret_cast<const u32x4*>(&lt[0][0][0]);
+  const u32x4* src = reinterpret_cast<const u32x4*>(&lt[0][0]);
   for (int q = tid; q < 2 * XP * C * C / 8; q += 512) {
     const int r = q / (C * C / 8), pl = r < XP ? r : r - XP;
     const int x = r < XP ? p0 + pl : (p0 + pl == 0 ? N / 2 : N - p0 - pl);
-    reinterpret_cast<u32x4*>(out + ((long)b * N + x) * C * C)[q - r * (C * C / 8)] = src[q];
+    reinterpret_cast<u32x4*>(out + ((long)b * N + x) * C * C)[q - r * (C * C / 8)] = src[q ^ ((q >> 4) & 3)];
   }
 }
 
-// Spectral weight gradient: G[kxi][ky][c][o] = sum_b conj(U[b][kxi][ky][c]) dV[b][kxi][ky][o].
-__global__ void __launch_bounds__(256) k_specgrad(const float2* __restrict__ U, const float2* __restrict__ dV,
-                                                  float2* __restrict__ G, int B) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (long)KX * KY * C * C) return;
-  const int o = (int)(e % C);
-  const int c = (int)((e / C) % C);
-  const long mode = e / (C * C);  // kxi * KY + ky
-  float2 acc = make_float2(0.f, 0.f);
-  for (int b = 0; b < B; ++b) {
-    const float2 u = U[((long)b * KX * KY + mode) * C + c];
-    const float2 d = dV[((long)b * KX * KY + mode) * C + o];
-    acc.x += u.x * d.x + u.y * d.y;
-    acc.y += u.x * d.y - u.y * d.x;
+// Spectral weight gradients of the four layers (blockIdx.y), one mode per block:
+//   G[kxi][ky][c][o] = sum_b conj(U[b][kxi][ky][c]) dV[b][kxi][ky][o].
+// Bound by the 4.2 MB a layer writes; one launch for the four layers, after
+// the last of them has its dV (10 us for 8 samples, four launches of a
+// thread per output 29).  A thread holds 2 x 2 outputs.
+struct SpecGrads {
+  const float2* U[4];
+  const float2* dV[4];
+  float2* G[4];
+};
+__global__ void __launch_bounds__(256) k_specgrad(SpecGrads t, int B) {
+  const int mode = blockIdx.x, l = blockIdx.y;  // kxi * KY + ky
+  const int o0 = (threadIdx.x & 15) * 2, c0 = (threadIdx.x >> 4) * 2;
+  const float2* U = t.U[l] + (long)mode * C + c0;
+  const float2* dV = t.dV[l] + (long)mode * C + o0;
+  constexpr long kS = (long)KX * KY * C;  // one sample's modes
+  float4 acc[2] = {};
+  auto add = [&](const float4& u, const float4& d) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const float ux = k ? u.z : u.x, uy = k ? u.w : u.y;
+      acc[k].x += ux * d.x + uy * d.y;
+      acc[k].y += ux * d.y - uy * d.x;
+      acc[k].z += ux * d.z + uy * d.w;
+      acc[k].w += ux * d.w - uy * d.z;
+    }
+  };
+  int b = 0;
+  for (; b + 8 <= B; b += 8) {
+    float4 u[8], d[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      u[k] = *reinterpret_cast<const float4*>(U + (b + k) * kS);
+      d[k] = *reinterpret_cast<const float4*>(dV + (b + k) * kS);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) add(u[k], d[k]);
   }
-  G[e] = acc;
+  for (; b < B; ++b)
+    add(*reinterpret_cast<const float4*>(U + b * kS), *reinterpret_cast<const float4*>(dV + b * kS));
+  // 8-byte stores: grad is only required to be aligned to its elements
+  float2* G = t.G[l] + ((long)mode * C + c0) * C + o0;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    G[k * C] = make_float2(acc[k].x, acc[k].y);
+    G[k * C + 1] = make_float2(acc[k].z, acc[k].w);
+  }
 }
 
 // ---------------------------------------------------------------------------
-// Per-cell GEMM with K = 64 and fused epilogue:
-//   out[p][o] = epi( sum_c P[p][c] A[o][c] + sum_k Q[y][k] R[b][x][o][k] + bias[o] )
-// EPI 0: identity, 1: GELU (pre-activation to pre_out when given),
-// 2: times GELU'(aux[p][o]).  The product is formed transposed (rows = output
-// channels, columns = 16 cells) so that lane l holds 4 consecutive channels of
-// cell l % 16 in both the B operand and the accumulator.  One wave covers 64
-// consecutive cells of a grid row.
-template <int EPI>
-__global__ void __launch_bounds__(256) k_pixel(const bf16* __restrict__ P, const bf16* __restrict__ Q,
-                                               const bf16* __restrict__ A, const bf16* __restrict__ R,
-                                               const float* __restrict__ bias, bf16* __restrict__ pre_out,
-                                               const bf16* __restrict__ aux, bf16* __restrict__ out, int N,
-                                               const int* done) {
-  if (skip(done)) return;
+// Per-cell GEMM of the backward pass (layers 3-1), K = 64:
+//   out[p][o] = (sum_c P[p][c] A[o][c] + sum_k Q[y][k] R[b][x][o][k]) GELU'(aux[p][o])
+// DZ: P is dh4, formed from dz (dproj8); otherwise P is read.  The product is
+// formed transposed (rows = output channels, columns = 16 cells) so that lane
+// l holds 4 consecutive channels of cell l % 16 in both the B operand and the
+// accumulator.  One wave covers 64 consecutive cells of a grid row: bound by
+// the 192 bytes per cell read and written (DZ: 136), so every operand of the
+// wave is in flight before its first product (21 and 17 us at N = 256, 8
+// samples: 4.8 and 4.2 TB/s).
+template <bool DZ>
+__global__ void __launch_bounds__(256) k_back_cells(const bf16* __restrict__ P, const float2* __restrict__ dz,
+                                                    const float* __restrict__ Wout, float is,
+                                                    const bf16* __restrict__ Q, const bf16* __restrict__ A,
+                                                    const bf16* __restrict__ R, const bf16* __restrict__ aux,
+                                                    bf16* __restrict__ out, int N) {
   // each wave stages its 16-cell tile (16 x 32 BF16, rows padded to 80 B) so
   // that every lane stores 16 contiguous bytes and a wave 1 KiB at once
-  __shared__ __align__(16) bf16 stage[2][4][16][40];
+  __shared__ __align__(16) bf16 stage[4][16][40];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const long wv = (long)blockIdx.x * 4 + w;  // every block is full: waves % 4 == 0
   const int segs = N / 64;
@@ -444,54 +595,119 @@ __global__ void __launch_bounds__(256) k_pixel(const bf16* __restrict__ P, const
   const int y0 = (int)(wv % segs) * 64;
   const int i = lane & 15, g = lane >> 4;
   const int rrow = lane >> 2, rcol = (lane & 3) * 8;
-  bf16x8 aw[2], ar[2];
-  float bs[2][4];
-#pragma unroll
-  for (int to = 0; to < 2; ++to) {
-    aw[to] = ld8(A + (16 * to + i) * C + 8 * g);
-    ar[to] = ld8(R + (bx * C + 16 * to + i) * C + 8 * g);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) bs[to][v] = bias ? bias[16 * to + 4 * g + v] : 0.f;
-  }
-  // all four tiles' operands in flight before the first MFMA
   bf16x8 bpt[4], bqt[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int y = y0 + 16 * t + i;
-    bpt[t] = ld8(P + (bx * N + y) * C + 8 * g);
-    bqt[t] = ld8(Q + (long)y * C + 8 * g);
-  }
+  float2 vd[4];
+  u32x2 ax[4][2];  // 4 channels of aux per accumulator
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int y = y0 + 16 * t + i;
     const long p = bx * N + y;
-    const bf16x8 bp = bpt[t];
-    const bf16x8 bq = bqt[t];
+    if (DZ)
+      vd[t] = dz[p];
+    else
+      bpt[t] = ld8(P + p * C + 8 * g);
+    bqt[t] = ld8(Q + (long)y * C + 8 * g);
+#pragma unroll
+    for (int to = 0; to < 2; ++to) ax[t][to] = *reinterpret_cast<const u32x2*>(aux + p * C + 16 * to + 4 * g);
+  }
+  bf16x8 aw[2], ar[2];
+#pragma unroll
+  for (int to = 0; to < 2; ++to) {
+    aw[to] = ld8(A + (16 * to + i) * C + 8 * g);
+    ar[to] = ld8(R + (bx * C + 16 * to + i) * C + 8 * g);
+  }
+  if (DZ) {
+    float wo[16];
+    dproj_weights(Wout, 8 * g, wo);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) bpt[t] = dproj8(vd[t], is, 8 * g, wo);
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
 #pragma unroll
     for (int to = 0; to < 2; ++to) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      acc = mma(aw[to], bp, acc);
-      acc = mma(ar[to], bq, acc);
-      const int o0 = 16 * to + 4 * g;
-      float r[4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) r[v] = acc[v] + bs[to][v];
-      if (EPI == 1) {
-        if (pre_out) st4(&stage[1][w][i][o0], r[0], r[1], r[2], r[3]);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) r[v] = gelu(r[v]);
-      } else if (EPI == 2) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) r[v] *= dgelu((float)aux[p * C + o0 + v]);
-      }
-      st4(&stage[0][w][i][o0], r[0], r[1], r[2], r[3]);
+      acc = mma(aw[to], bpt[t], acc);
+      acc = mma(ar[to], bqt[t], acc);
+      struct Q4 { bf16 v[4]; };
+      const Q4 x = __builtin_bit_cast(Q4, ax[t][to]);
+      st4(&stage[w][i][16 * to + 4 * g], acc[0] * dgelu((float)x.v[0]), acc[1] * dgelu((float)x.v[1]),
+          acc[2] * dgelu((float)x.v[2]), acc[3] * dgelu((float)x.v[3]));
     }
-    __syncthreads();
-    const long po = (bx * N + y0 + 16 * t + rrow) * C + rcol;
-    *(u32x4*)(out + po) = *(const u32x4*)&stage[0][w][rrow][rcol];
-    if (EPI == 1 && pre_out) *(u32x4*)(pre_out + po) = *(const u32x4*)&stage[1][w][rrow][rcol];
-    __syncthreads();
+    // the stage is the wave's own: LDS operations of a wave run in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    *(u32x4*)(out + (bx * N + y0 + 16 * t + rrow) * C + rcol) = *(const u32x4*)&stage[w][rrow][rcol];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
+}
+
+// The same GEMM at layer 0 (no activation below it) with the lift's
+// gradient.  dh0 is rounded to BF16 as an activation gradient is, but not
+// stored: the lift needs only
+//   part[blk] = (sum_p a_k dh0[p][c]  [k][c],  sum_p dh0[p][c])
+// with (a_0, a_1, a_2) = (chi chi_scale, s Re v, s Im v).  Waves step over
+// the 64-cell segments of all samples; a lane holds 8 channels of its cells
+// in 32 sums, joined across the block at the end.  12 us at N = 256, 8
+// samples; storing dh0 and a second kernel that read it took 30.
+__global__ void __launch_bounds__(256) k_back_lift(const bf16* __restrict__ P, const bf16* __restrict__ Q,
+                                                   const bf16* __restrict__ A, const bf16* __restrict__ R,
+                                                   const float* __restrict__ chi, float chi_scale,
+                                                   const float2* __restrict__ v, float s,
+                                                   float* __restrict__ part, int N, long nseg) {
+  __shared__ float red[4][4 * C];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int segs = N / 64;
+  const int i = lane & 15, g = lane >> 4;
+  bf16x8 aw[2];
+#pragma unroll
+  for (int to = 0; to < 2; ++to) aw[to] = ld8(A + (16 * to + i) * C + 8 * g);
+  float sum[32] = {};  // [a_0, a_1, a_2, 1][8 channels]
+  for (long wv = (long)blockIdx.x * 4 + w; wv < nseg; wv += (long)gridDim.x * 4) {
+    const long bx = wv / segs;  // sample * N + x
+    const int y0 = (int)(wv - bx * segs) * 64;
+    bf16x8 bpt[4], bqt[4], ar[2];
+    float cv[4];
+    float2 xv[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int y = y0 + 16 * t + i;
+      const long p = bx * N + y;
+      bpt[t] = ld8(P + p * C + 8 * g);
+      bqt[t] = ld8(Q + (long)y * C + 8 * g);
+      cv[t] = chi[p];
+      xv[t] = v[p];
+    }
+#pragma unroll
+    for (int to = 0; to < 2; ++to) ar[to] = ld8(R + (bx * C + 16 * to + i) * C + 8 * g);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float a[3] = {cv[t] * chi_scale, xv[t].x * s, xv[t].y * s};
+#pragma unroll
+      for (int to = 0; to < 2; ++to) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        acc = mma(aw[to], bpt[t], acc);
+        acc = mma(ar[to], bqt[t], acc);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float d = (float)(bf16)acc[q];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) sum[8 * k + 4 * to + q] += a[k] * d;
+          sum[24 + 4 * to + q] += d;
+        }
+      }
+    }
+  }
+  lane16_sums<32, 1>(sum, i);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int k = (2 * i + j) >> 3, q = (2 * i + j) & 7;
+    red[w][k * C + 16 * (q >> 2) + 4 * g + (q & 3)] = sum[j];
+  }
+  __syncthreads();
+  if (tid < 4 * C)
+    part[(long)blockIdx.x * 4 * C + tid] = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
 }
 
 // ---------------------------------------------------------------------------
@@ -769,7 +985,7 @@ __global__ void __launch_bounds__(512) k_lift_rows(LiftIn L, float2* vw, bf16* _
 //      e^{+2 pi i kx x/N}), which saves k_invx's launch but reads all of
 //      Vm[k] (128 KiB, from L2) per row: the better choice for one sample;
 //   2. h'[y] = GELU([h[y], F_y] [W; B_x] + b) for the row's N cells (16-cell
-//      tiles t = wave + 8u, as in k_pixel) to out (each lane stores the 4
+//      tiles t = wave + 8u) to out (each lane stores the 4
 //      channels it holds of one cell, 8 bytes) and channel-major into LDS
 //      (pre-activations to pre_out when given, for training);
 //   3. the row projection of h' into Anext[x], with the basis staged in LDS.
@@ -1143,7 +1359,7 @@ __global__ void __launch_bounds__(512) k_cell_rows_lift(LiftIn L, const bf16* __
 //   h4 = [h3, F_y] [W; B_x] + b,  z = s_id vv / *vnrm + (h4 W_out + b_out) / s
 // in FP32 (vnrm null: no scaling); h4 goes to hout as BF16 when given
 // (training).  Sample k reads vv and writes z at k * sV, k * sZ, its norm at
-// vnrm + k * sNrm bytes.  Grid as k_pixel.
+// vnrm + k * sNrm bytes.  One wave per 64 cells, as k_back_cells.
 __global__ void __launch_bounds__(256) k_cell_proj(const bf16* __restrict__ P, const bf16* __restrict__ Q,
                                                    const bf16* __restrict__ A, const bf16* __restrict__ R,
                                                    const float* __restrict__ bias, bf16* __restrict__ hout,
@@ -1223,101 +1439,104 @@ __global__ void __launch_bounds__(256) k_cell_proj(const bf16* __restrict__ P, c
 }
 
 
-// Block sums of NV per-thread values (every thread of the 256 passes vals);
-// thread k < NV writes the block's sum of value k to dst[k].
-template <int NV>
-__device__ inline void block_sums(const float* vals, float* dst) {
-  __shared__ float red[4][NV];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+// Gradients of the projection and of the identity path, with d = dz / s:
+//   part[blk] = (sum_p h[p][c] d_j  [c][j],  sum_p d_j,  sum_p Re(conj(dz) v))
+// Bound by the read of h, 64 bytes per cell: four lanes share a cell, 8
+// channels each, so a wave reads 1 KiB at once: 12 us at N = 256, 8 samples
+// (512 blocks 17; with one lane per cell and dh4 stored 26).
+__global__ void __launch_bounds__(256) k_proj_bwd(const float2* __restrict__ dz, const bf16* __restrict__ h,
+                                                  const float2* __restrict__ v, float is,
+                                                  float* __restrict__ part, long total) {
+  __shared__ float red[4][2 * C + 3];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int c8 = (tid & 3) * 8;
+  float acc[16] = {}, s0 = 0.f, s1 = 0.f, s2 = 0.f;
+  constexpr int U = 4;  // cells per thread and step, in flight together
+  const long step = (long)gridDim.x * 64;
+  for (long p0 = (long)blockIdx.x * 64 + (tid >> 2); p0 < total; p0 += U * step) {
+    bf16x8 hv[U];
+    float2 d[U], vv[U];
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const float t = wave_sum_f(vals[k]);
-    if (lane == 0) red[w][k] = t;
+    for (int u = 0; u < U; ++u) {
+      const long p = p0 + u * step < total ? p0 + u * step : total - 1;
+      hv[u] = ld8(h + p * C + c8);
+      d[u] = dz[p];
+      vv[u] = v[p];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (p0 + u * step >= total) break;
+      const float d0 = d[u].x * is, d1 = d[u].y * is;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const float x = (float)hv[u][k];
+        acc[2 * k] += x * d0;
+        acc[2 * k + 1] += x * d1;
+      }
+      s0 += d0;
+      s1 += d1;
+      s2 += d[u].x * vv[u].x + d[u].y * vv[u].y;
+    }
+  }
+  auto join = [&](float t) {
+#pragma unroll
+    for (int m = 4; m < 64; m *= 2) t += __shfl_xor(t, m, 64);
+    return t;
+  };
+  lane16_sums<16, 4>(acc, lane >> 2);
+  red[w][2 * c8 + (lane >> 2)] = acc[0];
+  s0 = join(s0);
+  s1 = join(s1);
+  s2 = join(s2);
+  if (lane == 0) {
+    red[w][2 * C] = s0;
+    red[w][2 * C + 1] = s1;
+    red[w][2 * C + 2] = s2;
   }
   __syncthreads();
-  for (int k = threadIdx.x; k < NV; k += 256) dst[k] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+  if (tid < 2 * C + 3)
+    part[(long)blockIdx.x * (2 * C + 3) + tid] = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
 }
 
-// projection backward: dz = dL/dz (re, im packed) -> d = dz / s;
-//   dh[p][c] = d0 W_out[c][0] + d1 W_out[c][1]   (BF16)
-//   part[blk] = (sum_p h[p][c] d_j  [c][j],  sum_p d_j,  sum_p Re(conj(dz) vv))
-__global__ void __launch_bounds__(256) k_proj_bwd(const float2* __restrict__ dz, const bf16* __restrict__ h,
-                                                  const float* __restrict__ P, const float2* __restrict__ v,
-                                                  float s, bf16* __restrict__ dh, float* __restrict__ part,
-                                                  long total) {
-  const float* W = P + kOffOut;
-  float acc[2 * C + 3];
-#pragma unroll
-  for (int k = 0; k < 2 * C + 3; ++k) acc[k] = 0.f;
-  const float is = 1.f / s;
-  for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < total; p += (long)gridDim.x * 256) {
-    const float2 d = dz[p];
-    const float d0 = d.x * is, d1 = d.y * is;
-#pragma unroll
-    for (int c8 = 0; c8 < C; c8 += 8) {
-      const bf16x8 hv = ld8(h + p * C + c8);
-      float r[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int c = c8 + k;
-        const float x = (float)hv[k];
-        acc[2 * c] += x * d0;
-        acc[2 * c + 1] += x * d1;
-        r[k] = d0 * W[2 * c] + d1 * W[2 * c + 1];
-      }
-      st4(dh + p * C + c8, r[0], r[1], r[2], r[3]);
-      st4(dh + p * C + c8 + 4, r[4], r[5], r[6], r[7]);
-    }
-    acc[2 * C] += d0;
-    acc[2 * C + 1] += d1;
-    const float2 vv = v[p];
-    acc[2 * C + 2] += d.x * vv.x + d.y * vv.y;
-  }
-  block_sums<2 * C + 3>(acc, part + (long)blockIdx.x * (2 * C + 3));
-}
-
-// lift backward: part[blk] = (sum_p a_i dh0[p][c]  [i][c],  sum_p dh0[p][c])
-__global__ void __launch_bounds__(256) k_lift_bwd(const bf16* __restrict__ dh0, const float* __restrict__ chi,
-                                                  float chi_scale, const float2* __restrict__ v, float s,
-                                                  float* __restrict__ part, long total) {
-  float acc[4 * C];
-#pragma unroll
-  for (int k = 0; k < 4 * C; ++k) acc[k] = 0.f;
-  for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < total; p += (long)gridDim.x * 256) {
-    const float2 vv = v[p];
-    const float a[3] = {chi[p] * chi_scale, vv.x * s, vv.y * s};
-#pragma unroll
-    for (int c8 = 0; c8 < C; c8 += 8) {
-      const bf16x8 hv = ld8(dh0 + p * C + c8);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float d = (float)hv[k];
-        acc[c8 + k] += a[0] * d;
-        acc[C + c8 + k] += a[1] * d;
-        acc[2 * C + c8 + k] += a[2] * d;
-        acc[3 * C + c8 + k] += d;
-      }
-    }
-  }
-  block_sums<4 * C>(acc, part + (long)blockIdx.x * 4 * C);
-}
-
-// out[k] = sum_g part[g * width + k]: 64 outputs per block, 16 strided
-// slices of g per output combined in a fixed order.
-__global__ void __launch_bounds__(1024) k_reduce_part(const float* __restrict__ part, int G, int width,
-                                                      float* __restrict__ out) {
+// out[k] = sum_g part[g * width + k] for every segment of the backward pass
+// (projection, the layers' weights and biases, lift) in one launch: 64 outputs per
+// block, 16 strided slices of g per output combined in a fixed order, sixteen
+// loads of a slice in flight: 8 us, where a launch per reduction took 6 x 6.
+struct ReduceSeg {
+  const float* part;
+  float* out;
+  int G, width, block0;  // block0: the segment's first block
+};
+constexpr int kReduceSegs = 6;
+struct ReduceList {
+  ReduceSeg seg[kReduceSegs];
+};
+__global__ void __launch_bounds__(1024) k_reduce_part(ReduceList list) {
   __shared__ float red[16][65];
+  ReduceSeg q = list.seg[0];
+#pragma unroll
+  for (int j = 1; j < kReduceSegs; ++j)
+    if ((int)blockIdx.x >= list.seg[j].block0) q = list.seg[j];
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  const int k = blockIdx.x * 64 + tx;
+  const int k = (blockIdx.x - q.block0) * 64 + tx;
   float s = 0.f;
-  if (k < width)
-    for (int gi = ty; gi < G; gi += 16) s += part[(long)gi * width + k];
+  if (k < q.width)
+    for (int g0 = ty; g0 < q.G; g0 += 256) {
+      float v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int gi = g0 + 16 * u;
+        v[u] = q.part[(long)(gi < q.G ? gi : ty) * q.width + k];
+      }
+#pragma unroll
+      for (int u = 0; u < 16; ++u) s += g0 + 16 * u < q.G ? v[u] : 0.f;
+    }
   red[ty][tx] = s;
   __syncthreads();
-  if (ty == 0 && k < width) {
+  if (ty == 0 && k < q.width) {
     float t = 0.f;
-    for (int q = 0; q < 16; ++q) t += red[q][tx];
-    out[k] = t;
+    for (int e = 0; e < 16; ++e) t += red[e][tx];
+    q.out[k] = t;
   }
 }
 
@@ -1357,11 +1576,10 @@ struct cgm_fno {
   float* A = nullptr;             // [B][N][32][32]
   float2* upart = nullptr;        // [B][N/XC][32][16][32]
   float2* U[4] = {};              // [B][32][16][32] (training)
-  float2* dV = nullptr;           // [B][32][16][32]
+  float2* dV[4] = {};             // [B][32][16][32] per layer
   float2* Vm = nullptr;           // [B][32][16][32] mixed modes
   bf16* Bt = nullptr;             // [B][N][32][32]
   float* part = nullptr;          // reduction partials
-  int Gp = 0;                     // blocks of the reducing kernels
   // saved by the last training forward
   int fwd_batch = 0;
   const float* chi_in = nullptr;
@@ -1373,42 +1591,59 @@ namespace {
 int fno_free(cgm_fno* f) {
   void* ptrs[] = {f->Wt, f->Wn, f->Ft, f->Fy, f->Ex, f->h[0], f->h[1], f->h[2], f->h[3], f->h[4],
                   f->pre[0], f->pre[1], f->pre[2], f->dh[0], f->dh[1], f->A, f->upart, f->U[0],
-                  f->U[1], f->U[2], f->U[3], f->dV, f->Vm, f->Bt, f->part};
+                  f->U[1], f->U[2], f->U[3], f->dV[0], f->dV[1], f->dV[2], f->dV[3], f->Vm, f->Bt, f->part};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   return CGM_SUCCESS;
 }
 
-int rowproj_grid(int rows) { return rows < 256 ? rows : 256; }
+// Blocks of the backward pass's reducing kernels: two row kernels per CU
+// (each holds the next row's loads in flight), enough waves of the two cell
+// kernels to fill the chip; each block leaves one set of partials.
+int back_rows_grid(int rows) { return rows < 512 ? rows : 512; }
+int back_cells_grid(long nseg) { return nseg / 4 < 1024 ? (int)(nseg / 4) : 1024; }
+constexpr int kProjGrid = 1024;
+constexpr int kRowPart = C * C + C, kProjPart = 2 * C + 3, kLiftPart = 4 * C;
 
-template <bool WZ>
-int launch_rowproj(cgm_fno* f, hipStream_t st, const bf16* Y, const bf16* Z, float* out, int B,
-                   const int* done) {
+// k_back_rows of a layer: Y, or dz with the output weights when Y is null.
+template <int NC>
+void launch_back_rows_n(const cgm_fno* f, hipStream_t st, const bf16* Y, const float2* dz, const bf16* Z,
+                        float* part, int B) {
   const int rows = B * f->N;
-  const int G = WZ ? f->Gp : rows;
-  const size_t lds = (size_t)(WZ ? 2 : 1) * f->N * S * sizeof(bf16);
-  hipLaunchKernelGGL((k_rowproj<WZ>), dim3(G), dim3(256), lds, st, f->Ft, Y, Z, out, f->part, f->N, rows,
-                     done);
+  const size_t lds = (size_t)2 * f->N * C * sizeof(bf16);
+  const float* Wout = f->params + kOffOut;
+  const float is = 1.f / (float)f->N;
+  const dim3 grid(back_rows_grid(rows)), block(512);
+  if (Y)
+    hipLaunchKernelGGL((k_back_rows<NC, false>), grid, block, lds, st, f->Ft, Y, dz, Wout, is, Z, f->A, part,
+                       f->N, rows);
+  else
+    hipLaunchKernelGGL((k_back_rows<NC, true>), grid, block, lds, st, f->Ft, Y, dz, Wout, is, Z, f->A, part,
+                       f->N, rows);
+}
+int launch_back_rows(const cgm_fno* f, hipStream_t st, const bf16* Y, const float2* dz, const bf16* Z, float* part,
+                     int B) {
+  if (f->N <= 128)
+    launch_back_rows_n<1>(f, st, Y, dz, Z, part, B);
+  else if (f->N <= 256)
+    launch_back_rows_n<2>(f, st, Y, dz, Z, part, B);
+  else if (f->N <= 512)
+    launch_back_rows_n<4>(f, st, Y, dz, Z, part, B);
+  else
+    launch_back_rows_n<8>(f, st, Y, dz, Z, part, B);
   CGM_HIP(hipGetLastError());
   return CGM_SUCCESS;
 }
 
-template <int EPI>
-int launch_pixel(cgm_fno* f, hipStream_t st, const bf16* P, const bf16* A, const bf16* R, const float* bias,
-                 bf16* pre_out, const bf16* aux, bf16* out, int B, const int* done) {
-  const long waves = (long)B * f->n / 64;  // N % 64 == 0, so waves % 4 == 0
-  CGM_CHECK(waves % 4 == 0, CGM_ERROR_UNSUPPORTED, "cell GEMM needs N %% 64 == 0");
-  hipLaunchKernelGGL((k_pixel<EPI>), dim3((unsigned)(waves / 4)), dim3(256), 0, st, P, f->Fy, A, R, bias, pre_out,
-                     aux, out, f->N, done);
-  CGM_HIP(hipGetLastError());
-  return CGM_SUCCESS;
-}
-
+// the most row pairs per work-group that still leave 256 of them, one per CU
 void launch_invx(cgm_fno* f, hipStream_t st, int B, const int* done) {
-  if (B >= 8)  // every work-group reads its vector's 128 KiB of modes: fewer, larger ones
+  const int pairs = f->N / 2 * B;
+  if (pairs >= 8 * 256)
     hipLaunchKernelGGL(k_invx<8>, dim3(f->N / 16, 1, B), dim3(512), 0, st, f->Vm, f->Bt, f->Ex, f->N, done);
-  else if (B >= 4)
+  else if (pairs >= 4 * 256)
     hipLaunchKernelGGL(k_invx<4>, dim3(f->N / 8, 1, B), dim3(512), 0, st, f->Vm, f->Bt, f->Ex, f->N, done);
+  else if (pairs >= 2 * 256)
+    hipLaunchKernelGGL(k_invx<2>, dim3(f->N / 4, 1, B), dim3(512), 0, st, f->Vm, f->Bt, f->Ex, f->N, done);
   else
     hipLaunchKernelGGL(k_invx<1>, dim3(f->N / 2, 1, B), dim3(512), 0, st, f->Vm, f->Bt, f->Ex, f->N, done);
 }
@@ -1569,41 +1804,59 @@ cgm_context* fno_context(const cgm_fno* f) { return f->ctx; }
 static int fno_backward(cgm_fno* f, const float2* dz, float* grad) {
   hipStream_t st = f->ctx->stream;
   const int B = f->fwd_batch;
-  const long total = (long)B * f->n;
-  const float s = (float)f->N;
+  const long total = (long)B * f->n, nseg = total / 64;  // N % 64 == 0, so nseg % 4 == 0
+  const int rows = B * f->N;
+  const float s = (float)f->N, is = 1.f / s;
+  const float* Wout = f->params + kOffOut;
   int rc;
-  const int Gr = 256;
-  // projection
-  hipLaunchKernelGGL(k_proj_bwd, dim3(Gr), dim3(256), 0, st, dz, f->h[4], f->params, f->v_in, s, f->dh[0], f->part,
-                     total);
-  hipLaunchKernelGGL(k_reduce_part, dim3(2), dim3(1024), 0, st, f->part, Gr, 2 * C + 3, grad + kOffOut);
+  // partials of every reduction, summed by one launch at the end
+  ReduceList list;
+  float* part = f->part;
+  int nb = 0, ns = 0;
+  auto segment = [&](int G, int width, float* out) {
+    float* p = part;
+    list.seg[ns++] = ReduceSeg{p, out, G, width, nb};
+    nb += (width + 63) / 64;
+    part += (size_t)G * width;
+    return p;
+  };
+  SpecGrads sg;
+  hipLaunchKernelGGL(k_proj_bwd, dim3(kProjGrid), dim3(256), 0, st, dz, f->h[4], f->v_in, is,
+                     segment(kProjGrid, kProjPart, grad + kOffOut), total);
   CGM_HIP(hipGetLastError());
-  // layer 3 has no activation: dPre_3 = dh4
-  int cur = 0;
+  // layer 3 has no activation: its pre-activation gradient is dh4, which its
+  // kernels form from dz
+  const bf16* dpre = nullptr;
   for (int l = 3; l >= 0; --l) {
     const float* Lp = f->params + layer_off(l);
     float* Lg = grad + layer_off(l);
-    const bf16* dpre = f->dh[cur];
     // g_B rows (basis F), dW_l and db_l partials
-    if ((rc = launch_rowproj<true>(f, st, dpre, f->h[l], f->A, B, nullptr))) return rc;
-    hipLaunchKernelGGL(k_reduce_part, dim3((C * C + C + 63) / 64), dim3(1024), 0, st, f->part, f->Gp, C * C + C,
-                       Lg);
+    if ((rc = launch_back_rows(f, st, dpre, dz, f->h[l], segment(back_rows_grid(rows), kRowPart, Lg), B)))
+      return rc;
     // spectral adjoint: dV (saved), dA rows into Bt
-    if ((rc = spectral(f, st, (const float2*)(Lp + C * C + C), f->dV, true, B, nullptr))) return rc;
-    hipLaunchKernelGGL(k_specgrad, dim3(KX * KY * C * C / 256), dim3(256), 0, st, f->U[l], f->dV,
-                       (float2*)(Lg + C * C + C), B);
-    CGM_HIP(hipGetLastError());
+    if ((rc = spectral(f, st, (const float2*)(Lp + C * C + C), f->dV[l], true, B, nullptr))) return rc;
+    sg.U[l] = f->U[l];
+    sg.dV[l] = f->dV[l];
+    sg.G[l] = (float2*)(Lg + C * C + C);
     const bf16* Wl = f->Wn + l * C * C;
-    if (l > 0)
-      rc = launch_pixel<2>(f, st, dpre, Wl, f->Bt, nullptr, nullptr, f->pre[l - 1], f->dh[cur ^ 1], B, nullptr);
-    else
-      rc = launch_pixel<0>(f, st, dpre, Wl, f->Bt, nullptr, nullptr, nullptr, f->dh[cur ^ 1], B, nullptr);
-    if (rc) return rc;
-    cur ^= 1;
+    bf16* dnext = f->dh[l & 1];
+    const dim3 grid((unsigned)(nseg / 4));
+    if (l == 3)
+      hipLaunchKernelGGL(k_back_cells<true>, grid, dim3(256), 0, st, dpre, dz, Wout, is, f->Fy, Wl, f->Bt,
+                         f->pre[l - 1], dnext, f->N);
+    else if (l > 0)
+      hipLaunchKernelGGL(k_back_cells<false>, grid, dim3(256), 0, st, dpre, dz, Wout, is, f->Fy, Wl, f->Bt,
+                         f->pre[l - 1], dnext, f->N);
+    else {
+      const int G = back_cells_grid(nseg);
+      hipLaunchKernelGGL(k_back_lift, dim3(G), dim3(256), 0, st, dpre, f->Fy, Wl, f->Bt, f->chi_in, f->chi_scale,
+                         f->v_in, s, segment(G, kLiftPart, grad), f->N, nseg);
+    }
+    CGM_HIP(hipGetLastError());
+    dpre = dnext;
   }
-  hipLaunchKernelGGL(k_lift_bwd, dim3(Gr), dim3(256), 0, st, f->dh[cur], f->chi_in, f->chi_scale, f->v_in, s,
-                     f->part, total);
-  hipLaunchKernelGGL(k_reduce_part, dim3(2), dim3(1024), 0, st, f->part, Gr, 4 * C, grad);
+  hipLaunchKernelGGL(k_specgrad, dim3(KX * KY, 4), dim3(256), 0, st, sg, B);
+  hipLaunchKernelGGL(k_reduce_part, dim3(nb), dim3(1024), 0, st, list);
   CGM_HIP(hipGetLastError());
   return CGM_SUCCESS;
 }
@@ -1649,13 +1902,12 @@ extern "C" int cgm_fno_create(cgm_ctx_t c, int batch, float chi_scale, cgm_fno_t
   alloc((void**)&f->A, sizeof(float) * (size_t)batch * N * C * C);
   alloc((void**)&f->upart, sizeof(float2) * (size_t)batch * (N / XC) * KX * KY * C);
   for (int l = 0; l < 4; ++l) alloc((void**)&f->U[l], sizeof(float2) * (size_t)batch * KX * KY * C);
-  alloc((void**)&f->dV, sizeof(float2) * (size_t)batch * KX * KY * C);
+  for (int l = 0; l < 4; ++l) alloc((void**)&f->dV[l], sizeof(float2) * (size_t)batch * KX * KY * C);
   alloc((void**)&f->Vm, sizeof(float2) * (size_t)batch * KX * KY * C);
   alloc((void**)&f->Bt, sizeof(bf16) * (size_t)batch * N * C * C);
-  f->Gp = rowproj_grid(batch * N);
-  size_t pw = (size_t)f->Gp * (C * C + C);
-  if (pw < (size_t)256 * 4 * C) pw = (size_t)256 * 4 * C;
-  alloc((void**)&f->part, sizeof(float) * pw);
+  alloc((void**)&f->part, sizeof(float) * ((size_t)4 * back_rows_grid(batch * N) * kRowPart +
+                                           (size_t)kProjGrid * kProjPart +
+                                           (size_t)back_cells_grid(batch * f->n / 64) * kLiftPart));
   if (rc) {
     fno_free(f);
     delete f;
@@ -1682,10 +1934,13 @@ extern "C" int cgm_fno_create(cgm_ctx_t c, int batch, float chi_scale, cgm_fno_t
   CGM_HIP(hipMemcpy(f->Ft, ft.data(), sizeof(bf16) * ft.size(), hipMemcpyHostToDevice));
   CGM_HIP(hipMemcpy(f->Fy, fy.data(), sizeof(bf16) * fy.size(), hipMemcpyHostToDevice));
   CGM_HIP(hipMemcpy(f->Ex, ex.data(), sizeof(float2) * ex.size(), hipMemcpyHostToDevice));
-  const size_t lds2 = (size_t)2 * N * S * sizeof(bf16);
-  CGM_HIP(hipFuncSetAttribute((const void*)k_rowproj<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2));
-  CGM_HIP(hipFuncSetAttribute((const void*)k_rowproj<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)(lds2 / 2)));
+  const void* backk[] = {(const void*)k_back_rows<1, false>, (const void*)k_back_rows<1, true>,
+                         (const void*)k_back_rows<2, false>, (const void*)k_back_rows<2, true>,
+                         (const void*)k_back_rows<4, false>, (const void*)k_back_rows<4, true>,
+                         (const void*)k_back_rows<8, false>, (const void*)k_back_rows<8, true>};
+  for (const void* k : backk)
+    CGM_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)((size_t)2 * N * C * sizeof(bf16))));
   CGM_HIP(hipFuncSetAttribute((const void*)k_lift_row, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)row_kernel_lds(N)));
   const void* rowk[] = {(const void*)k_cell_row<true, false>, (const void*)k_cell_row<false, false>,
@@ -1739,7 +1994,7 @@ extern "C" int cgm_fno_backward(cgm_fno_t f, const cgm_complex64* dz, float* gra
 // Average device time (ms, HIP events on the context stream, reps launches
 // after two warm-ups) of each kernel of the network on `batch` vectors
 // (contiguous [batch][N*N] chi, v, z): ms[0] lift with the first row projection (k_lift_row),
-// [1] row projection alone (k_rowproj, used by the backward pass), [2] x-DFT,
+// [1] row projection with the weight gradient (k_back_rows, the backward pass), [2] x-DFT,
 // [3] mixing, [4] inverse x-DFT, [5] cell GEMM with GELU and the next row
 // projection (k_cell_row of layers 1-2, forming B_x itself for batch 1), [6]
 // last cell GEMM with the projection (k_cell_proj), [7] one whole forward
@@ -1772,7 +2027,7 @@ extern "C" int cgm_fno_profile(cgm_fno_t f, const float* chi, const cgm_complex6
         case 0:  // the first warm-up also stores h0, which cases 1 and 5 read
           launch_lift(f, st, rows, L, nullptr, r == -2 ? f->h[0] : nullptr, nullptr);
           break;
-        case 1: rc = launch_rowproj<false>(f, st, f->h[0], nullptr, f->A, B, nullptr); break;
+        case 1: rc = launch_back_rows(f, st, f->h[0], nullptr, f->h[1], f->part, B); break;
         case 2: nch = launch_dftx(f, st, 0, B, nullptr); break;
         case 3:
           hipLaunchKernelGGL((k_mix<false>), dim3(KY, KX / KXG, B), dim3(256), 0, st, f->upart, nch, W, nullptr,

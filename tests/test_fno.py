@@ -199,6 +199,16 @@ def test_fno_backward_matches_oracle(gpu, N, B):
         assert e < 2e-2, name
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,B", [(64, 1), (64, 9), (192, 3), (320, 2), (576, 1), (1024, 1)])
+def test_fno_backward_row_sizes(gpu, N, B):
+    """Edges of the backward row kernel: half a work-group of items (N = 64),
+    rows that end inside a step of 128 cells (192, 320, 576), the largest row,
+    fewer rows than work-groups (64), B not a multiple of the four samples
+    taken together (9); the same bounds as above."""
+    test_fno_backward_matches_oracle(gpu, N, B)
+
+
 def _small_problem(N, seed=0):
     from cugmres_amd import problems
     chi, b, _ = problems.config_plain(N, seed)
