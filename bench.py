@@ -841,7 +841,7 @@ def profile_fno(ctx, net, dchi, db, batch=1):
     st = lib().cgm_fno_profile(net.handle, ctypes.c_void_p(dchi.data_ptr()), ctypes.c_void_p(v.data_ptr()),
                                ctypes.c_void_p(z.data_ptr()), batch, 50, ms)
     _lib.check(st, "cgm_fno_profile")
-    names = ["fno_lift", "fno_rowproj", "fno_dftx", "fno_mix", "fno_invx", "fno_cell_gemm", "fno_proj",
+    names = ["fno_lift", "fno_rowproj", "fno_spectral", None, "fno_invx", "fno_cell_gemm", "fno_proj",
              "fno_forward_total", "fno_cell_gemm_lift"]
     # launches per forward pass: fno_lift = k_lift_row / k_lift_rows (lift +
     # layer-0 row projection; h0 stays in LDS); fno_cell_gemm = k_cell_row /
@@ -856,24 +856,25 @@ def profile_fno(ctx, net, dchi, db, batch=1):
     # k_invx runs for layer 3 only; for more, k_invx forms every B_x.  The
     # row projection with the weight-gradient partials (k_back_rows) runs only
     # in the backward pass.  Algorithmic bytes per launch: BF16 activations 64 B per cell, complex64 vectors 8 B,
-    # chi 4 B; FP32 row projections 4 KiB per grid row, x-DFT partials
-    # 128 KiB per 64 rows, spectral weights 4 MiB per layer, mixed modes
+    # chi 4 B; FP32 row projections 4 KiB per grid row, spectral weights 4 MiB per layer, mixed modes
     # 128 KiB per vector, row twiddles 256 B per row, BF16 per-row mixing
     # matrices 2 KiB per row
     # (per vector; the spectral weights once per launch)
-    part = (N // 64) * 16384 * 8   # x-DFT partials: one per 64 rows
     Bv = batch
     bx = 128 * 1024 if batch == 1 else N * 2048   # B_x source per vector: modes (folded) or k_invx's rows
-    bytes_ = {"fno_lift": Bv * (n * (4 + 8) + N * 4096), "fno_rowproj": Bv * (n * 128 + N * 4096) + min(512, Bv * N) * 4224,
-              "fno_dftx": Bv * (N * 4096 + part) + N * 256, "fno_mix": Bv * (part + 16384 * 8) + 4 * 1024 * 1024,
+    bytes_ = {"fno_lift": Bv * (n * (4 + 8) + N * 4096),
+              "fno_rowproj": Bv * (n * 128 + N * 4096) + min(512, Bv * N) * 4224,
+              "fno_spectral": Bv * (N * 4096 + 16384 * 8) + N * 256 + 4 * 1024 * 1024,
               "fno_invx": Bv * (16384 * 8 + N * 2048) + N * 256,
               "fno_cell_gemm": Bv * (n * 128 + N * 4096 + bx) + N * 256,
               "fno_cell_gemm_lift": Bv * (n * (4 + 8 + 64) + N * 4096 + bx) + N * 256,
               "fno_proj": Bv * (n * (64 + 16) + N * 2048)}
-    per_step = {"fno_lift": 1, "fno_rowproj": 0, "fno_dftx": 4, "fno_mix": 4, "fno_invx": 1 if batch == 1 else 4,
+    per_step = {"fno_lift": 1, "fno_rowproj": 0, "fno_spectral": 4, "fno_invx": 1 if batch == 1 else 4,
                 "fno_cell_gemm": 2, "fno_cell_gemm_lift": 1, "fno_proj": 1}
     kernels = {}
     for i, k in enumerate(names):
+        if k is None:
+            continue
         us = ms[i] * 1e3
         e = {"us": us}
         if k in bytes_:

@@ -26,15 +26,15 @@
 // transforms are GEMMs against an N x 32 basis F[y,2ky] = cos(2 pi ky y/N),
 // F[y,2ky+1] = -sin(2 pi ky y/N), and every layer is
 //   row projection : A_x = F^T H_x          per grid row x (K = N, MFMA)
-//   k_dftx         : DFT of A along x at the 32 kx (FP32)
-//   k_mix          : channel mixing per mode (FP32)
+//   k_spectral     : DFT of A along x at the 32 kx and the channel mixing per
+//                    mode (FP32)
 //   k_invx         : inverse DFT along x (FP32) -> B_x
 //   cell GEMM      : h' = act([h, F_y] [W; B_x] + b)  per cell (K = 64, MFMA)
 // In the forward pass the row projection of each layer's input runs inside
 // the kernel that produces it (k_lift_row, k_cell_row), for one sample the
 // inverse x-DFT of each row of layers 0-2 runs in the cell GEMM of that row,
 // and the last cell GEMM carries the 32 -> 2 projection (k_cell_proj):
-// 1 + 3 x 3 + 4 launches for one sample, 1 + 4 x 4 for more.  h0 is a
+// 1 + 3 x 2 + 3 launches for one sample, 1 + 4 x 3 for more.  h0 is a
 // pointwise function of (chi, v): outside training it never reaches global
 // memory, and layer 0's cell GEMM lifts its row again.  The
 // backward pass has separate kernels (k_back_rows, k_back_cells) with the roles
@@ -61,7 +61,6 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 constexpr int C = 32;   // channels
 constexpr int KY = 16;  // retained column frequencies
 constexpr int KX = 32;  // retained row frequencies
-constexpr int XC = 32;  // fewest rows per partial of k_dftx (sizes the partials)
 constexpr int S = 36;   // LDS row stride (bf16) of a lifted row: 16-bank offset between lane groups
 constexpr int kLayerParams = C * C + C + KX * KY * C * C * 2;
 constexpr long kOffLayer0 = 4 * C;
@@ -300,152 +299,187 @@ __global__ void __launch_bounds__(512, NC <= 4 ? 4 : 2) k_back_rows(const bf16* 
 }
 
 // ---------------------------------------------------------------------------
-// DFT along x at the retained kx, one chunk of XR rows per block:
-//   out[b][chunk][kxi][ky][c] = s_ky sum_{x in chunk} (in[b][x][2ky][c] + i in[b][x][2ky+1][c]) e^{-2 pi i kx x/N}
-// with s_ky = 1 (forward) or w_ky / N^2 (backward of the inverse transform).
-// A chunk is XR/2 row pairs: pair p >= 1 is rows (p, N - p), whose twiddles
-// are conjugate (kx integer), so with P = A_x + A_{N-x}, M = A_x - A_{N-x}
-// and e = e^{2 pi i kx x/N} = c + is the pair adds c P - i s M (half the
-// products of two rows); pair 0 is rows 0 and N/2 (twiddles 1 and
-// (-1)^kx = (-1)^kxi: P at even kxi, M at odd).  The partials of all chunks
-// sum to the whole transform.  Thread (kp, cp) of 256 accumulates the 2 x 2
-// outputs kxi in {2kp, 2kp+1}, c in {cp, cp + 16}.
-template <int XR>
-__global__ void __launch_bounds__(256) k_dftx(const float* __restrict__ in, float2* __restrict__ outp,
-                                              const float2* __restrict__ Ex, int N, int scaled,
-                                              const int* done) {
+// Spectral path of a layer from the row projections to the mixed modes, one
+// block per (ky, KG retained kx, sample):
+//   U[kxi][ch] = s sum_x (in[b][x][2ky][ch] + i in[b][x][2ky+1][ch]) e^{-2 pi i kx x/N}   (saved to usave)
+//   forward : s = 1,            V[kxi][o] = w_ky / N^2 sum_c U[kxi][c] W[kxi][ky][c][o]
+//   backward: s = w_ky / N^2,   V[kxi][c] = sum_o conj(W[kxi][ky][c][o]) U[kxi][o]
+// (w_0 = 1, else 2).  V goes to vout[b][kxi][ky][ch].
+//
+// Rows go in pairs: pair p >= 1 is rows (p, N - p), whose twiddles are
+// conjugate (kx integer), so with P = A_x + A_{N-x}, M = A_x - A_{N-x} and
+// e = e^{2 pi i kx x/N} = c + is the pair adds c P - i s M (half the products
+// of two rows); pair 0 is rows 0 and N/2 (twiddles 1 and (-1)^kx = (-1)^kxi:
+// P at even kxi, M at odd).  32 pairs make a chunk; the sums of the chunks
+// are formed by separate threads and added in order, so a sum does not depend
+// on KG, which is chosen by the number of blocks.  Sums and products are
+// written out as fused or not: every KG rounds alike.
+//
+// Bound by latencies (the loads of the block's 256 bytes of each row, then a
+// chain of 32 pairs, then the mixing), so 512 threads take CP chunks at once:
+// thread (chunk, kp, cp) holds RK frequencies x 2 channels.  One sample of
+// N = 512 takes 7.9 us, 8 of N = 256 11.4 (12.3 backward); a transform that
+// left its chunks' partial sums to a mixing kernel took 5.0 + 4.0 and
+// 7.0 + 5.5 (7.1), and a launch more.
+constexpr int kPairs = 32;  // row pairs per chunk
+template <int KG>
+struct SpecShape {
+  static constexpr int RK = KG >= 16 ? 2 : 1;   // frequencies per thread
+  static constexpr int TPC = KG / RK * 16;      // threads per chunk
+  static constexpr int CP = 512 / TPC < 8 ? 512 / TPC : 8;  // chunks at once (8: 128 KiB of P and M)
+  static size_t lds(int N) {
+    const int nch = N / 64, cp = nch < CP ? nch : CP;
+    return (size_t)cp * kPairs * C * 2 * sizeof(float2) + (size_t)KG * (cp * kPairs + 1) * sizeof(float2) +
+           (size_t)nch * KG * C * sizeof(float2);
+  }
+};
+template <int KG, bool BWD>
+__global__ void __launch_bounds__(512) k_spectral(const float* __restrict__ in, const float2* __restrict__ Ex,
+                                                  const float2* __restrict__ W, float2* __restrict__ usave,
+                                                  float2* __restrict__ vout, int N, const int* done) {
+#pragma clang fp contract(off)
   if (skip(done)) return;
-  constexpr int XH = XR / 2;  // pairs per chunk
-  __shared__ float2 sp[XH][C + 1];
-  __shared__ float2 sm[XH][C + 1];
-  __shared__ float2 se[KX][XH + 1];
-  const int chunk = blockIdx.x, ky = blockIdx.y, b = blockIdx.z;
-  const int nch = gridDim.x;
+  typedef SpecShape<KG> Sh;
+  constexpr int RK = Sh::RK, TPC = Sh::TPC, CP = Sh::CP;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int nch = N / 64, ncp = nch < CP ? nch : CP;
+  float2* sp = reinterpret_cast<float2*>(smem_raw);  // [chunk pair][C]
+  float2* sm = sp + ncp * kPairs * C;
+  float2* part = sm + ncp * kPairs * C;               // [chunk][KG][C]
+  float2* se = part + nch * KG * C;                   // [KG][ncp kPairs + 1]
+  const int els = ncp * kPairs + 1;
+  const int ky = blockIdx.x, k0 = blockIdx.y * KG, b = blockIdx.z;
   const int tid = threadIdx.x;
-  const int p0 = chunk * XH;
-  // every load of the staging first, then the LDS writes (a load-wait-write
-  // chain per item would expose the load latency once per item)
-  constexpr int NA = XH * C / 256, NE = KX * XH / 256;
-  static_assert(NA * 256 == XH * C && NE * 256 == KX * XH, "staging items must fill the work-group");
-  float2 u1[NA], u2[NA], ev[NE];
+  // this thread's output of the mixing
+  const int kl = tid >> 5, ch = tid & 31, kxi = k0 + kl;
+  const bool mixes = tid < KG * C;
+  const float2* Wm = W + (long)((mixes ? kxi : k0) * KY + ky) * C * C;
+  const int cl = tid / TPC, kp = tid % TPC / 16, cp = tid & 15;
+  const float sc = BWD ? (ky == 0 ? 1.f : 2.f) / ((float)N * (float)N) : 1.f;
+  auto stage = [&](int g0) {  // P, M and the twiddles of the group's chunks to LDS
+    const int pg = g0 * kPairs;                                   // first pair of the group
+    const int np = (nch - g0 < CP ? nch - g0 : CP) * kPairs;      // its pairs
+    constexpr int NI = CP * kPairs * C / 4 / 512;  // items of 4 channels of a pair per thread
+    float4 u1[NI][2], u2[NI][2];
 #pragma unroll
-  for (int k = 0; k < NA; ++k) {
-    const int e = tid + 256 * k, pl = e >> 5, c = e & 31;
-    const int x = p0 + pl, x2 = x == 0 ? N / 2 : N - x;
-    const float* r1 = in + ((long)(b * N + x) * C + 2 * ky) * C;
-    const float* r2 = in + ((long)(b * N + x2) * C + 2 * ky) * C;
-    u1[k] = make_float2(r1[c], r1[C + c]);
-    u2[k] = make_float2(r2[c], r2[C + c]);
-  }
-#pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    const int e = tid + 256 * k, q = e / XH, pl = e % XH;
-    ev[k] = Ex[(long)q * N + p0 + pl];  // frequency q at row p0 + pl
-  }
-#pragma unroll
-  for (int k = 0; k < NA; ++k) {
-    const int e = tid + 256 * k, pl = e >> 5, c = e & 31;
-    sp[pl][c] = make_float2(u1[k].x + u2[k].x, u1[k].y + u2[k].y);
-    sm[pl][c] = make_float2(u1[k].x - u2[k].x, u1[k].y - u2[k].y);
-  }
-#pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    const int e = tid + 256 * k;
-    se[e / XH][e % XH] = ev[k];
-  }
-  __syncthreads();
-  const int kp = tid >> 4, cp = tid & 15;
-  float2 acc[2][2] = {};
-  int pl0 = 0;
-  if (p0 == 0) {  // rows 0 and N/2: P at kxi = 2kp, M at 2kp + 1
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      acc[0][c] = sp[0][cp + 16 * c];
-      acc[1][c] = sm[0][cp + 16 * c];
+    for (int k = 0; k < NI; ++k) {
+      if (64 * k >= np) break;
+      int pl = (tid + 512 * k) >> 3;
+      pl = pl < np ? pl : np - 1;
+      const int c4 = (tid & 7) * 4, x = pg + pl, x2 = x == 0 ? N / 2 : N - x;
+      const float* r1 = in + ((long)(b * N + x) * C + 2 * ky) * C + c4;
+      const float* r2 = in + ((long)(b * N + x2) * C + 2 * ky) * C + c4;
+      u1[k][0] = *reinterpret_cast<const float4*>(r1);
+      u1[k][1] = *reinterpret_cast<const float4*>(r1 + C);
+      u2[k][0] = *reinterpret_cast<const float4*>(r2);
+      u2[k][1] = *reinterpret_cast<const float4*>(r2 + C);
     }
-    pl0 = 1;
-  }
-#pragma unroll 4
-  for (int pl = pl0; pl < XH; ++pl) {
-    const float2 e[2] = {se[2 * kp][pl], se[2 * kp + 1][pl]};
-    const float2 P[2] = {sp[pl][cp], sp[pl][cp + 16]};
-    const float2 M[2] = {sm[pl][cp], sm[pl][cp + 16]};
+    for (int q = tid; q < KG * np; q += 512) {
+      const int kq = q / np, pl = q - kq * np;
+      se[kq * els + pl] = Ex[(long)(k0 + kq) * N + pg + pl];
+    }
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int k = 0; k < NI; ++k) {
+      const int pl = (tid + 512 * k) >> 3, c4 = (tid & 7) * 4;
+      if (pl >= np) break;
+      const float4 a = u1[k][0], ai = u1[k][1], d = u2[k][0], di = u2[k][1];
+      float4* p4 = reinterpret_cast<float4*>(sp + pl * C + c4);
+      float4* m4 = reinterpret_cast<float4*>(sm + pl * C + c4);
+      p4[0] = make_float4(a.x + d.x, ai.x + di.x, a.y + d.y, ai.y + di.y);
+      p4[1] = make_float4(a.z + d.z, ai.z + di.z, a.w + d.w, ai.w + di.w);
+      m4[0] = make_float4(a.x - d.x, ai.x - di.x, a.y - d.y, ai.y - di.y);
+      m4[1] = make_float4(a.z - d.z, ai.z - di.z, a.w - d.w, ai.w - di.w);
+    }
+  };
+  auto transform = [&](int g0) {
+    const int np = (nch - g0 < CP ? nch - g0 : CP) * kPairs;
+    if (cl < CP && cl * kPairs < np) {
+      const float2* P = sp + cl * kPairs * C + cp;
+      const float2* M = sm + cl * kPairs * C + cp;
+      const float2* E = se + RK * kp * els + cl * kPairs;
+      float2 acc[RK][2] = {};
+      auto add = [&](int pl) {
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        acc[a][c].x += e[a].x * P[c].x + e[a].y * M[c].y;  // c P - i s M
-        acc[a][c].y += e[a].x * P[c].y - e[a].y * M[c].x;
+        for (int a = 0; a < RK; ++a)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const float2 e = E[a * els + pl], p = P[pl * C + 16 * c], m = M[pl * C + 16 * c];
+            acc[a][c].x = acc[a][c].x + __builtin_fmaf(e.x, p.x, e.y * m.y);  // c P - i s M
+            acc[a][c].y = acc[a][c].y + __builtin_fmaf(e.x, p.y, -(e.y * m.x));
+          }
+      };
+      if (g0 + cl == 0) {  // rows 0 and N/2: P at even kxi, M at odd
+#pragma unroll
+        for (int a = 0; a < RK; ++a)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) acc[a][c] = (RK * kp + a) & 1 ? M[16 * c] : P[16 * c];
+      } else {
+        add(0);
       }
-  }
-  float sc = 1.f;
-  if (scaled) sc = (ky == 0 ? 1.f : 2.f) / ((float)N * (float)N);
+#pragma unroll 8
+      for (int pl = 1; pl < kPairs; ++pl) add(pl);
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+      for (int a = 0; a < RK; ++a)
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
-      outp[(((long)(b * nch + chunk) * KX + 2 * kp + a) * KY + ky) * C + cp + 16 * c] =
-          make_float2(acc[a][c].x * sc, acc[a][c].y * sc);
-}
-
-// ---------------------------------------------------------------------------
-// Channel mixing per mode, one (ky, sample) per block:
-//   U[kxi][ch] = sum of the k_dftx partials             (saved to usave)
-//   forward : V[kxi][o] = s_ky sum_c U[kxi][c] W[kxi][ky][c][o],  s_ky = w_ky / N^2
-//   backward: V[kxi][c] = sum_o conj(W[kxi][ky][c][o]) U[kxi][o]
-// V goes to vout[b][kxi][ky][ch].
-constexpr int KXG = 8;  // retained kx per block of k_mix
-template <bool BWD>
-__global__ void __launch_bounds__(256) k_mix(const float2* __restrict__ upart, int nch,
-                                             const float2* __restrict__ W, float2* __restrict__ usave,
-                                             float2* __restrict__ vout, int N, const int* done) {
-  if (skip(done)) return;
-  __shared__ float2 su[KXG][C + 1];
-  const int ky = blockIdx.x, b = blockIdx.z;
-  const int tid = threadIdx.x;
-  const int kl = tid >> 5, ch = tid & 31;
-  const int kxi = blockIdx.y * KXG + kl;
-  float2 acc = make_float2(0.f, 0.f);
-  for (int k0 = 0; k0 < nch; k0 += 8) {
-    float2 u[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      u[j] = (k0 + j < nch) ? upart[(((long)(b * nch + k0 + j) * KX + kxi) * KY + ky) * C + ch]
-                            : make_float2(0.f, 0.f);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      acc.x += u[j].x;
-      acc.y += u[j].y;
+        for (int c = 0; c < 2; ++c)
+          part[((g0 + cl) * KG + RK * kp + a) * C + cp + 16 * c] = make_float2(acc[a][c].x * sc, acc[a][c].y * sc);
     }
-  }
-  su[kl][ch] = acc;
-  const long slot = (((long)b * KX + kxi) * KY + ky) * C + ch;
-  if (usave) usave[slot] = acc;
-  __syncthreads();
-  const float2* Wm = W + (long)(kxi * KY + ky) * C * C;
-  float2 v = make_float2(0.f, 0.f);
+  };
+  stage(0);
+  // this thread's 32 weights of the mixing, in flight during the transform
+  // (forward: a column of the mode's matrix, coalesced over ch)
+  float2 wv[C];
   if (!BWD) {
-    // all 32 weights of this output in flight at once (8 at a time would
-    // expose the load latency four times)
-    float2 wv[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) wv[c] = Wm[c * C + ch];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-      const float2 uu = su[kl][c];
-      v.x += uu.x * wv[c].x - uu.y * wv[c].y;
-      v.y += uu.x * wv[c].y + uu.y * wv[c].x;
-    }
-    const float sc = (ky == 0 ? 1.f : 2.f) / ((float)N * (float)N);
-    v.x *= sc;
-    v.y *= sc;
   } else {
-#pragma unroll 8
-    for (int o = 0; o < C; ++o) {
-      const float2 uu = su[kl][o], wv = Wm[ch * C + o];
-      v.x += wv.x * uu.x + wv.y * uu.y;  // conj(w) * u
-      v.y += wv.x * uu.y - wv.y * uu.x;
+    const float4* wr = reinterpret_cast<const float4*>(Wm + ch * C);
+#pragma unroll
+    for (int c = 0; c < C / 2; ++c) {
+      const float4 q = wr[c];
+      wv[2 * c] = make_float2(q.x, q.y);
+      wv[2 * c + 1] = make_float2(q.z, q.w);
     }
+  }
+  __syncthreads();
+  transform(0);
+  for (int g0 = CP; g0 < nch; g0 += CP) {
+    __syncthreads();
+    stage(g0);
+    __syncthreads();
+    transform(g0);
+  }
+  __syncthreads();
+  float2* su = sp;  // [KG][C]
+  const long slot = (((long)b * KX + kxi) * KY + ky) * C + ch;
+  if (mixes) {
+    float2 u = make_float2(0.f, 0.f);
+    for (int k = 0; k < nch; ++k) {
+      const float2 t = part[(k * KG + kl) * C + ch];
+      u.x = u.x + t.x;
+      u.y = u.y + t.y;
+    }
+    su[kl * C + ch] = u;
+    if (usave) usave[slot] = u;
+  }
+  __syncthreads();
+  if (!mixes) return;
+  float2 v = make_float2(0.f, 0.f);
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const float2 u = su[kl * C + c], w = wv[c];
+    if (!BWD) {
+      v.x = v.x + __builtin_fmaf(u.x, w.x, -(u.y * w.y));
+      v.y = v.y + __builtin_fmaf(u.y, w.x, u.x * w.y);
+    } else {  // conj(w) u
+      v.x = v.x + __builtin_fmaf(w.x, u.x, w.y * u.y);
+      v.y = v.y + __builtin_fmaf(w.x, u.y, -(w.y * u.x));
+    }
+  }
+  if (!BWD) {
+    const float so = (ky == 0 ? 1.f : 2.f) / ((float)N * (float)N);
+    v.x *= so;
+    v.y *= so;
   }
   vout[slot] = v;
 }
@@ -1574,7 +1608,6 @@ struct cgm_fno {
   bf16* pre[3] = {};              // pre-activations (training)
   bf16* dh[2] = {};               // backward ping-pong
   float* A = nullptr;             // [B][N][32][32]
-  float2* upart = nullptr;        // [B][N/XC][32][16][32]
   float2* U[4] = {};              // [B][32][16][32] (training)
   float2* dV[4] = {};             // [B][32][16][32] per layer
   float2* Vm = nullptr;           // [B][32][16][32] mixed modes
@@ -1590,7 +1623,7 @@ namespace {
 
 int fno_free(cgm_fno* f) {
   void* ptrs[] = {f->Wt, f->Wn, f->Ft, f->Fy, f->Ex, f->h[0], f->h[1], f->h[2], f->h[3], f->h[4],
-                  f->pre[0], f->pre[1], f->pre[2], f->dh[0], f->dh[1], f->A, f->upart, f->U[0],
+                  f->pre[0], f->pre[1], f->pre[2], f->dh[0], f->dh[1], f->A, f->U[0],
                   f->U[1], f->U[2], f->U[3], f->dV[0], f->dV[1], f->dV[2], f->dV[3], f->Vm, f->Bt, f->part};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -1648,24 +1681,40 @@ void launch_invx(cgm_fno* f, hipStream_t st, int B, const int* done) {
     hipLaunchKernelGGL(k_invx<1>, dim3(f->N / 2, 1, B), dim3(512), 0, st, f->Vm, f->Bt, f->Ex, f->N, done);
 }
 
-// x-DFT of A (B vectors) into partials over chunks of 64 rows, whatever B
-// (the same partial sums for one vector and for a batch); returns the number
-// of chunks
-int launch_dftx(cgm_fno* f, hipStream_t st, int scaled, int B, const int* done) {
-  hipLaunchKernelGGL(k_dftx<64>, dim3(f->N / 64, KY, B), dim3(256), 0, st, f->A, f->upart, f->Ex, f->N, scaled, done);
-  return f->N / 64;
+// A of B vectors to the mixed modes Vm, with the most frequencies per block
+// (16, 8, 4, 2) that leave 256 blocks, one per CU: a block reads its part of A
+// once for all its frequencies (8 samples of N = 256: 16 per block takes
+// 11.4 us, 8 per block 15.9; one of N = 512: 2 per block 7.9, 4 per block 8.7).
+template <int KG>
+void launch_spectral_n(const cgm_fno* f, hipStream_t st, const float2* W, float2* usave, bool bwd, int B,
+                       const int* done) {
+  hipLaunchKernelGGL((bwd ? k_spectral<KG, true> : k_spectral<KG, false>), dim3(KY, KX / KG, B), dim3(512),
+                     SpecShape<KG>::lds(f->N), st, f->A, f->Ex, W, usave, f->Vm, f->N, done);
+}
+void launch_spectral(const cgm_fno* f, hipStream_t st, const float2* W, float2* usave, bool bwd, int B,
+                     const int* done) {
+  const int kg = KY * KX * B / 256;
+  if (kg >= 16)
+    launch_spectral_n<16>(f, st, W, usave, bwd, B, done);
+  else if (kg >= 8)
+    launch_spectral_n<8>(f, st, W, usave, bwd, B, done);
+  else if (kg >= 4)
+    launch_spectral_n<4>(f, st, W, usave, bwd, B, done);
+  else
+    launch_spectral_n<2>(f, st, W, usave, bwd, B, done);
+}
+template <int KG>
+int spectral_limits(int N) {
+  const void* k[] = {(const void*)k_spectral<KG, false>, (const void*)k_spectral<KG, true>};
+  for (const void* p : k)
+    CGM_HIP(hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SpecShape<KG>::lds(N)));
+  return CGM_SUCCESS;
 }
 
 // spectral path of one layer: A (row projections) -> Bt (per-row mixing matrices)
 int spectral(cgm_fno* f, hipStream_t st, const float2* W, float2* usave, bool bwd, int B, const int* done,
              bool invx = true) {
-  const int nch = launch_dftx(f, st, bwd ? 1 : 0, B, done);
-  if (!bwd)
-    hipLaunchKernelGGL((k_mix<false>), dim3(KY, KX / KXG, B), dim3(256), 0, st, f->upart, nch, W, usave, f->Vm,
-                       f->N, done);
-  else
-    hipLaunchKernelGGL((k_mix<true>), dim3(KY, KX / KXG, B), dim3(256), 0, st, f->upart, nch, W, usave, f->Vm,
-                       f->N, done);
+  launch_spectral(f, st, W, usave, bwd, B, done);
   if (invx)
     launch_invx(f, st, B, done);
   CGM_HIP(hipGetLastError());
@@ -1900,7 +1949,6 @@ extern "C" int cgm_fno_create(cgm_ctx_t c, int batch, float chi_scale, cgm_fno_t
   for (int l = 0; l < 3; ++l) alloc((void**)&f->pre[l], act);
   for (int l = 0; l < 2; ++l) alloc((void**)&f->dh[l], act);
   alloc((void**)&f->A, sizeof(float) * (size_t)batch * N * C * C);
-  alloc((void**)&f->upart, sizeof(float2) * (size_t)batch * (N / XC) * KX * KY * C);
   for (int l = 0; l < 4; ++l) alloc((void**)&f->U[l], sizeof(float2) * (size_t)batch * KX * KY * C);
   for (int l = 0; l < 4; ++l) alloc((void**)&f->dV[l], sizeof(float2) * (size_t)batch * KX * KY * C);
   alloc((void**)&f->Vm, sizeof(float2) * (size_t)batch * KX * KY * C);
@@ -1934,6 +1982,9 @@ extern "C" int cgm_fno_create(cgm_ctx_t c, int batch, float chi_scale, cgm_fno_t
   CGM_HIP(hipMemcpy(f->Ft, ft.data(), sizeof(bf16) * ft.size(), hipMemcpyHostToDevice));
   CGM_HIP(hipMemcpy(f->Fy, fy.data(), sizeof(bf16) * fy.size(), hipMemcpyHostToDevice));
   CGM_HIP(hipMemcpy(f->Ex, ex.data(), sizeof(float2) * ex.size(), hipMemcpyHostToDevice));
+  if ((rc = spectral_limits<2>(N)) || (rc = spectral_limits<4>(N)) || (rc = spectral_limits<8>(N)) ||
+      (rc = spectral_limits<16>(N)))
+    return rc;
   const void* backk[] = {(const void*)k_back_rows<1, false>, (const void*)k_back_rows<1, true>,
                          (const void*)k_back_rows<2, false>, (const void*)k_back_rows<2, true>,
                          (const void*)k_back_rows<4, false>, (const void*)k_back_rows<4, true>,
@@ -1994,8 +2045,8 @@ extern "C" int cgm_fno_backward(cgm_fno_t f, const cgm_complex64* dz, float* gra
 // Average device time (ms, HIP events on the context stream, reps launches
 // after two warm-ups) of each kernel of the network on `batch` vectors
 // (contiguous [batch][N*N] chi, v, z): ms[0] lift with the first row projection (k_lift_row),
-// [1] row projection with the weight gradient (k_back_rows, the backward pass), [2] x-DFT,
-// [3] mixing, [4] inverse x-DFT, [5] cell GEMM with GELU and the next row
+// [1] row projection with the weight gradient (k_back_rows, the backward pass), [2] x-DFT
+// with the mode mixing (k_spectral), [3] unused (0), [4] inverse x-DFT, [5] cell GEMM with GELU and the next row
 // projection (k_cell_row of layers 1-2, forming B_x itself for batch 1), [6]
 // last cell GEMM with the projection (k_cell_proj), [7] one whole forward
 // pass, [8] the cell GEMM of layer 0 (k_cell_row lifting its row from chi
@@ -2011,7 +2062,6 @@ extern "C" int cgm_fno_profile(cgm_fno_t f, const float* chi, const cgm_complex6
   const long total = (long)B * f->n;
   const unsigned rows = (unsigned)(B * f->N);
   const float s = (float)f->N;
-  int nch = 0;
   const float* Lp = f->params + layer_off(0);
   const float2* W = (const float2*)(Lp + C * C + C);
   const size_t lds = row_kernel_lds(f->N);
@@ -2024,15 +2074,12 @@ extern "C" int cgm_fno_profile(cgm_fno_t f, const float* chi, const cgm_complex6
     for (int r = -2; r < reps && !rc; ++r) {
       if (r == 0) CGM_HIP(hipEventRecord(e0, st));
       switch (k) {
+        case 3: break;
         case 0:  // the first warm-up also stores h0, which cases 1 and 5 read
           launch_lift(f, st, rows, L, nullptr, r == -2 ? f->h[0] : nullptr, nullptr);
           break;
         case 1: rc = launch_back_rows(f, st, f->h[0], nullptr, f->h[1], f->part, B); break;
-        case 2: nch = launch_dftx(f, st, 0, B, nullptr); break;
-        case 3:
-          hipLaunchKernelGGL((k_mix<false>), dim3(KY, KX / KXG, B), dim3(256), 0, st, f->upart, nch, W, nullptr,
-                             f->Vm, f->N, nullptr);
-          break;
+        case 2: launch_spectral(f, st, W, nullptr, false, B, nullptr); break;
         case 4:
           launch_invx(f, st, B, nullptr);
           break;
@@ -2065,7 +2112,7 @@ extern "C" int cgm_fno_profile(cgm_fno_t f, const float* chi, const cgm_complex6
     CGM_HIP(hipEventSynchronize(e1));
     float t = 0.f;
     CGM_HIP(hipEventElapsedTime(&t, e0, e1));
-    ms[k] = t / reps;
+    ms[k] = k == 3 ? 0.f : t / reps;
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);

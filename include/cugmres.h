@@ -516,8 +516,9 @@ int cgm_profile_step(cgm_ctx_t ctx, const cgm_complex64* dev_gamma, const float*
 
 /* Average device time (ms, HIP events on the context stream, reps launches
  * each) of the preconditioner's kernels on `batch` vectors ([batch][N*N] chi,
- * v, z): ms[0] lift with the first row projection, [1] stand-alone row
- * projection (backward pass), [2] x-DFT, [3] mode mixing, [4] inverse x-DFT,
+ * v, z): ms[0] lift with the first row projection, [1] row projection with
+ * the weight gradient (backward pass), [2] x-DFT with the mode mixing, [3]
+ * unused (0), [4] inverse x-DFT,
  * [5] cell GEMM with GELU and the next row projection (layers 1-2), [6] last
  * cell GEMM with the projection, [7] a whole forward pass, [8] the cell GEMM
  * of layer 0, which lifts its row from chi and v itself (ms holds 9
