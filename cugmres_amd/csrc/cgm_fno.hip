@@ -318,7 +318,7 @@ __global__ void __launch_bounds__(512, NC <= 4 ? 4 : 2) k_back_rows(const bf16* 
 // Bound by latencies (the loads of the block's 256 bytes of each row, then a
 // chain of 32 pairs, then the mixing), so 512 threads take CP chunks at once:
 // thread (chunk, kp, cp) holds RK frequencies x 2 channels.  One sample of
-// N = 512 takes 7.9 us, 8 of N = 256 11.4 (12.3 backward); a transform that
+// N = 512 takes 7.4 us, 8 of N = 256 10.1 (11.1 backward); a transform that
 // left its chunks' partial sums to a mixing kernel took 5.0 + 4.0 and
 // 7.0 + 5.5 (7.1), and a launch more.
 constexpr int kPairs = 32;  // row pairs per chunk
@@ -374,10 +374,12 @@ __global__ void __launch_bounds__(512) k_spectral(const float* __restrict__ in, 
       u2[k][0] = *reinterpret_cast<const float4*>(r2);
       u2[k][1] = *reinterpret_cast<const float4*>(r2 + C);
     }
-    for (int q = tid; q < KG * np; q += 512) {
-      const int kq = q / np, pl = q - kq * np;
-      se[kq * els + pl] = Ex[(long)(k0 + kq) * N + pg + pl];
-    }
+    // twiddles: 16 groups of 32 threads, frequency kq, 32 pairs per item
+    constexpr int NE = KG * CP * kPairs / 512, SE = 16 / KG * kPairs;
+    const int kq = (tid >> 5) % KG, pe = (tid >> 5) / KG * kPairs + (tid & 31);
+    float2 ev[NE];
+#pragma unroll
+    for (int k = 0; k < NE; ++k) ev[k] = Ex[(long)(k0 + kq) * N + pg + (pe + SE * k < np ? pe + SE * k : 0)];
 #pragma unroll
     for (int k = 0; k < NI; ++k) {
       const int pl = (tid + 512 * k) >> 3, c4 = (tid & 7) * 4;
@@ -390,6 +392,9 @@ __global__ void __launch_bounds__(512) k_spectral(const float* __restrict__ in, 
       m4[0] = make_float4(a.x - d.x, ai.x - di.x, a.y - d.y, ai.y - di.y);
       m4[1] = make_float4(a.z - d.z, ai.z - di.z, a.w - d.w, ai.w - di.w);
     }
+#pragma unroll
+    for (int k = 0; k < NE; ++k)
+      if (pe + SE * k < np) se[kq * els + pe + SE * k] = ev[k];
   };
   auto transform = [&](int g0) {
     const int np = (nch - g0 < CP ? nch - g0 : CP) * kPairs;
@@ -774,25 +779,25 @@ inline size_t row_kernel_lds(int N) {
 // a clamped item, so that no branch waits for one load before the next is
 // issued).
 template <int NT>
-__device__ inline void basis_to_lds(const bf16* __restrict__ Xt, bf16* lb, int N) {
+__device__ inline void basis_to_lds(const bf16* __restrict__ Xt, bf16* lb, int N, int tid = threadIdx.x) {
   const int per_row = N / 8, items = C * per_row;
   u32x4 v[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    int q = threadIdx.x + k * NT;
+    int q = tid + k * NT;
     q = q < items ? q : items - 1;
     const int a = q / per_row, y8 = (q - a * per_row) * 8;
     v[k] = *reinterpret_cast<const u32x4*>(Xt + (long)a * N + y8);
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int q = threadIdx.x + k * NT;
+    const int q = tid + k * NT;
     if (q < items) {
       const int a = q / per_row, y8 = (q - a * per_row) * 8;
       *reinterpret_cast<u32x4*>(lb + a * basis_ld(N) + y8) = v[k];
     }
   }
-  for (int q = threadIdx.x + 4 * NT; q < items; q += NT) {  // N > 16 NT / C only
+  for (int q = tid + 4 * NT; q < items; q += NT) {  // N > 16 NT / C only
     const int a = q / per_row, y8 = (q - a * per_row) * 8;
     *reinterpret_cast<u32x4*>(lb + a * basis_ld(N) + y8) = *reinterpret_cast<const u32x4*>(Xt + (long)a * N + y8);
   }
@@ -805,8 +810,8 @@ __device__ inline void basis_to_lds(const bf16* __restrict__ Xt, bf16* lb, int N
 // in halves and the upper half adds into the lower through red.
 template <int NW>
 __device__ inline void row_project(const bf16* __restrict__ Xt, int ldx, const bf16* lt, int N,
-                                   float* __restrict__ o, float* red) {
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+                                   float* __restrict__ o, float* red, int tid = threadIdx.x) {
+  const int lane = tid & 63, w = tid >> 6;
   const int i = lane & 15, g = lane >> 4;
   const int ta = (w >> 1) & 1, tc = w & 1;
   const int kh = NW == 8 ? (w >> 2) : 0;
@@ -1195,6 +1200,135 @@ __global__ void __launch_bounds__(512) k_cell_row(const bf16* __restrict__ P, Li
     __syncthreads();
   }
   row_project<8>(lbas, basis_ld(N), lt, N, Anext + bx * C * C, red);
+}
+
+// k_cell_row<true, LIFT> on the two grid rows of a pair (p, N - p; 0 and N/2
+// for p = 0) of one sample, 512 threads per row, for N <= 512 (a wave owns at
+// most four 16-cell tiles; both rows fit the LDS).  The pair's B_x come from
+// the same four sums, so the modes are read and summed once for two rows, and
+// the basis is staged once.  The arithmetic of a row is k_cell_row's.  At
+// N = 512: 14.4 us (lifting 15.3), where single rows, two work-groups per CU,
+// take 16.4 (16.7), 3 of them for the modes.
+inline size_t cell_pair_lds(int N, bool lift) {
+  const size_t t = (size_t)C * basis_ld(N), r = (size_t)2 * N * S;
+  return (2 * t + (lift && r > t ? r : t)) * sizeof(bf16);
+}
+template <bool LIFT>
+__global__ void __launch_bounds__(1024) k_cell_pair(const bf16* __restrict__ P, LiftIn L,
+                                                    const bf16* __restrict__ Q, const bf16* __restrict__ A,
+                                                    const float2* __restrict__ Vm, const float2* __restrict__ Ex,
+                                                    const float* __restrict__ bias, bf16* __restrict__ pre_out,
+                                                    bf16* __restrict__ out, const bf16* __restrict__ Xt,
+                                                    float* __restrict__ Anext, int N, const int* done) {
+  if (skip(done)) return;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ float red[2][4 * 64 * 4];
+  __shared__ __align__(16) bf16 lb[2][C][C + 8];  // B_x of the two rows as [o][k], rows padded to 80 B
+  const int half = threadIdx.x >> 9, tid = threadIdx.x & 511, lane = tid & 63, w = tid >> 6;
+  const int p = blockIdx.x;  // the pair's first row
+  const int xr = half == 0 ? p : p == 0 ? N / 2 : N - p;
+  const long ks = blockIdx.y, bx = ks * N + xr;
+  bf16* lt = reinterpret_cast<bf16*>(smem_raw) + half * C * basis_ld(N);  // h' channel-major
+  bf16* lbas = reinterpret_cast<bf16*>(smem_raw) + 2 * C * basis_ld(N);   // the basis, with LIFT first
+  bf16* lrow = lbas + half * N * S;                                       // the lifted rows
+  const int i = lane & 15, g = lane >> 4;
+  const int ntile = N / 16;
+  bf16x8 bpt[4], bqt[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    int t = w + 8 * u;
+    t = t < ntile ? t : ntile - 1;
+    const int y = 16 * t + i;
+    if (!LIFT) bpt[u] = ld8(P + (bx * N + y) * C + 8 * g);
+    bqt[u] = ld8(Q + (long)y * C + 8 * g);
+  }
+  if (LIFT) {
+    float wl[32];
+    lift_weights(L, wl);
+    for (int q0 = tid; q0 < N * 4; q0 += 4 * 512) {
+      LiftRegs lg;
+      lift_load<512>(L, ks, xr, N, q0, lg);
+      lift_store<512, false>(L, lg, wl, ks, xr, N, q0, lrow, nullptr, nullptr);
+    }
+  }
+  if (half == 0) {  // the sums and their order of k_invx
+    const int ky = tid >> 5, o = tid & 31;
+    const float2* Vs = Vm + (ks * KX * KY + ky) * C + o;
+    float2 vq[KX];
+#pragma unroll
+    for (int q = 0; q < KX; ++q) vq[q] = Vs[(long)q * KY * C];
+    float s1 = 0.f, s2 = 0.f, s3 = 0.f, s4 = 0.f;
+#pragma unroll
+    for (int q = 0; q < KX; ++q) {
+      const float2 e = Ex[(long)q * N + p];
+      s1 += vq[q].x * e.x;
+      s2 += vq[q].y * e.y;
+      s3 += vq[q].x * e.y;
+      s4 += vq[q].y * e.x;
+    }
+    lb[0][o][2 * ky] = (bf16)(s1 - s2);
+    lb[0][o][2 * ky + 1] = (bf16)(s3 + s4);
+    if (p == 0) {  // row N/2
+      s1 = s4 = s2 = s3 = 0.f;
+#pragma unroll
+      for (int q = 0; q < KX; q += 2) {
+        s1 += vq[q].x - vq[q + 1].x;
+        s4 += vq[q].y - vq[q + 1].y;
+      }
+    }
+    lb[1][o][2 * ky] = (bf16)(s1 + s2);
+    lb[1][o][2 * ky + 1] = (bf16)(s4 - s3);
+  } else if (!LIFT) {
+    basis_to_lds<512>(Xt, lbas, N, tid);
+  }
+  bf16x8 aw[2];
+  float bs[2][4];
+#pragma unroll
+  for (int to = 0; to < 2; ++to) {
+    aw[to] = ld8(A + (16 * to + i) * C + 8 * g);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) bs[to][v] = bias[16 * to + 4 * g + v];
+  }
+  __syncthreads();
+  bf16x8 ar[2];
+#pragma unroll
+  for (int to = 0; to < 2; ++to) ar[to] = *reinterpret_cast<const bf16x8*>(&lb[half][16 * to + i][8 * g]);
+  if (LIFT) {  // every wave takes its cells, then the basis replaces the rows
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      int t = w + 8 * u;
+      t = t < ntile ? t : ntile - 1;
+      const u32x2* sp = reinterpret_cast<const u32x2*>(lrow + (16 * t + i) * S + 8 * g);
+      const u32x2 lo = sp[0], hi = sp[1];
+      bpt[u] = __builtin_bit_cast(bf16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+    }
+    __syncthreads();
+    basis_to_lds<1024>(Xt, lbas, N);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int t = w + 8 * u;
+    if (t >= ntile) break;
+    const int y = 16 * t + i;
+#pragma unroll
+    for (int to = 0; to < 2; ++to) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      acc = mma(aw[to], bpt[u], acc);
+      acc = mma(ar[to], bqt[u], acc);
+      const int oc0 = 16 * to + 4 * g;
+      float r[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) r[v] = acc[v] + bs[to][v];
+      if (pre_out) st4(pre_out + (bx * N + y) * C + oc0, r[0], r[1], r[2], r[3]);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) r[v] = gelu(r[v]);
+      st4(out + (bx * N + y) * C + oc0, r[0], r[1], r[2], r[3]);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) lt[(oc0 + v) * basis_ld(N) + y] = (bf16)r[v];
+    }
+  }
+  __syncthreads();
+  row_project<8>(lbas, basis_ld(N), lt, N, Anext + bx * C * C, red[half], tid);
 }
 
 // k_cell_row<false, false> (B_x from R, the cells from P) with RPW
@@ -1683,8 +1817,9 @@ void launch_invx(cgm_fno* f, hipStream_t st, int B, const int* done) {
 
 // A of B vectors to the mixed modes Vm, with the most frequencies per block
 // (16, 8, 4, 2) that leave 256 blocks, one per CU: a block reads its part of A
-// once for all its frequencies (8 samples of N = 256: 16 per block takes
-// 11.4 us, 8 per block 15.9; one of N = 512: 2 per block 7.9, 4 per block 8.7).
+// once for all its frequencies (measured with the twiddles staged one by one:
+// 8 samples of N = 256: 16 per block 11.4 us, 8 per block 15.9; one of N = 512:
+// 2 per block 7.9, 4 per block 8.7).
 template <int KG>
 void launch_spectral_n(const cgm_fno* f, hipStream_t st, const float2* W, float2* usave, bool bwd, int B,
                        const int* done) {
@@ -1757,6 +1892,21 @@ void launch_cell_rows_lift(const cgm_fno* f, hipStream_t st, int rows, const Lif
                        nullptr, nullptr, bias, pre, out, f->Ft, f->A, f->N, done);
 }
 
+// Cell GEMM of layers 0-2 on one sample, B_x from the mixed modes: in pairs
+// of rows where single rows would be more blocks than CUs and the pair fits.
+void launch_cell_fold(const cgm_fno* f, hipStream_t st, int rows, bool lift, const bf16* P, const LiftIn& L,
+                      const bf16* W, const float* bias, bf16* pre, bf16* out, const int* done) {
+  if (f->N > 256 && f->N <= 512) {
+    auto kern = lift ? k_cell_pair<true> : k_cell_pair<false>;
+    hipLaunchKernelGGL(kern, dim3(f->N / 2, rows / f->N), dim3(1024), cell_pair_lds(f->N, lift), st, P, L, f->Fy, W,
+                       f->Vm, f->Ex, bias, pre, out, f->Ft, f->A, f->N, done);
+  } else {
+    auto kern = lift ? k_cell_row<true, true> : k_cell_row<true, false>;
+    hipLaunchKernelGGL(kern, dim3(rows), dim3(512), row_kernel_lds(f->N), st, P, L, f->Fy, W, f->Bt, f->Vm, f->Ex,
+                       bias, pre, out, f->Ft, f->A, f->N, done);
+  }
+}
+
 // Cell GEMM of layers 1-2 on B > 1 samples (B_x from R): the most rows per
 // work-group (8, 4 or 2) that leave at least 1024 work-groups.
 void launch_cell_rows(const cgm_fno* f, hipStream_t st, int rows, const bf16* P, const bf16* W, const float* bias,
@@ -1804,14 +1954,13 @@ int fno_forward_io(cgm_fno* f, hipStream_t st, const FnoIO& io, int B, bool trai
                        !fold_l)))
       return rc;
     const bf16* Wl = f->Wt + l * C * C;
-    if (l > 0 && l < 3 && !fold) {
+    if (l < 3 && (l > 0 || train) && !fold) {  // training has h0 in memory: reading it beats lifting again
       launch_cell_rows(f, st, rows, f->h[l], Wl, Lp + C * C, train ? f->pre[l] : nullptr, f->h[l + 1], done);
     } else if (l == 0 && !fold) {
       launch_cell_rows_lift(f, st, rows, L0, Wl, Lp + C * C, train ? f->pre[0] : nullptr, f->h[1], done);
     } else if (l < 3) {
-      auto kern = l == 0 ? k_cell_row<true, true> : k_cell_row<true, false>;
-      hipLaunchKernelGGL(kern, dim3(rows), dim3(512), lds, st, f->h[l], L0, f->Fy, Wl, f->Bt, f->Vm, f->Ex,
-                         Lp + C * C, train ? f->pre[l] : nullptr, f->h[l + 1], f->Ft, f->A, f->N, done);
+      launch_cell_fold(f, st, rows, l == 0, f->h[l], L0, Wl, Lp + C * C, train ? f->pre[l] : nullptr, f->h[l + 1],
+                       done);
     } else {
       const long waves = (long)B * f->n / 64;
       CGM_CHECK(waves % 4 == 0, CGM_ERROR_UNSUPPORTED, "cell GEMM needs N %% 64 == 0");
@@ -1994,6 +2143,12 @@ extern "C" int cgm_fno_create(cgm_ctx_t c, int batch, float chi_scale, cgm_fno_t
                                 (int)((size_t)2 * N * C * sizeof(bf16))));
   CGM_HIP(hipFuncSetAttribute((const void*)k_lift_row, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)row_kernel_lds(N)));
+  if (N <= 512) {
+    CGM_HIP(hipFuncSetAttribute((const void*)k_cell_pair<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)cell_pair_lds(N, false)));
+    CGM_HIP(hipFuncSetAttribute((const void*)k_cell_pair<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)cell_pair_lds(N, true)));
+  }
   const void* rowk[] = {(const void*)k_cell_row<true, false>, (const void*)k_cell_row<false, false>,
                         (const void*)k_cell_row<true, true>,  (const void*)k_cell_row<false, true>,
                         (const void*)k_cell_rows<2>,          (const void*)k_cell_rows<4>,
@@ -2085,15 +2240,13 @@ extern "C" int cgm_fno_profile(cgm_fno_t f, const float* chi, const cgm_complex6
           break;
         case 5:
           if (B == 1)
-            hipLaunchKernelGGL((k_cell_row<true, false>), dim3(rows), dim3(512), lds, st, f->h[0], L, f->Fy, f->Wt,
-                               f->Bt, f->Vm, f->Ex, Lp + C * C, nullptr, f->h[1], f->Ft, f->A, f->N, nullptr);
+            launch_cell_fold(f, st, rows, false, f->h[0], L, f->Wt, Lp + C * C, nullptr, f->h[1], nullptr);
           else
             launch_cell_rows(f, st, rows, f->h[0], f->Wt, Lp + C * C, nullptr, f->h[1], nullptr);
           break;
         case 8:
           if (B == 1)
-            hipLaunchKernelGGL((k_cell_row<true, true>), dim3(rows), dim3(512), lds, st, nullptr, L, f->Fy, f->Wt,
-                               f->Bt, f->Vm, f->Ex, Lp + C * C, nullptr, f->h[1], f->Ft, f->A, f->N, nullptr);
+            launch_cell_fold(f, st, rows, true, nullptr, L, f->Wt, Lp + C * C, nullptr, f->h[1], nullptr);
           else
             launch_cell_rows_lift(f, st, rows, L, f->Wt, Lp + C * C, nullptr, f->h[1], nullptr);
           break;
