@@ -691,7 +691,7 @@ def profile_tiles(ctx, tl, v, reps=20):
     N, T = ctx.N, tl.T
     b = tl.apply_bytes(1)
     full = (N // T) ** 2 * T ** 4 * (4 if T == 64 else 8)
-    return {"kernel": "tile application (k_tile_ws, k_tile_wsum, FFT convolution, combine)" if T >= 64
+    return {"kernel": "tile application (k_tile_ws, k_tile_wsum, FFT convolution, output)" if T >= 64
             else "k_tile_apply",
             "us": us, "bytes": b,
             "GBps": b / (us * 1e-6) / 1e9, "kept_fraction": (b - 16 * N * N) / full,

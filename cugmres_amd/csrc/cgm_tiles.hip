@@ -36,7 +36,7 @@
 // W_t = (D_S^{-1} - G_SS)^{-1}, and only the lower triangle of its 128 x 128
 // blocks is stored and streamed), then G_t u_t for all tiles at once as a
 // batch of T x T convolutions through the operator's own FFT passes at size
-// 2T with the tile's spectrum, then y = x + G_t u_t.  On the benchmark maps
+// 2T with the tile's spectrum, the last of which adds x: y = x + G_t u_t.  On the benchmark maps
 // 3/8 of the cells carry chi != 0, so a 128 x 128 tile streams about 4 % of
 // the entries of its dense inverse, and the inversion work drops by about
 // 20x; that makes 128 x 128 tiles affordable, which take 1,032 Krylov steps
@@ -51,6 +51,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "cgm_fft.h"
 #include "cgm_internal.h"
 #include "cgm_special.h"
 
@@ -118,7 +119,6 @@ struct cgm_tiles {
   float2* Cw = nullptr;            // n_max x kBlk column block (factor)
   size_t cw_cap = 0;
   float2* U = nullptr;             // [sys][nt * nt][M2] u_t scattered on the tile (apply)
-  float2* Y = nullptr;             // [sys][nt * nt][M2] G_t u_t (apply)
   float2* Tm = nullptr;            // [sys][nt * nt][T * 2T] FFT scratch (apply)
   int scratch_sys = 0;             // systems the apply scratch holds
   Plan P;                          // tile convolution: N' = T, M' = 2T
@@ -782,30 +782,32 @@ k_tile_xs(const int* __restrict__ ncol, const unsigned short* __restrict__ cols,
   __shared__ float red[16];
   const int nt = N / T;
   const int s = blockIdx.y, t = blockIdx.x / parts, part = blockIdx.x % parts;
-  if (done && *boff(done, (long)s * sd)) return;
+  // two latencies, of n and cols and of v behind them: the norm and the flag
+  // are tested once those loads are in flight
+  const int dn = done ? *boff(done, (long)s * sd) : 0;
   const long tb = (long)(maps1 ? 0 : s) * nt * nt + t;
   const int n = ncol[tb];
-  if (n == 0) return;
-  const int np = (n + kBlkW - 1) / kBlkW * kBlkW;
   const unsigned short* ct = cols + tb * M2;
+  const float2* v = io.v + (long)s * io.sV;
+  float2 xv[PT];
+  int cell[PT];
+#pragma unroll
+  for (int k = 0; k < PT; ++k) cell[k] = ct[threadIdx.x + 1024 * k];
+#pragma unroll
+  for (int k = 0; k < PT; ++k) {  // padding slots load a cell too, so that no load waits behind a branch
+    if ((int)threadIdx.x + 1024 * k >= n) cell[k] = kPadCol;
+    xv[k] = v[tile_cell(t, cell[k] == kPadCol ? 0 : cell[k], nt, T, N)];
+  }
   float sc = 1.f;
   if (io.nrm) {
     const double d = *boff(io.nrm, (long)s * io.sNrm);
     sc = d > 0.0 ? (float)(1.0 / d) : 0.f;
   }
-  const float2* v = io.v + (long)s * io.sV;
-  float2 xv[PT];
-  int cell[PT];
+  if (dn || n == 0) return;
+  const int np = (n + kBlkW - 1) / kBlkW * kBlkW;
   float mx = 0.f;
 #pragma unroll
   for (int k = 0; k < PT; ++k) {
-    const int p = threadIdx.x + 1024 * k;
-    cell[k] = ct[p < M2 ? p : 0];
-    if (p >= n) cell[k] = kPadCol;
-  }
-#pragma unroll
-  for (int k = 0; k < PT; ++k) {  // padding slots load a cell too, so that no load waits behind a branch
-    xv[k] = v[tile_cell(t, cell[k] == kPadCol ? 0 : cell[k], nt, T, N)];
     xv[k].x = cell[k] == kPadCol ? 0.f : xv[k].x * sc;
     xv[k].y = cell[k] == kPadCol ? 0.f : xv[k].y * sc;
     mx = fmaxf(mx, fmaxf(fabsf(xv[k].x), fabsf(xv[k].y)));
@@ -1148,28 +1150,55 @@ k_tile_wsum(const float* __restrict__ ksc, const float* __restrict__ xinv, const
   }
 }
 
-// z = x + Y (Y in tile-major order) for system blockIdx.y; x is io.v scaled
-// as in k_tile_xs and is written to io.vw when io.nrm and io.vw are given.
+// Last pass of the tile convolution and the application's result, z = x + G_t
+// u_t: the inverse row transforms of k_pass3 (rows of tile blockIdx.y % tiles,
+// system blockIdx.y / tiles), whose rows are then read and written in the
+// grid's order; x is io.v scaled as in k_tile_xs and is written to io.vw when
+// io.nrm and io.vw are given.  Bound by memory: T x 2T transformed values in, x
+// in, z out; a kernel of its own for the sum read and wrote T x T more, 21 of
+// 523 us for 16 systems at N = 512, T = 128, and its launch 2 of 33 us for one
+// system at N = 128, T = 64.
+template <int T>
+struct TileOut {
+  static constexpr int M = 2 * T, E = kFftE<M>, NT = FftShape<M, E>::NT, ROWS = 256 / NT;
+};
 template <int T>
 __global__ void __launch_bounds__(256)
-k_tile_combine(FnoIO io, const float2* __restrict__ Y, const int* __restrict__ done, long sd, int N) {
-  const int s = blockIdx.y;
-  if (done && *boff(done, (long)s * sd)) return;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (long)N * N) return;
+k_tile_out(FnoIO io, const float2* __restrict__ Tm, const float2* __restrict__ tw, const int* __restrict__ done,
+           long sd, int N) {
+  typedef TileOut<T> S;
+  constexpr int M = S::M, E = S::E, NT = S::NT;
+  __shared__ __align__(16) float2 smem[S::ROWS * LdsLen<M>::value];
+  const int nt = N / T;
+  const int s = blockIdx.y / (nt * nt), tile = blockIdx.y % (nt * nt);
+  const int dn = done ? *boff(done, (long)s * sd) : 0;  // tested once the loads are in flight
+  const int t = threadIdx.x % NT, rl = threadIdx.x / NT, row = blockIdx.x * S::ROWS + rl;
+  Tm += (long)blockIdx.y * T * M;
+  FftTwiddles<float, M, E> tws;
+  tws.load(tw, t);
+  float2 v[E], xv[E / 2];
+#pragma unroll
+  for (int k = 0; k < E; ++k) v[k] = Tm[tpos(row, t + k * NT, T)];
+  const long cell = (long)(tile / nt * T + row) * N + tile % nt * T;
+#pragma unroll
+  for (int k = 0; k < E / 2; ++k) xv[k] = io.v[(long)s * io.sV + cell + t + k * NT];
   float sc = 1.f;
   if (io.nrm) {
     const double d = *boff(io.nrm, (long)s * io.sNrm);
     sc = d > 0.0 ? (float)(1.0 / d) : 0.f;
   }
-  const int i = (int)(e / N), j = (int)(e % N);
-  const int nt = N / T;
-  float2 xv = io.v[(long)s * io.sV + e];
-  xv.x *= sc;
-  xv.y *= sc;
-  if (io.nrm && io.vw) io.vw[(long)s * io.sV + e] = xv;
-  const float2 g = Y[((long)s * nt * nt + (i / T) * nt + j / T) * (T * T) + (i % T) * T + j % T];
-  io.z[(long)s * io.sZ + e] = cadd(xv, g);
+  if (dn) return;
+  reg_fft<float, M, +1, false, true, E>(v, smem + rl * LdsLen<M>::value, tws, t);  // columns < T are used
+  constexpr float inv = 1.f / ((float)M * (float)M);
+#pragma unroll
+  for (int k = 0; k < E / 2; ++k) {
+    const long e = cell + t + k * NT;
+    float2 x = xv[k];
+    x.x *= sc;
+    x.y *= sc;
+    if (io.nrm && io.vw) io.vw[(long)s * io.sV + e] = x;
+    io.z[(long)s * io.sZ + e] = cadd(x, cscale(v[k], inv));
+  }
 }
 
 // Inputs and partial products of the applications to scratch_sys systems.
@@ -1188,14 +1217,13 @@ int ensure_scratch(cgm_tiles* t, int nsys) {
   if (nsys <= t->scratch_sys) return CGM_SUCCESS;
   const size_t n = (size_t)t->N * t->N;
   const size_t tm = (size_t)t->nt * t->nt * t->T * t->P.M;
-  void* ptrs[] = {t->U, t->Y, t->Tm};
+  void* ptrs[] = {t->U, t->Tm};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
-  t->bytes -= (2 * n + tm) * sizeof(float2) * t->scratch_sys;
-  t->U = t->Y = t->Tm = nullptr;
+  t->bytes -= (n + tm) * sizeof(float2) * t->scratch_sys;
+  t->U = t->Tm = nullptr;
   t->scratch_sys = 0;
   if (hipMalloc((void**)&t->U, sizeof(float2) * n * nsys) != hipSuccess ||
-      hipMalloc((void**)&t->Y, sizeof(float2) * n * nsys) != hipSuccess ||
       hipMalloc((void**)&t->Tm, sizeof(float2) * tm * nsys) != hipSuccess) {
     cgm_set_last_error("tile preconditioner: scratch allocation for %d systems failed", nsys);
     return CGM_ERROR_ALLOC;
@@ -1206,7 +1234,7 @@ int ensure_scratch(cgm_tiles* t, int nsys) {
     return CGM_ERROR_DEVICE;
   }
   t->scratch_sys = nsys;
-  t->bytes += (2 * n + tm) * sizeof(float2) * nsys;
+  t->bytes += (n + tm) * sizeof(float2) * nsys;
   return grow_products(t);
 }
 
@@ -1269,19 +1297,16 @@ int launch_apply_red(const cgm_tiles* tl, hipStream_t st, const FnoIO& io, const
   bs.T = (long)tl->T * tl->P.M;
   rc = launch_pass1<float>(tl->P, st, tl->U, nullptr, nullptr, nullptr, kModeGreen, tl->Tm, tl->tw32, nullptr, B, bs);
   if (!rc) rc = launch_pass2<float, float2>(tl->P, st, tl->Tm, tl->gq, tl->tw32, nullptr, B, bs);
-  if (!rc)
-    rc = launch_pass3<float>(tl->P, st, tl->Tm, tl->U, nullptr, nullptr, tl->Y, kModeGreen, tl->tw32, nullptr, B, bs);
   if (rc) {
     cgm_set_last_error("tile convolution at T = %d failed", tl->T);
     return rc;
   }
-  const long n = (long)tl->N * tl->N;
   if (tl->T == 64)
-    hipLaunchKernelGGL((k_tile_combine<64>), dim3((n + 255) / 256, nsys), dim3(256), 0, st, io, tl->Y, done, sd,
-                       tl->N);
+    hipLaunchKernelGGL((k_tile_out<64>), dim3(64 / TileOut<64>::ROWS, B), dim3(256), 0, st, io, tl->Tm, tl->tw32,
+                       done, sd, tl->N);
   else
-    hipLaunchKernelGGL((k_tile_combine<128>), dim3((n + 255) / 256, nsys), dim3(256), 0, st, io, tl->Y, done, sd,
-                       tl->N);
+    hipLaunchKernelGGL((k_tile_out<128>), dim3(128 / TileOut<128>::ROWS, B), dim3(256), 0, st, io, tl->Tm, tl->tw32,
+                       done, sd, tl->N);
   CGM_HIP(hipGetLastError());
   return CGM_SUCCESS;
 }
@@ -1318,7 +1343,10 @@ int layout_reduced(cgm_tiles* t, const std::vector<int>& nc, int maps) {
     struct Item { int work, tile, i, j; };
     std::vector<Item> items;
     // long strips move fewer partial products and short ones keep more
-    // work-groups busy: the longest of which each CU gets two or more
+    // work-groups busy: the longest of which each CU gets four or more, and
+    // single rows only where two leave CUs idle (four 64 x 64 tiles, 84
+    // strips of two rows: 36.4 us with two, 33.4 with one; 16 tiles, 336
+    // strips: 52.1 and 54.5)
     int R = 8;
     for (;; R /= 2) {
       items.clear();
@@ -1331,7 +1359,7 @@ int layout_reduced(cgm_tiles* t, const std::vector<int>& nc, int maps) {
             items.push_back({work, tl, i, j});
           }
       }
-      if (R == 2 || items.size() >= 1024) break;
+      if (R == 1 || items.size() >= (R == 2 ? 256 : 1024)) break;
     }
     const int spos0 = (int)spos.size();
     int slots = 0;
@@ -1668,7 +1696,7 @@ extern "C" int cgm_tiles_destroy(cgm_tiles_t t) {
                   t->ids,  t->bloc, t->sloc, t->stab, t->spos, t->sstart, t->scount, t->ssize,
                   t->Pw,   t->Xs,   t->xinv, t->koff, t->nl,
                   t->W16,  t->Kw,   t->Pb,    t->Rw,   t->Cw,
-                  t->U,    t->Y,    t->Tm,   t->tw32, t->tw64, t->blkT,  t->gq};
+                  t->U,    t->Tm,   t->tw32, t->tw64, t->blkT,  t->gq};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (t->h) (void)rocblas_destroy_handle(t->h);
