@@ -884,7 +884,7 @@ k_tile_xs(const int* __restrict__ ncol, const unsigned short* __restrict__ cols,
 // compiler's waits know how many loads are younger than the ones waited for.
 //
 // At N = 512, T = 128 on a map of the benchmark (1.33 GB of W; a plain
-// non-temporal read of as much takes 190 us): one system 242 us (5.5 TB/s),
+// non-temporal read of as much takes 190 us): one system 229-236 us (5.7 TB/s),
 // 16 systems 337 us.  The vector-ALU kernel before it, which took one block
 // and one system at a time, took 272 and 3,000 us (202 us of arithmetic per
 // system).  One FP16 part instead of three would save 19 us at one system.
@@ -926,10 +926,12 @@ k_tile_ws(const unsigned* __restrict__ W16, const Strip* __restrict__ stab, cons
     for (int c = 0; c < 4; ++c)
       A[k % D][c] = __builtin_nontemporal_load(reinterpret_cast<const uint2_t*>(Bp + voff + 2 * c * B * sizeof(unsigned)));
   };
-  // x_i at the wave's rows, loaded a block ahead of its first use and before the loads of W that follow it
+  // x_i at the wave's rows, loaded a block ahead of its first use and before the loads of W that follow it; the
+  // columns not in use repeat column 0 (with one system, 14 of 16: 21 of every 152 KB read)
+  const int ax = a < ncols ? a : 0;
   uint4_t xr[2][kSplits], xn[2][kSplits];
   const auto load_x = [&](int i, uint4_t (*to)[kSplits]) {
-    const unsigned* xi = X + (long)i * kXsBlk + 32 * w + a * B + 4 * g;
+    const unsigned* xi = X + (long)i * kXsBlk + 32 * w + ax * B + 4 * g;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
