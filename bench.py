@@ -849,7 +849,7 @@ def profile_fno(ctx, net, dchi, db, batch=1):
     # layers 1-2); fno_cell_gemm_lift = the same for layer 0 (k_cell_row /
     # k_cell_rows_lift), lifting its row from chi and v; fno_proj =
     # k_cell_proj (layer-3 cell GEMM + the 32 -> 2 projection).  Batches of
-    # at least 2048 grid rows take the *_rows kernels, several grid rows per
+    # at least 1024 grid rows take the *_rows kernels, several grid rows per
     # work-group; the algorithmic bytes are the same.
     # For one vector the row kernels of
     # layers 0-2 form B_x themselves (inverse x-DFT from the mixed modes) and

@@ -317,30 +317,34 @@ __global__ void __launch_bounds__(512, NC <= 4 ? 4 : 2) k_back_rows(const bf16* 
 //
 // Bound by latencies (the loads of the block's 256 bytes of each row, then a
 // chain of 32 pairs, then the mixing), so 512 threads take CP chunks at once:
-// thread (chunk, kp, cp) holds RK frequencies x 2 channels.  One sample of
+// thread (chunk, kp, cp) holds RK frequencies x 2 channels.  With 8 and 16
+// frequencies CP is 4; five and six chunks (N = 320, 384) take 768 threads
+// and CP = 6 (SIX) instead of a second round for the fifth.  One sample of
 // N = 512 takes 7.4 us, 8 of N = 256 10.1 (11.1 backward); a transform that
 // left its chunks' partial sums to a mixing kernel took 5.0 + 4.0 and
 // 7.0 + 5.5 (7.1), and a launch more.
 constexpr int kPairs = 32;  // row pairs per chunk
-template <int KG>
+template <int KG, bool SIX = false>
 struct SpecShape {
   static constexpr int RK = KG >= 16 ? 2 : 1;   // frequencies per thread
   static constexpr int TPC = KG / RK * 16;      // threads per chunk
-  static constexpr int CP = 512 / TPC < 8 ? 512 / TPC : 8;  // chunks at once (8: 128 KiB of P and M)
+  // chunks at once: 512 threads' (at most 8: 128 KiB of P and M), or six
+  static constexpr int CP = SIX ? 6 : 512 / TPC < 8 ? 512 / TPC : 8;
+  static constexpr int NTHR = SIX ? 6 * TPC : 512;
   static size_t lds(int N) {
     const int nch = N / 64, cp = nch < CP ? nch : CP;
     return (size_t)cp * kPairs * C * 2 * sizeof(float2) + (size_t)KG * (cp * kPairs + 1) * sizeof(float2) +
            (size_t)nch * KG * C * sizeof(float2);
   }
 };
-template <int KG, bool BWD>
-__global__ void __launch_bounds__(512) k_spectral(const float* __restrict__ in, const float2* __restrict__ Ex,
+template <int KG, bool BWD, bool SIX>
+__global__ void __launch_bounds__((SpecShape<KG, SIX>::NTHR)) k_spectral(const float* __restrict__ in, const float2* __restrict__ Ex,
                                                   const float2* __restrict__ W, float2* __restrict__ usave,
                                                   float2* __restrict__ vout, int N, const int* done) {
 #pragma clang fp contract(off)
   if (skip(done)) return;
-  typedef SpecShape<KG> Sh;
-  constexpr int RK = Sh::RK, TPC = Sh::TPC, CP = Sh::CP;
+  typedef SpecShape<KG, SIX> Sh;
+  constexpr int RK = Sh::RK, TPC = Sh::TPC, CP = Sh::CP, NTHR = Sh::NTHR;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int nch = N / 64, ncp = nch < CP ? nch : CP;
   float2* sp = reinterpret_cast<float2*>(smem_raw);  // [chunk pair][C]
@@ -359,12 +363,12 @@ __global__ void __launch_bounds__(512) k_spectral(const float* __restrict__ in, 
   auto stage = [&](int g0) {  // P, M and the twiddles of the group's chunks to LDS
     const int pg = g0 * kPairs;                                   // first pair of the group
     const int np = (nch - g0 < CP ? nch - g0 : CP) * kPairs;      // its pairs
-    constexpr int NI = CP * kPairs * C / 4 / 512;  // items of 4 channels of a pair per thread
+    constexpr int NI = CP * kPairs * C / 4 / NTHR;  // items of 4 channels of a pair per thread
     float4 u1[NI][2], u2[NI][2];
 #pragma unroll
     for (int k = 0; k < NI; ++k) {
-      if (64 * k >= np) break;
-      int pl = (tid + 512 * k) >> 3;
+      if (NTHR / 8 * k >= np) break;
+      int pl = (tid + NTHR * k) >> 3;
       pl = pl < np ? pl : np - 1;
       const int c4 = (tid & 7) * 4, x = pg + pl, x2 = x == 0 ? N / 2 : N - x;
       const float* r1 = in + ((long)(b * N + x) * C + 2 * ky) * C + c4;
@@ -374,7 +378,7 @@ __global__ void __launch_bounds__(512) k_spectral(const float* __restrict__ in, 
       u2[k][0] = *reinterpret_cast<const float4*>(r2);
       u2[k][1] = *reinterpret_cast<const float4*>(r2 + C);
     }
-    // twiddles: 16 groups of 32 threads, frequency kq, 32 pairs per item
+    // twiddles: 16 groups of 32 of the first 512 threads, frequency kq, 32 pairs per item
     constexpr int NE = KG * CP * kPairs / 512, SE = 16 / KG * kPairs;
     const int kq = (tid >> 5) % KG, pe = (tid >> 5) / KG * kPairs + (tid & 31);
     float2 ev[NE];
@@ -382,7 +386,7 @@ __global__ void __launch_bounds__(512) k_spectral(const float* __restrict__ in, 
     for (int k = 0; k < NE; ++k) ev[k] = Ex[(long)(k0 + kq) * N + pg + (pe + SE * k < np ? pe + SE * k : 0)];
 #pragma unroll
     for (int k = 0; k < NI; ++k) {
-      const int pl = (tid + 512 * k) >> 3, c4 = (tid & 7) * 4;
+      const int pl = (tid + NTHR * k) >> 3, c4 = (tid & 7) * 4;
       if (pl >= np) break;
       const float4 a = u1[k][0], ai = u1[k][1], d = u2[k][0], di = u2[k][1];
       float4* p4 = reinterpret_cast<float4*>(sp + pl * C + c4);
@@ -394,7 +398,7 @@ __global__ void __launch_bounds__(512) k_spectral(const float* __restrict__ in, 
     }
 #pragma unroll
     for (int k = 0; k < NE; ++k)
-      if (pe + SE * k < np) se[kq * els + pe + SE * k] = ev[k];
+      if ((NTHR == 512 || tid < 512) && pe + SE * k < np) se[kq * els + pe + SE * k] = ev[k];
   };
   auto transform = [&](int g0) {
     const int np = (nch - g0 < CP ? nch - g0 : CP) * kPairs;
@@ -500,9 +504,9 @@ __global__ void __launch_bounds__(512) k_spectral(const float* __restrict__ in, 
 // block's 2 XP x 32 x 32 outputs are assembled in LDS, where the 16-byte
 // chunk j of channel ch is at j ^ (ch / 4 % 4) (a wave's writes, one word per
 // channel, then touch 32 banks and not 4), and leave as 16-byte stores of
-// whole 2 KiB rows.  Every block reads its sample's 128 KiB of modes, so XP
-// is the largest that still gives every CU a block (N = 256, 8 samples: XP 4
-// takes 6.8 us; XP 8, half the CUs, and unswizzled 2-byte LDS writes 10.2).
+// whole 2 KiB rows.  Every block reads its sample's 128 KiB of modes, so few
+// blocks are better as long as every CU has one (N = 256, 8 samples: XP 4 takes
+// 6.8 us; XP 8, half the CUs, and unswizzled 2-byte LDS writes 10.2).
 template <int XP>
 __global__ void __launch_bounds__(512) k_invx(const float2* __restrict__ V, bf16* __restrict__ out,
                                               const float2* __restrict__ Ex, int N, const int* done) {
@@ -1802,47 +1806,61 @@ int launch_back_rows(const cgm_fno* f, hipStream_t st, const bf16* Y, const floa
   return CGM_SUCCESS;
 }
 
-// the most row pairs per work-group that still leave 256 of them, one per CU
+// One row pair per work-group while that is at most one per CU, then two, four
+// from twice as many on, and eight where they still give every CU one: the
+// forward pass of three samples of N = 320 (480 pairs) takes 124.5 us with two
+// and 130.1 with one, of two of N = 256 (256 pairs) 86.2 and 85.1; eight samples
+// of N = 256 (1,024 pairs): k_invx 7.0 us with four, 8.9 with eight.
 void launch_invx(cgm_fno* f, hipStream_t st, int B, const int* done) {
   const int pairs = f->N / 2 * B;
   if (pairs >= 8 * 256)
     hipLaunchKernelGGL(k_invx<8>, dim3(f->N / 16, 1, B), dim3(512), 0, st, f->Vm, f->Bt, f->Ex, f->N, done);
-  else if (pairs >= 4 * 256)
+  else if (pairs > 2 * 256)
     hipLaunchKernelGGL(k_invx<4>, dim3(f->N / 8, 1, B), dim3(512), 0, st, f->Vm, f->Bt, f->Ex, f->N, done);
-  else if (pairs >= 2 * 256)
+  else if (pairs > 256)
     hipLaunchKernelGGL(k_invx<2>, dim3(f->N / 4, 1, B), dim3(512), 0, st, f->Vm, f->Bt, f->Ex, f->N, done);
   else
     hipLaunchKernelGGL(k_invx<1>, dim3(f->N / 2, 1, B), dim3(512), 0, st, f->Vm, f->Bt, f->Ex, f->N, done);
 }
 
-// A of B vectors to the mixed modes Vm, with the most frequencies per block
-// (16, 8, 4, 2) that leave 256 blocks, one per CU: a block reads its part of A
-// once for all its frequencies (measured with the twiddles staged one by one:
-// 8 samples of N = 256: 16 per block 11.4 us, 8 per block 15.9; one of N = 512:
-// 2 per block 7.9, 4 per block 8.7).
+// A of B vectors to the mixed modes Vm, with the fewest frequencies per block
+// (2, 4, 8, 16) that need no more than 256 blocks: the LDS holds one block per
+// CU, so more of them are a second round (8 samples of N = 256: 16 per block
+// 11.4 us, 8 per block 15.9; one of N = 512: 2 per block 7.9, 4 per block 8.7;
+// six of N = 512: 8 per block 20.8, 16 per block 13.5).
+template <int KG, bool SIX>
+void launch_spectral_k(const cgm_fno* f, hipStream_t st, const float2* W, float2* usave, bool bwd, int B,
+                       const int* done) {
+  typedef SpecShape<KG, SIX> Sh;
+  hipLaunchKernelGGL((bwd ? k_spectral<KG, true, SIX> : k_spectral<KG, false, SIX>), dim3(KY, KX / KG, B),
+                     dim3(Sh::NTHR), Sh::lds(f->N), st, f->A, f->Ex, W, usave, f->Vm, f->N, done);
+}
 template <int KG>
 void launch_spectral_n(const cgm_fno* f, hipStream_t st, const float2* W, float2* usave, bool bwd, int B,
                        const int* done) {
-  hipLaunchKernelGGL((bwd ? k_spectral<KG, true> : k_spectral<KG, false>), dim3(KY, KX / KG, B), dim3(512),
-                     SpecShape<KG>::lds(f->N), st, f->A, f->Ex, W, usave, f->Vm, f->N, done);
+  const int nch = f->N / 64;
+  if constexpr (KG >= 8) {
+    if (nch == 5 || nch == 6) return launch_spectral_k<KG, true>(f, st, W, usave, bwd, B, done);
+  }
+  launch_spectral_k<KG, false>(f, st, W, usave, bwd, B, done);
 }
 void launch_spectral(const cgm_fno* f, hipStream_t st, const float2* W, float2* usave, bool bwd, int B,
                      const int* done) {
-  const int kg = KY * KX * B / 256;
-  if (kg >= 16)
+  const int kg = KY * KX * B / 256;  // at least this many
+  if (kg > 8)
     launch_spectral_n<16>(f, st, W, usave, bwd, B, done);
-  else if (kg >= 8)
+  else if (kg > 4)
     launch_spectral_n<8>(f, st, W, usave, bwd, B, done);
-  else if (kg >= 4)
+  else if (kg > 2)
     launch_spectral_n<4>(f, st, W, usave, bwd, B, done);
   else
     launch_spectral_n<2>(f, st, W, usave, bwd, B, done);
 }
-template <int KG>
+template <int KG, bool SIX = false>
 int spectral_limits(int N) {
-  const void* k[] = {(const void*)k_spectral<KG, false>, (const void*)k_spectral<KG, true>};
+  const void* k[] = {(const void*)k_spectral<KG, false, SIX>, (const void*)k_spectral<KG, true, SIX>};
   for (const void* p : k)
-    CGM_HIP(hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SpecShape<KG>::lds(N)));
+    CGM_HIP(hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SpecShape<KG, SIX>::lds(N)));
   return CGM_SUCCESS;
 }
 
@@ -1861,15 +1879,17 @@ int spectral(cgm_fno* f, hipStream_t st, const float2* W, float2* usave, bool bw
 namespace cgm {
 
 // Two grid rows per block where N allows it (N even, N <= 512) and the
-// grid still holds at least 1024 blocks.
-inline bool two_rows(int N, int rows) { return N % 2 == 0 && N <= 512 && rows / 2 >= 1024; }
+// grid still holds at least 512 blocks, two per CU, from as many on four: one pass
+// over four samples of N = 256 takes 106 us (116.6 with single rows), over four of
+// N = 512 211 with four rows per block and 221 with two.
+inline bool two_rows(int N, int rows) { return N % 2 == 0 && N <= 512 && rows / 2 >= 512; }
 
 // The lift with layer 0's first row projection (k_lift_row / k_lift_rows):
-// four rows per block where the grid still holds 1024 blocks, else two.
+// four rows per block where the grid still holds 512 blocks, else two.
 void launch_lift(const cgm_fno* f, hipStream_t st, int rows, const LiftIn& L, float2* vw, bf16* h0,
                  const int* done) {
   const size_t lds = row_kernel_lds(f->N);
-  if (f->N % 4 == 0 && f->N <= 512 && rows / 4 >= 1024)
+  if (f->N % 4 == 0 && f->N <= 512 && rows / 4 >= 512)
     hipLaunchKernelGGL(k_lift_rows<4>, dim3(rows / 4), dim3(512), lds, st, L, vw, h0, f->Ft, f->A, f->N, done);
   else if (two_rows(f->N, rows))
     hipLaunchKernelGGL(k_lift_rows<2>, dim3(rows / 2), dim3(512), lds, st, L, vw, h0, f->Ft, f->A, f->N, done);
@@ -1881,7 +1901,7 @@ void launch_lift(const cgm_fno* f, hipStream_t st, int rows, const LiftIn& L, fl
 void launch_cell_rows_lift(const cgm_fno* f, hipStream_t st, int rows, const LiftIn& L, const bf16* W,
                            const float* bias, bf16* pre, bf16* out, const int* done) {
   const size_t lds = row_kernel_lds(f->N);
-  if (f->N % 4 == 0 && f->N <= 512 && rows / 4 >= 1024)
+  if (f->N % 4 == 0 && f->N <= 512 && rows / 4 >= 512)
     hipLaunchKernelGGL(k_cell_rows_lift<4>, dim3(rows / 4), dim3(512), lds, st, L, f->Fy, W, f->Bt, bias, pre, out,
                        f->Ft, f->A, f->N, done);
   else if (two_rows(f->N, rows))
@@ -1908,14 +1928,14 @@ void launch_cell_fold(const cgm_fno* f, hipStream_t st, int rows, bool lift, con
 }
 
 // Cell GEMM of layers 1-2 on B > 1 samples (B_x from R): the most rows per
-// work-group (8, 4 or 2) that leave at least 1024 work-groups.
+// work-group (8, 4 or 2) that leave at least 1024 work-groups (4: 512).
 void launch_cell_rows(const cgm_fno* f, hipStream_t st, int rows, const bf16* P, const bf16* W, const float* bias,
                       bf16* pre, bf16* out, const int* done) {
   const size_t lds = row_kernel_lds(f->N);
   if (f->N % 8 == 0 && f->N <= 512 && rows / 8 >= 1024)
     hipLaunchKernelGGL(k_cell_rows<8>, dim3(rows / 8), dim3(512), lds, st, P, f->Fy, W, f->Bt, bias, pre, out, f->Ft,
                        f->A, f->N, done);
-  else if (f->N % 4 == 0 && f->N <= 512 && rows / 4 >= 1024)
+  else if (f->N % 4 == 0 && f->N <= 512 && rows / 4 >= 512)
     hipLaunchKernelGGL(k_cell_rows<4>, dim3(rows / 4), dim3(512), lds, st, P, f->Fy, W, f->Bt, bias, pre, out, f->Ft,
                        f->A, f->N, done);
   else if (two_rows(f->N, rows))
@@ -2132,7 +2152,8 @@ extern "C" int cgm_fno_create(cgm_ctx_t c, int batch, float chi_scale, cgm_fno_t
   CGM_HIP(hipMemcpy(f->Fy, fy.data(), sizeof(bf16) * fy.size(), hipMemcpyHostToDevice));
   CGM_HIP(hipMemcpy(f->Ex, ex.data(), sizeof(float2) * ex.size(), hipMemcpyHostToDevice));
   if ((rc = spectral_limits<2>(N)) || (rc = spectral_limits<4>(N)) || (rc = spectral_limits<8>(N)) ||
-      (rc = spectral_limits<16>(N)))
+      (rc = spectral_limits<16>(N)) ||
+      (N <= 384 && ((rc = spectral_limits<8, true>(N)) || (rc = spectral_limits<16, true>(N)))))
     return rc;
   const void* backk[] = {(const void*)k_back_rows<1, false>, (const void*)k_back_rows<1, true>,
                          (const void*)k_back_rows<2, false>, (const void*)k_back_rows<2, true>,

@@ -210,11 +210,11 @@ def test_fno_backward_row_sizes(gpu, N, B):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("N,B", [(64, 2), (128, 5), (320, 8), (1024, 4)])
+@pytest.mark.parametrize("N,B", [(64, 2), (128, 5), (320, 4), (384, 8), (448, 5), (1024, 4)])
 def test_spectral_blocks_round_alike(gpu, N, B):
     """The spectral kernel takes 2, 4, 8 or 16 frequencies per block by B (1, 2,
-    5, 8) and its chunks of 64 rows in one or several groups (N = 64: one chunk,
-    320: five, 1024: sixteen): a batch equals its single vectors bit for bit."""
+    4, from 5) and its chunks of 64 rows in one or several groups (N = 64: one chunk,
+    320 and 384: five and six taken at once, 448: seven, 1024: sixteen): a batch equals its single vectors bit for bit."""
     test_fno_forward_batch_equals_single_vectors(gpu, N, B)
 
 
