@@ -255,8 +255,25 @@ k_tile_apply8(const float2* __restrict__ K, long sK, FnoIO io, const int* __rest
     if (live[v]) io.z[(long)(s0 + v) * io.sZ + cell] = acc[v];
 }
 
+// io.vw = io.v over its norm, system blockIdx.y, before an application that is
+// to normalise its input in place: several work-groups of k_tile_apply read a
+// tile, so none of them can write to it (a late one would divide again).
+__global__ void __launch_bounds__(256)
+k_tile_scale(FnoIO io, const int* __restrict__ done, long sd, long n) {
+  const int s = blockIdx.y;
+  if (done && *boff(done, (long)s * sd)) return;
+  const long e = (long)blockIdx.x * 256 + threadIdx.x;
+  if (e >= n) return;
+  const double d = *boff(io.nrm, (long)s * io.sNrm);
+  const float sc = d > 0.0 ? (float)(1.0 / d) : 0.f;
+  float2 x = io.v[(long)s * io.sV + e];
+  x.x *= sc;
+  x.y *= sc;
+  io.vw[(long)s * io.sV + e] = x;
+}
+
 // Tiles of side 16 and 32: blockIdx.x = tile and block of 128 rows, blockIdx.y =
-// group of NV systems.
+// group of NV systems.  io.vw must not be io.v (k_tile_scale).
 //
 // The stream of K bounds it (8 T^4 bytes per tile; column-major, so rows are
 // independent and a row block needs no sum with another).  A wave reads two
@@ -407,9 +424,16 @@ int launch_apply_m(const cgm_tiles* tl, hipStream_t st, const FnoIO& io, const i
     else
       hipLaunchKernelGGL(k_tile_apply8<1>, dim3(ntiles, groups), dim3(64), 0, st, tl->K, sK, io, done, sd, tl->N, tl->T, nsys);
   } else {
+    FnoIO in = io;
+    if (io.nrm && io.vw == io.v) {
+      const long n = (long)tl->N * tl->N;
+      hipLaunchKernelGGL(k_tile_scale, dim3((unsigned)((n + 255) / 256), nsys), dim3(256), 0, st, io, done, sd, n);
+      in.nrm = nullptr;
+      in.vw = nullptr;
+    }
 #define CGM_DENSE(NV, S)                                                                                              \
   hipLaunchKernelGGL((k_tile_apply<M2, NV>), dim3(ntiles * (M2 / 128), groups), dim3(64 * kTileWaves), 0, st, tl->K, S, \
-                     io, done, sd, tl->N, tl->T, nsys)
+                     in, done, sd, tl->N, tl->T, nsys)
     switch (nv) {
       case 8: CGM_DENSE(8, 0L); break;
       case 4: CGM_DENSE(4, 0L); break;

@@ -423,3 +423,50 @@ def _oracle_right_pc_gmres(A, P, b, tol, m=400):
         if np.linalg.norm(e1 - H[:j + 2, :j + 1] @ y) <= tol * bn:
             break
     return y @ Z[:j + 1], j + 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,T", [(448, 16), (448, 32), (160, 32), (64, 8)])
+def test_two_pass_fgmres_normalises_its_input_in_place(N, T):
+    """The two-pass cycle (restart <= 64, N no power of two or path 1) hands the
+    tile inverses the same buffer to read v from and to write v / ||v|| to, with
+    ||b|| = N for the first vector.  Several work-groups read a tile of side 16
+    or 32: 1,568 of them on both grids of N = 448, more than run at once.  The
+    estimate history equals that of the same cycle written out with the
+    out-of-place call, P(v) = tl.apply(v / ||v||), in FP64 between the calls, to
+    1e-4 of ||r0|| (as the fused and the two-pass cycles agree above)."""
+    import torch
+    from cugmres_amd import problems, solver, tiles as gt
+    print(f"two-pass fgmres N={N} T={T}", flush=True)
+    m = 8
+    ctx = solver.Context(N, 0)
+    ctx.set_arnoldi_path(1)
+    g = ctx.spectrum_helmholtz(problems.KH)
+    chi, b = _problem(N, 5)
+    dchi = ctx.to_device(chi, "f32")
+    tl = gt.Tiles(ctx, T, 1).factor(ctx.block_helmholtz(problems.KH), dchi)
+    _, info = ctx.fgmres(g, dchi, ctx.to_device(b), precond=tl, restart=m, tol=1e-9, max_cycles=1, stall_ratio=0.0,
+                         history=True)
+    n = N * N
+    V = np.zeros((m + 1, n), complex)
+    H = np.zeros((m + 1, m), complex)
+    V[0] = b / np.linalg.norm(b)
+    want = [np.linalg.norm(b)]
+    for j in range(m):
+        z = tl.apply(ctx.to_device(V[j].astype(np.complex64)))
+        w = ctx.matvec(g, dchi, z).cpu().numpy().astype(complex)
+        for _ in range(2):
+            h = V[:j + 1].conj() @ w
+            w = w - h @ V[:j + 1]
+            H[:j + 1, j] += h
+        H[j + 1, j] = np.linalg.norm(w)
+        V[j + 1] = w / H[j + 1, j]
+        e1 = np.zeros(j + 2, complex)
+        e1[0] = want[0]
+        y = np.linalg.lstsq(H[:j + 2, :j + 1], e1, rcond=None)[0]
+        want.append(np.linalg.norm(e1 - H[:j + 2, :j + 1] @ y))
+    got = info["history"]
+    assert len(got) == m + 1
+    assert np.abs(got - want).max() < 1e-4 * want[0], (got, want)
+    tl.close()
+    ctx.close()
