@@ -150,6 +150,7 @@ int grow(cgm_tiles* t, P** p, size_t* cap, size_t need) {
   }
   if (hipMalloc((void**)p, need * sizeof(P)) != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();  // the caller reports it; the next launch's check must not
     cgm_set_last_error("tile preconditioner: allocation of %zu MiB failed", need * sizeof(P) >> 20);
     return CGM_ERROR_ALLOC;
   }
@@ -1227,11 +1228,11 @@ k_tile_out(FnoIO io, const float2* __restrict__ Tm, const float2* __restrict__ t
   }
 }
 
-// Inputs and partial products of the applications to scratch_sys systems.
+// Inputs and partial products of the applications to up to nsys systems.
 // One map serves groups of 8 or 16 systems; systems with maps of their own
 // are groups of one.
-int grow_products(cgm_tiles* t) {
-  const size_t sys = (size_t)std::max(t->scratch_sys, 1);
+int grow_products(cgm_tiles* t, int nsys) {
+  const size_t sys = (size_t)std::max(nsys, 1);
   const size_t groups = t->maps1 ? (sys + 15) / 16 : sys, per = t->maps1 ? std::min<size_t>(sys, 16) : 1;
   int rc = grow(t, &t->Pw, &t->pw_cap, groups * t->plen_max * 64 * per);
   if (!rc) rc = grow(t, &t->Xs, &t->xs_cap, groups * t->xblk_max * kXsBlk);
@@ -1239,29 +1240,43 @@ int grow_products(cgm_tiles* t) {
   return rc;
 }
 
-int ensure_scratch(cgm_tiles* t, int nsys) {
-  if (nsys <= t->scratch_sys) return CGM_SUCCESS;
-  const size_t n = (size_t)t->N * t->N;
-  const size_t tm = (size_t)t->nt * t->nt * t->T * t->P.M;
+void release_scratch(cgm_tiles* t) {
   void* ptrs[] = {t->U, t->Tm};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
-  t->bytes -= (n + tm) * sizeof(float2) * t->scratch_sys;
   t->U = t->Tm = nullptr;
+  const size_t n = (size_t)t->N * t->N, tm = (size_t)t->nt * t->nt * t->T * t->P.M;
+  t->bytes -= (n + tm) * sizeof(float2) * t->scratch_sys;
   t->scratch_sys = 0;
+}
+
+// The apply scratch for nsys systems; where one of its buffers cannot be had,
+// none counts (scratch_sys = 0) and the next application asks for all again.
+int ensure_scratch(cgm_tiles* t, int nsys) {
+  if (nsys <= t->scratch_sys) return CGM_SUCCESS;
+  release_scratch(t);
+  const size_t n = (size_t)t->N * t->N;
+  const size_t tm = (size_t)t->nt * t->nt * t->T * t->P.M;
+  int rc = CGM_SUCCESS;
   if (hipMalloc((void**)&t->U, sizeof(float2) * n * nsys) != hipSuccess ||
       hipMalloc((void**)&t->Tm, sizeof(float2) * tm * nsys) != hipSuccess) {
+    (void)hipGetLastError();
     cgm_set_last_error("tile preconditioner: scratch allocation for %d systems failed", nsys);
-    return CGM_ERROR_ALLOC;
+    rc = CGM_ERROR_ALLOC;
   }
   // the cells with chi = 0 keep u = 0: the application writes only the cells of S
-  if (hipMemset(t->U, 0, sizeof(float2) * n * nsys) != hipSuccess) {
+  if (!rc && hipMemset(t->U, 0, sizeof(float2) * n * nsys) != hipSuccess) {
     cgm_set_last_error("tile preconditioner: scratch clear failed");
-    return CGM_ERROR_DEVICE;
+    rc = CGM_ERROR_DEVICE;
+  }
+  if (!rc) rc = grow_products(t, nsys);
+  if (rc) {
+    release_scratch(t);
+    return rc;
   }
   t->scratch_sys = nsys;
   t->bytes += (n + tm) * sizeof(float2) * nsys;
-  return grow_products(t);
+  return CGM_SUCCESS;
 }
 
 // u_t = W_t x_t[S] of every tile for nsys systems; NT = 1: groups of up to 8
@@ -1411,7 +1426,7 @@ int layout_reduced(cgm_tiles* t, const std::vector<int>& nc, int maps) {
   if ((rc = grow(t, &t->W16, &t->w16_cap, (size_t)std::max(total, 1L)))) return rc;
   if ((rc = grow(t, &t->stab, &t->stab_cap, std::max<size_t>(stab.size(), 1)))) return rc;
   if ((rc = grow(t, &t->spos, &t->spos_cap, std::max<size_t>(spos.size(), 1)))) return rc;
-  if ((rc = grow_products(t))) return rc;
+  if ((rc = grow_products(t, t->scratch_sys))) return rc;
   CGM_HIP(hipMemcpyAsync(t->woff, off.data(), sizeof(long) * nb, hipMemcpyHostToDevice, st));
   CGM_HIP(hipMemcpyAsync(t->bloc, bloc.data(), sizeof(int) * nb, hipMemcpyHostToDevice, st));
   CGM_HIP(hipMemcpyAsync(t->sloc, sloc.data(), sizeof(int) * nb, hipMemcpyHostToDevice, st));

@@ -470,3 +470,31 @@ def test_two_pass_fgmres_normalises_its_input_in_place(N, T):
     assert np.abs(got - want).max() < 1e-4 * want[0], (got, want)
     tl.close()
     ctx.close()
+
+
+@pytest.mark.gpu
+def test_reduced_tiles_after_a_failed_scratch_allocation():
+    """A batch whose partial products (425 GB: 1,056 strips of one full 128 x 128
+    tile for 4,096 groups of 16 systems) do not fit the device is refused, a second
+    time too, before any launch; then a single vector gives the same result as
+    before, and the workspace counts the same bytes."""
+    import torch
+    from cugmres_amd import _lib, problems, solver, tiles as gt
+    N = T = 128
+    print("tiles scratch allocation failure", flush=True)
+    ctx = solver.Context(N, 0)
+    chi = ctx.to_device(np.random.default_rng(1).uniform(0.1, 0.5, N * N), "f32")
+    tl = gt.Tiles(ctx, T, 1).factor(ctx.block_helmholtz(problems.KH), chi)
+    x = ctx.to_device(problems.plane_wave(N, problems.KH, 0.4).reshape(-1))
+    want = tl.apply(x)
+    held = tl.memory_bytes()
+    many = torch.empty((65535, N * N), dtype=torch.complex64, device=ctx.device)
+    for _ in range(2):
+        with pytest.raises(_lib.CgmError, match="allocation"):
+            tl.apply(many, out=many.new_empty((65535, N * N)))
+    assert torch.equal(tl.apply(x), want)
+    assert tl.memory_bytes() == held
+    tl.close()
+    ctx.close()
+    del many
+    torch.cuda.empty_cache()
