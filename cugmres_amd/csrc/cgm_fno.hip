@@ -1856,11 +1856,44 @@ void launch_spectral(const cgm_fno* f, hipStream_t st, const float2* W, float2* 
   else
     launch_spectral_n<2>(f, st, W, usave, bwd, B, done);
 }
-template <int KG, bool SIX = false>
-int spectral_limits(int N) {
-  const void* k[] = {(const void*)k_spectral<KG, false, SIX>, (const void*)k_spectral<KG, true, SIX>};
-  for (const void* p : k)
-    CGM_HIP(hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SpecShape<KG, SIX>::lds(N)));
+// Lets a kernel ask for all the LDS that its static part leaves.  The limit
+// belongs to the kernel, not to a network: one set to what this network's N
+// needs would be lowered by a smaller network created later.
+int whole_lds(const void* kernel) {
+  hipFuncAttributes at;
+  CGM_HIP(hipFuncGetAttributes(&at, kernel));
+  CGM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)(kMaxLds - at.sharedSizeBytes)));
+  return CGM_SUCCESS;
+}
+template <int KG, bool SIX>
+constexpr const void* spectral_kernel(bool bwd) {
+  return bwd ? (const void*)k_spectral<KG, true, SIX> : (const void*)k_spectral<KG, false, SIX>;
+}
+// Of every kernel with an N-dependent LDS size, on the current device.
+int lds_limits() {
+  const void* kernels[] = {
+      spectral_kernel<2, false>(false),       spectral_kernel<2, false>(true),
+      spectral_kernel<4, false>(false),       spectral_kernel<4, false>(true),
+      spectral_kernel<8, false>(false),       spectral_kernel<8, false>(true),
+      spectral_kernel<16, false>(false),      spectral_kernel<16, false>(true),
+      spectral_kernel<8, true>(false),        spectral_kernel<8, true>(true),
+      spectral_kernel<16, true>(false),       spectral_kernel<16, true>(true),
+      (const void*)k_back_rows<1, false>,     (const void*)k_back_rows<1, true>,
+      (const void*)k_back_rows<2, false>,     (const void*)k_back_rows<2, true>,
+      (const void*)k_back_rows<4, false>,     (const void*)k_back_rows<4, true>,
+      (const void*)k_back_rows<8, false>,     (const void*)k_back_rows<8, true>,
+      (const void*)k_lift_row,                (const void*)k_cell_pair<false>,
+      (const void*)k_cell_pair<true>,         (const void*)k_cell_row<true, false>,
+      (const void*)k_cell_row<false, false>,  (const void*)k_cell_row<true, true>,
+      (const void*)k_cell_row<false, true>,   (const void*)k_cell_rows<2>,
+      (const void*)k_cell_rows<4>,            (const void*)k_cell_rows<8>,
+      (const void*)k_cell_rows_lift<2>,       (const void*)k_cell_rows_lift<4>,
+      (const void*)k_lift_rows<2>,            (const void*)k_lift_rows<4>};
+  for (const void* k : kernels) {
+    const int rc = whole_lds(k);
+    if (rc) return rc;
+  }
   return CGM_SUCCESS;
 }
 
@@ -2148,36 +2181,18 @@ extern "C" int cgm_fno_create(cgm_ctx_t c, int batch, float chi_scale, cgm_fno_t
       ex[(size_t)q * N + y] = make_float2((float)cos(ph), (float)sin(ph));
     }
   }
-  CGM_HIP(hipMemcpy(f->Ft, ft.data(), sizeof(bf16) * ft.size(), hipMemcpyHostToDevice));
-  CGM_HIP(hipMemcpy(f->Fy, fy.data(), sizeof(bf16) * fy.size(), hipMemcpyHostToDevice));
-  CGM_HIP(hipMemcpy(f->Ex, ex.data(), sizeof(float2) * ex.size(), hipMemcpyHostToDevice));
-  if ((rc = spectral_limits<2>(N)) || (rc = spectral_limits<4>(N)) || (rc = spectral_limits<8>(N)) ||
-      (rc = spectral_limits<16>(N)) ||
-      (N <= 384 && ((rc = spectral_limits<8, true>(N)) || (rc = spectral_limits<16, true>(N)))))
-    return rc;
-  const void* backk[] = {(const void*)k_back_rows<1, false>, (const void*)k_back_rows<1, true>,
-                         (const void*)k_back_rows<2, false>, (const void*)k_back_rows<2, true>,
-                         (const void*)k_back_rows<4, false>, (const void*)k_back_rows<4, true>,
-                         (const void*)k_back_rows<8, false>, (const void*)k_back_rows<8, true>};
-  for (const void* k : backk)
-    CGM_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)((size_t)2 * N * C * sizeof(bf16))));
-  CGM_HIP(hipFuncSetAttribute((const void*)k_lift_row, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)row_kernel_lds(N)));
-  if (N <= 512) {
-    CGM_HIP(hipFuncSetAttribute((const void*)k_cell_pair<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)cell_pair_lds(N, false)));
-    CGM_HIP(hipFuncSetAttribute((const void*)k_cell_pair<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)cell_pair_lds(N, true)));
+  if (hipMemcpy(f->Ft, ft.data(), sizeof(bf16) * ft.size(), hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(f->Fy, fy.data(), sizeof(bf16) * fy.size(), hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(f->Ex, ex.data(), sizeof(float2) * ex.size(), hipMemcpyHostToDevice) != hipSuccess) {
+    cgm_set_last_error("cgm_fno_create: copy of the bases failed");
+    rc = CGM_ERROR_DEVICE;
   }
-  const void* rowk[] = {(const void*)k_cell_row<true, false>, (const void*)k_cell_row<false, false>,
-                        (const void*)k_cell_row<true, true>,  (const void*)k_cell_row<false, true>,
-                        (const void*)k_cell_rows<2>,          (const void*)k_cell_rows<4>,
-                        (const void*)k_cell_rows<8>,
-                        (const void*)k_cell_rows_lift<2>,     (const void*)k_cell_rows_lift<4>,
-                        (const void*)k_lift_rows<2>,          (const void*)k_lift_rows<4>};
-  for (const void* k : rowk)
-    CGM_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)row_kernel_lds(N)));
+  if (!rc) rc = lds_limits();
+  if (rc) {
+    fno_free(f);
+    delete f;
+    return rc;
+  }
   *out = f;
   return CGM_SUCCESS;
 }

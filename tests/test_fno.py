@@ -335,3 +335,35 @@ def test_validation_based_stop_keeps_the_best_held_out_parameters(gpu):
     assert kept < 0.9 * learn.validation_loss(ctx, g, untrained, chi_v, v_v)
     tl.close()
 
+
+
+@pytest.mark.gpu
+def test_networks_of_different_sizes_in_turn(gpu):
+    """The kernels of a small and a large network are the same, with 11 to 145 KB
+    of LDS: a small one created while a large one is alive changes nothing for the
+    large one, forward and backward bit for bit."""
+    import torch
+    solver, fno = gpu
+    nets = {}
+
+    def step(N):
+        net, chi, v = nets[N]
+        z = net.forward(chi, v, train=True)
+        return z, net.backward(v)
+
+    def create(N, B):
+        ctx = solver.Context(N)
+        rng = np.random.default_rng(N)
+        chi = torch.as_tensor(rng.uniform(0.0, 11.1, (B, N * N)).astype(np.float32)).to(ctx.device)
+        v = rng.standard_normal((B, N * N)) + 1j * rng.standard_normal((B, N * N))
+        v = torch.as_tensor((v / np.linalg.norm(v, axis=1, keepdims=True)).astype(np.complex64)).to(ctx.device)
+        nets[N] = fno.Preconditioner(ctx, batch=B, params=fno.init_params(1, zero_out=False)), chi, v
+    print("networks of N = 1024, 384 and 64 in turn", flush=True)
+    create(1024, 1)
+    create(384, 2)
+    alone = {N: step(N) for N in (1024, 384)}
+    create(64, 1)
+    step(64)
+    for N in (1024, 384):
+        for a, b in zip(alone[N], step(N)):
+            assert torch.equal(a, b), N
