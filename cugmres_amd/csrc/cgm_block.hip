@@ -470,7 +470,8 @@ extern "C" int cgm_block_orthonormalise(cgm_ctx_t c, const cgm_complex64* basis,
   if (!B.ticket) {
     unsigned* p = nullptr;
     CGM_HIP(hipMalloc((void**)&p, sizeof(unsigned)));
-    if (hipMemset(p, 0, sizeof(unsigned)) != hipSuccess) {
+    // cleared before the launches below, whose stream need not wait for the null stream's
+    if (hipMemset(p, 0, sizeof(unsigned)) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
       (void)hipFree(p);
       cgm_set_last_error("block orthonormalisation: ticket clear failed");
       return CGM_ERROR_DEVICE;

@@ -1264,8 +1264,10 @@ int ensure_scratch(cgm_tiles* t, int nsys) {
     cgm_set_last_error("tile preconditioner: scratch allocation for %d systems failed", nsys);
     rc = CGM_ERROR_ALLOC;
   }
-  // the cells with chi = 0 keep u = 0: the application writes only the cells of S
-  if (!rc && hipMemset(t->U, 0, sizeof(float2) * n * nsys) != hipSuccess) {
+  // the cells with chi = 0 keep u = 0: the application writes only the cells of
+  // S, on a stream that need not wait for the null stream's clear
+  if (!rc && (hipMemset(t->U, 0, sizeof(float2) * n * nsys) != hipSuccess ||
+              hipStreamSynchronize(nullptr) != hipSuccess)) {
     cgm_set_last_error("tile preconditioner: scratch clear failed");
     rc = CGM_ERROR_DEVICE;
   }

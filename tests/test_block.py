@@ -270,3 +270,30 @@ def test_device_orthonormalisation(n, k, s):
         dW[s - 1] = dW[0]
         assert call(dW)[-1].real in (1.0, 2.0)
     ctx.close()
+
+
+@pytest.mark.gpu
+def test_block_solve_on_a_stream_of_its_own():
+    """A context bound to a side stream, whose work need not wait for the null
+    stream: its first block step and the first application to more systems than
+    the tiles' workspace holds (which allocate and clear) give the bits of the
+    default stream."""
+    import torch
+    from cugmres_amd import block, problems, solver, tiles as gt
+    N, T, s = 128, 64, 5
+    print("block solve on a side stream", flush=True)
+    out = []
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            ctx = solver.Context(N, 0)
+            g = ctx.spectrum_helmholtz(problems.KH)
+            chi = ctx.to_device(problems.block_eps_map(N, 8, 0.5, 0.75, seed=3, eps_hi=2.25) - 1.0, "f32")
+            B = torch.stack([ctx.to_device(problems.plane_wave(N, problems.KH, 0.3 + k).reshape(-1)) for k in range(s)])
+            tl = gt.Tiles(ctx, T, 1).factor(ctx.block_helmholtz(problems.KH), chi)
+            X, info = block.solve_map(ctx, g, chi, B, tiles=tl, restart=12, tol=1e-12, max_cycles=1)
+            stream.synchronize()
+            out.append((X.cpu(), info["block_steps"]))
+            tl.close()
+            ctx.close()
+    assert out[0][1] == out[1][1] == 12
+    assert torch.equal(out[0][0], out[1][0])
