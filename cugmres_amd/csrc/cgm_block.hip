@@ -440,6 +440,7 @@ int ensure(void** p, size_t* cap, size_t need) {
   *cap = 0;
   if (hipMalloc(p, need) != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();  // the caller reports it; the next launch's check must not
     cgm_set_last_error("block orthonormalisation: allocation of %zu MiB failed", need >> 20);
     return CGM_ERROR_ALLOC;
   }

@@ -297,3 +297,29 @@ def test_block_solve_on_a_stream_of_its_own():
             ctx.close()
     assert out[0][1] == out[1][1] == 12
     assert torch.equal(out[0][0], out[1][0])
+
+
+@pytest.mark.gpu
+def test_a_refused_block_workspace_leaves_no_error_behind():
+    """k = 2e9 basis rows ask for 512 GB of partial sums and are refused before
+    any launch; the call after that succeeds."""
+    import ctypes
+    import torch
+    from cugmres_amd import _lib, solver
+    n, s = 64, 2
+    ctx = solver.Context(64, 0)
+    rng = np.random.default_rng(4)
+    W = torch.as_tensor((rng.standard_normal((s, n)) + 1j * rng.standard_normal((s, n))).astype(np.complex64))
+    w, out = W.to(ctx.device), torch.empty((s, n), dtype=torch.complex64, device=ctx.device)
+    h = torch.zeros(s * s + 1, dtype=torch.complex128, device=ctx.device)
+    print("block workspace refused", flush=True)
+
+    def call(k):
+        p = [ctypes.c_void_p(t.data_ptr()) for t in (w, out, h)]
+        return _lib.lib().cgm_block_orthonormalise(ctx.handle, p[0], k, p[0], p[1], s, n, 1e-12, p[2])
+    assert call(2_000_000_000) == _lib.ERROR_ALLOC
+    assert call(0) == _lib.SUCCESS
+    torch.cuda.synchronize()
+    Q = out.cpu().numpy().astype(complex)
+    assert np.abs(Q.conj() @ Q.T - np.eye(s)).max() < 5e-7
+    ctx.close()
