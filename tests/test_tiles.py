@@ -498,3 +498,33 @@ def test_reduced_tiles_after_a_failed_scratch_allocation():
     ctx.close()
     del many
     torch.cuda.empty_cache()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,T,systems", [(32, 32, 1), (96, 32, 16), (64, 32, 5), (32, 16, 2), (80, 16, 3), (48, 16, 4),
+                                         (64, 16, 9), (96, 16, 17), (64, 8, 2), (40, 8, 5)])
+def test_dense_tiles_system_groups(orc, N, T, systems):
+    """Every number of systems per pass over the dense inverses and a remainder
+    of each, from a single tile on: the first and the last system against the
+    oracle (1e-4, FP32 LU of the tile operators), every system equal bit for bit
+    to its own application at T = 16 and 32."""
+    import torch
+    from cugmres_amd import problems, solver, tiles as gt
+    from oracle import tiles
+    print(f"dense tiles N={N} T={T} systems={systems}", flush=True)
+    ctx = solver.Context(N, 0)
+    ref_blk = orc.baseline_green_block(N, problems.KH)
+    chi, _ = _problem(N, N + systems)
+    tl = gt.Tiles(ctx, T, 1).factor(ctx.block_helmholtz(problems.KH), ctx.to_device(chi, "f32"))
+    rng = np.random.default_rng(systems)
+    V = (rng.standard_normal((systems, N * N)) + 1j * rng.standard_normal((systems, N * N))).astype(np.complex64)
+    dV = torch.as_tensor(V).to(ctx.device)
+    y = tl.apply(dV)
+    K = tiles.tile_inverses(ref_blk, chi, N, T)
+    for k in sorted({0, systems - 1}):
+        assert rel(y[k].cpu().numpy(), tiles.tile_apply(K, V[k].astype(np.complex128), N, T)) < 1e-4
+    for n in range(1, systems + 1) if T > 8 else ():
+        assert torch.equal(tl.apply(dV[:n].contiguous()), y[:n]), n
+        assert torch.equal(tl.apply(dV[n - 1].contiguous()), y[n - 1]), n
+    tl.close()
+    ctx.close()
