@@ -43,3 +43,34 @@ def test_products_on_ragged_grids(N):
         ref = _torch_matvec(torch, blk, chi[0], x[0], N, ctx.M, mode)
         assert rel(y64.cpu().numpy(), ref.cpu().numpy()) < 1e-12, mode
     ctx.close()
+
+
+# one N with a remainder for each embedding that the grids above leave out: M =
+# 192, 512, 1024 (two-wave and one-wave form, radices 8 8 4 4 and 16 8 8) and 2048
+# (16 elements per thread in complex64)
+@pytest.mark.parametrize("N,plan", [(67, 0), (200, 0), (401, 0), (401, 1), (511, 0), (511, 1), (901, 0)])
+def test_products_on_the_other_embeddings(N, plan):
+    """Bounds as above: complex64 to 2e-6, complex128 to 1e-12 of the product by
+    torch.fft, single and batched products equal bit for bit, all modes."""
+    import torch
+    from cugmres_amd import problems, solver
+    print(f"ragged grid N={N} plan={plan}", flush=True)
+    ctx = solver.Context(N, 0)
+    g, g64 = ctx.spectrum_helmholtz(problems.KH, fp64=True)
+    blk = ctx.block_helmholtz(problems.KH)
+    rng = np.random.default_rng(N)
+    B = 3
+    chi = torch.as_tensor(rng.uniform(0.0, 11.1, (B, N * N))).to(ctx.device)
+    x = torch.as_tensor(rng.standard_normal((B, N * N)) + 1j * rng.standard_normal((B, N * N))).to(ctx.device)
+    c32, x32 = chi.to(torch.float32), x.to(torch.complex64)
+    ctx.set_radix_plan(plan)
+    for mode in (0, 1, 2):
+        own = ctx.matvec_batched(g, c32, x32, mode)
+        for k in range(B):
+            ref = _torch_matvec(torch, blk, c32[k].to(torch.float64), x32[k].to(torch.complex128), N, ctx.M, mode)
+            assert rel(own[k].cpu().numpy(), ref.cpu().numpy()) < 2e-6, (mode, k)
+            assert torch.equal(own[k], ctx.matvec(g, c32[k].contiguous(), x32[k].contiguous(), mode)), (mode, k)
+        y64 = ctx.matvec_c128(g64, chi[0].contiguous(), x[0].contiguous(), mode)
+        ref = _torch_matvec(torch, blk, chi[0], x[0], N, ctx.M, mode)
+        assert rel(y64.cpu().numpy(), ref.cpu().numpy()) < 1e-12, mode
+    ctx.close()
