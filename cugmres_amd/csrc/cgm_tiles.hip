@@ -273,38 +273,61 @@ k_tile_scale(FnoIO io, const int* __restrict__ done, long sd, long n) {
   io.vw[(long)s * io.sV + e] = x;
 }
 
-// Tiles of side 16 and 32: blockIdx.x = tile and block of 128 rows, blockIdx.y =
-// group of NV systems.  io.vw must not be io.v (k_tile_scale).
+// Tiles of side 16 and 32: a work-group takes a tile, a block of 128 of its rows
+// and a group of NV systems.  io.vw must not be io.v (k_tile_scale).
 //
 // The stream of K bounds it (8 T^4 bytes per tile; column-major, so rows are
 // independent and a row block needs no sum with another).  A wave reads two
 // rows per lane (1 KB of a column per load) of every eighth group of four
-// columns, kU loads ahead; the waves' sums meet in LDS.  Eight waves on 128 rows,
-// instead of one thread per row through all columns, keep 16 waves per CU on 256
-// tiles of side 16 where there were four, and 64 tiles of side 32 on all CUs.
-// One / four / sixteen systems of one map, us: N = 256, T = 16 (134 MB): 20.7 /
-// 34.3 / 48.9 before, 21.7 / 22.5 / 47 now; N = 512, T = 16 (537 MB): 90.6 / 101 /
-// 387 before, 88 / 95 / 207 now; N = 256, T = 32 (537 MB): 201 / 210 / 202 before,
-// 89 / 95 / 198 now.  Non-temporal loads are slower (the inverses of smaller
-// grids stay in the Infinity Cache): 25.3 / 26.5 / 55 at N = 256, T = 16.
+// columns, kU loads ahead, each register loaded again as soon as it is used and
+// not at all in the last round; the waves' sums meet in LDS.  Eight waves on 128
+// rows, instead of one thread per row through all columns, keep 16 waves per CU
+// on 256 tiles of side 16 where there were four, and 64 tiles of side 32 on all
+// CUs.
+//
+// Work-groups L, L + 8, L + 16.. run on one XCD one after the other: they take the
+// groups of systems of one row block (up to 16 per blockIdx.y, so that its L2
+// serves all but the first), then the tile's other row blocks.  In the order
+// (row block, then tile; groups in blockIdx.y) the second group read K from memory
+// again: N = 256, T = 16, nine systems 45 us, now 33.5; T = 32, sixteen 198, now
+// 126.  `units` are tiles, or pairs (map, tile) of systems with their own maps
+// (NV = 1); fewer than eight would leave XCDs idle, so their row blocks are dealt
+// out over the XCDs instead (T = 32, four tiles, one system: 14.0 us on four XCDs,
+// 12.2 on eight).
+//
+// NTL: inverses beyond the 256 MB of Infinity Cache that are read once, without
+// a place in the caches (N = 512, T = 16, one system: 91 -> 79 us; N = 384, 302 MB:
+// 45.9 -> 44.7; N = 352, 254 MB, is faster with: 36.4 against 37.7).
+//
+// One / four / sixteen systems of one map, us, against one thread per row: N = 256,
+// T = 16 (134 MB): 20.4 / 30.6 / 43.0, here 20.1 / 21.7 / 32.6; N = 512, T = 16 (537
+// MB): 91 / 102 / 388, here 79 / 85 / 146; N = 256, T = 32 (537 MB): 201 / 209 / 190,
+// here 78 / 81 / 126.  At N = 320, T = 16 (800 work-groups, 3.1 per CU) one system is
+// 1.5 us behind it (29.9, here 31.4).  kU = 16 and 4 for up to four systems: 20.5 and
+// 20.4 at N = 256, T = 16, 31.5 and 32.4 at N = 320.
 constexpr int kTileWaves = 8;
-template <int M2, int NV>
+template <int M2, int NV, bool NTL>
 __global__ void __launch_bounds__(64 * kTileWaves)
 k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restrict__ done, long sd, int N, int T,
-             int nsys) {
+             int nsys, int units, int ngroups) {
   constexpr int kWaves = kTileWaves;
   constexpr int RB = 128, kBlocks = M2 / RB;
-  constexpr int kUnit = 4;             // loads of one turn of a wave
-  constexpr int kU = NV > 4 ? 4 : 8;   // loads ahead: one turn or two
-  static_assert(M2 % (2 * kUnit * kWaves) == 0, "whole rounds of loads");
+  constexpr int kUnit = 4;  // loads of one turn of a wave
+  constexpr int kU = 8;     // loads ahead: two turns
+  static_assert(M2 % (kU * kWaves) == 0, "whole rounds of loads");
   constexpr size_t kXsLen = sizeof(float2) * M2 * NV, kRedLen = sizeof(float4) * (kWaves / 2) * NV * 64;
   __shared__ __align__(16) unsigned char smem[kXsLen > kRedLen ? kXsLen : kRedLen];  // the inputs, then the waves' sums
   float2(*xs)[NV] = reinterpret_cast<float2(*)[NV]>(smem);
   float4(*red)[NV][64] = reinterpret_cast<float4(*)[NV][64]>(smem);
   const int nt = N / T;
-  const int t = blockIdx.x / kBlocks, rb = blockIdx.x % kBlocks;
+  const int xcd = blockIdx.x & 7, step = blockIdx.x >> 3;
+  const int row = NV > 1 ? step / ngroups : step;  // row blocks before this one on the XCD
+  const int u = units < 8 ? (row * 8 + xcd) / kBlocks : row / kBlocks * 8 + xcd;
+  const int rb = (units < 8 ? row * 8 + xcd : row) % kBlocks;
+  const int t = NV > 1 ? u : u % (nt * nt);
+  const int s0 = NV > 1 ? (blockIdx.y * ngroups + step % ngroups) * NV : u / (nt * nt);
+  if (u >= units || s0 >= nsys) return;
   const int a = t / nt, b = t % nt;
-  const int s0 = blockIdx.y * NV;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   bool live[NV];
   bool any = false;
@@ -317,7 +340,11 @@ k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restr
   if (!any) return;  // uniform over the work-group
   const float4* Kt = reinterpret_cast<const float4*>(K + (long)(NV == 1 ? s0 : 0) * sK + (long)t * M2 * M2 + rb * RB) + lane;
   typedef float f4v __attribute__((ext_vector_type(4)));
-  const auto load = [&](int q) { return *reinterpret_cast<const f4v*>(Kt + (long)q * (M2 / 2)); };  // rows 2 lane, + 1
+  const auto load = [&](int q) {  // rows 2 lane, + 1
+    const f4v* p = reinterpret_cast<const f4v*>(Kt + (long)q * (M2 / 2));
+    if constexpr (NTL) return __builtin_nontemporal_load(p);
+    else return *p;
+  };
   f4v k[kU];
   // load u of a round: the wave's turns come in the same order for every NV, so
   // a system's sums do not depend on the others
@@ -352,27 +379,28 @@ k_tile_apply(const float2* __restrict__ K, long sK, FnoIO io, const int* __restr
   float4 acc[NV];  // the two rows
 #pragma unroll
   for (int v = 0; v < NV; ++v) acc[v] = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int q = 0; q < M2; q += kStep) {
-    f4v c[kU];
+  const auto add_column = [&](int q, f4v c) {
 #pragma unroll
-    for (int u = 0; u < kU; ++u) c[u] = k[u];
-    const int qn = q + kStep < M2 ? q + kStep : q;
-#pragma unroll
-    for (int u = 0; u < kU; ++u) k[u] = load(qn + col(u));
-    __builtin_amdgcn_sched_barrier(0);
+    for (int v = 0; v < NV; ++v) {
+      const float2 xv = xs[q][v];
+      // two fused multiply-adds each (a product of its own and an addition otherwise)
+      acc[v].x = fmaf(-c[1], xv.y, fmaf(c[0], xv.x, acc[v].x));
+      acc[v].y = fmaf(c[1], xv.x, fmaf(c[0], xv.y, acc[v].y));
+      acc[v].z = fmaf(-c[3], xv.y, fmaf(c[2], xv.x, acc[v].z));
+      acc[v].w = fmaf(c[3], xv.x, fmaf(c[2], xv.y, acc[v].w));
+    }
+  };
+  int q = 0;
+#pragma unroll 1
+  for (; q < M2 - kStep; q += kStep)
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        const float2 xv = xs[q + col(u)][v];
-        // two fused multiply-adds each (a product of its own and an addition otherwise)
-        acc[v].x = fmaf(-c[u][1], xv.y, fmaf(c[u][0], xv.x, acc[v].x));
-        acc[v].y = fmaf(c[u][1], xv.x, fmaf(c[u][0], xv.y, acc[v].y));
-        acc[v].z = fmaf(-c[u][3], xv.y, fmaf(c[u][2], xv.x, acc[v].z));
-        acc[v].w = fmaf(c[u][3], xv.x, fmaf(c[u][2], xv.y, acc[v].w));
-      }
+      add_column(q + col(u), k[u]);
+      k[u] = load(q + kStep + col(u));
+      if (u % 2) __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of their use
     }
-  }
+#pragma unroll
+  for (int u = 0; u < kU; ++u) add_column(q + col(u), k[u]);
   // sums of the eight waves: the upper four to the lower four, then those four
   const auto add = [](float4& o, const float4& p) {
     o.x += p.x;
@@ -432,9 +460,14 @@ int launch_apply_m(const cgm_tiles* tl, hipStream_t st, const FnoIO& io, const i
       in.nrm = nullptr;
       in.vw = nullptr;
     }
-#define CGM_DENSE(NV, S)                                                                                              \
-  hipLaunchKernelGGL((k_tile_apply<M2, NV>), dim3(ntiles * (M2 / 128), groups), dim3(64 * kTileWaves), 0, st, tl->K, S, \
-                     in, done, sd, tl->N, tl->T, nsys)
+    // every entry read once, and more of them than the Infinity Cache holds
+    const size_t bytes = sizeof(float2) * sK * (tl->maps == 1 ? 1 : nsys);
+    const bool ntl = (tl->maps > 1 || groups == 1) && bytes > (size_t)256 << 20;
+    const int units = nv > 1 ? ntiles : ntiles * groups, ng = nv > 1 ? std::min(groups, 16) : 1;
+    const dim3 grid((units + 7) / 8 * 8 * (M2 / 128) * ng, nv > 1 ? (groups + ng - 1) / ng : 1);
+#define CGM_DENSE(NV, S)                                                                                             \
+  hipLaunchKernelGGL((ntl ? k_tile_apply<M2, NV, true> : k_tile_apply<M2, NV, false>), grid, dim3(64 * kTileWaves), 0, \
+                     st, tl->K, S, in, done, sd, tl->N, tl->T, nsys, units, ng)
     switch (nv) {
       case 8: CGM_DENSE(8, 0L); break;
       case 4: CGM_DENSE(4, 0L); break;

@@ -528,3 +528,50 @@ def test_dense_tiles_system_groups(orc, N, T, systems):
         assert torch.equal(tl.apply(dV[n - 1].contiguous()), y[n - 1]), n
     tl.close()
     ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,T,systems", [(192, 32, 9), (32, 16, 133)])
+def test_dense_tiles_routes_round_alike(N, T, systems):
+    """302 MB of inverses are read past the caches by one group of systems and
+    through them by two; 17 groups are more than a row block's XCD takes in one
+    go.  Every system equals its own application bit for bit."""
+    import torch
+    from cugmres_amd import problems, solver, tiles as gt
+    print(f"dense tiles routes N={N} T={T} systems={systems}", flush=True)
+    ctx = solver.Context(N, 0)
+    chi, _ = _problem(N, 8)
+    tl = gt.Tiles(ctx, T, 1).factor(ctx.block_helmholtz(problems.KH), ctx.to_device(chi, "f32"))
+    rng = np.random.default_rng(systems)
+    V = (rng.standard_normal((systems, N * N)) + 1j * rng.standard_normal((systems, N * N))).astype(np.complex64)
+    dV = torch.as_tensor(V).to(ctx.device)
+    y = tl.apply(dV)
+    for k in range(systems):
+        assert torch.equal(tl.apply(dV[k].contiguous()), y[k]), k
+    assert torch.equal(tl.apply(dV[:8].contiguous()), y[:8])
+    tl.close()
+    ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,T,maps", [(32, 32, 3), (64, 32, 3), (48, 16, 2), (16, 16, 5)])
+def test_dense_tiles_of_several_maps_equal_one_map_each(N, T, maps):
+    """Pairs (map, tile) from three on, fewer and more than the XCDs: every system
+    equals the application of its map's inverses alone, bit for bit."""
+    import torch
+    from cugmres_amd import problems, solver, tiles as gt
+    print(f"dense tiles own maps N={N} T={T} maps={maps}", flush=True)
+    ctx = solver.Context(N, 0)
+    blk = ctx.block_helmholtz(problems.KH)
+    chis = torch.stack([ctx.to_device(_problem(N, 70 + k)[0], "f32") for k in range(maps)])
+    rng = np.random.default_rng(maps)
+    V = (rng.standard_normal((maps, N * N)) + 1j * rng.standard_normal((maps, N * N))).astype(np.complex64)
+    dV = torch.as_tensor(V).to(ctx.device)
+    tl = gt.Tiles(ctx, T, maps).factor(blk, chis)
+    y = tl.apply(dV)
+    for k in range(maps):
+        one = gt.Tiles(ctx, T, 1).factor(blk, chis[k])
+        assert torch.equal(one.apply(dV[k].contiguous()), y[k]), k
+        one.close()
+    tl.close()
+    ctx.close()
