@@ -57,7 +57,7 @@
 
 using namespace cgm;
 
-// One work-group's share of a tile's W (k_tile_ws): block columns j0, j0 + 1
+// One work-group's share of a tile's W (k_tile_ws): block column j0 (and j0 + 1)
 // and the block rows from i0 on.
 struct Strip {
   long woff;   // the tile's first block in W16
@@ -65,6 +65,9 @@ struct Strip {
   int nB;      // block rows of the tile
   int i0, j0;
 };
+// Strips of two block columns and several rows, of two columns and one row, of
+// one column and one row.
+enum StripKind { kLongStrip, kRowStrip, kBlockStrip };
 
 struct cgm_tiles {
   cgm_context* ctx = nullptr;
@@ -94,12 +97,13 @@ struct cgm_tiles {
   size_t stab_cap = 0, spos_cap = 0;
   int* sstart = nullptr;           // [B] first entry of each map's list in stab
   int* scount = nullptr;           // [B] strips of each map
-  int* ssize = nullptr;            // [B] block rows of a map's strips
+  int* ssize = nullptr;            // [B] block rows of a map's strips and, << 8, their block columns
   int scount_max = 0;              // largest strip count over the factored maps
-  long plen_max = 0;               // largest scount * (2 + ssize)
+  unsigned kinds = 0;              // which StripKinds the maps have (bits)
+  long plen_max = 0;               // largest scount * (columns + rows of a strip)
   int xblk_max = 0;                // largest number of block rows of a map
   int nbmax = 0;                   // largest number of block rows of a tile
-  float4* Pw = nullptr;            // [group][strip][2 + ssize][64 systems of the group] partial products (apply)
+  float4* Pw = nullptr;            // [group][strip][columns, rows][64 systems of the group] partial products (apply)
   size_t pw_cap = 0;
   unsigned* Xs = nullptr;          // [group][xblk_max][kXsBlk] inputs in FP16 parts (apply)
   size_t xs_cap = 0;
@@ -910,11 +914,11 @@ k_tile_xs(const int* __restrict__ ncol, const unsigned short* __restrict__ cols,
 // The products with W_t of up to VP = 8 NT systems of one map.  W_t is complex
 // symmetric (W_t = (D_S^{-1} - G_SS)^{-1}, G symmetric), so only its lower
 // triangle is stored, in kBlkW x kBlkW blocks.  A work-group takes a strip of
-// them: block columns j0 = 2 sj and j0 + 1 of its tile, block rows i of
-// [si R, si R + R) with i >= j0 (R = 2, 4 or 8, by map), and forms for every
-// block (i, j) B x_j (added up over the two columns, per row) and, for j < i,
-// B^T x_i (added up over the rows, per column): 2 + R partial products of kBlkW
-// values per system, which k_tile_wsum adds up.
+// them: block columns j0 = 2 sj and j0 + 1 of its tile (SC = 1: column j0 = sj
+// alone), block rows i of [si R, si R + R) with i >= j0 (R = 1, 2, 4 or 8, by
+// map), and forms for every block (i, j) B x_j (added up over the columns, per row)
+// and, for j < i, B^T x_i (added up over the rows, per column): SC + R partial
+// products of kBlkW values per system, which k_tile_wsum adds up.
 //
 // What bounds it is the stream of W (64 KB a block), which is read once.  The
 // contraction runs on the matrix cores (FP16 inputs, FP32 sums): W is FP16 as
@@ -941,6 +945,12 @@ k_tile_xs(const int* __restrict__ ncol, const unsigned short* __restrict__ cols,
 // unconditionally (the last block again where there is no next), so that the
 // compiler's waits know how many loads are younger than the ones waited for.
 //
+// KIND: strips of one row need no second set of x_i, and their last block is known
+// when compiled, so nothing is loaded in vain: three work-groups per CU instead of
+// two cover each other's first loads and last sums (sixteen maps at N = 128, T =
+// 64: 114 us with strips of two blocks, two per CU; 96 with three; 94.6 with
+// single blocks).
+//
 // At N = 512, T = 128 on a map of the benchmark (1.33 GB of W; a plain
 // non-temporal read of as much takes 190 us): one system 229-236 us (5.7 TB/s),
 // 16 systems 337 us.  The vector-ALU kernel before it, which took one block
@@ -948,25 +958,28 @@ k_tile_xs(const int* __restrict__ ncol, const unsigned short* __restrict__ cols,
 // system).  One FP16 part instead of three would save 19 us at one system.
 // Two groups of 4 waves with 8 K-steps in flight took 249 us; R = 4 and 16
 // (rows per strip) instead of 8 took 252 and 241 us.
-template <int NT>
-__global__ void __launch_bounds__(256, 2)
+template <int NT, int KIND>
+__global__ void __launch_bounds__(256, KIND != kLongStrip && NT == 1 ? 3 : 2)
 k_tile_ws(const unsigned* __restrict__ W16, const Strip* __restrict__ stab, const int* __restrict__ sstart,
           const int* __restrict__ scount, const int* __restrict__ ssize, int maps1, int nsys,
           const unsigned* __restrict__ Xs, long sXs, float4_t* __restrict__ Pw, long spw,
           const int* __restrict__ done, long sd) {
   constexpr int B = kBlkW, VP = 8 * NT, KS = B / 16;
+  constexpr int SC = KIND == kBlockStrip ? 1 : 2;
+  constexpr bool ONE = KIND != kLongStrip;          // one block row
   constexpr int D = NT == 1 ? 4 : 2;                // K-steps of W in flight (2 KB per wave each)
   constexpr int kSlot = kSplits * 16 * kXsRow;      // dwords of one block row's inputs in LDS
-  __shared__ unsigned lds[2 * kSlot];
+  static_assert(SC * kSlot * sizeof(unsigned) >= 3 * KS * 64 * sizeof(float4_t), "the waves' sums fit the inputs' LDS");
+  __shared__ unsigned lds[SC * kSlot];
   const int grp = blockIdx.y, map = maps1 ? 0 : grp;
-  if ((int)blockIdx.x >= scount[map]) return;
+  const int size = ssize[map], R = ONE ? 1 : size & 255;
+  if ((int)blockIdx.x >= scount[map] || size >> 8 != SC) return;
   const int nv = maps1 ? (nsys - grp * VP < VP ? nsys - grp * VP : VP) : 1;
   if (done) {  // uniform over the work-group
     bool all = true;
     for (int k = 0; k < nv; ++k) all &= *boff(done, (long)((maps1 ? grp * VP : grp) + k) * sd) != 0;
     if (all) return;
   }
-  const int R = ssize[map];
   const Strip sp = stab[sstart[map] + blockIdx.x];
   const int nB = sp.nB, j0 = sp.j0, i0 = sp.i0, iend = i0 + R < nB ? i0 + R : nB;
   const int ibeg = i0 > j0 ? i0 : j0;
@@ -1001,7 +1014,7 @@ k_tile_ws(const unsigned* __restrict__ W16, const Strip* __restrict__ stab, cons
 
   {  // x_j of the two columns, the columns in use, into LDS
     const unsigned* src = X + (long)j0 * kXsBlk;
-    const int per = ncols * (B / 4), all = (j0 + 1 < nB ? 2 : 1) * kSplits * per;
+    const int per = ncols * (B / 4), all = (SC == 2 && j0 + 1 < nB ? 2 : 1) * kSplits * per;
     for (int e0 = tid; e0 < all; e0 += 4 * 256) {
       uint4_t v[4];
 #pragma unroll
@@ -1027,17 +1040,17 @@ k_tile_ws(const unsigned* __restrict__ W16, const Strip* __restrict__ stab, cons
     Iim[2 * c + 1] = one;
   }
   const float4_t zero = {0.f, 0.f, 0.f, 0.f};
-  float4_t Z[2][KS][NT];
+  float4_t Z[SC][KS][NT];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < SC; ++h)
 #pragma unroll
     for (int k = 0; k < KS; ++k)
 #pragma unroll
       for (int n = 0; n < NT; ++n) Z[h][k][n] = zero;
 
-  // partial products: [strip][2 columns, R rows][positions / 4][system][re, im] float4
+  // partial products: [strip][SC columns, R rows][positions / 4][system][re, im] float4
   const long qlen = 64 * nv;
-  float4_t* P = Pw + (long)grp * spw + (long)blockIdx.x * (2 + R) * qlen;
+  float4_t* P = Pw + (long)grp * spw + (long)blockIdx.x * (SC + R) * qlen;
   const auto put_p = [&](float4_t* Pq, int k, const float4_t* acc) {  // positions 16 k + 4 g .. + 3
     float4_t* q = Pq + (k * 4 + g) * 2 * nv;
     if constexpr (NT == 2) {
@@ -1060,9 +1073,10 @@ k_tile_ws(const unsigned* __restrict__ W16, const Strip* __restrict__ stab, cons
     }
   };
   float4_t Y[2 * NT];
-  // block (i, j): its row sums to Y, with `columns` its column sums to Zj (not on the diagonal, where the block is whole and its row
-  // sums are all), and the loads of block (ni, nj)
-  const auto product = [&](auto columns, int i, int j, int ni, int nj, const unsigned* xj, float4_t (&Zj)[KS][NT]) {
+  // block (i, j): its row sums to Y, with `columns` its column sums to Zj (not on the diagonal, where the block is
+  // whole and its row sums are all), and the loads of block (ni, nj), unless it is the `last`
+  const auto product = [&](auto columns, auto last, int i, int j, int ni, int nj, const unsigned* xj,
+                           float4_t (&Zj)[KS][NT]) {
     int xoff = a * kXsRow + 4 * g;
     asm volatile("" : "+v"(xoff));  // x_j is read from LDS for every block: 96 registers otherwise
     unsigned keep = i != j ? 0xFFFFFFFFu : 0u;
@@ -1076,7 +1090,7 @@ k_tile_ws(const unsigned* __restrict__ W16, const Strip* __restrict__ stab, cons
         f[1] = __builtin_bit_cast(half8_t, (uint4_t{Ak[0].y, Ak[1].y, Ak[2].y, Ak[3].y}));
       }
       if (k + D < KS) load_a(i, j, k + D);
-      else load_a(ni, nj, k + D - KS);
+      else if constexpr (!decltype(last)::value) load_a(ni, nj, k + D - KS);
 #pragma unroll
       for (int q = 0; q < kSplits; ++q) {
         const uint4_t v = *reinterpret_cast<const uint4_t*>(xj + xoff + q * 16 * kXsRow + 16 * k);
@@ -1101,39 +1115,51 @@ k_tile_ws(const unsigned* __restrict__ W16, const Strip* __restrict__ stab, cons
   };
   const auto store_y = [&](int i) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) put_p(P + (2 + i - i0) * qlen, 2 * w + h, Y + h * NT);
+    for (int h = 0; h < 2; ++h) put_p(P + (SC + i - i0) * qlen, 2 * w + h, Y + h * NT);
   };
   __syncthreads();
+  typedef std::true_type yes;
+  typedef std::false_type no;
   int i = ibeg;
   if (i == j0) {
 #pragma unroll
     for (int k = 0; k < 2 * NT; ++k) Y[k] = zero;
     const bool more = i + 1 < iend;
-    product(std::false_type(), i, j0, more ? i + 1 : i, j0, lds, Z[0]);
+    product(no(), std::integral_constant<bool, ONE>(), i, j0, more ? i + 1 : i, j0, lds, Z[0]);
     store_y(i);
     ++i;
   }
-  for (; i < iend; ++i) {
-    const bool more = i + 1 < iend;
+  if constexpr (ONE) {
+    if (i < iend) {
 #pragma unroll
-    for (int k = 0; k < 2 * NT; ++k) Y[k] = zero;
-    product(std::true_type(), i, j0, i, j0 + 1, lds, Z[0]);
-    if constexpr (NT == 1) load_x(more ? i + 1 : i, xn);
-    product(std::true_type(), i, j0 + 1, more ? i + 1 : i, more ? j0 : j0 + 1, lds + kSlot, Z[1]);
-    store_y(i);
-    if constexpr (NT == 1) {
+      for (int k = 0; k < 2 * NT; ++k) Y[k] = zero;
+      product(yes(), std::integral_constant<bool, SC == 1>(), i, j0, i, j0 + 1, lds, Z[0]);
+      if constexpr (SC == 2) product(yes(), yes(), i, j0 + 1, i, j0 + 1, lds + kSlot, Z[SC - 1]);
+      store_y(i);
+    }
+  } else {
+    for (; i < iend; ++i) {
+      const bool more = i + 1 < iend;
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int k = 0; k < 2 * NT; ++k) Y[k] = zero;
+      product(yes(), no(), i, j0, i, j0 + 1, lds, Z[0]);
+      if constexpr (NT == 1) load_x(more ? i + 1 : i, xn);
+      product(yes(), no(), i, j0 + 1, more ? i + 1 : i, more ? j0 : j0 + 1, lds + kSlot, Z[SC - 1]);
+      store_y(i);
+      if constexpr (NT == 1) {
 #pragma unroll
-        for (int q = 0; q < kSplits; ++q) xr[h][q] = xn[h][q];
-    } else {
-      load_x(more ? i + 1 : i, xr);
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int q = 0; q < kSplits; ++q) xr[h][q] = xn[h][q];
+      } else {
+        load_x(more ? i + 1 : i, xr);
+      }
     }
   }
   // Z over the four waves: wave w keeps positions 32 w .. 32 w + 31
   float4_t* red = reinterpret_cast<float4_t*>(lds);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < SC; ++h) {
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       __syncthreads();
@@ -1174,7 +1200,7 @@ k_tile_wsum(const float* __restrict__ ksc, const float* __restrict__ xinv, const
   const long tb = (long)map * nt * nt + t;
   const int n = ncol[tb], nB = (n + B - 1) / B;
   if (i >= nB) return;
-  const int R = ssize[map], si = i / R, sj = i >> 1;
+  const int R = ssize[map] & 255, SC = ssize[map] >> 8, si = i / R, sj = SC == 2 ? i >> 1 : i;
   const int nS = (nB + R - 1) / R;
   const int e = threadIdx.x & 63, sl = threadIdx.x >> 6;
   const long qlen = 64 * nv;
@@ -1186,7 +1212,7 @@ k_tile_wsum(const float* __restrict__ ksc, const float* __restrict__ xinv, const
 #pragma unroll 4
   for (int k = sl; k < terms; k += 4) {
     const int r = k <= sj ? si : si + k - sj - 1, c = k <= sj ? k : sj;
-    acc += P[((long)pos[r * 64 + c] * (2 + R) + (k <= sj ? 2 + i - si * R : (i & 1))) * qlen];
+    acc += P[((long)pos[r * 64 + c] * (SC + R) + (k <= sj ? SC + i - si * R : i & (SC - 1))) * qlen];
   }
   red[sl][e] = acc;
   __syncthreads();
@@ -1332,8 +1358,17 @@ int launch_ws(const cgm_tiles* tl, hipStream_t st, const FnoIO& io, const int* d
   hipLaunchKernelGGL((k_tile_xs<T, VP>), dim3(ntiles * parts, nsys), dim3(1024), 0, st, tl->ncol, tl->cols, tl->bloc, m1, parts, io,
                      tl->Xs, sxs, tl->xinv, done, sd, tl->N);
   if (ev) CGM_HIP(hipEventRecord(ev[0], st));
-  hipLaunchKernelGGL((k_tile_ws<NT>), dim3(tl->scount_max, groups), dim3(256), 0, st,
-                     reinterpret_cast<const unsigned*>(tl->W16), tl->stab, tl->sstart, tl->scount, tl->ssize, m1, nsys, tl->Xs, sxs, Pw, spw, done, sd);
+  const auto ws = [&](auto kind) {
+    hipLaunchKernelGGL((k_tile_ws<NT, decltype(kind)::value>), dim3(tl->scount_max, groups), dim3(256), 0, st,
+                       reinterpret_cast<const unsigned*>(tl->W16), tl->stab, tl->sstart, tl->scount, tl->ssize, m1,
+                       nsys, tl->Xs, sxs, Pw, spw, done, sd);
+  };
+  // single rows have a launch of their own only where no map has longer strips
+  // (a second launch costs more than it gives: three maps at N = 192, T = 64,
+  // 68 us with it and 63.7 without)
+  if (tl->kinds & 1u << kLongStrip) ws(std::integral_constant<int, kLongStrip>());
+  else if (tl->kinds & 1u << kRowStrip) ws(std::integral_constant<int, kRowStrip>());
+  if (tl->kinds & 1u << kBlockStrip) ws(std::integral_constant<int, kBlockStrip>());
   if (ev) CGM_HIP(hipEventRecord(ev[1], st));
   hipLaunchKernelGGL((k_tile_wsum<T, VP>), dim3(ntiles * tl->nbmax, per, groups), dim3(256), 0, st, tl->kscale,
                      tl->xinv, tl->ncol, tl->cols, tl->sloc, tl->spos, tl->ssize, m1, nsys, tl->nbmax, Pw, spw, tl->U,
@@ -1402,12 +1437,29 @@ int layout_reduced(cgm_tiles* t, const std::vector<int>& nc, int maps) {
   t->kept.assign(maps, 0.0);
   t->nbmax = t->scount_max = t->xblk_max = 0;
   t->plen_max = 0;
+  t->kinds = 0;
   t->maps1 = maps == 1;
+  const auto blocks = [&](int m, int tl) { return (nc[m * ntiles + tl] + kBlkW - 1) / kBlkW; };
+  struct Item { int work, tile, i, j; };
+  // map m in strips of R block rows and C block columns
+  const auto strips = [&](int m, int R, int C) {
+    std::vector<Item> items;
+    for (int tl = 0; tl < ntiles; ++tl) {
+      const int nB = blocks(m, tl);
+      for (int i = 0; i * R < nB; ++i)
+        for (int j = 0; C * j < std::min(nB, i * R + R); ++j) {
+          int work = 0;
+          for (int r = i * R; r < std::min(nB, i * R + R); ++r) work += std::max(0, std::min(C, r - C * j + 1));
+          items.push_back({work, tl, i, j});
+        }
+    }
+    return items;
+  };
   for (int m = 0; m < maps; ++m) {
     int rows = 0;
     for (int tl = 0; tl < ntiles; ++tl) {
       const int k = m * ntiles + tl;
-      const int nB = (nc[k] + kBlkW - 1) / kBlkW;
+      const int nB = blocks(m, tl);
       const int nblk = nB * (nB + 1) / 2;
       off[k] = total;
       total += nblk * BB;
@@ -1416,45 +1468,36 @@ int layout_reduced(cgm_tiles* t, const std::vector<int>& nc, int maps) {
       rows += nB;
       t->nbmax = std::max(t->nbmax, nB);
     }
-    struct Item { int work, tile, i, j; };
-    std::vector<Item> items;
     // long strips move fewer partial products and short ones keep more
-    // work-groups busy: the longest of which each CU gets four or more, and
-    // single rows only where two leave CUs idle (four 64 x 64 tiles, 84
-    // strips of two rows: 36.4 us with two, 33.4 with one; 16 tiles, 336
-    // strips: 52.1 and 54.5)
-    int R = 8;
-    for (;; R /= 2) {
-      items.clear();
-      for (int tl = 0; tl < ntiles; ++tl) {
-        const int nB = (nc[m * ntiles + tl] + kBlkW - 1) / kBlkW;
-        for (int i = 0; i * R < nB; ++i)
-          for (int j = 0; 2 * j < std::min(nB, i * R + R); ++j) {
-            int work = 0;
-            for (int r = i * R; r < std::min(nB, i * R + R); ++r) work += std::max(0, std::min(2, r - 2 * j + 1));
-            items.push_back({work, tl, i, j});
-          }
-      }
-      if (R == 1 || items.size() >= (R == 2 ? 256 : 1024)) break;
-    }
+    // work-groups busy: the longest of which each CU gets four or more; single
+    // rows where two leave CUs idle (16 tiles of side 64, 336 strips of two: 52.1 us,
+    // of one 54.5), and single blocks where those do (four tiles, 168 strips of
+    // one row, sixteen systems: 43.2 us, single blocks 40.6; one tile, nine systems:
+    // 33.2 and 28.7).  The map alone decides, so that its rounding does not depend
+    // on the others.
+    int R = 8, C = 2;
+    std::vector<Item> items = strips(m, R, C);
+    while (R > 1 && items.size() < (R == 2 ? 256 : 1024)) items = strips(m, R /= 2, C);
+    if (R == 1 && items.size() < 256) items = strips(m, R, C = 1);
+    ssize[m] = R | C << 8;
+    if (!items.empty()) t->kinds |= 1u << (R > 1 ? kLongStrip : C == 2 ? kRowStrip : kBlockStrip);
     const int spos0 = (int)spos.size();
     int slots = 0;
     for (int tl = 0; tl < ntiles; ++tl) {
       sloc[m * ntiles + tl] = spos0 + slots;
-      slots += ((nc[m * ntiles + tl] + kBlkW - 1) / kBlkW + R - 1) / R * 64;
+      slots += (blocks(m, tl) + R - 1) / R * 64;
     }
     spos.resize(spos0 + slots);
     std::stable_sort(items.begin(), items.end(), [](const Item& x, const Item& y) { return x.work > y.work; });
     sstart[m] = (int)stab.size();
     for (size_t k = 0; k < items.size(); ++k) {
-      spos[sloc[m * ntiles + items[k].tile] + items[k].i * 64 + items[k].j] = (int)k;
       const int q = m * ntiles + items[k].tile;
-      stab.push_back({off[q], bloc[q], (nc[q] + kBlkW - 1) / kBlkW, items[k].i * R, items[k].j * 2});
+      spos[sloc[q] + items[k].i * 64 + items[k].j] = (int)k;
+      stab.push_back({off[q], bloc[q], blocks(m, items[k].tile), items[k].i * R, items[k].j * C});
     }
     scount[m] = (int)items.size();
-    ssize[m] = R;
     t->scount_max = std::max(t->scount_max, scount[m]);
-    t->plen_max = std::max(t->plen_max, (long)scount[m] * (2 + R));
+    t->plen_max = std::max(t->plen_max, (long)scount[m] * (C + R));
     t->xblk_max = std::max(t->xblk_max, rows);
   }
   int rc;

@@ -575,3 +575,59 @@ def test_dense_tiles_of_several_maps_equal_one_map_each(N, T, maps):
         one.close()
     tl.close()
     ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,systems", [(64, 1), (64, 8), (64, 17), (128, 9), (128, 16)])
+def test_reduced_tiles_in_single_blocks(orc, N, systems):
+    """One and four 64 x 64 tiles of the benchmark's map (42 and 168 strips of one
+    block row, fewer than CUs) take W block by block, in groups of 8 and 16 systems
+    and their remainders: the first and the last system against the oracle's
+    reduced form (1e-2, FP16 W), every system equal to its own application."""
+    import torch
+    from cugmres_amd import problems, solver, tiles as gt
+    from oracle import tiles
+    T = 64
+    print(f"tiles single blocks N={N} systems={systems}", flush=True)
+    ctx = solver.Context(N, 0)
+    ref_blk = orc.baseline_green_block(N, problems.KH)
+    chi, _ = _problem(N, 21)
+    tl = gt.Tiles(ctx, T, 1).factor(ctx.block_helmholtz(problems.KH), ctx.to_device(chi, "f32"))
+    rng = np.random.default_rng(systems)
+    V = (rng.standard_normal((systems, N * N)) + 1j * rng.standard_normal((systems, N * N))).astype(np.complex64)
+    dV = torch.as_tensor(V).to(ctx.device)
+    y = tl.apply(dV)
+    R = tiles.tile_reduced(ref_blk, chi, N, T)
+    for k in range(systems):
+        if k in (0, systems - 1):
+            assert rel(y[k].cpu().numpy(), tiles.tile_apply_reduced(R, ref_blk, V[k].astype(np.complex128), N, T)) < 1e-2
+        assert torch.equal(tl.apply(dV[k].contiguous()), y[k]), k
+    tl.close()
+    ctx.close()
+
+
+@pytest.mark.gpu
+def test_reduced_tiles_of_maps_with_different_strips():
+    """Four maps at N = 128, T = 64 whose W are taken in strips of several rows (chi
+    != 0 everywhere), of one row (315 strips), in single blocks, and not at all
+    (chi = 0): together and alone each gives the same bits."""
+    import torch
+    from cugmres_amd import problems, solver, tiles as gt
+    N, T = 128, 64
+    print("tiles of maps with different strips", flush=True)
+    ctx = solver.Context(N, 0)
+    blk = ctx.block_helmholtz(problems.KH)
+    rng = np.random.default_rng(6)
+    maps = [rng.uniform(0.1, 0.5, N * N), _sparse_pattern_map(N, 2), _problem(N, 9)[0], np.zeros(N * N)]
+    V = (rng.standard_normal((4, N * N)) + 1j * rng.standard_normal((4, N * N))).astype(np.complex64)
+    dV = torch.as_tensor(V).to(ctx.device)
+    for order in ((0, 1, 2, 3), (3, 1, 2), (2, 1)):
+        chis = torch.stack([ctx.to_device(maps[k], "f32") for k in order])
+        tl = gt.Tiles(ctx, T, len(order)).factor(blk, chis)
+        y = tl.apply(dV[list(order)].contiguous())
+        for j, k in enumerate(order):
+            one = gt.Tiles(ctx, T, 1).factor(blk, chis[j])
+            assert torch.equal(one.apply(dV[k].contiguous()), y[j]), (order, k)
+            one.close()
+        tl.close()
+    ctx.close()
