@@ -18,9 +18,10 @@
 //
 // The passes hold their transforms in registers and cross threads through LDS
 // between stages only (cgm_fft.h): S stages take S - 1 exchanges, where transforms
-// kept in LDS took S + 1.  N = 301, two vectors: 33.4 -> 24.1 us; N = 512, 16
-// vectors: 124 -> 107 us (20 + 58 + 25; pass 2 is bound by its vector
-// arithmetic, about 40 us at full issue, passes 1 and 3 by memory).
+// kept in LDS took S + 1.  N = 301, two vectors: 33.4 -> 23.0 us; N = 512, one
+// vector: 25 -> 20.6 us (replays of a graph; 5.0 + 7.9 + 5.2 in the passes alone),
+// 16 vectors: 124 -> 105 us (20 + 50 + 26; pass 2 is bound by its vector arithmetic, 35
+// us at full issue, passes 1 and 3 by memory).
 #include <math.h>
 #include <string.h>
 
@@ -37,10 +38,11 @@ namespace cgm {
 // rows/columns per work-group); double kernels keep the tighter bound that
 // avoids register spills of the FP64 transforms.
 // Elements per thread of the pass kernels: 16 saves one of four stages at 2048
-// and 4096 points in single precision (N = 1024, four vectors: 128 against 157
-// us); at 128-512 points the fewer waves cost more (N = 128, one vector: 15.1
-// against 11.0 us), and so do the registers of 16 double elements (N = 1024:
-// 90.6 against 82.7 us) and of 24 elements at 3 * 2^k (N = 384: 50.8 against 38.3 us).
+// and 4096 points in single precision (N = 1024, four vectors: 133.6 against 149.1
+// us); at 128-512 points the fewer waves cost more (N = 128, one vector: 13.3
+// against 10.0 us), and so do the registers of 16 double elements (N = 1024:
+// 88.8 against 83.2 us) and of 24 elements at 3 * 2^k (N = 384, four vectors: 48.0
+// against 40.0 us).
 template <typename T, int M> constexpr int kPassE = sizeof(T) == 4 && (M == 2048 || M == 4096) ? 16 : kFftE<M>;
 // At M = 1024 in single precision both 8 and 16 pay, by pass and batch (the
 // autotuner's radix plan): with 16 a transform is one wave (radices 16, 8, 8),
@@ -126,32 +128,29 @@ k_pass2(cplx<T>* __restrict__ Tm, const G* __restrict__ gq, int N, int cols_per_
   constexpr int ML = LdsLen<M>::value;
   const int grp = xcd_tile(blockIdx.x, gridDim.x);
   const int c0 = grp * cols_per_wg;
-  const int nthr = blockDim.x;  // cols_per_wg * NT
   const int t = threadIdx.x % NT;
   const int cl = threadIdx.x / NT;
   FftTwiddles<T, M, E> tws;
   tws.load(tw, t);
   // gather the column tile: consecutive threads read consecutive columns; N <=
-  // M/2, so each thread gathers at most EPT/2 values
+  // M/2, so each thread gathers at most EPT/2 values, of column c and rows r0 + k NT
+  // (the work-group is cols_per_wg * NT threads).  A division by cols_per_wg for
+  // each value was a third of the kernel's vector instructions (M = 1024, one wave
+  // per column: 2,007 of them, now 1,320).
   constexpr int GR = EPT / 2;
+  const int r0 = threadIdx.x / cols_per_wg, c = threadIdx.x - r0 * cols_per_wg;
   {
     cplx<T> gv[GR];
 #pragma unroll
     for (int k = 0; k < GR; ++k) {
-      const int idx = threadIdx.x + k * nthr;
-      if (idx < N * cols_per_wg) {
-        const int r = idx / cols_per_wg, c = idx - r * cols_per_wg;
-        gv[k] = Tm[tpos(r, c0 + c, N)];
-      }
+      const int r = r0 + k * NT;
+      if (r < N) gv[k] = Tm[tpos(r, c0 + c, N)];
     }
     if (dn) return;
 #pragma unroll
     for (int k = 0; k < GR; ++k) {
-      const int idx = threadIdx.x + k * nthr;
-      if (idx < N * cols_per_wg) {
-        const int r = idx / cols_per_wg, c = idx - r * cols_per_wg;
-        smem[c * ML + lpad(r)] = gv[k];
-      }
+      const int r = r0 + k * NT;
+      if (r < N) smem[c * ML + lpad(r)] = gv[k];
     }
   }
   // the column's multipliers, loaded ahead of the transform
@@ -192,11 +191,8 @@ k_pass2(cplx<T>* __restrict__ Tm, const G* __restrict__ gq, int N, int cols_per_
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < GR; ++k) {
-    const int idx = threadIdx.x + k * nthr;
-    if (idx < N * cols_per_wg) {
-      const int r = idx / cols_per_wg, c = idx - r * cols_per_wg;
-      Tm[tpos(r, c0 + c, N)] = smem[c * ML + lpad(r)];
-    }
+    const int r = r0 + k * NT;
+    if (r < N) Tm[tpos(r, c0 + c, N)] = smem[c * ML + lpad(r)];
   }
 }
 
@@ -261,10 +257,11 @@ k_pass3(const cplx<T>* __restrict__ Tm, const cplx<T>* __restrict__ x, const T* 
 // passes.  The transforms are those of k_pass1..3: results are equal bit for bit.
 //
 // Such a product is a chain of latencies: three launches that each wait for the
-// one before, with a few work-groups each.  N = 24, one vector: 6.5 us instead of
-// 12.1 (FP64: 7.0 instead of 13.6); N = 48, four vectors: 12.4 instead of 13.3.
+// one before, with a few work-groups each.  N = 24, one vector: 6.6 us instead of
+// 10.9 (FP64: 7.4 instead of 13.2).  At N = 48 the two are level: 12.3 us against
+// 11.6 in replays of a graph, 12.4 against 13.3 where the host issues the launches.
 // At M = 128 one CU's LDS traffic costs more than the launches (N = 64, one
-// vector: 14.5 against 10.6 us).
+// vector: 15.6 against 9.7 us).
 // ---------------------------------------------------------------------------
 template <int M> struct SmallShape {
   static constexpr int E = kFftE<M>;
