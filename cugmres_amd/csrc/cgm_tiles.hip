@@ -825,8 +825,9 @@ __device__ inline int xrow(int q) { return (q & ~31) | (q & 15) << 1 | (q >> 4 &
 // by 1 / *(io.nrm + s sNrm bytes) when io.nrm is given), as the right-hand
 // operand of k_tile_ws: every value is scaled by the power of two that brings
 // the tile's largest component to [2^14, 2^15) and cut into kSplits FP16
-// parts, x = hi + mid + lo, which hold all 24 bits of the FP32 value (down to
-// 2^-39 of the tile's largest).  Group v = s / VP of the systems, column
+// parts, x = hi + mid + lo, which hold all 24 bits of the FP32 values down to 2^-15
+// of the tile's largest and resolve smaller ones to 2^-39 of it (W is stored to
+// 2^-11).  Group v = s / VP of the systems, column
 // n(s) = s % VP: with VP = 16 one dword (re, im) per value and column n; with
 // VP = 8 the two columns 2n and 2n + 1 hold (re, -im) and (im, re).  Layout
 // [group][block row][part][16 columns][kBlkW], rows at xpos().  xinv[s][tile] is the inverse
@@ -923,7 +924,7 @@ k_tile_xs(const int* __restrict__ ncol, const unsigned short* __restrict__ cols,
 // What bounds it is the stream of W (64 KB a block), which is read once.  The
 // contraction runs on the matrix cores (FP16 inputs, FP32 sums): W is FP16 as
 // stored, and the FP32 inputs enter as three FP16 parts (k_tile_xs), so the
-// products are those of the FP32 values.  Complex arithmetic is real arithmetic
+// products are those of the FP32 values down to 2^-15 of a tile's largest.  Complex arithmetic is real arithmetic
 // on interleaved parts: a dword (re, im) of W meets the dword (re, -im) of x
 // for the real part and (im, re) for the imaginary part, 16 complex values of
 // K per MFMA.

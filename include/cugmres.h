@@ -366,7 +366,9 @@ int cgm_tiles_factor(cgm_tiles_t tiles, const cgm_complex128* dev_block, const f
 /* y[b] = P x[b] for b < batch ([batch][N*N]; map b, or the one map).
  * Asynchronous on the context stream.  With one map and several systems the
  * reduced form (T >= 64) applies W to up to 16 systems per pass over it on the
- * matrix cores (FP32 inputs as three FP16 parts each, FP32 sums); the dense
+ * matrix cores (FP32 sums; FP32 inputs as three FP16 parts each under one scale
+ * per tile, which keeps the 24 bits of components down to 2^-15 of the tile's
+ * largest and 2^-39 of it in smaller ones; W itself is stored in FP16); the dense
  * form (T <= 32) applies each inverse to eight systems per pass (T = 8: four).  A system's
  * result does not depend on the others. */
 int cgm_tiles_apply(cgm_tiles_t tiles, const cgm_complex64* dev_x, cgm_complex64* dev_y, int batch);
