@@ -12,7 +12,7 @@ uses seed --seed-offset + k (warm-up steps first).
 Methods (each system is solved from scratch; the time of a solve includes
 everything that depends on its map):
   - learned: flexible GMRES with the two-level preconditioner - the exact
-    inverses of the operator on 32 x 32 tiles (--tile; factored per map on the
+    inverses of the operator on 128 x 128 tiles (--tile; factored per map on the
     device), then the FNO network as a correction on the residual they leave
     (cugmres_amd.tiles.TwoLevel) - with the long-recurrence path (the whole
     Krylov basis in HBM, up to --lr-restart steps).  The network is trained
@@ -476,13 +476,12 @@ def c3_run(a, rhs=16, mem_budget=150e9):
     """Batched workload: per instance one map and `rhs` plane waves at angles
     2 pi k / rhs.  --c3-method block (default): block GMRES over the map's
     right-hand sides with its tile inverses (cugmres_amd.block.solve_map: one
-    shared block Krylov space, the projection V^H W as batched complex GEMMs,
+    shared block Krylov space, the projection V^H W on the matrix cores,
     cycles of --block-restart block steps that restart from the FP64 true
     residual with the solution kept in complex128).  --c3-method lockstep: the
     right-hand sides are solved in lockstep by flexible GMRES with the tile inverses
     of that map (factored once; the dense form streams each inverse once per
-    four right-hand sides, the reduced form runs the systems of one W block
-    back to back on one XCD) on the long-recurrence path with cycles of --lr-restart
+    eight right-hand sides, the reduced form once per sixteen) on the long-recurrence path with cycles of --lr-restart
     steps (two at most).  The right-hand sides run in lockstep groups as large
     as mem_budget bytes of Krylov bases allow (all 16 up to N = 256, fewer
     above).  A right-hand side left above the tolerance (on the hardest maps
@@ -593,7 +592,7 @@ def c3_run(a, rhs=16, mem_budget=150e9):
     return {"workload": f"{a.instances} instances x {rhs} plane waves, N in {list(C3_SIZES)}, blocks 4-8, "
                         f"eps in {{1,12.1}}, tol {a.tol:g}",
             "method": ("block GMRES over each map's 16 right-hand sides with its tile inverses (one "
-                       "factorisation per map), projection V^H W as batched complex GEMMs, cycles restarting from "
+                       "factorisation per map), projection V^H W on FP32 MFMA, cycles restarting from "
                        "the FP64 true residual" if a.c3_method == "block" else
                        "FGMRES with tile inverses, lockstep, one factorisation per map; FP64 refinement from "
                        "where it stopped for a system left at the complex64 floor"),
@@ -844,10 +843,10 @@ def profile_fno(ctx, net, dchi, db, batch=1):
     names = ["fno_lift", "fno_rowproj", "fno_spectral", None, "fno_invx", "fno_cell_gemm", "fno_proj",
              "fno_forward_total", "fno_cell_gemm_lift"]
     # launches per forward pass: fno_lift = k_lift_row / k_lift_rows (lift +
-    # layer-0 row projection; h0 stays in LDS); fno_cell_gemm = k_cell_row /
-    # k_cell_rows (B_x of the row, cell GEMM + GELU + next row projection,
-    # layers 1-2); fno_cell_gemm_lift = the same for layer 0 (k_cell_row /
-    # k_cell_rows_lift), lifting its row from chi and v; fno_proj =
+    # layer-0 row projection; h0 stays in LDS); fno_cell_gemm = k_cell_row,
+    # k_cell_pair (one vector, 256 < N <= 512) or k_cell_rows (B_x of the row, cell GEMM + GELU + next row projection,
+    # layers 1-2); fno_cell_gemm_lift = the same for layer 0 (k_cell_row,
+    # k_cell_pair or k_cell_rows_lift), lifting its row from chi and v; fno_proj =
     # k_cell_proj (layer-3 cell GEMM + the 32 -> 2 projection).  Batches of
     # at least 1024 grid rows take the *_rows kernels, several grid rows per
     # work-group; the algorithmic bytes are the same.

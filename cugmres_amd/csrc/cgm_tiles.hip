@@ -953,7 +953,7 @@ k_tile_xs(const int* __restrict__ ncol, const unsigned short* __restrict__ cols,
 // single blocks).
 //
 // At N = 512, T = 128 on a map of the benchmark (1.33 GB of W; a plain
-// non-temporal read of as much takes 190 us): one system 229-236 us (5.7 TB/s),
+// non-temporal read of as much takes 190 us): one system 225-236 us (5.8 TB/s),
 // 16 systems 337 us.  The vector-ALU kernel before it, which took one block
 // and one system at a time, took 272 and 3,000 us (202 us of arithmetic per
 // system).  One FP16 part instead of three would save 19 us at one system.
